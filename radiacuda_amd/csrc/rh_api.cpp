@@ -443,8 +443,15 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
         if (e == hipSuccess) e = up(&md.in_geo, F.in_geo);
         if (e == hipSuccess) e = up(&md.in_F, F.in_F);
         if (e == hipSuccess) e = up(&md.tile_box, F.tile_box);
-        if (e == hipSuccess) e = up(&md.edge_cont, F.edge_cont);
-        if (e == hipSuccess) e = up(&md.face_cont, F.face_cont);
+        std::vector<int32_t> eflag(F.edge_cont.size()), fflag(F.face_cont.size());
+        for (size_t i = 0; i < eflag.size(); i++) eflag[i] = (F.edge_cont[i] == 1.0) ? rh::kMeshCont : 0;
+        for (size_t i = 0; i < fflag.size(); i++) {
+            fflag[i] = (F.face_cont[i] == 1.0 || F.face_cont[i] == 3.0) ? rh::kMeshCont : 0;
+            for (size_t k = 0; k < 3; k++)
+                if (F.face_edge[3 * i + k] >= 0) fflag[i] |= 1 << k;
+        }
+        if (e == hipSuccess) e = up(&md.edge_flag, eflag);
+        if (e == hipSuccess) e = up(&md.face_flag, fflag);
         if (e == hipSuccess) e = up(&md.face_edge, F.face_edge);
         md.ne_free = F.ne_free;
         md.nf_tri = F.nf_tri;

@@ -116,7 +116,7 @@ RH_HD void eval_mixed(int kind, const double* __restrict__ rec, const double xl[
 {
     bool near = near_element<KIND>(kind, rec, xl);
 #ifdef __HIP_DEVICE_COMPILE__
-    near = __any(near);
+    near = rh_any(near);
 #endif
     if (near)
         eval_k<double, KIND>(kind, rec, xl, q6);
@@ -186,7 +186,7 @@ RH_HD bool near32(int kind, const double* __restrict__ rec, const double* __rest
     if (crec) return tet_near32(crec, x);
     bool near = near_field<KIND>(kind, rec, x);
 #ifdef __HIP_DEVICE_COMPILE__
-    near = __any(near);
+    near = rh_any(near);
 #endif
     return near;
 }

@@ -325,23 +325,23 @@ constexpr int kTetTile = 32;
 #ifndef RH_TET_WAVES
 #define RH_TET_WAVES 3
 #endif
-// mesh sweep: occupancy floor (waves per SIMD) and edge and face records
-// staged per LDS tile.  FP64: 6 waves (80 VGPRs, 8 bytes of spill outside
-// the record loops) measured 50.9 / 566 ms on the C-yoke / Halbach ring
-// against 51.3 / 569 ms at 5 waves (85 VGPRs); FP32: 7 waves (72 VGPRs),
-// the records near a wave evaluated in FP64 after each tile's loop.
+// mesh sweep with N points per lane: occupancy floor (waves per SIMD).  Two
+// points share a record's LDS reads, branches and votes and give each other
+// independent instructions; on the C-yoke (FP64, 1M points) two points at 3
+// waves (149 VGPRs, no spill) take 36.9 ms and at 4 waves 37.1 ms, one point
+// at 4 to 6 waves 40-47 ms; FP32 on the Halbach ring (250,007 points) two
+// points 37.5 ms at 4 waves and 39.7 at 3, one point 39.4 ms at 5.
 #ifndef RH_MESH_WAVES32
-#define RH_MESH_WAVES32 7
+#define RH_MESH_WAVES32 4
 #endif
 #ifndef RH_MESH_WAVES
-#define RH_MESH_WAVES 6
+#define RH_MESH_WAVES 3
 #endif
-#ifndef RH_MESH_STAGE32
-#define RH_MESH_STAGE32 64
-#endif
-#ifndef RH_MESH_STAGE
-#define RH_MESH_STAGE 64
-#endif
+template <class R, int N>
+constexpr int mesh_waves() { return N == 1 ? 4 : (sizeof(R) == 4 ? RH_MESH_WAVES32 : RH_MESH_WAVES); }
+// records per LDS tile (at most 64: one bit of a mask each; even, for the
+// pairwise unrolled loops)
+constexpr int kMeshStage = 64;
 
 template <class R, bool SYM, int PASS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RH_TET_WAVES))) void k_field_tet(DevModel m, const double* __restrict__ pts,
@@ -426,21 +426,18 @@ __global__ __launch_bounds__(256) void k_mesh_charge_edges(MeshDev md, const dou
     }
     const double* g = md.edge_geo + kMeshEdgeGeo * i;
     double* o = md.ch_edge + kMeshEdge * i;
-    for (int k = 0; k < kMeshEdgeGeo; k++) o[k] = g[k];
+    for (int k = 0; k < kMeshEdgeGeo - 1; k++) o[k] = g[k];
+    o[9] = 2.0 * g[9];
     o[10] = w[0];
     o[11] = w[1];
     o[12] = w[2];
-    o[13] = md.edge_cont[i];
+    o[13] = 0.0;
     if (pack32) {
+        // slot 6: 2 len and the near distance of the FP32 sweep (kNear32 lengths)
         float* f = reinterpret_cast<float*>(o + 6);
-        const float t0 = float(g[6]), t1 = float(g[7]), t2 = float(g[8]), len = float(g[9]);
-        f[0] = t0;
-        f[1] = t1;
-        f[2] = t2;
-        f[3] = len;
-        // slot 8: the near distance of the FP32 sweep (kNear32 lengths)
-        f[4] = kNear32 * len;
-        f[5] = 0.0f;
+        const float len = float(g[9]);
+        f[0] = 2.0f * len;
+        f[1] = kNear32 * len;
     }
 }
 
@@ -457,35 +454,50 @@ __global__ __launch_bounds__(256) void k_mesh_charge_faces(MeshDev md, const dou
         s += v[0] * M[3 * j] + v[1] * M[3 * j + 1] + v[2] * M[3 * j + 2];
     }
     double* o = md.ch_face + kMeshFace * i;
-    for (int k = 0; k < kMeshFaceGeo; k++) o[k] = g[k];
-    o[18] = s * n0;
-    o[19] = s * n1;
-    o[20] = s * n2;
-    o[21] = md.face_cont[i];
-    // owned edges: length and the net weight of the charged edge record
+    const bool tri = !(g[17] > 3.5);
+    const double a1 = g[15], a2 = g[16];
+    const double nk = tri ? 2.0 * a1 : 1.0;  // triangles: n scaled by four times the area
+    for (int k = 0; k < 12; k++) o[k] = g[k];
+    o[12] = nk * n0;
+    o[13] = nk * n1;
+    o[14] = nk * n2;
+    o[15] = 2.0 * a1;
+    o[16] = 2.0 * a2;
+    o[17] = g[17];
+    // squared distances of (v0,v1), (v1,v2), (v0,v2), (v2,v3), (v0,v3)
+    const int pa[5] = {0, 1, 0, 2, 0}, pb[5] = {1, 2, 2, 3, 3};
+    double l2[5];
+    for (int k = 0; k < 5; k++) {
+        const double* u = g + 3 * pa[k];
+        const double* v = g + 3 * pb[k];
+        l2[k] = (tri && k > 2) ? 0.0 : sq3(v[0] - u[0], v[1] - u[1], v[2] - u[2]);
+        o[kMeshFaceLen2 + k] = l2[k];
+    }
+    o[kMeshFaceLen2 + 5] = 0.0;
+    o[18] = -2.0 * (s * n0);
+    o[19] = -2.0 * (s * n1);
+    o[20] = -2.0 * (s * n2);
+    o[21] = 0.0;
+    // owned edges: twice the length and the net weight of the charged edge record
     // (charged before the faces, on the same stream)
-    int32_t mask = 0;
     for (int k = 0; k < 3; k++) {
         const int64_t e = md.face_edge[3 * i + k];
         double* d = o + kMeshFaceEdges + 4 * k;
         if (e >= 0) {
             const double* ce = md.ch_edge + kMeshEdge * e;
-            d[0] = md.edge_geo[kMeshEdgeGeo * e + 9];
+            d[0] = 2.0 * md.edge_geo[kMeshEdgeGeo * e + 9];
             d[1] = ce[10];
             d[2] = ce[11];
             d[3] = ce[12];
-            mask |= 1 << k;
         } else {
             d[0] = d[1] = d[2] = d[3] = 0.0;
         }
     }
-    int32_t* mk = reinterpret_cast<int32_t*>(o + kMeshFaceEdges + 12);
-    mk[0] = mask;
-    mk[1] = 0;
+    o[kMeshFaceEdges + 12] = 0.0;
     o[kMeshFaceEdges + 13] = 0.0;
     if (pack32) {
         // slot 35: the near distance of the FP32 sweep (kNear32 longest sides)
-        const int nv = g[17] > 3.5 ? 4 : 3;
+        const int nv = tri ? 3 : 4;
         double lmax = 0.0;
         for (int k = 0; k < nv; k++) {
             const double* a = g + 3 * k;
@@ -497,13 +509,14 @@ __global__ __launch_bounds__(256) void k_mesh_charge_faces(MeshDev md, const dou
     }
     if (pack32) {
         float* f = reinterpret_cast<float*>(o + 12);
-        const float a1 = float(g[15]), a2 = float(g[16]);
-        f[0] = float(n0);
-        f[1] = float(n1);
-        f[2] = float(n2);
-        f[3] = a1;
-        f[4] = a2;
+        f[0] = float(nk * n0);
+        f[1] = float(nk * n1);
+        f[2] = float(nk * n2);
+        f[3] = float(2.0 * a1);
+        f[4] = float(2.0 * a2);
         f[5] = 0.0f;
+        float* l = reinterpret_cast<float*>(o + kMeshFaceLen2);
+        for (int k = 0; k < 5; k++) l[k] = float(l2[k]);
     }
 }
 
@@ -523,73 +536,114 @@ __global__ __launch_bounds__(256) void k_mesh_charge_in(MeshDev md, const double
     for (int k = 0; k < 4 * kMeshPlanes; k++) o[4 + k] = g[1 + k];
 }
 
-// Field sweep of the mesh form: slice blockIdx.y of the unique edges, unique
-// faces and inside tiles, each staged through LDS in tiles of kMeshTile
-// records read at wave-uniform addresses.  Inside tiles whose bounding box
-// holds no point of the wave are skipped (wave-uniform vote).
-template <class R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? RH_MESH_WAVES32 : RH_MESH_WAVES))) void
+// Field sweep of the mesh form: slice blockIdx.y of the unique edges no face
+// owns, the unique faces and the inside tiles.  Every lane evaluates the same
+// record for its own N points; records are staged through LDS in tiles of
+// kMeshStage and read there at wave-uniform addresses (broadcast), their
+// branch flags through the scalar cache.
+//
+// Bound by FP64 vector issue: 119 instructions per wave of points and
+// tetrahedron on the C-yoke (185 with logarithm-ratio edges, dot products and
+// one point per lane), 80 % of the issue slots.  1M points: 35.0 ms against
+// 49.3; FP32 on the 20,000-element ring, 250,007 points: 35.4 ms against 45.8.
+// Reading the records through the scalar cache instead of LDS freed the vector
+// registers but left each wave waiting on scalar loads: 52 ms.
+//
+// FP32: the records of a chunk that the wave is near (mesh32_near) are marked
+// in `defer` and evaluated in FP64 after the chunk's loop, where the loop's
+// carried values are dead, so the FP64 code does not add to the loop's
+// registers.
+template <class R, int N>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(mesh_waves<R, N>()))) void
 k_field_mesh(DevModel m, const double* __restrict__ pts, int64_t np, int64_t S, int64_t slice0,
              double* __restrict__ B, double* __restrict__ H, double* __restrict__ part)
 {
-    constexpr int kStage = (sizeof(R) == 4) ? RH_MESH_STAGE32 : RH_MESH_STAGE;
-    __shared__ __align__(16) double tile[kStage * kMeshFace > kMeshTile * kMeshIn ? kStage * kMeshFace
-                                                                                     : kMeshTile * kMeshIn];
+    constexpr bool f32 = sizeof(R) == 4;
+    using Vtx = MeshVtxN<R, N>;
+    __shared__ __align__(16) double tile[kMeshStage * kMeshFace];
     const MeshDev& md = m.mesh;
-    const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    // a wave's 64 N points are consecutive
+    const int64_t p = int64_t(blockIdx.x) * (256 * N) + (threadIdx.x >> 6) * (64 * N) + (threadIdx.x & 63);
     const bool live = p < np;
     const int64_t y = blockIdx.y;
-    double x[3] = {0.0, 0.0, 0.0};
-    if (live) {
-        x[0] = pts[3 * p];
-        x[1] = pts[3 * p + 1];
-        x[2] = pts[3 * p + 2];
+    double x[N][3];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        // a point past the end repeats the lane's first one, unstored
+        const int64_t q = (p + 64 * i < np) ? p + 64 * i : p;
+        for (int k = 0; k < 3; k++) x[i][k] = live ? pts[3 * q + k] : 0.0;
     }
-    double h[3] = {0.0, 0.0, 0.0}, min[3] = {0.0, 0.0, 0.0};
-    double2* dst = reinterpret_cast<double2*>(tile);
-    // unique edges that no triangle owns (edges of quadrilaterals only):
-    // + L_e w_e, along paths: a continued edge takes its first vertex's
-    // offset and distance from the previous edge.  The loop is unrolled by
-    // two with the vertex slots P, Q swapping roles, so the carried values
-    // stay in place (no register copies per edge).
-    // FP32: the records of a tile that the wave is near (mesh32_near) are
-    // marked in `defer` and evaluated in FP64 after the tile's loop, where
-    // the loop's carried values are dead, so the FP64 code does not add to
-    // the loop's registers
-    static_assert(kStage <= 64, "one bit per staged record");
-    uint64_t defer = 0;
+    // records [base, base + cnt) of `size` doubles each into the tile
+    auto stage = [&](const double* __restrict__ rec, int cnt, int size) {
+        const double2* src = reinterpret_cast<const double2*>(rec);
+        double2* dst = reinterpret_cast<double2*>(tile);
+        __syncthreads();  // the previous tile has been consumed
+        for (int i = threadIdx.x; i < cnt * (size / 2); i += 256) dst[i] = src[i];
+        __syncthreads();
+    };
+    double h[N][3];
+#pragma unroll
+    for (int i = 0; i < N; i++) h[i][0] = h[i][1] = h[i][2] = 0.0;
+    auto add = [&](const R (&v)[N], const double* __restrict__ w) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            h[i][0] += double(v[i]) * w[0];
+            h[i][1] += double(v[i]) * w[1];
+            h[i][2] += double(v[i]) * w[2];
+        }
+    };
+    // FP32: whether a point of the wave is near the record with these vertices
+    auto near32 = [&](const Vtx* const (&v)[4], int nv, float thr) {
+        float d = float(v[0]->d[0]);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                if (k < nv) d = fminf(d, float(v[k]->d[i]));
+        return mesh32_near(d, thr);
+    };
+    // leading coefficients of the far tiers, kept in vector registers
+    double a_top = kAtan32Top, e_top = kEdge6Top;
+    if constexpr (!f32) asm("" : "+v"(a_top), "+v"(e_top));
+    // an edge from its ends and the sum of their distances: + L_e w_e, e its
+    // 2 len and w
+    auto edge_term = [&](const Vtx& u, const Vtx& v, const R (&suv)[N], const double* __restrict__ e, R len2) {
+        R L[N];
+        edge_L2(u.r, u.d, v.r, v.d, suv, len2, e_top, L);
+        add(L, e + 1);
+    };
+    // unique edges that no face owns, along paths: a continued edge takes its
+    // first vertex's offset and distance from the previous edge.  The loop is
+    // unrolled by two with the vertex slots P, Q swapping roles, so the
+    // carried values stay in place (no register copies per edge).
     {
-        MeshVtx<R> P{}, Q{};
+        Vtx P{}, Q{};
         const int64_t e0 = md.ne_free * y / S, e1 = md.ne_free * (y + 1) / S;
-        auto edge = [&](int64_t g, int q, MeshVtx<R>& a, MeshVtx<R>& b) {
+        const MeshFlags flags = mesh_flags(md.edge_flag);
+        uint64_t defer = 0;
+        auto edge = [&](int64_t g, int q, Vtx& a, Vtx& b) {
             const double* rec = tile + kMeshEdge * q;
-            if (!(mesh_code(rec + 13) == 1 && g != e0)) a = mesh_vtx<R>(rec, x);
-            b = mesh_vtx<R>(rec + 3, x);
-            // L_e from the end offsets, distances and the length (the
-            // FP32 records carry the length as a float in slot 7, and keep
-            // it in FP64 in slot 9 for the waves near the edge)
-            if constexpr (sizeof(R) == 4) {
-                if (mesh32_near(fminf(a.d, b.d), mesh32(rec, 8)[0])) {
+            if (!(flags[g] & kMeshCont) || g == e0) mesh_vtx<R, N>(rec, x, a);
+            mesh_vtx<R, N>(rec + 3, x, b);
+            if constexpr (f32) {
+                const float* f = reinterpret_cast<const float*>(rec + 6);
+                const Vtx* const v[4] = {&a, &b, &b, &b};
+                if (near32(v, 2, f[1])) {
                     defer |= uint64_t(1) << q;
-                } else {
-                    const double L = double(edge_L(a.r, a.d, b.r, b.d, mesh32(rec, 6)[3]));
-                    h[0] += L * rec[10];
-                    h[1] += L * rec[11];
-                    h[2] += L * rec[12];
+                    return;
                 }
+                R s[N];
+                mesh_sum<R, N>(a, b, s);
+                edge_term(a, b, s, rec + 9, f[0]);
             } else {
-                const double L = double(edge_L(a.r, a.d, b.r, b.d, R(rec[9])));
-                h[0] += L * rec[10];
-                h[1] += L * rec[11];
-                h[2] += L * rec[12];
+                R s[N];
+                mesh_sum<R, N>(a, b, s);
+                edge_term(a, b, s, rec + 9, rec[9]);
             }
         };
-        for (int64_t base = e0; base < e1; base += kStage) {
-            const int cnt = int((e1 - base < kStage) ? (e1 - base) : kStage);
-            const double2* src = reinterpret_cast<const double2*>(md.ch_edge + kMeshEdge * base);
-            __syncthreads();
-            for (int i = threadIdx.x; i < cnt * (kMeshEdge / 2); i += 256) dst[i] = src[i];
-            __syncthreads();
+        for (int64_t base = e0; base < e1; base += kMeshStage) {
+            const int cnt = int((e1 - base < kMeshStage) ? (e1 - base) : kMeshStage);
+            stage(md.ch_edge + kMeshEdge * base, cnt, kMeshEdge);
             if (!live) continue;
             int q = 0;
 #pragma unroll 1
@@ -597,210 +651,179 @@ k_field_mesh(DevModel m, const double* __restrict__ pts, int64_t np, int64_t S, 
                 edge(base + q, q, P, Q);
                 edge(base + q + 1, q + 1, Q, P);
             }
-            if (q < cnt) {
-                edge(base + q, q, P, Q);
-                P = Q;
-            }
-            if constexpr (sizeof(R) == 4) {
+            if (q < cnt) edge(base + q, q, P, Q);  // the last edge of the slice
+            if constexpr (f32) {
                 for (; defer; defer &= defer - 1) {
                     const double* rec = tile + kMeshEdge * __builtin_ctzll(defer);
-                    const double L = mesh_edge_L_near(rec, x);
-                    h[0] += L * rec[10];
-                    h[1] += L * rec[11];
-                    h[2] += L * rec[12];
+#pragma unroll
+                    for (int i = 0; i < N; i++) {
+                        const double L = mesh_edge_L_near(rec, x[i]);
+                        for (int k = 0; k < 3; k++) h[i][k] += L * rec[10 + k];
+                    }
                 }
             }
         }
     }
     // unique faces: - Omega_f g_f, triangles along strips: a continued
-    // triangle takes its first two vertices (and their dot product) from the
-    // previous one.  Unrolled by three with the slots A, B, C rotating.  A
-    // triangle also evaluates the edges it owns (+ L_e w_e) from the
-    // offsets, distances and dot products of its vertices.
+    // triangle takes its first two vertices (and the sum of their distances)
+    // from the previous one.  Unrolled by three with the slots A, B, C
+    // rotating.  A triangle also evaluates the edges it owns from the offsets
+    // and distances of its vertices.
     {
-        MeshVtx<R> A{}, Bv{}, C{}, QA{}, QB{}, QC{}, QD{};
-        R dAB = R(0), dBC = R(0), dCA = R(0), dQAB = R(0), dQCD = R(0);
         // this slice's faces: triangles [f0, ft), then quadrilaterals [fq, f1)
         const int64_t f0 = md.nf * y / S, f1 = md.nf * (y + 1) / S;
         const int64_t ft = f1 < md.nf_tri ? f1 : md.nf_tri, fq = f0 > md.nf_tri ? f0 : md.nf_tri;
-        // an edge owned by the current face: the offsets and distances of its
-        // ends and their dot product are already at hand
-        auto owned = [&](const MeshVtx<R>& u, const MeshVtx<R>& v, R duv, const double* e) {
-            const double L = double(edge_L(u.r, u.d, v.r, v.d, duv, R(e[0])));
-            h[0] += L * e[1];
-            h[1] += L * e[2];
-            h[2] += L * e[3];
-        };
-        // FP64 for the records of the tile the wave is near
-        auto deferred = [&]() {
-            if constexpr (sizeof(R) == 4) {
+        const MeshFlags flags = mesh_flags(md.face_flag);
+        uint64_t defer = 0;
+        // FP64 for the records of the tile from `base` that the wave is near
+        auto deferred = [&](int64_t base) {
+            if constexpr (f32) {
                 for (; defer; defer &= defer - 1) {
-                    const double* rec = tile + kMeshFace * __builtin_ctzll(defer);
-                    const MeshFace64 t = mesh_face_near(rec, mesh_mask(rec + kMeshFaceEdges + 12), x);
-                    h[0] += t.h0 - t.om * rec[18];
-                    h[1] += t.h1 - t.om * rec[19];
-                    h[2] += t.h2 - t.om * rec[20];
-                }
-            }
-        };
-        auto tri = [&](int64_t g, int q, MeshVtx<R>& a, MeshVtx<R>& b, MeshVtx<R>& c, R& dab, R& dbc) {
-            const double* rec = tile + kMeshFace * q;
-            if (!(mesh_code(rec + 21) == 1 && g != f0)) {
-                a = mesh_vtx<R>(rec, x);
-                b = mesh_vtx<R>(rec + 3, x);
-                dab = dot(a.r, b.r);
-            }
-            c = mesh_vtx<R>(rec + 6, x);
-            dbc = dot(b.r, c.r);
-            double om;
-            if constexpr (sizeof(R) == 4) {
-                // a near record only sets its bit; the carried values
-                // (b, c, dbc) are in place either way
-                if (mesh32_near(fminf(fminf(a.d, b.d), c.d), mesh32(rec, kMeshFaceEdges + 13)[0])) {
-                    defer |= uint64_t(1) << q;
-                    return;
-                }
-                const R dca = dot(c.r, a.r);
-                const int mask = mesh_mask(rec + kMeshFaceEdges + 12);
-                om = double(mesh32_tri_omega(a.r, a.d, b.r, b.d, c.r, c.d, dab, dbc, dca, rec));
-                if (mask & 1) owned(a, b, dab, rec + kMeshFaceEdges);
-                if (mask & 2) owned(b, c, dbc, rec + kMeshFaceEdges + 4);
-                if (mask & 4) owned(c, a, dca, rec + kMeshFaceEdges + 8);
-            } else {
-                const R dca = dot(c.r, a.r);
-                const int mask = mesh_mask(rec + kMeshFaceEdges + 12);
-                om = mesh_tri_omega_from<R>(a.r, a.d, b.r, b.d, c.r, c.d, dab, dbc, dca, rec);
-                if (mask & 1) owned(a, b, dab, rec + kMeshFaceEdges);
-                if (mask & 2) owned(b, c, dbc, rec + kMeshFaceEdges + 4);
-                if (mask & 4) owned(c, a, dca, rec + kMeshFaceEdges + 8);
-            }
-            h[0] -= om * rec[18];
-            h[1] -= om * rec[19];
-            h[2] -= om * rec[20];
-        };
-        // a quadrilateral with the sides (v0,v1), (v1,v2), (v2,v3) it owns,
-        // along strips: a continued quadrilateral takes v0, v1 and their dot
-        // product from the previous one's v2, v3 (slots a, b, dab)
-        auto quad = [&](int64_t g, int q, MeshVtx<R>& a, MeshVtx<R>& b, MeshVtx<R>& c, MeshVtx<R>& d, R& dab,
-                        R& dcd) {
-            const double* rec = tile + kMeshFace * q;
-            if (!(mesh_code(rec + 21) == 3 && g != fq)) {
-                a = mesh_vtx<R>(rec, x);
-                b = mesh_vtx<R>(rec + 3, x);
-                dab = dot(a.r, b.r);
-            }
-            c = mesh_vtx<R>(rec + 6, x);
-            d = mesh_vtx<R>(rec + 9, x);
-            dcd = dot(c.r, d.r);
-            if constexpr (sizeof(R) == 4) {
-                if (mesh32_near(fminf(fminf(a.d, b.d), fminf(c.d, d.d)), mesh32(rec, kMeshFaceEdges + 13)[0])) {
-                    defer |= uint64_t(1) << q;
-                    return;
-                }
-            }
-            const MeshVtx<R> v[4] = {a, b, c, d};
-            const R dbc = dot(b.r, c.r);
-            const double om =
-                double(mesh_quad_omega_from<R>(v, dab, dot(a.r, c.r), dot(a.r, d.r), dbc, dcd, rec));
-            const int mask = mesh_mask(rec + kMeshFaceEdges + 12);
-            if (mask & 1) owned(a, b, dab, rec + kMeshFaceEdges);
-            if (mask & 2) owned(b, c, dbc, rec + kMeshFaceEdges + 4);
-            if (mask & 4) owned(c, d, dcd, rec + kMeshFaceEdges + 8);
-            h[0] -= om * rec[18];
-            h[1] -= om * rec[19];
-            h[2] -= om * rec[20];
-        };
-        for (int64_t base = f0; base < ft; base += kStage) {
-            const int cnt = int((ft - base < kStage) ? (ft - base) : kStage);
-            const double2* src = reinterpret_cast<const double2*>(md.ch_face + kMeshFace * base);
-            __syncthreads();
-            for (int i = threadIdx.x; i < cnt * (kMeshFace / 2); i += 256) dst[i] = src[i];
-            __syncthreads();
-            if (!live) continue;
-            int q = 0;
-#pragma unroll 1
-            for (; q + 3 <= cnt; q += 3) {
-                tri(base + q, q, A, Bv, C, dAB, dBC);
-                tri(base + q + 1, q + 1, Bv, C, A, dBC, dCA);
-                tri(base + q + 2, q + 2, C, A, Bv, dCA, dAB);
-            }
-            // remainder, then the carried pair back into (A, B)
-            if (q < cnt) {
-                tri(base + q, q, A, Bv, C, dAB, dBC);
-                if (q + 1 < cnt) {
-                    tri(base + q + 1, q + 1, Bv, C, A, dBC, dCA);
-                    Bv = A;
-                    A = C;
-                    dAB = dCA;
-                } else {
-                    A = Bv;
-                    Bv = C;
-                    dAB = dBC;
-                }
-            }
-            deferred();
-        }
-        for (int64_t base = fq; base < f1; base += kStage) {
-            const int cnt = int((f1 - base < kStage) ? (f1 - base) : kStage);
-            const double2* src = reinterpret_cast<const double2*>(md.ch_face + kMeshFace * base);
-            __syncthreads();
-            for (int i = threadIdx.x; i < cnt * (kMeshFace / 2); i += 256) dst[i] = src[i];
-            __syncthreads();
-            if (!live) continue;
-            int q = 0;
-#pragma unroll 1
-            for (; q + 2 <= cnt; q += 2) {
-                quad(base + q, q, QA, QB, QC, QD, dQAB, dQCD);
-                quad(base + q + 1, q + 1, QC, QD, QA, QB, dQCD, dQAB);
-            }
-            // remainder, then the carried pair back into (QA, QB)
-            if (q < cnt) {
-                quad(base + q, q, QA, QB, QC, QD, dQAB, dQCD);
-                QA = QC;
-                QB = QD;
-                dQAB = dQCD;
-            }
-            deferred();
-        }
-    }
-    // inside tests: B gets the magnetization of the element holding the point
-    {
-        const int64_t t0 = md.ntiles * y / S, t1 = md.ntiles * (y + 1) / S;
-        for (int64_t t = t0; t < t1; t++) {
-            const double* bx = md.tile_box + 6 * t;
-            const bool near = live && x[0] >= bx[0] && x[1] >= bx[1] && x[2] >= bx[2] &&
-                              x[0] <= bx[3] && x[1] <= bx[4] && x[2] <= bx[5];
-            if (!__syncthreads_or(near ? 1 : 0)) continue;
-            const int64_t base = t * kMeshTile;
-            const int cnt = int((md.ni - base < kMeshTile) ? (md.ni - base) : kMeshTile);
-            const double2* src = reinterpret_cast<const double2*>(md.ch_in + kMeshIn * base);
-            for (int i = threadIdx.x; i < cnt * (kMeshIn / 2); i += 256) dst[i] = src[i];
-            __syncthreads();
-            if (near) {
-                for (int q = 0; q < cnt; q++) {
-                    const double* rec = tile + kMeshIn * q;
-                    if (mesh_inside(rec, x)) {
-                        min[0] += rec[1];
-                        min[1] += rec[2];
-                        min[2] += rec[3];
+                    const int q = __builtin_ctzll(defer);
+                    const double* rec = tile + kMeshFace * q;
+                    const int flag = flags[base + q];
+#pragma unroll
+                    for (int i = 0; i < N; i++) {
+                        const MeshFace64 f = mesh_face_near(rec, flag, x[i]);
+                        h[i][0] += f.h0 + f.om * rec[18];
+                        h[i][1] += f.h1 + f.om * rec[19];
+                        h[i][2] += f.h2 + f.om * rec[20];
                     }
                 }
             }
-            __syncthreads();
+        };
+        auto owned = [&](const Vtx& u, const Vtx& v, const R (&suv)[N], const double* __restrict__ e) {
+            edge_term(u, v, suv, e, R(e[0]));
+        };
+        {
+            Vtx A{}, Bv{}, C{};
+            R sAB[N] = {}, sBC[N] = {}, sCA[N] = {};
+            auto tri = [&](int64_t g, int q, Vtx& a, Vtx& b, Vtx& c, R (&sab)[N], R (&sbc)[N]) {
+                const double* rec = tile + kMeshFace * q;
+                const int flag = flags[g];
+                if (!(flag & kMeshCont) || g == f0) {
+                    mesh_vtx<R, N>(rec, x, a);
+                    mesh_vtx<R, N>(rec + 3, x, b);
+                    mesh_sum<R, N>(a, b, sab);
+                }
+                mesh_vtx<R, N>(rec + 6, x, c);
+                mesh_sum<R, N>(b, c, sbc);
+                if constexpr (f32) {
+                    // a near record only sets its bit; the carried values
+                    // (b, c, sbc) are in place either way
+                    const Vtx* const v[4] = {&a, &b, &c, &c};
+                    if (near32(v, 3, reinterpret_cast<const float*>(rec + kMeshFaceEdges + 13)[0])) {
+                        defer |= uint64_t(1) << q;
+                        return;
+                    }
+                }
+                R sca[N], om[N];
+                mesh_sum<R, N>(c, a, sca);
+                mesh_tri_half_omega<R, N>(a, b, c, sab, sbc, sca, rec, a_top, om);
+                add(om, rec + 18);
+                if (flag & 1) owned(a, b, sab, rec + kMeshFaceEdges);
+                if (flag & 2) owned(b, c, sbc, rec + kMeshFaceEdges + 4);
+                if (flag & 4) owned(c, a, sca, rec + kMeshFaceEdges + 8);
+            };
+            // tiles hold whole turns of the slots
+            constexpr int kTri = kMeshStage / 3 * 3;
+            for (int64_t base = f0; base < ft; base += kTri) {
+                const int cnt = int((ft - base < kTri) ? (ft - base) : kTri);
+                stage(md.ch_face + kMeshFace * base, cnt, kMeshFace);
+                if (!live) continue;
+                int q = 0;
+#pragma unroll 1
+                for (; q + 3 <= cnt; q += 3) {
+                    tri(base + q, q, A, Bv, C, sAB, sBC);
+                    tri(base + q + 1, q + 1, Bv, C, A, sBC, sCA);
+                    tri(base + q + 2, q + 2, C, A, Bv, sCA, sAB);
+                }
+                // the last triangles of the slice
+                if (q < cnt) tri(base + q, q, A, Bv, C, sAB, sBC);
+                if (q + 1 < cnt) tri(base + q + 1, q + 1, Bv, C, A, sBC, sCA);
+                deferred(base);
+            }
+        }
+        {
+            Vtx QA{}, QB{}, QC{}, QD{};
+            R sQAB[N] = {}, sQCD[N] = {};
+            // a quadrilateral with the sides (v0,v1), (v1,v2), (v2,v3) it
+            // owns, along strips: a continued quadrilateral takes v0, v1 and
+            // their sum from the previous one's v2, v3 (slots a, b, sab)
+            auto quad = [&](int64_t g, int q, Vtx& a, Vtx& b, Vtx& c, Vtx& d, R (&sab)[N], R (&scd)[N]) {
+                const double* rec = tile + kMeshFace * q;
+                const int flag = flags[g];
+                if (!(flag & kMeshCont) || g == fq) {
+                    mesh_vtx<R, N>(rec, x, a);
+                    mesh_vtx<R, N>(rec + 3, x, b);
+                    mesh_sum<R, N>(a, b, sab);
+                }
+                mesh_vtx<R, N>(rec + 6, x, c);
+                mesh_vtx<R, N>(rec + 9, x, d);
+                mesh_sum<R, N>(c, d, scd);
+                if constexpr (f32) {
+                    const Vtx* const v[4] = {&a, &b, &c, &d};
+                    if (near32(v, 4, reinterpret_cast<const float*>(rec + kMeshFaceEdges + 13)[0])) {
+                        defer |= uint64_t(1) << q;
+                        return;
+                    }
+                }
+                R sbc[N], om[N];
+                mesh_sum<R, N>(b, c, sbc);
+                mesh_quad_half_omega<R, N>(a, b, c, d, sab, sbc, scd, rec, a_top, om);
+                add(om, rec + 18);
+                if (flag & 1) owned(a, b, sab, rec + kMeshFaceEdges);
+                if (flag & 2) owned(b, c, sbc, rec + kMeshFaceEdges + 4);
+                if (flag & 4) owned(c, d, scd, rec + kMeshFaceEdges + 8);
+            };
+            for (int64_t base = fq; base < f1; base += kMeshStage) {
+                const int cnt = int((f1 - base < kMeshStage) ? (f1 - base) : kMeshStage);
+                stage(md.ch_face + kMeshFace * base, cnt, kMeshFace);
+                if (!live) continue;
+                int q = 0;
+#pragma unroll 1
+                for (; q + 2 <= cnt; q += 2) {
+                    quad(base + q, q, QA, QB, QC, QD, sQAB, sQCD);
+                    quad(base + q + 1, q + 1, QC, QD, QA, QB, sQCD, sQAB);
+                }
+                if (q < cnt) quad(base + q, q, QA, QB, QC, QD, sQAB, sQCD);
+                deferred(base);
+            }
         }
     }
     if (!live) return;
-    for (int k = 0; k < 3; k++) h[k] *= kInv4Pi;
-    if (part) {
-        double* o = part + ((slice0 + y) * np + p) * 6;
-        for (int k = 0; k < 3; k++) {
-            o[k] = h[k] + min[k];
-            o[3 + k] = h[k];
+    // inside tests: B gets the magnetization of the element holding the
+    // point.  Tiles whose bounding box holds no point of the wave are skipped
+    // (wave-uniform vote).
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const int64_t pi = p + 64 * i;
+        if (pi >= np) break;
+        double min[3] = {0.0, 0.0, 0.0};
+        const int64_t t0 = md.ntiles * y / S, t1 = md.ntiles * (y + 1) / S;
+        for (int64_t t = t0; t < t1; t++) {
+            const double* bx = md.tile_box + 6 * t;
+            const bool near = x[i][0] >= bx[0] && x[i][1] >= bx[1] && x[i][2] >= bx[2] && x[i][0] <= bx[3] &&
+                              x[i][1] <= bx[4] && x[i][2] <= bx[5];
+            if (!rh_any(near)) continue;
+            const int64_t base = t * kMeshTile;
+            const int cnt = int((md.ni - base < kMeshTile) ? (md.ni - base) : kMeshTile);
+            for (int q = 0; q < cnt; q++) {
+                const double* rec = md.ch_in + kMeshIn * (base + q);
+                if (near && mesh_inside(rec, x[i]))
+                    for (int k = 0; k < 3; k++) min[k] += rec[1 + k];
+            }
         }
-    } else {
+        double* o = part ? part + ((slice0 + y) * np + pi) * 6 : nullptr;
         for (int k = 0; k < 3; k++) {
-            if (B) B[3 * p + k] = h[k] + min[k];
-            if (H) H[3 * p + k] = h[k];
+            const double hk = h[i][k] * kInv4Pi;
+            if (o) {
+                o[k] = hk + min[k];
+                o[3 + k] = hk;
+            } else {
+                if (B) B[3 * pi + k] = hk + min[k];
+                if (H) H[3 * pi + k] = hk;
+            }
         }
     }
 }
@@ -1911,10 +1934,10 @@ hipError_t launch_assemble(const DevModel& m, void* Q, int elem_bytes, int64_t l
 
 namespace {
 // element splits for one kind slot: enough workgroups to fill the chip
-int64_t slot_splits(int64_t np, int64_t cnt)
+int64_t slot_splits(int64_t np, int64_t cnt, int64_t per_block = 256)
 {
     if (cnt == 0) return 0;
-    const int64_t blocks = (np + 255) / 256;
+    const int64_t blocks = (np + per_block - 1) / per_block;
     if (blocks >= 2048 || cnt < 64) return 1;
     int64_t sp = (2048 + blocks - 1) / blocks;
     sp = std::min<int64_t>(sp, std::max<int64_t>(1, cnt / 16));
@@ -1955,13 +1978,25 @@ void field_slot(const DevModel& m, const double* M, const double* pts, int64_t n
 
 bool mesh_on(const DevModel& m) { return m.use_mesh && m.mesh.active; }
 
+// Points per lane of the mesh sweep.  Two from 1e8 (point, entity) pairs on:
+// below that a sweep is too short to fill the chip with half as many waves and
+// its latency decides.  Measured (FP64, us, one / two points per lane):
+// 1,000 points on the 8,000-tetrahedron yoke (2.9e7 pairs) 142 / 171, 8,000
+// points (2.3e8) 441 / 409, 32,000 points 1,513 / 1,317; 8,000 points on the
+// 1,000-tetrahedron yoke (2.9e7) 135 / 152; 1,000 points on the 20,000-element
+// ring (1.3e8) 344 / 327.
+int64_t mesh_points(const DevModel& m, int64_t np)
+{
+    return double(np) * double(m.mesh.ne + m.mesh.nf) >= 1e8 ? 2 : 1;
+}
+
 // slices per kind slot (0 blocks, 1 tetrahedra, 2 general polyhedra); in the
 // mesh form slot 1 carries the whole mesh and slot 2 is empty
 void slot_plan(const DevModel& m, int64_t np, int64_t sp[3], int64_t work_cap)
 {
     sp[0] = slot_splits(np, m.koff[1] - m.koff[0]);
     if (mesh_on(m)) {
-        sp[1] = slot_splits(np, m.mesh.ne + m.mesh.nf);
+        sp[1] = slot_splits(np, m.mesh.ne + m.mesh.nf, 256 * mesh_points(m, np));
         sp[2] = 0;
     } else {
         sp[1] = slot_splits(np, m.koff[2] - m.koff[1]);
@@ -1995,9 +2030,12 @@ hipError_t field_all(const DevModel& m, const double* M, const double* pts, int6
     if (sp[0]) field_slot<R, SYM, 0>(m, M, pts, np, sp[0], slice0, B, H, part, s);
     slice0 += sp[0];
     if (sp[1] && mesh_on(m)) {
-        const dim3 grid{unsigned((np + 255) / 256), unsigned(sp[1]), 1u};
-        hipLaunchKernelGGL((k_field_mesh<R>), grid, dim3(256), 0, s, m, pts, np, sp[1], slice0, B, H,
-                           part);
+        const int64_t per = 256 * mesh_points(m, np);
+        const dim3 grid{unsigned((np + per - 1) / per), unsigned(sp[1]), 1u};
+        if (mesh_points(m, np) == 2)
+            hipLaunchKernelGGL((k_field_mesh<R, 2>), grid, dim3(256), 0, s, m, pts, np, sp[1], slice0, B, H, part);
+        else
+            hipLaunchKernelGGL((k_field_mesh<R, 1>), grid, dim3(256), 0, s, m, pts, np, sp[1], slice0, B, H, part);
     } else if (sp[1]) {
         field_slot<R, SYM, 1>(m, M, pts, np, sp[1], slice0, B, H, part, s);
     }

@@ -26,8 +26,8 @@ struct MeshDev {
     const double* in_geo = nullptr;
     const double* in_F = nullptr;        // 9 per inside record
     const double* tile_box = nullptr;
-    const double* edge_cont = nullptr;
-    const double* face_cont = nullptr;
+    const int32_t* edge_flag = nullptr;  // kMeshCont
+    const int32_t* face_flag = nullptr;  // owned sides (bits 0-2), kMeshCont
     int64_t ne_free = 0;                // edges [0, ne_free) are swept on their own
     int64_t nf_tri = 0;                 // faces [0, nf_tri) are triangles, the rest quadrilaterals
     const int64_t* face_edge = nullptr;  // 3 per face: owned edge record or -1

@@ -42,6 +42,13 @@
 
 namespace rh {
 
+#ifdef __HIPCC__
+// Votes over the active lanes, straight from the comparison's mask (__all and
+// __any first turn the lane's answer into an integer and compare that again).
+__device__ __forceinline__ bool rh_all(bool c) { return __builtin_amdgcn_ballot_w64(!c) == 0; }
+__device__ __forceinline__ bool rh_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
+#endif
+
 constexpr double kInv4Pi = 0.079577471545947667884441881686257181;  // 1/(4 pi)
 
 // Element record kinds in the packed element data.
@@ -146,9 +153,9 @@ RH_HD float rh_log1p(float x)
 // normal arguments.  The library routines round correctly over the whole
 // domain and cost about 90 (log), 100 (atan2) and 15 (sqrt) vector
 // instructions each on gfx950; the forms below cost about a third:
-//  * reciprocal: the hardware seed refined by two Newton-Raphson steps;
-//  * square root: the hardware reciprocal-square-root seed, one Goldschmidt
-//    step and one Newton correction;
+//  * reciprocal and division: the hardware seed and the second-order series
+//    of its error;
+//  * square root: the hardware reciprocal-square-root seed, likewise;
 //  * ln(num/den): exponents split off, ln(a/b) = 2 atanh(s) for the
 //    mantissas a, b in [1/2, 1) with s = (a - b)/(a + b) exact in the
 //    numerator, |s| < 1/3, and a degree-9 polynomial in s^2;
@@ -184,24 +191,60 @@ static __constant__ double d_atan_p[11] = {
 static __constant__ double d_atan16_p[7] = {-0.33333333333333237, 0.19999999999760989, -0.14285714188882722,
                                             0.11111096372965646,  -0.090898379007095286, 0.076521309422432607,
                                             -0.059098572131161474};
+// the same on |t| <= 1/32, degree 3 (within 2e-20 of atan t)
+static __constant__ double d_atan32_p[4] = {-0.3333333333333327, 0.19999999997886797, -0.1428570346460735,
+                                            0.11093375583013043};
+// ln((1 + X/2)/(1 - X/2)) = X + X^3 P(X^2): P on X <= 1/6 (degree 4, within
+// 1.7e-17 of the result, relative) and on X <= 1/2 (degree 7, 3.1e-17),
+// Chebyshev interpolants fitted at 60 digits
+static __constant__ double d_edge6_p[5] = {0.08333333333333395, 0.01249999999889163, 0.0022321431761517696,
+                                           0.00043399566660258694, 9.009544000788967e-05};
+static __constant__ double d_edge2_p[8] = {0.08333333333333322,   0.012500000000060307,  0.002232142852088486,
+                                           0.0004340279388094421, 8.877589708906781e-05, 1.8801225959087634e-05,
+                                           3.971004714131101e-06, 1.128428632788004e-06};
 #endif
+// Coefficients of a branch that few waves take: read there (the address is
+// hidden from the compiler, which would otherwise load every branch's
+// coefficients ahead of the sweep's loop and spill scalar registers for them).
+#ifdef __HIP_DEVICE_COMPILE__
+typedef const __attribute__((address_space(4))) double* CoefPtr;
+__device__ __forceinline__ CoefPtr rh_coef_rare(const double* c)
+{
+    uint64_t a = reinterpret_cast<uint64_t>(c);
+    asm volatile("" : "+s"(a));
+    return (CoefPtr)a;
+}
+#endif
+constexpr double kAtan32Top = 0.11093375583013043, kEdge6Top = 9.009544000788967e-05;
 constexpr double kTanPi16 = 0.19891236737965800;
 constexpr double kLn2Hi = 0.6931471803691238;  // ln 2 to 32 bits: k * kLn2Hi is exact
 constexpr double kLn2Lo = 1.9082149292705877e-10;
 constexpr double kTanPi8 = 0.41421356237309503;
 constexpr double kPi4 = 0.7853981633974483, kPi2 = 1.5707963267948966, kPi = 3.141592653589793;
 
-RH_HD double rh_rcp(double d)
+RH_HD double rh_rcp_seed(double d)
 {
 #ifdef __HIP_DEVICE_COMPILE__
-    double r = __builtin_amdgcn_rcp(d);
+    return __builtin_amdgcn_rcp(d);
 #else
-    double r = 1.0 / d;
+    return 1.0 / d;
 #endif
-    double e = fma(-d, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-d, r, 1.0);
-    return fma(r, e, r);
+}
+// 1/d and y/d from the seed r = (1 - e)/d, |e| < 2^-24 (measured on gfx950):
+// 1/d = r (1 + e + e^2 + ...), cut after e^2 (2^-72), one operation fewer
+// than two Newton steps.
+RH_HD double rh_rcp(double d)
+{
+    const double r = rh_rcp_seed(d);
+    const double e = fma(-d, r, 1.0);
+    return fma(r, fma(e, e, e), r);
+}
+RH_HD double rh_div(double y, double d)
+{
+    const double r = rh_rcp_seed(d);
+    const double e = fma(-d, r, 1.0);
+    const double t = y * r;
+    return fma(t, fma(e, e, e), t);
 }
 
 RH_HD double rh_sqrt(double x)
@@ -211,14 +254,13 @@ RH_HD double rh_sqrt(double x)
 #else
     const double y = 1.0 / sqrt(x);
 #endif
-    // the seed is within 2^-24 (measured on gfx950): the Goldschmidt step
-    // leaves 2^-48, the Newton correction the rounding error
-    double g = x * y, h = 0.5 * y;
-    const double r = fma(-h, g, 0.5);
-    g = fma(g, r, g);
-    h = fma(h, r, h);
-    const double d = fma(-g, g, x);
-    return fma(d, h, g);
+    // the seed is within 2^-24 (measured on gfx950): with g = x y and
+    // e = 1 - g y (exact but for its last rounding), sqrt(x) = g / sqrt(1 - e)
+    // up to half of g's own rounding error; the series is cut after e^2
+    // (5/16 e^3 < 2^-70)
+    const double g = x * y;
+    const double e = fma(-g, y, 1.0);
+    return fma(g * e, fma(e, 0.375, 0.5), g);
 }
 
 RH_HD void rh_frexp(double x, double& m, int& e)
@@ -233,7 +275,8 @@ RH_HD void rh_frexp(double x, double& m, int& e)
 
 // ln(num/den), num and den positive, finite and normal: with the mantissas
 // a, b in [1/2, 1), s = (a - b)/(a + b) (numerator exact), |s| < 1/3.
-RH_HD double rh_log_ratio(double num, double den)
+template <class C>
+RH_HD double rh_log_ratio_c(double num, double den, C c)
 {
     double a, b;
     int ea, eb;
@@ -242,20 +285,24 @@ RH_HD double rh_log_ratio(double num, double den)
     const double k = double(ea - eb);
     const double s = (a - b) * rh_rcp(a + b);
     const double v = s * s;
-#ifdef __HIP_DEVICE_COMPILE__
-    const double* c = d_log_p;
-#else
-    const double* c = kLogP;
-#endif
     double p = c[9];
 #pragma unroll
     for (int i = 8; i >= 0; i--) p = fma(p, v, c[i]);
     const double r = fma(s * v, p, 2.0 * s);
     return fma(k, kLn2Hi, fma(k, kLn2Lo, r));
 }
+RH_HD double rh_log_ratio(double num, double den)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return rh_log_ratio_c(num, den, d_log_p);
+#else
+    return rh_log_ratio_c(num, den, kLogP);
+#endif
+}
 RH_HD float rh_log_ratio(float num, float den) { return logf(num / den); }
 
-RH_HD double rh_atan2(double y, double x)
+template <class C>
+RH_HD double rh_atan2_c(double y, double x, C c)
 {
     const double ax = fabs(x), ay = fabs(y);
     const double mx = fmax(ax, ay), mn = fmin(ax, ay);
@@ -263,11 +310,6 @@ RH_HD double rh_atan2(double y, double x)
     const double t0 = (big ? mn - mx : mn) * rh_rcp(big ? mn + mx : mx);
     const double t = (mx > 0.0) ? t0 : 0.0;
     const double u = t * t;
-#ifdef __HIP_DEVICE_COMPILE__
-    const double* c = d_atan_p;
-#else
-    const double* c = kAtanP;
-#endif
     double p = c[10];
 #pragma unroll
     for (int i = 9; i >= 0; i--) p = fma(p, u, c[i]);
@@ -277,9 +319,19 @@ RH_HD double rh_atan2(double y, double x)
     a = (x < 0.0) ? kPi - a : a;
     return copysign(a, y);
 }
+RH_HD double rh_atan2(double y, double x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return rh_atan2_c(y, x, d_atan_p);
+#else
+    return rh_atan2_c(y, x, kAtanP);
+#endif
+}
 
-// atan2 for sweeps in which most angles are small.  Three tiers, chosen per
+// atan2 for sweeps in which most angles are small.  Four tiers, chosen per
 // wave by a vote over its active lanes:
+// - every lane has x > 0 and |y| <= x / 32: a degree-3 polynomial in t^2
+//   fitted to that range (within 2e-20 of atan t in exact arithmetic);
 // - every lane has x > 0 and |y| < tan(pi/16) x: a degree-6 polynomial in t^2
 //   on t = y/x fitted to that range (within 7.4e-18 of atan t in exact
 //   arithmetic);
@@ -293,31 +345,72 @@ RH_HD double rh_atan2(double y, double x)
 // decide, and the two differ by rounding (about 1e-17 absolute).  A sweep's
 // result for one point can change at that level with the order or batching
 // of the points.
+#ifdef __HIPCC__
+template <int N>
+__device__ __forceinline__ void rh_atan2_wave(const double (&y)[N], const double (&x)[N], double top_c,
+                                              double (&a)[N])
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    // waves whose angles are all below 1/32 or pi/16 (distant faces) take a
+    // shorter polynomial (same accuracy on that range)
+    bool c32 = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) c32 = c32 && (fabs(y[i]) <= 0.03125 * x[i]);
+    if (rh_all(c32)) {
+        const double* c = d_atan32_p;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const double t = rh_div(y[i], x[i]), u = t * t;
+            const double p = fma(fma(fma(top_c, u, c[2]), u, c[1]), u, c[0]);
+            a[i] = fma(t * u, p, t);
+        }
+        return;
+    }
+    bool c16 = true, c8 = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        c16 = c16 && (fabs(y[i]) < kTanPi16 * x[i]);
+        c8 = c8 && (fabs(y[i]) < kTanPi8 * x[i]);
+    }
+    if (rh_all(c16)) {
+        const CoefPtr c = rh_coef_rare(d_atan16_p);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const double t = rh_div(y[i], x[i]), u = t * t;
+            double p = c[6];
+#pragma unroll
+            for (int k = 5; k >= 0; k--) p = fma(p, u, c[k]);
+            a[i] = fma(t * u, p, t);
+        }
+        return;
+    }
+    const CoefPtr c = rh_coef_rare(d_atan_p);
+    const bool all8 = rh_all(c8);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        if (all8) {
+            const double t = rh_div(y[i], x[i]), u = t * t;
+            double p = c[10];
+#pragma unroll
+            for (int k = 9; k >= 0; k--) p = fma(p, u, c[k]);
+            a[i] = fma(t * u, p, t);
+        } else {
+            a[i] = rh_atan2_c(y[i], x[i], c);
+        }
+    }
+#endif
+}
+#endif
 RH_HD double rh_atan2_wave(double y, double x)
 {
 #ifdef __HIP_DEVICE_COMPILE__
-    // waves whose angles are all below pi/16 (distant faces) take a shorter
-    // polynomial (same accuracy on that range)
-    if (__all(fabs(y) < kTanPi16 * x)) {
-        const double t = y * rh_rcp(x);
-        const double u = t * t;
-        const double* c = d_atan16_p;
-        double p = c[6];
-#pragma unroll
-        for (int i = 5; i >= 0; i--) p = fma(p, u, c[i]);
-        return fma(t * u, p, t);
-    }
-    if (__all(fabs(y) < kTanPi8 * x)) {
-        const double t = y * rh_rcp(x);
-        const double u = t * t;
-        const double* c = d_atan_p;
-        double p = c[10];
-#pragma unroll
-        for (int i = 9; i >= 0; i--) p = fma(p, u, c[i]);
-        return fma(t * u, p, t);
-    }
-#endif
+    const double yy[1] = {y}, xx[1] = {x};
+    double a[1];
+    rh_atan2_wave(yy, xx, kAtan32Top, a);
+    return a[0];
+#else
     return rh_atan2(y, x);
+#endif
 }
 // FP32 counterpart: degree 2 below pi/16 (within 9e-9 of atan t in float
 // arithmetic, 1.6e-9 in exact arithmetic) and degree 4 below pi/8 (1.8e-8);
@@ -327,13 +420,13 @@ RH_HD float rh_atan2_wave(float y, float x)
 {
 #ifdef __HIP_DEVICE_COMPILE__
     // below pi/16: degree 2 in t^2 (within 9e-9 of atan t in float arithmetic)
-    if (__all(fabsf(y) < 0.19891237f * x)) {
+    if (rh_all(fabsf(y) < 0.19891237f * x)) {
         const float t = y * rh_rcp(x);
         const float u = t * t;
         const float p = -0.3333331346511841f + u * (0.19990657269954681f + u * -0.13649502396583557f);
         return fmaf(t * u, p, t);
     }
-    if (__all(fabsf(y) < 0.41421356f * x)) {
+    if (rh_all(fabsf(y) < 0.41421356f * x)) {
         const float t = y * rh_rcp(x);
         const float u = t * t;
         const float p = -0.3333333134651184f +
@@ -344,6 +437,26 @@ RH_HD float rh_atan2_wave(float y, float x)
 #endif
     return rh_atan2(y, x);
 }
+#ifdef __HIPCC__
+template <int N>
+__device__ __forceinline__ void rh_atan2_wave(const float (&y)[N], const float (&x)[N], double, float (&a)[N])
+{
+    bool c16 = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) c16 = c16 && (fabsf(y[i]) < 0.19891237f * x[i]);
+    if (rh_all(c16)) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const float t = y[i] * rh_rcp(x[i]), u = t * t;
+            const float p = -0.3333331346511841f + u * (0.19990657269954681f + u * -0.13649502396583557f);
+            a[i] = fmaf(t * u, p, t);
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) a[i] = rh_atan2_wave(y[i], x[i]);
+}
+#endif
 
 // Vertex relative to the observation point, formed in FP64 then rounded to R.
 template <class R>
@@ -407,13 +520,14 @@ RH_HD R edge_log1p(const V3<R>& ra, R Ra, const V3<R>& rb, R Rb, const V3<R>& t,
 // |ra x rb|^2 / (Ra Rb - ra . rb), again without cancellation.  A wave whose
 // lanes all have ra . rb >= 0 skips the cross product; each lane's result
 // does not depend on the branch its wave takes.
-RH_HD double edge_L(const V3<double>& ra, double Ra, const V3<double>& rb, double Rb, double dab, double len)
+RH_HD void edge_L_ratio(const V3<double>& ra, double Ra, const V3<double>& rb, double Rb, double dab, double len,
+                        double& num, double& den)
 {
     const double q = len * (len + (Ra + Rb));
-    double den = fma(Ra, Rb, dab);
-    double num = den + q;
+    den = fma(Ra, Rb, dab);
+    num = den + q;
 #ifdef __HIP_DEVICE_COMPILE__
-    if (!__all(dab >= 0.0))
+    if (!rh_all(dab >= 0.0))
 #endif
     {
         RH_KEEP_BRANCH();
@@ -423,6 +537,11 @@ RH_HD double edge_L(const V3<double>& ra, double Ra, const V3<double>& rb, doubl
             num = fma(q, fma(Ra, Rb, -dab), den);
         }
     }
+}
+RH_HD double edge_L(const V3<double>& ra, double Ra, const V3<double>& rb, double Rb, double dab, double len)
+{
+    double num, den;
+    edge_L_ratio(ra, Ra, rb, Rb, dab, len, num, den);
     return rh_log_ratio(num, den);
 }
 
@@ -432,7 +551,7 @@ RH_HD float edge_L(const V3<float>& ra, float Ra, const V3<float>& rb, float Rb,
     const float q = len * (len + (Ra + Rb));
     float delta = q * rh_rcp(fmaf(Ra, Rb, dab));
 #ifdef __HIP_DEVICE_COMPILE__
-    if (!__all(dab >= 0.0f))
+    if (!rh_all(dab >= 0.0f))
 #endif
     {
         RH_KEEP_BRANCH();
@@ -449,6 +568,99 @@ RH_HD R edge_L(const V3<R>& ra, R Ra, const V3<R>& rb, R Rb, R len)
 {
     return edge_L(ra, Ra, rb, Rb, dot(ra, rb), len);
 }
+
+#ifdef __HIPCC__
+// The same integral from twice the length and the sum S = Ra + Rb at N points
+// of a lane, for sweeps in which most edges are short against their distance:
+// with X = 2 len / S, L = 2 atanh(X/2) = X + X^3 P(X^2).  No term cancels, so the error is relative
+// to L.  Waves whose points all have X <= 1/6, or all X <= 1/2, take that
+// tier's polynomial; any other wave (a point within about two lengths) forms
+// the ratio above, where 1 - X/2 would lose digits next to the edge.  An edge
+// costs about 20 issue slots instead of 40.  A point's result depends on its
+// wave-mates' tier at rounding level.  top_c: the first tier's leading
+// coefficient (kEdge6Top) in a vector register: an FMA of two scalar operands
+// needs a move first.
+template <int N>
+__device__ __forceinline__ void edge_L2(const V3<double> (&ra)[N], const double (&Ra)[N], const V3<double> (&rb)[N],
+                                        const double (&Rb)[N], const double (&S)[N], double len2, double top_c,
+                                        double (&L)[N])
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    double X[N], u[N], top = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        X[i] = rh_div(len2, S[i]);
+        u[i] = X[i] * X[i];
+        top = (i == 0) ? X[0] : fmax(top, X[i]);
+    }
+    if (rh_all(top <= 1.0 / 6.0)) {
+        const double* c = d_edge6_p;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const double p = fma(fma(fma(fma(top_c, u[i], c[3]), u[i], c[2]), u[i], c[1]), u[i], c[0]);
+            L[i] = fma(X[i] * u[i], p, X[i]);
+        }
+        return;
+    }
+    if (rh_all(top <= 0.5)) {
+        const double* c = d_edge2_p;
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            double p = c[7];
+#pragma unroll
+            for (int k = 6; k >= 0; k--) p = fma(p, u[i], c[k]);
+            L[i] = fma(X[i] * u[i], p, X[i]);
+        }
+        return;
+    }
+    RH_KEEP_BRANCH();
+    const CoefPtr c = rh_coef_rare(d_log_p);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        double num, den;
+        edge_L_ratio(ra[i], Ra[i], rb[i], Rb[i], dot(ra[i], rb[i]), 0.5 * len2, num, den);
+        L[i] = rh_log_ratio_c(num, den, c);
+    }
+#endif
+}
+// FP32: degree 2 on X <= 1/4 and degree 5 on X <= 1 (5.4e-9 relative), from
+// the same Chebyshev fits; the quotient carries about 2 ulp.
+template <int N>
+__device__ __forceinline__ void edge_L2(const V3<float> (&ra)[N], const float (&Ra)[N], const V3<float> (&rb)[N],
+                                        const float (&Rb)[N], const float (&S)[N], float len2, double, float (&L)[N])
+{
+    float X[N], u[N], top = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        X[i] = len2 * rh_rcp(S[i]);
+        u[i] = X[i] * X[i];
+        top = (i == 0) ? X[0] : fmaxf(top, X[i]);
+    }
+    if (rh_all(top <= 0.25f)) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const float p = fmaf(fmaf(0.002273426156f, u[i], 0.01249902845f), u[i], 0.08333333671f);
+            L[i] = fmaf(X[i] * u[i], p, X[i]);
+        }
+        return;
+    }
+    if (rh_all(top <= 1.0f)) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            float p = fmaf(3.845649477e-5f, u[i], 6.341298406e-5f);
+            p = fmaf(p, u[i], 0.0004480419985f);
+            p = fmaf(p, u[i], 0.002228746852f);
+            p = fmaf(p, u[i], 0.01250029582f);
+            p = fmaf(p, u[i], 0.08333332921f);
+            L[i] = fmaf(X[i] * u[i], p, X[i]);
+        }
+        return;
+    }
+    RH_KEEP_BRANCH();
+#pragma unroll
+    for (int i = 0; i < N; i++) L[i] = edge_L(ra[i], Ra[i], rb[i], Rb[i], 0.5f * len2);
+}
+#endif
 
 // Solid-angle factor of triangle (r1, r2, r3) as a complex number whose
 // argument is half the signed solid angle (Van Oosterom & Strackee 1983).
@@ -706,7 +918,7 @@ RH_HD bool tet_near32(const double* __restrict__ rec, const double p[3])
     }
     bool near = d < kNear32 * float(rec[kChargedM + 3]);
 #ifdef __HIP_DEVICE_COMPILE__
-    near = __any(near);
+    near = rh_any(near);
 #endif
     return near;
 }

@@ -17,22 +17,29 @@
 
 namespace rh {
 
-// Charged edge record: a(3), b(3), t(3), len, w(3), cont (1: a is the
-// previous record's b).  The FP32 sweep's records hold t(3), len and the
-// near distance as floats in slots 6-8.
+// Charged edge record: a(3), b(3), t(3), 2 len, w(3), cont (1: a is the
+// previous record's b).  The FP32 sweep's records hold 2 len and the near
+// distance as floats in slot 6 (the near pass reads slot 9).
 constexpr int kMeshEdge = 14;
-// Charged face record: v0..v3 (12), n(3), 2*area(v0,v1,v2), 2*area(v0,v2,v3),
-// nv, g(3), code (0 triangle, 1 triangle whose v0, v1 are the previous
+// Charged face record: v0..v3 (12), n(3), 4*area(v0,v1,v2), 4*area(v0,v2,v3),
+// nv, -2 g(3), code (0 triangle, 1 triangle whose v0, v1 are the previous
 // record's v1, v2, 2 quadrilateral, 3 quadrilateral whose v0, v1 are the
 // previous record's v2, v3), then the edges the face owns: for the sides
 // (v0,v1), (v1,v2), (v2,v0) of a triangle or (v0,v1), (v1,v2), (v2,v3) of a
-// quadrilateral in turn len and w(3) (slots 22-33), and
-// the mask of owned sides as an integer in the low word of slot 34; slot 35:
-// the FP32 sweep's near distance (a float).  A face's vertices may come in
-// either direction of its loop: its solid angle below takes the fan
-// triangles' triple products from n and their areas, not from the order.
-constexpr int kMeshFace = 36;
+// quadrilateral in turn 2 len and w(3) (slots 22-33); slot 35: the FP32
+// sweep's near distance (a float); slots 36-40: the squared distances of
+// (v0,v1), (v1,v2), (v0,v2), (v2,v3), (v0,v3) (the last two of
+// quadrilaterals; FP32 records: five floats from slot 36).  A face's vertices
+// may come in either direction of its loop: its solid angle below takes the
+// fan triangles' triple products from n and their areas, not from the order.
+// Constant factors are charged into the records, so that the sweep spends no
+// instruction on them: lengths are doubled (edge_L2), the charge is -2 g
+// (the sweep adds half the solid angle), and a triangle's n is scaled by
+// 4*area.  (The host build's mesh_edge_L and mesh_face_omega read records
+// with plain len, n, 2*area and g.)
+constexpr int kMeshFace = 42;
 constexpr int kMeshFaceEdges = 22;
+constexpr int kMeshFaceLen2 = 36;
 // Inside-test record: nplanes, M(3), up to 8 planes (n(3), d) with outward n:
 // inside iff n.p < d for every plane.
 constexpr int kMeshPlanes = 8;
@@ -74,28 +81,16 @@ RH_HD double mesh_face_omega(const double* __restrict__ rec, const double p[3])
     return 2.0 * double(rh_atan2_wave(im, re));
 }
 
-// Wave-uniform integer of a 0/1/2/3 code stored as a double: its high word
-// (0, 0x3ff00000, 0x40000000, 0x40080000) read into a scalar register.
-RH_HD int mesh_code(const double* __restrict__ slot)
-{
-#ifdef __HIP_DEVICE_COMPILE__
-    const int hi = __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(slot)[1]);
-#else
-    const int hi = int(uint64_t(__builtin_bit_cast(uint64_t, *slot)) >> 32);
+#ifdef __HIPCC__
+// What the sweep has to know of a record before it reads the record itself is
+// read through the scalar cache (the address is the same in every lane), so
+// that its branches wait for no vector instruction.
+typedef const __attribute__((address_space(4))) int* MeshFlags;
+__device__ __forceinline__ MeshFlags mesh_flags(const int32_t* p) { return (MeshFlags)(uintptr_t)p; }
 #endif
-    return hi == 0 ? 0 : (hi == 0x3ff00000 ? 1 : (hi == 0x40000000 ? 2 : 3));
-}
-
-// The owned-side mask of a face record (an integer in the slot's low word),
-// wave-uniform on the device.
-RH_HD int mesh_mask(const double* __restrict__ slot)
-{
-#ifdef __HIP_DEVICE_COMPILE__
-    return __builtin_amdgcn_readfirstlane(reinterpret_cast<const int*>(slot)[0]);
-#else
-    return int(uint32_t(__builtin_bit_cast(uint64_t, *slot) & 0xffffffffu));
-#endif
-}
+// Flags of a face or edge record: bits 0-2 the sides a face owns, bit 3 the
+// record continues the previous one (faces: code 1 or 3).
+constexpr int kMeshCont = 8;
 
 // A vertex relative to the observation point and its distance.
 template <class R>
@@ -109,45 +104,84 @@ RH_HD MeshVtx<R> mesh_vtx(const double* __restrict__ v, const double p[3])
     const V3<R> r = rel<R>(v, p);
     return MeshVtx<R>{r, rh_sqrt(dot(r, r))};
 }
+// The same for the N points of a lane.
+template <class R, int N>
+struct MeshVtxN {
+    V3<R> r[N];
+    R d[N];
+};
 
-// Signed solid angle of a charged triangle from the offsets and distances of
-// its vertices and r0 . r1.
-template <class R>
-RH_HD double mesh_tri_omega_from(const V3<R>& r0, R R0, const V3<R>& r1, R R1, const V3<R>& r2, R R2, R d01,
-                                 R d12, R d20, const double* __restrict__ rec)
-{
-    const V3<R> n = v3(R(rec[12]), R(rec[13]), R(rec[14]));
-    const R im = R(rec[15]) * dot(r0, n);
-    const R re = R0 * R1 * R2 + d01 * R2 + d20 * R1 + d12 * R0;
-    return 2.0 * double(rh_atan2_wave(im, re));
-}
-
+#ifdef __HIPCC__
 // FP32 sweep records: the geometry the lanes use in FP32 is stored as floats
-// when the records are charged (edge slots 6-7: t(3), len; face slots 12-14:
-// n(3), the two doubled areas), so the sweep converts none of it per record;
-// vertices (offsets are formed in FP64) and the weights w and g (the sums are
-// accumulated in FP64) stay FP64.
-RH_HD const float* mesh32(const double* __restrict__ rec, int slot)
+// when the records are charged (edge slot 6: 2 len, near distance; face slots
+// 12-14: n(3), the two doubled areas), so the sweep converts none of it per
+// record; vertices (offsets are formed in FP64) and the weights w and g (the
+// sums are accumulated in FP64) stay FP64.
+template <class R>
+struct MeshGeo {
+    R n0, n1, n2, a1, a2, l01, l12, l02, l23, l03;
+};
+template <class R>
+__device__ __forceinline__ MeshGeo<R> mesh_geo(const double* __restrict__ rec)
 {
-    return reinterpret_cast<const float*>(rec + slot);
+    if constexpr (sizeof(R) == 4) {
+        const float* f = reinterpret_cast<const float*>(rec + 12);
+        const float* l = reinterpret_cast<const float*>(rec + kMeshFaceLen2);
+        return MeshGeo<R>{f[0], f[1], f[2], f[3], f[4], l[0], l[1], l[2], l[3], l[4]};
+    } else {
+        const double* l = rec + kMeshFaceLen2;
+        return MeshGeo<R>{rec[12], rec[13], rec[14], rec[15], rec[16], l[0], l[1], l[2], l[3], l[4]};
+    }
 }
 
-RH_HD float mesh32_tri_omega(const V3<float>& r0, float R0, const V3<float>& r1, float R1, const V3<float>& r2,
-                             float R2, float d01, float d12, float d20, const double* __restrict__ rec)
+template <class R, int N>
+__device__ __forceinline__ void mesh_vtx(const double* __restrict__ v, const double (&p)[N][3], MeshVtxN<R, N>& o)
 {
-    const float* f = mesh32(rec, 12);
-    const float im = f[3] * dot(r0, v3(f[0], f[1], f[2]));
-    const float re = R0 * R1 * R2 + d01 * R2 + d20 * R1 + d12 * R0;
-    return 2.0f * rh_atan2_wave(im, re);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        o.r[i] = rel<R>(v, p[i]);
+        o.d[i] = rh_sqrt(dot(o.r[i], o.r[i]));
+    }
+}
+// S = Ra + Rb
+template <class R, int N>
+__device__ __forceinline__ void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b, R (&o)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N; i++) o[i] = a.d[i] + b.d[i];
 }
 
-// FP64 solid angle of a face of an FP32 sweep record, whose normal and areas
-// are stored as floats: the fan triangles' triple products r0 . (r1 x r2)
+// Half the signed solid angle of a charged triangle from the offset of its
+// first vertex, the distances and their sums.  The formula of Van Oosterom and
+// Strackee, tan(Omega/2) = r0 . (r1 x r2) / (R0 R1 R2 + (r0.r1) R2 + (r2.r0) R1
+// + (r1.r2) R0), with r_i . r_j = (R_i^2 + R_j^2 - l_ij^2) / 2: the denominator
+// is ((R0+R1)(R1+R2)(R2+R0) - R2 l01^2 - R1 l02^2 - R0 l12^2) / 2.  Each term
+// keeps the error of the dot products' form (a few ulp of R^3), no dot product
+// is formed, and the sums are those that the edges' integrals divide by.
+template <class R, int N>
+__device__ __forceinline__ void mesh_tri_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
+                                                    const MeshVtxN<R, N>& c, const R (&sab)[N], const R (&sbc)[N],
+                                                    const R (&sca)[N], const double* __restrict__ rec, double top_c,
+                                                    R (&om)[N])
+{
+    const MeshGeo<R> g = mesh_geo<R>(rec);
+    R im[N], re[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        im[i] = dot(a.r[i], v3(g.n0, g.n1, g.n2));
+        re[i] = (sab[i] * sbc[i]) * sca[i] - (c.d[i] * g.l01 + b.d[i] * g.l02 + a.d[i] * g.l12);
+    }
+    rh_atan2_wave(im, re, top_c, om);
+}
+#endif
+
+// FP64 half solid angle of a face of an FP32 sweep record, whose normal and
+// areas are stored as floats: the fan triangles' triple products r0 . (r1 x r2)
 // are taken as r0 . ((v1 - v0) x (v2 - v0)) from the FP64 vertices, signed by
 // the stored normal (the same quantity as area * (r0 . n) of the FP64 sweep).
-RH_HD double mesh_face_omega_near(const double* __restrict__ rec, const double p[3])
+RH_HD double mesh_face_half_omega_near(const double* __restrict__ rec, const double p[3])
 {
-    const float* f = mesh32(rec, 12);
+    const float* f = reinterpret_cast<const float*>(rec + 12);
     const V3<double> e1 = v3(rec[3] - rec[0], rec[4] - rec[1], rec[5] - rec[2]);
     const V3<double> e2 = v3(rec[6] - rec[0], rec[7] - rec[1], rec[8] - rec[2]);
     const V3<double> c1 = cross(e1, e2);
@@ -167,32 +201,32 @@ RH_HD double mesh_face_omega_near(const double* __restrict__ rec, const double p
         re = pr;
         im = pi;
     }
-    return 2.0 * rh_atan2_wave(im, re);
+    return rh_atan2_wave(im, re);
 }
 
 // Near test of the FP32 mesh sweep: FP32 offsets carry eps32 of the distance,
 // so a term's relative error grows like eps32 * size / distance.  A wave with
 // a point within kNear32 entity sizes of a vertex (faces: the longest side;
 // edges: the length) evaluates that entity in FP64.  thr: kNear32 sizes, as
-// the record carries it (faces: slot 35, edges: slot 8).
+// the record carries it (faces: slot 35, edges: slot 6, second float).
 RH_HD bool mesh32_near(float dmin, float thr)
 {
     bool near = dmin < thr;
 #ifdef __HIP_DEVICE_COMPILE__
-    near = __any(near);
+    near = rh_any(near);
 #endif
     return near;
 }
 
-// L_e of an FP32 sweep edge record in FP64 (vertices in slots 0-5, the FP64
-// length in slot 9).
+// L_e of an FP32 sweep edge record in FP64 (vertices in slots 0-5, twice the
+// FP64 length in slot 9).
 RH_HD double mesh_edge_L_near(const double* __restrict__ rec, const double p[3])
 {
     const MeshVtx<double> a = mesh_vtx<double>(rec, p), b = mesh_vtx<double>(rec + 3, p);
-    return edge_L(a.r, a.d, b.r, b.d, rec[9]);
+    return edge_L(a.r, a.d, b.r, b.d, 0.5 * rec[9]);
 }
 
-// A face of an FP32 sweep record in FP64 (triangle or quadrilateral): its
+// A face of an FP32 sweep record in FP64 (triangle or quadrilateral): half its
 // solid angle and the sum of L_e w_e over the sides it owns.
 struct MeshFace64 {
     double om, h0, h1, h2;
@@ -200,13 +234,13 @@ struct MeshFace64 {
 RH_HD MeshFace64 mesh_face_near(const double* __restrict__ rec, int mask, const double p[3])
 {
     const int nv = rec[17] > 3.5 ? 4 : 3;
-    MeshFace64 t{mesh_face_omega_near(rec, p), 0.0, 0.0, 0.0};
+    MeshFace64 t{mesh_face_half_omega_near(rec, p), 0.0, 0.0, 0.0};
     for (int k = 0; k < 3; k++) {
         if (!(mask & (1 << k))) continue;
         const double* e = rec + kMeshFaceEdges + 4 * k;
         const int k1 = (k + 1 == nv) ? 0 : k + 1;
         const MeshVtx<double> a = mesh_vtx<double>(rec + 3 * k, p), b = mesh_vtx<double>(rec + 3 * k1, p);
-        const double L = edge_L(a.r, a.d, b.r, b.d, dot(a.r, b.r), e[0]);
+        const double L = edge_L(a.r, a.d, b.r, b.d, dot(a.r, b.r), 0.5 * e[0]);
         t.h0 += L * e[1];
         t.h1 += L * e[2];
         t.h2 += L * e[3];
@@ -214,27 +248,30 @@ RH_HD MeshFace64 mesh_face_near(const double* __restrict__ rec, int mask, const 
     return t;
 }
 
-// A quadrilateral face record at p from its vertex offsets, distances and
-// dot products: the signed solid angle (fans (v0,v1,v2) and (v0,v2,v3)
-// multiplied as complex numbers).  FP64 records hold n and the doubled fan
-// areas in slots 12-16, FP32 records as floats in slots 12-14.
-template <class R>
-RH_HD R mesh_quad_omega_from(const MeshVtx<R> v[4], R d01, R d02, R d03, R d12, R d23,
-                             const double* __restrict__ rec)
+#ifdef __HIPCC__
+// Half the signed solid angle of a quadrilateral record, likewise: the fans
+// (v0,v1,v2) and (v0,v2,v3) multiplied as complex numbers.
+template <class R, int N>
+__device__ __forceinline__ void mesh_quad_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
+                                                     const MeshVtxN<R, N>& c, const MeshVtxN<R, N>& d,
+                                                     const R (&sab)[N], const R (&sbc)[N], const R (&scd)[N],
+                                                     const double* __restrict__ rec, double top_c, R (&om)[N])
 {
-    R n0, n1, n2, a1, a2;
-    if constexpr (sizeof(R) == 4) {
-        const float* f = mesh32(rec, 12);
-        n0 = f[0], n1 = f[1], n2 = f[2], a1 = f[3], a2 = f[4];
-    } else {
-        n0 = R(rec[12]), n1 = R(rec[13]), n2 = R(rec[14]), a1 = R(rec[15]), a2 = R(rec[16]);
+    const MeshGeo<R> g = mesh_geo<R>(rec);
+    R im[N], re[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const R h = dot(a.r[i], v3(g.n0, g.n1, g.n2));
+        const R i1 = g.a1 * h, i2 = g.a2 * h;
+        const R sac = a.d[i] + c.d[i], sad = a.d[i] + d.d[i];
+        const R r1 = (sab[i] * sbc[i]) * sac - (c.d[i] * g.l01 + b.d[i] * g.l02 + a.d[i] * g.l12);
+        const R r2 = (sac * scd[i]) * sad - (d.d[i] * g.l02 + c.d[i] * g.l03 + a.d[i] * g.l23);
+        im[i] = r1 * i2 + i1 * r2;
+        re[i] = r1 * r2 - i1 * i2;
     }
-    const R h = dot(v[0].r, v3(n0, n1, n2));
-    const R im = a1 * h, im2 = a2 * h;
-    const R re = v[0].d * v[1].d * v[2].d + d01 * v[2].d + d02 * v[1].d + d12 * v[0].d;
-    const R re2 = v[0].d * v[2].d * v[3].d + d02 * v[3].d + d03 * v[2].d + d23 * v[0].d;
-    return R(2) * rh_atan2_wave(re * im2 + im * re2, re * re2 - im * im2);
+    rh_atan2_wave(im, re, top_c, om);
 }
+#endif
 
 // Plane test of one inside record.
 RH_HD bool mesh_inside(const double* __restrict__ rec, const double p[3])
