@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "rh_current.hpp"
 #include "rh_eval.hpp"
@@ -828,20 +829,40 @@ k_field_mesh(DevModel m, const double* __restrict__ pts, int64_t np, int64_t S, 
     }
 }
 
+// Sums the `splits` partial rows of 6 np values (B and H of each point) in a
+// fixed order: a workgroup owns 256/G columns, G threads take every G-th row
+// of a column and the first adds their G sums.  With one thread per point a
+// sweep of 64 points over 1,790 slices of the 8,000-tetrahedron yoke spent
+// 0.5 ms here, in one thread's chain of additions; G by the number of rows.
+template <int G>
 __global__ __launch_bounds__(256) void k_field_reduce(int64_t np, int64_t splits,
                                                       const double* __restrict__ part,
                                                       double* __restrict__ B, double* __restrict__ H)
 {
-    const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (p >= np) return;
-    double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (int64_t s = 0; s < splits; s++) {
-        const double* o = part + (s * np + p) * 6;
-        for (int k = 0; k < 6; k++) acc[k] += o[k];
+    constexpr int C = 256 / G;
+    __shared__ double red[G > 1 ? 256 : 1];
+    const int col = threadIdx.x % C, g = threadIdx.x / C;
+    const int64_t c = int64_t(blockIdx.x) * C + col, w = 6 * np;
+    double acc = 0.0;
+    if (c < w) {
+#pragma unroll 4
+        for (int64_t s = g; s < splits; s += G) acc += part[s * w + c];
     }
-    for (int k = 0; k < 3; k++) {
-        if (B) B[3 * p + k] = acc[k];
-        if (H) H[3 * p + k] = acc[3 + k];
+    if constexpr (G > 1) {
+        red[threadIdx.x] = acc;
+        __syncthreads();
+        if (g == 0) {
+#pragma unroll
+            for (int k = 1; k < G; k++) acc += red[k * C + col];
+        }
+    }
+    if (g != 0 || c >= w) return;
+    const int64_t p = c / 6;
+    const int k = int(c - 6 * p);
+    if (k < 3) {
+        if (B) B[3 * p + k] = acc;
+    } else {
+        if (H) H[3 * p + k - 3] = acc;
     }
 }
 
@@ -2043,8 +2064,18 @@ hipError_t field_all(const DevModel& m, const double* M, const double* pts, int6
     if (sp[2]) field_slot<R, SYM, 2>(m, M, pts, np, sp[2], slice0, B, H, part, s);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || total <= 1) return e;
-    hipLaunchKernelGGL(k_field_reduce, dim3(unsigned((np + 255) / 256)), dim3(256), 0, s, np, total,
-                       part, B, H);
+    // about 16 rows per thread: fewer threads per column read longer lines,
+    // more shorten the chain of additions
+    auto reduce = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        const int64_t cols = 256 / G;
+        hipLaunchKernelGGL(k_field_reduce<G>, dim3(unsigned((6 * np + cols - 1) / cols)), dim3(256), 0, s, np, total,
+                           part, B, H);
+    };
+    if (total <= 16) reduce(std::integral_constant<int, 1>{});
+    else if (total <= 64) reduce(std::integral_constant<int, 4>{});
+    else if (total <= 256) reduce(std::integral_constant<int, 16>{});
+    else reduce(std::integral_constant<int, 64>{});
     return hipGetLastError();
 }
 }  // namespace
