@@ -232,6 +232,7 @@ struct rh_model {
     double* d_rowt = nullptr;
     int32_t* d_kidx = nullptr;
     double* d_charged = nullptr;  // field-only tetrahedron records, rebuilt per field call
+    double* d_far = nullptr;      // far-form tetrahedron records of the assembly
     // adjoint geometry, uploaded on the first adjoint call
     double* d_adj = nullptr;
     int64_t* d_adj_off = nullptr;
@@ -305,6 +306,7 @@ void free_model(rh_model* m)
     dfree(m->d_rowt);
     dfree(m->d_kidx);
     dfree(m->d_charged);
+    dfree(m->d_far);
     dfree(m->d_adj);
     dfree(m->d_adj_off);
     dfree(m->d_vert_off);
@@ -397,12 +399,7 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
     if (e == hipSuccess) e = upload(&m->d_kidx, P.kind_idx, s);
     if (e == hipSuccess)
         e = dalloc(&m->d_charged, size_t(rh::kChargedTet * (P.kind_off[2] - P.kind_off[1])));
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-        std::string msg = std::string("model upload: ") + hipGetErrorString(e);
-        free_model(m);
-        return fail(e == hipErrorOutOfMemory ? RH_ERR_NOMEM : RH_ERR_HIP, msg);
-    }
+    if (e == hipSuccess) e = dalloc(&m->d_far, size_t(rh::far_tet_doubles(P.kind_off[2] - P.kind_off[1])));
     rh::DevModel& d = m->dev;
     d.n = P.n;
     d.kind = m->d_kind;
@@ -413,9 +410,17 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
     d.colloc = m->d_colloc;
     d.rowt = m->d_rowt;
     d.kidx = m->d_kidx;
+    d.far_tet = m->d_far;
     for (int k = 0; k < 4; k++) d.koff[k] = P.kind_off[k];
     d.sym = P.sym;
     d.rowt_identity = P.rowt_identity;
+    if (e == hipSuccess) e = rh::launch_far_records(d, m->d_far, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (e != hipSuccess) {
+        std::string msg = std::string("model upload: ") + hipGetErrorString(e);
+        free_model(m);
+        return fail(e == hipErrorOutOfMemory ? RH_ERR_NOMEM : RH_ERR_HIP, msg);
+    }
     if (P.mesh.active) {
         const rh::MeshForm& F = P.mesh;
         rh::MeshDev& md = d.mesh;

@@ -17,6 +17,7 @@
 
 #include "rh_current.hpp"
 #include "rh_eval.hpp"
+#include "rh_far.hpp"
 #include "rh_geom.hpp"
 #include "rh_kernels.hpp"
 #include "rh_mesh.hpp"
@@ -41,22 +42,71 @@ __global__ __launch_bounds__(256) void k_charge_tets(DevModel m, const double* _
     charge_tet(m.data + m.off[j], mm, out + kChargedTet * (k - m.koff[1]));
 }
 
+// Far-form records of the tetrahedra (one lane each).
+__global__ __launch_bounds__(256) void k_far_records(DevModel m, double* __restrict__ out)
+{
+    const int64_t k = m.koff[1] + int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (k >= m.koff[2]) return;
+    far_tet_record(m.data + m.off[m.kidx[k]], out + kFarTet * (k - m.koff[1]));
+}
+
+// The far form of a tetrahedron's block at x when every lane of the wave is
+// far (else false).  FAR32: FP32 integrals beyond two circumradii of the
+// vertex mean, as block_Q_mixed takes them (vertices come first in the far
+// record, as in the element record).
+template <bool FAR32>
+__device__ __forceinline__ bool tet_fp32(const double* __restrict__ far, const double x[3])
+{
+    if constexpr (FAR32) return !rh_any(near_element<1>(EK_TET, far, x));
+    else return false;
+}
+template <bool FAR32>
+__device__ __forceinline__ bool far_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
+{
+    auto eval = [&](auto zero) {
+        using R = decltype(zero);
+        FarTet<R> t;
+        if (!far_tet_open<R>(far, x, t)) return false;
+        far_tet_block<R>(far, t, q5);
+        return true;
+    };
+    if constexpr (FAR32) {
+        if (tet_fp32<FAR32>(far, x)) return eval(float(0));
+    }
+    return eval(double(0));
+}
+template <bool FAR32>
+__device__ __forceinline__ bool near_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
+{
+    if constexpr (FAR32) {
+        if (tet_fp32<FAR32>(far, x)) return near_tet_block<float>(far, x, q5);
+    }
+    return near_tet_block<double>(far, x, q5);
+}
+
 template <class T>
 __device__ __forceinline__ void store_out(T* p, double v) { *p = T(v); }
 
 // ---------------------------------------------------------------- assembly
 // Rows of elements [r0, r1) into Q (Q holds row 3*r0 first); block columns
-// are the elements kidx[k0 .. k1) of one kind slot.  Each lane owns one row
-// element and the wave sweeps the sources with uniform records.  A lane's
-// 3x3 blocks for S consecutive sources are staged in LDS and the wave then
-// writes the 3*64 matrix rows of the tile as contiguous row segments of 96
-// bytes (4 sources in FP64, 8 in FP32), so that a cache line is written by
-// at most two consecutive tiles of one wave instead of by 64 rows' worth of
-// interleaved 24-byte stores; the tile (20 KB) still allows two waves per
-// SIMD.  Measured on the 8,000-tetrahedron yoke: 2.95 ms against 4.15 ms
-// unstaged (FP64), 2.41 against 3.03 ms (FP32); wider tiles cost occupancy.
-// Sources whose columns are not consecutive (mixed kinds) are stored
-// directly.
+// are the elements kidx[k0 .. k1) of one kind slot.  A workgroup's four waves
+// own the same 64 row elements (one per lane) and split the sources of a tile
+// between them, sweeping uniform records; the lanes' 3x3 blocks of the tile's
+// S sources are staged in one LDS tile, and the 256 threads write its rows as
+// contiguous segments of 128 bytes (symmetric-block planes: 16 sources in FP64,
+// 32 in FP32) or 192 bytes (row-major blocks: 8 and 16 sources).  Sources
+// whose columns are not consecutive (mixed kinds) are stored directly.
+//
+// Measured with the integrals left out, the stores alone take (8,000 rows,
+// FP64 planes) 2.09 ms in 32-byte segments, 1.03 in 64-byte and 0.72 in
+// 128-byte ones, which fill whole lines.  With one wave per tile 128-byte
+// segments leave LDS for one wave per SIMD; four waves to a tile allow three.
+// Tetrahedra take the far form of rh_far.hpp, staged through LDS, where every
+// lane is far (84 % of the sources a wave of the C-yoke meets, 92 % on the
+// 24,000-tetrahedron yoke).  Measured: C-yoke FP64 2.09 -> 1.35 ms; 23,999
+// tetrahedra mixed 14.05 -> 8.4 ms; 1,500 blocks x 4 copies mixed 259 -> 240 us.
+// What bounds it now: vector issue about half of the time, the rest the four
+// waves' wait for the one that met near sources, and the stores' 0.72 ms.
 //
 // Symmetric-block layout (PK = 5 or 6): without transform copies and row
 // transforms every block is the symmetric tensor Q(x_i) of source j, so an
@@ -66,22 +116,16 @@ __device__ __forceinline__ void store_out(T* p, double v) { *p = T(v); }
 // block with a trace beyond 1/4 (a collocation point inside another element)
 // sets *flag, and the caller stores the matrix with 6 planes instead.
 #ifndef RH_ASM_S64
-#define RH_ASM_S64 4
+#define RH_ASM_S64 8
 #endif
 #ifndef RH_ASM_S32
-#define RH_ASM_S32 8
+#define RH_ASM_S32 16
 #endif
-// symmetric-block tiles: 8 (FP64) or 16 (FP32) sources, 64-byte plane
-// segments; on the 40,000-tetrahedron yoke 49.2 / 38.5 ms against 55.1 / 40.4
-// with 4 / 8 sources and 80.7 / 48.1 with 2 / 4 (padded tiles); unpadded
-// swizzled tiles 46.2 / 37.2 against 47.4 / 39.0 ms padded.  Three waves
-// per SIMD (RH_ASM_WAVES=3: 154 VGPRs) with 4 / 8 sources measured 58-63 /
-// 40 ms: the wider plane segments matter more than the occupancy
 #ifndef RH_ASM_P64
-#define RH_ASM_P64 8
+#define RH_ASM_P64 16
 #endif
 #ifndef RH_ASM_P32
-#define RH_ASM_P32 16
+#define RH_ASM_P32 32
 #endif
 template <class OUT, int PK>
 struct AsmTile {
@@ -92,9 +136,8 @@ struct AsmTile {
     static constexpr int U = VPS * S * int(sizeof(OUT)) / 8;  // 8-byte units per row segment
     static constexpr int EPU = 8 / int(sizeof(OUT));          // elements per 8-byte unit
     // LDS row stride (elements): row-major tiles pad a unit against bank
-    // conflicts; plane tiles are unpadded (20 KB per wave, so that two waves
-    // per SIMD fit the CU's LDS) with the units of the rows of lane l stored
-    // at unit index u ^ (l & SWZ) instead
+    // conflicts; plane tiles are unpadded with the units of the rows of lane l
+    // stored at unit index u ^ (l & SWZ) instead
     static constexpr int W = (PK ? U : U + 1) * EPU;
     static constexpr int SWZ = PK ? U - 1 : 0;
     static_assert(!PK || (U & (U - 1)) == 0, "plane tiles swizzle a power-of-two number of units");
@@ -102,24 +145,37 @@ struct AsmTile {
     __device__ static int at(int r, int c) { return r * W + (((c / EPU) ^ ((r / RPE) & SWZ)) * EPU + c % EPU); }
 };
 
-#ifdef RH_ASM_WAVES
-#define RH_ASM_ATTR __attribute__((amdgpu_waves_per_eu(RH_ASM_WAVES)))
-#else
-#define RH_ASM_ATTR
-#endif
+// occupancy floor (waves per SIMD): tetrahedra 3 (the LDS tiles allow 3), the
+// other kinds 2 (their integrals need more than 168 registers)
+template <int KIND, bool SYM>
+constexpr int asm_waves() { return KIND == 1 ? (SYM ? 2 : 3) : 2; }
+// far-form tetrahedron records staged at a time
+constexpr int kFarChunk = 16;
+static_assert(kFarTet % 2 == 0, "16-byte loads of whole records");
 // FAR32: far blocks in FP32 arithmetic, near ones in FP64 (block_Q_mixed).
 // PK: 0 row-major 3x3 blocks, 5 or 6 the symmetric-block planes (then ld is
 // the plane stride and SYM, ROWT are false).
 template <class R, bool SYM, bool ROWT, class OUT, int KIND, bool FAR32 = false, int PK = 0>
-__global__ __launch_bounds__(64) RH_ASM_ATTR void k_assemble(DevModel m, OUT* __restrict__ Q, int64_t ld,
-                                                 double* __restrict__ qdiag, int64_t jt, int64_t r0,
-                                                 int64_t r1, int32_t* __restrict__ flag)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(asm_waves<KIND, SYM>()))) void
+k_assemble(DevModel m, OUT* __restrict__ Q, int64_t ld, double* __restrict__ qdiag, int64_t jt, int64_t r0, int64_t r1,
+           int32_t* __restrict__ flag)
 {
     static_assert(PK == 0 || (!SYM && !ROWT), "the symmetric-block layout needs lab-frame blocks");
     using TL = AsmTile<OUT, PK>;
     constexpr int S = TL::S, W = TL::W, RPE = TL::RPE, VPS = TL::VPS;
-    __shared__ OUT tile[RPE * 64 * W];
-    const int lane = threadIdx.x;
+    static_assert(S % 4 == 0 && S <= 32, "a quarter of the tile's sources per wave, one bit each");
+    __shared__ __align__(16) OUT tile[RPE * 64 * W];
+    // tetrahedra: the far records of the next CH sources, fetched one chunk
+    // ahead into registers.  (Read through the scalar cache a record's 620
+    // bytes cost six dependent batches of scalar loads, each a miss of its
+    // own wave: 2.8 ms on the C-yoke with one wave per tile, against 2.1
+    // without the far form.)
+    constexpr bool kFar = KIND == 1;
+    constexpr int CH = S < kFarChunk ? S : kFarChunk;
+    constexpr int kLoads = (CH * kFarTet / 2 + 255) / 256;
+    __shared__ __align__(16) double fsrc[kFar ? CH * kFarTet : 2];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
     const int64_t i0 = r0 + int64_t(blockIdx.x) * 64;
     const int64_t i = i0 + lane;
     const bool live = i < r1;
@@ -135,17 +191,53 @@ __global__ __launch_bounds__(64) RH_ASM_ATTR void k_assemble(DevModel m, OUT* __
         for (int k = 0; k < 9; k++) rt[k] = m.rowt[9 * ic + k];
     OUT* row = Q + (RPE * (ic - r0)) * ld;
     bool traced = false;
+    double2 ahead[kFar ? kLoads : 1];
+    auto fetch = [&](int64_t k) {
+        if constexpr (kFar) {
+            const double2* src = reinterpret_cast<const double2*>(m.far_tet + kFarTet * (k - m.koff[1]));
+            const int cnt = int((k1 - k < CH) ? (k1 - k) : CH) * (kFarTet / 2);
+#pragma unroll
+            for (int t = 0; t < kLoads; t++)
+                if (int(threadIdx.x) + 256 * t < cnt) ahead[t] = src[threadIdx.x + 256 * t];
+        }
+    };
+    auto chunk = [&](int64_t k) {
+        if constexpr (kFar) {
+            __syncthreads();  // the previous chunk has been consumed
+            double2* dst = reinterpret_cast<double2*>(fsrc);
+#pragma unroll
+            for (int t = 0; t < kLoads; t++)
+                if (int(threadIdx.x) + 256 * t < CH * (kFarTet / 2)) dst[threadIdx.x + 256 * t] = ahead[t];
+            __syncthreads();
+            if (k + CH < k1) fetch(k + CH);
+        }
+    };
+    if constexpr (kFar) {
+#pragma unroll
+        for (int t = 0; t < kLoads; t++) ahead[t] = double2{0.0, 0.0};
+        fetch(k0);
+    }
     for (int64_t kb = k0; kb < k1; kb += S) {
         const int cnt = int((k1 - kb < S) ? (k1 - kb) : S);
         const int64_t jb = m.kidx[kb];
         const bool run = (m.kidx[kb + cnt - 1] - jb == cnt - 1);  // consecutive columns
-        for (int s = 0; s < cnt; s++) {
-            const int64_t j = m.kidx[kb + s];
-            double q[9];
-            if constexpr (FAR32)
-                block_Q_mixed<SYM, KIND>(mv, j, x, q);
-            else
-                block_Q<R, SYM, KIND>(mv, j, x, q);
+        // a lane's stored values of source s: into the tile, or straight to its row
+        auto put = [&](int s, const double (&v)[RPE * VPS]) {
+            if (run) {
+#pragma unroll
+                for (int a = 0; a < RPE; a++)
+#pragma unroll
+                    for (int b = 0; b < VPS; b++) tile[TL::at(RPE * lane + a, VPS * s + b)] = OUT(v[VPS * a + b]);
+            } else if (live) {
+                OUT* o = row + VPS * m.kidx[kb + s];
+#pragma unroll
+                for (int a = 0; a < RPE; a++)
+#pragma unroll
+                    for (int b = 0; b < VPS; b++) store_out(o + a * ld + b, v[VPS * a + b]);
+            }
+        };
+        // the block q of source s (element j): row transform, self block, storage
+        auto finish = [&](int s, int64_t j, double (&q)[9]) {
             if (ROWT) {
                 double t[9];
                 for (int a = 0; a < 3; a++)
@@ -173,28 +265,113 @@ __global__ __launch_bounds__(64) RH_ASM_ATTR void k_assemble(DevModel m, OUT* __
                 v[4] = 0.5 * (q[5] + q[7]);
                 if constexpr (PK == 6) v[5] = q[8];
             }
-            if (run) {
+            put(s, v);
+        };
+        if constexpr (kFar && SYM) {
+            // tetrahedra with transform copies: copy by copy, far or not
+#pragma unroll 1
+            for (int c = 0; c < cnt; c += CH) {
+                chunk(kb + c);
+#pragma unroll 1
+                for (int t = 0; t < CH / 4; t++) {
+                    const int f = wave * (CH / 4) + t, s = c + f;
+                    if (s >= cnt) break;
+                    const int64_t j = m.kidx[kb + s];
+                    double q[9];
 #pragma unroll
-                for (int a = 0; a < RPE; a++)
+                    for (int k = 0; k < 9; k++) q[k] = 0.0;
+#pragma unroll 1
+                    for (int64_t cc = m.copy_off[j]; cc < m.copy_off[j + 1]; cc++) {
+                        const double* cp = m.copies + 24 * cc;
+                        double xl[3], g[5];
+                        apply_inv(cp, x, xl);
+                        double zz = 0.0;
+                        if (!far_tet_eval<FAR32>(fsrc + kFarTet * f, xl, g))
+                            zz = near_tet_eval<FAR32>(fsrc + kFarTet * f, xl, g) ? -1.0 : 0.0;
+                        zz -= g[0] + g[3];
+                        const double l[9] = {g[0], g[1], g[2], g[1], g[3], g[4], g[2], g[4], zz};
+                        const double* F = cp + 12;
 #pragma unroll
-                    for (int b = 0; b < VPS; b++) tile[TL::at(RPE * lane + a, VPS * s + b)] = OUT(v[VPS * a + b]);
-            } else if (live) {
-                OUT* o = row + VPS * j;
+                        for (int a = 0; a < 3; a++)
 #pragma unroll
-                for (int a = 0; a < RPE; a++)
+                            for (int b = 0; b < 3; b++)
+                                q[3 * a + b] += F[3 * a] * l[b] + F[3 * a + 1] * l[3 + b] + F[3 * a + 2] * l[6 + b];
+                    }
+                    finish(s, j, q);
+                }
+            }
+        } else if constexpr (kFar) {
+            // stores a tetrahedron's block: xx, xy, xz, yy, yz and zz
+            auto put6 = [&](int s, const double (&q)[5], double zz) {
+                double v[RPE * VPS];
+                if constexpr (PK == 0) {
+                    v[0] = q[0];
+                    v[1] = v[3] = q[1];
+                    v[2] = v[6] = q[2];
+                    v[4] = q[3];
+                    v[5] = v[7] = q[4];
+                    v[8] = zz;
+                } else {
 #pragma unroll
-                    for (int b = 0; b < VPS; b++) store_out(o + a * ld + b, v[VPS * a + b]);
+                    for (int k = 0; k < 5; k++) v[k] = q[k];
+                    if constexpr (PK == 6) v[5] = zz;
+                }
+                put(s, v);
+            };
+#pragma unroll 1
+            for (int c = 0; c < cnt; c += CH) {
+                chunk(kb + c);
+                // far sources first; the others' bits are set and they follow
+                // after the loop, where the far form's registers are free
+                uint32_t near = 0;
+#pragma unroll 1
+                for (int t = 0; t < CH / 4; t++) {
+                    const int f = wave * (CH / 4) + t, s = c + f;
+                    if (s >= cnt) break;
+                    double q[5];
+                    if (far_tet_eval<FAR32>(fsrc + kFarTet * f, x, q))
+                        put6(s, q, -(q[0] + q[3]));
+                    else
+                        near |= 1u << f;
+                }
+#pragma unroll 1
+                for (; near; near &= near - 1) {
+                    const int f = __builtin_ctz(near), s = c + f;
+                    double q[5];
+                    const bool in = near_tet_eval<FAR32>(fsrc + kFarTet * f, x, q);
+                    double zz = -(q[0] + q[3]) - (in ? 1.0 : 0.0);
+                    if (live && m.kidx[kb + s] == i) {
+                        const double d[9] = {q[0], q[1], q[2], q[1], q[3], q[4], q[2], q[4], zz};
+                        for (int k = 0; k < 9; k++) qdiag[9 * i + k] = d[k];
+                        for (int k = 0; k < 5; k++) q[k] = 0.0;
+                        zz = 0.0;
+                    } else if (PK == 5) {
+                        traced |= in;
+                    }
+                    put6(s, q, zz);
+                }
+            }
+        } else {
+#pragma unroll 1
+            for (int s = wave * (S / 4); s < (wave + 1) * (S / 4) && s < cnt; s++) {
+                const int64_t j = m.kidx[kb + s];
+                double q[9];
+                if constexpr (FAR32)
+                    block_Q_mixed<SYM, KIND>(mv, j, x, q);
+                else
+                    block_Q<R, SYM, KIND>(mv, j, x, q);
+                finish(s, j, q);
             }
         }
         if (run) {
             __syncthreads();
             OUT* base = Q + (RPE * (i0 - r0)) * ld + VPS * jb;
-            constexpr int U = TL::U, RP = 64 / U;  // rows per pass
-            constexpr int TR = RPE * 64;            // stored rows of a full tile
+            constexpr int U = TL::U, RP = 256 / U;  // rows per pass
+            constexpr int TR = RPE * 64;             // stored rows of a full tile
             if (cnt == S && nrow == 64 && ((VPS * jb * int64_t(sizeof(OUT))) & 7) == 0) {
                 // full tile: 8-byte units, RP rows of U units per pass, offsets
                 // in 32 bits from a uniform base (the tile spans < 2^32 bytes)
-                const int lr = lane / U, lc = lane - U * lr;
+                const int lr = threadIdx.x / U, lc = threadIdx.x - U * lr;
                 if (lr < RP) {
                     constexpr int WU = W / TL::EPU;
                     const uint64_t* src = reinterpret_cast<const uint64_t*>(tile);
@@ -203,9 +380,21 @@ __global__ __launch_bounds__(64) RH_ASM_ATTR void k_assemble(DevModel m, OUT* __
                     char* dst = reinterpret_cast<char*>(base);  // uniform, advanced per pass
                     const int64_t step = int64_t(RP) * ld * int64_t(sizeof(OUT));
                     const uint32_t off = uint32_t(lr) * uint32_t(ld * sizeof(OUT)) + uint32_t(8 * lc);
-                    constexpr int full = TR / RP;  // passes with every lane's row in the tile
-#pragma unroll 4
-                    for (int it = 0; it < full; it++) {
+                    constexpr int full = TR / RP;  // passes with every thread's row in the tile
+                    constexpr int G = full % 5 == 0 ? 5 : (full % 4 == 0 ? 4 : 3);  // reads in flight
+#pragma unroll 1
+                    for (int it = 0; it < full / G * G; it += G) {
+                        uint64_t u[G];
+#pragma unroll
+                        for (int k = 0; k < G; k++) u[k] = unit(lr + RP * (it + k));
+#pragma unroll
+                        for (int k = 0; k < G; k++) {
+                            *reinterpret_cast<uint64_t*>(dst + off) = u[k];
+                            dst += step;
+                        }
+                    }
+#pragma unroll
+                    for (int it = full / G * G; it < full; it++) {
                         *reinterpret_cast<uint64_t*>(dst + off) = unit(lr + RP * it);
                         dst += step;
                     }
@@ -214,9 +403,9 @@ __global__ __launch_bounds__(64) RH_ASM_ATTR void k_assemble(DevModel m, OUT* __
             } else {
                 // partial tile: the RPE*nrow stored rows, VPS*cnt values each
                 const int cols = VPS * cnt, total = RPE * nrow * cols;
-                const int step_r = 64 / cols, step_c = 64 - step_r * cols;
-                int r = lane / cols, c = lane - r * cols;
-                for (int e = lane; e < total; e += 64) {
+                const int step_r = 256 / cols, step_c = 256 - step_r * cols;
+                int r = threadIdx.x / cols, c = threadIdx.x - r * cols;
+                for (int e = threadIdx.x; e < total; e += 256) {
                     base[int64_t(r) * ld + c] = tile[TL::at(r, c)];
                     c += step_c;
                     r += step_r;
@@ -244,22 +433,22 @@ hipError_t asm_dispatch(const DevModel& m, OUT* Q, int64_t ld, double* qdiag, in
         // enough workgroups to fill 256 CUs several times over; column tiles
         // are whole LDS tiles
         constexpr int S = AsmTile<OUT, PK>::S;
-        const int64_t gy_target = std::max<int64_t>(1, (8192 + gx - 1) / gx);
+        const int64_t gy_target = std::max<int64_t>(1, (4096 + gx - 1) / gx);
         int64_t jt = std::max<int64_t>(4, (cnt + gy_target - 1) / gy_target);
         jt = std::min<int64_t>((jt + S - 1) / S * S, 256);
         const dim3 grid{unsigned(gx), unsigned((cnt + jt - 1) / jt), 1u};
         // FP32 storage: far blocks in FP32 arithmetic (general polyhedra stay FP64)
         constexpr bool mixed = sizeof(OUT) == 4;
         if (slot == 0 && mixed && far32)
-            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 0, mixed, PK>), grid, dim3(64), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
+            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 0, mixed, PK>), grid, dim3(256), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
         else if (slot == 0)
-            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 0, false, PK>), grid, dim3(64), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
+            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 0, false, PK>), grid, dim3(256), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
         else if (slot == 1 && mixed && far32)
-            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 1, mixed, PK>), grid, dim3(64), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
+            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 1, mixed, PK>), grid, dim3(256), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
         else if (slot == 1)
-            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 1, false, PK>), grid, dim3(64), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
+            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 1, false, PK>), grid, dim3(256), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
         else
-            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 2, false, PK>), grid, dim3(64), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
+            hipLaunchKernelGGL((k_assemble<double, SYM, ROWT, OUT, 2, false, PK>), grid, dim3(256), 0, s, m, Q, ld, qdiag, jt, r0, r1, flag);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -1931,6 +2120,16 @@ __global__ __launch_bounds__(256) void k_current(int64_t ns, const int32_t* __re
 }  // namespace
 
 // ---------------------------------------------------------------- launchers
+int64_t far_tet_doubles(int64_t ntet) { return kFarTet * ntet; }
+
+hipError_t launch_far_records(const DevModel& m, double* out, hipStream_t s)
+{
+    const int64_t ntet = m.koff[2] - m.koff[1];
+    if (ntet == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_far_records, dim3(unsigned((ntet + 255) / 256)), dim3(256), 0, s, m, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_assemble(const DevModel& m, void* Q, int elem_bytes, int64_t ld, double* qdiag,
                            int64_t r0, int64_t r1, hipStream_t s, bool far32, int planes, int32_t* flag)
 {
