@@ -11,7 +11,6 @@
 #include <array>
 #include <cmath>
 #include <cstring>
-#include <map>
 #include <utility>
 
 #include "rh_math.hpp"
@@ -154,41 +153,92 @@ void pack_tet(std::vector<Vec> V, std::vector<double>& d)
     }
 }
 
+// Ids of vertices, edges and faces in order of first occurrence:
+// open addressing over a table of ids at most half full, keys stored in id
+// order (no allocation per key).  The key's words are mixed by a multiplication
+// each.  Models are packed on every geometry change, so this is on the path of
+// a gradient step: with ordered maps and a vector per face the 1,000 polyhedra
+// of an undulator took 13 ms of one core here and take 3.4 ms (a step over them
+// 12.8 -> 7.8 ms).
+using VKey = std::array<uint64_t, 3>;   // bits of the coordinates
+using EKey = std::array<int32_t, 2>;    // ascending vertex ids
+using FKey = std::array<int32_t, 4>;    // ascending vertex ids, a triangle's first one -1
+inline uint64_t mix(uint64_t h, uint64_t w)
+{
+    h = (h ^ w) * 0x9E3779B97F4A7C15ull;
+    return h ^ (h >> 29);
+}
+inline uint64_t word2(int32_t a, int32_t b) { return (uint64_t(uint32_t(a)) << 32) | uint32_t(b); }
+inline uint64_t hash_key(const VKey& k) { return mix(mix(mix(1, k[0]), k[1]), k[2]); }
+inline uint64_t hash_key(const EKey& k) { return mix(1, word2(k[0], k[1])); }
+inline uint64_t hash_key(const FKey& k) { return mix(mix(1, word2(k[0], k[1])), word2(k[2], k[3])); }
+
+template <class Key>
+class IdMap {
+public:
+    explicit IdMap(size_t expect)
+    {
+        keys_.reserve(expect);
+        size_t n = 16;
+        while (n < 2 * expect) n *= 2;
+        slot_.assign(n, -1);
+    }
+    // id of the key, a new one if it is not there
+    int32_t add(const Key& k)
+    {
+        size_t i = place(k);
+        if (slot_[i] >= 0) return slot_[i];
+        if (2 * (keys_.size() + 1) > slot_.size()) {
+            slot_.assign(2 * slot_.size(), -1);
+            for (size_t q = 0; q < keys_.size(); q++) slot_[place(keys_[q])] = int32_t(q);
+            i = place(k);
+        }
+        keys_.push_back(k);
+        return slot_[i] = int32_t(keys_.size() - 1);
+    }
+    int32_t find(const Key& k) const { return slot_[place(k)]; }
+    size_t size() const { return keys_.size(); }
+    const Key& operator[](size_t id) const { return keys_[id]; }
+
+private:
+    size_t place(const Key& k) const
+    {
+        const size_t m = slot_.size() - 1;
+        size_t i = size_t(hash_key(k)) & m;
+        while (slot_[i] >= 0 && keys_[size_t(slot_[i])] != k) i = (i + 1) & m;
+        return i;
+    }
+    std::vector<Key> keys_;
+    std::vector<int32_t> slot_;
+};
+
+EKey ekey(int32_t a, int32_t b) { return {std::min(a, b), std::max(a, b)}; }
 void pack_gen(const std::vector<Vec>& V, const std::vector<Face>& F, std::vector<double>& d)
 {
     // unique undirected edges with their W
-    std::map<std::pair<int, int>, int> eid;
-    std::vector<std::pair<int, int>> edges;
+    size_t sides = 0;
+    for (const Face& f : F) sides += f.v.size();
+    IdMap<EKey> edges(sides / 2);
     std::vector<std::array<double, 6>> W;
+    W.reserve(sides / 2);
     for (const Face& f : F) {
         const size_t k = f.v.size();
         for (size_t i = 0; i < k; i++) {
             int p = f.v[i], q = f.v[(i + 1) % k];
-            auto key = std::make_pair(std::min(p, q), std::max(p, q));
-            auto it = eid.find(key);
-            int id;
-            if (it == eid.end()) {
-                id = int(edges.size());
-                eid[key] = id;
-                edges.push_back(key);
-                W.push_back({0, 0, 0, 0, 0, 0});
-            } else {
-                id = it->second;
-            }
+            const size_t id = size_t(edges.add(ekey(p, q)));
+            if (id == W.size()) W.push_back({0, 0, 0, 0, 0, 0});
             Vec tf = sub(V[q], V[p]);
             tf = scl(tf, 1.0 / nrm(tf));
             add_mn(W[id].data(), crs(tf, f.n), f.n);
         }
     }
-    int nfv = 0;
-    for (const Face& f : F) nfv += int(f.v.size());
     d.push_back(double(V.size()));
     d.push_back(double(edges.size()));
     d.push_back(double(F.size()));
-    d.push_back(double(nfv));
+    d.push_back(double(sides));
     for (const Vec& v : V) append(d, v);
     for (size_t e = 0; e < edges.size(); e++) {
-        int a = edges[e].first, b = edges[e].second;
+        int a = edges[e][0], b = edges[e][1];
         Vec t = sub(V[b], V[a]);
         double len = nrm(t);
         t = scl(t, 1.0 / len);
@@ -232,6 +282,10 @@ rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err)
     for (int64_t f = 0; f < nf_all; f++) fstart[f + 1] = fstart[f] + d->face_len[f];
     P.adj_off.assign(size_t(n + 1), 0);
     P.vert_off.assign(size_t(n + 1), 0);
+    // one element's vertices, faces and triangles, kept from element to element
+    std::vector<Vec> V;
+    std::vector<Face> F;
+    std::vector<double> tri;
     for (int64_t e = 0; e < n; e++) {
         P.off[e] = int64_t(P.data.size());
         P.adj_off[e] = int64_t(P.adj.size());
@@ -257,7 +311,7 @@ rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err)
             return RH_ERR_UNSUPPORTED;
         }
         const int64_t v0 = d->vert_off[e], v1 = d->vert_off[e + 1];
-        std::vector<Vec> V;
+        V.clear();
         for (int64_t v = v0; v < v1; v++)
             V.push_back({d->verts[3 * v], d->verts[3 * v + 1], d->verts[3 * v + 2]});
         // centroid: mean of the vertices in the order given
@@ -268,9 +322,10 @@ rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err)
         cent[3 * e + 1] = b * s.y;
         cent[3 * e + 2] = b * s.z;
         // faces of this element (face_idx is flat over all faces of all elements)
-        std::vector<Face> F;
+        F.resize(size_t(std::max<int64_t>(0, d->face_off[e + 1] - d->face_off[e])));
         for (int64_t f = d->face_off[e]; f < d->face_off[e + 1]; f++) {
-            Face fc;
+            Face& fc = F[size_t(f - d->face_off[e])];
+            fc.v.clear();
             if (d->face_len[f] < 3) {
                 *err = "face with fewer than 3 vertices";
                 return RH_ERR_GEOMETRY;
@@ -283,12 +338,11 @@ rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err)
                 }
                 fc.v.push_back(vi);
             }
-            F.push_back(fc);
         }
         rh_status st = orient_faces(V, F, err);
         if (st != RH_OK) return st;
         {
-            std::vector<double> tri;
+            tri.clear();
             for (const Face& f : F)
                 for (size_t k = 1; k + 1 < f.v.size(); k++) {
                     tri.push_back(double(f.v[0]));
@@ -394,7 +448,6 @@ rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err)
 }
 
 namespace {
-using VKey = std::array<uint64_t, 3>;
 
 VKey vkey(const double* v)
 {
@@ -403,52 +456,73 @@ VKey vkey(const double* v)
     return k;
 }
 
-// One polyhedron seen through its packed record: vertices, edges (vertex
-// pair and W6), faces (vertex loop CCW about the outward normal, n).
-struct ElemView {
-    int nv = 0;
-    const double* verts = nullptr;
-    std::vector<std::array<int, 2>> edges;
-    std::vector<const double*> edge_w;
-    std::vector<std::vector<int>> faces;
-    std::vector<const double*> face_n;
+// a face piece: its loop of 3 or 4 unique vertices
+struct Piece {
+    int32_t v[4];
+    int n;
+    FKey key() const
+    {
+        FKey k{-1, -1, -1, -1};
+        for (int i = 0; i < n; i++) k[size_t(i)] = v[i];
+        std::sort(k.begin(), k.end());
+        return k;
+    }
 };
 
-ElemView view_elem(const PackedModel& P, int64_t j)
-{
-    ElemView v;
-    const double* rec = P.data.data() + P.off[j];
-    if (P.kind[j] == EK_TET) {
-        v.nv = 4;
-        v.verts = rec;
-        for (int e = 0; e < 6; e++) {
-            v.edges.push_back({kTetEdgeA[e], kTetEdgeB[e]});
-            v.edge_w.push_back(rec + 12 + kTetEdge * e + 4);
-        }
-        for (int f = 0; f < 4; f++) {
-            v.faces.push_back({kTetFace[f][0], kTetFace[f][1], kTetFace[f][2]});
-            v.face_n.push_back(rec + 12 + 6 * kTetEdge + kTetFaceRec * f);
-        }
-        return v;
+// One polyhedron seen through its packed record: vertices, edges (vertex
+// pair and W6), faces (vertex loop CCW about the outward normal, n).  The
+// vertex numbers of all views stand in one array.
+struct Loop {
+    const int32_t* v;
+    size_t n;
+    size_t size() const { return n; }
+    int32_t operator[](size_t k) const { return v[k]; }
+};
+struct ElemView {
+    int nv, ne, nf;
+    const double* verts;
+    const double* w;  // W6 of edge 0, the next one ws further
+    int ws;
+    const double* fn;  // n of face 0, the next one fs further
+    int fs;
+    size_t at;  // in the array: vertex pairs, offsets of the nf loops and their end, loops
+    const double* edge_w(int e) const { return w + ws * e; }
+    const double* face_n(int f) const { return fn + fs * f; }
+    const int32_t* edge(const std::vector<int32_t>& a, int e) const { return &a[at + size_t(2 * e)]; }
+    Loop face(const std::vector<int32_t>& a, int f) const
+    {
+        const int32_t* o = &a[at + size_t(2 * ne + f)];
+        return {&a[at] + o[0], size_t(o[1] - o[0])};
     }
-    const int nv = int(rec[0]), ne = int(rec[1]), nf = int(rec[2]);
-    v.nv = nv;
-    v.verts = rec + kGenHdr;
-    const double* E = v.verts + 3 * nv;
+};
+
+ElemView view_elem(const PackedModel& P, int64_t j, std::vector<int32_t>& a)
+{
+    const double* rec = P.data.data() + P.off[j];
+    const size_t at = a.size();
+    if (P.kind[j] == EK_TET) {
+        for (int e = 0; e < 6; e++) {
+            a.push_back(kTetEdgeA[e]);
+            a.push_back(kTetEdgeB[e]);
+        }
+        for (int f = 0; f <= 4; f++) a.push_back(17 + 3 * f);
+        for (int f = 0; f < 4; f++) a.insert(a.end(), kTetFace[f], kTetFace[f] + 3);
+        return {4, 6, 4, rec, rec + 12 + 4, kTetEdge, rec + 12 + 6 * kTetEdge, kTetFaceRec, at};
+    }
+    const int nv = int(rec[0]), ne = int(rec[1]), nf = int(rec[2]), nfv = int(rec[3]);
+    const double* verts = rec + kGenHdr;
+    const double* E = verts + 3 * nv;
     const double* F = E + kGenEdge * ne;
     const double* fv = F + kGenFace * nf;
     for (int e = 0; e < ne; e++) {
-        v.edges.push_back({int(E[kGenEdge * e]), int(E[kGenEdge * e + 1])});
-        v.edge_w.push_back(E + kGenEdge * e + 6);
+        a.push_back(int32_t(E[kGenEdge * e]));
+        a.push_back(int32_t(E[kGenEdge * e + 1]));
     }
-    for (int f = 0; f < nf; f++) {
-        const double* fr = F + kGenFace * f;
-        std::vector<int> loop;
-        for (int k = 0; k < int(fr[4]); k++) loop.push_back(int(fv[int(fr[3]) + k]));
-        v.faces.push_back(loop);
-        v.face_n.push_back(fr);
-    }
-    return v;
+    const int32_t l0 = 2 * ne + nf + 1;
+    for (int f = 0; f < nf; f++) a.push_back(l0 + int32_t(F[kGenFace * f + 3]));
+    a.push_back(l0 + nfv);
+    for (int k = 0; k < nfv; k++) a.push_back(int32_t(fv[k]));
+    return {nv, ne, nf, verts, E + 6, kGenEdge, F, kGenFace, at};
 }
 }  // namespace
 
@@ -459,9 +533,11 @@ void build_mesh_form(PackedModel& P)
     if (P.kind_off[3] - P.kind_off[1] < 2) return;
     std::vector<int64_t> elems(P.kind_idx.begin() + P.kind_off[1], P.kind_idx.begin() + P.kind_off[3]);
     std::vector<ElemView> views;
+    std::vector<int32_t> nums;
+    views.reserve(elems.size());
     for (int64_t j : elems) {
-        views.push_back(view_elem(P, j));
-        if (int(views.back().faces.size()) > kMeshPlanes) return;
+        views.push_back(view_elem(P, j, nums));
+        if (views.back().nf > kMeshPlanes) return;
     }
     // Every element copy is a mesh element in the laboratory frame: copy c
     // maps points x -> M_c x + V_c and fields by F_c = s_c M_c (M_c
@@ -473,113 +549,118 @@ void build_mesh_form(PackedModel& P)
     // n, exactly.
     struct Inst {
         int32_t j;
-        const double* F;               // F_c, row-major
-        std::vector<double> verts;     // laboratory frame
-        std::vector<double> normals;   // laboratory frame, 3 per face
+        const double* cp;  // Minv, V, F_c (row-major)
         const ElemView* v;
     };
     std::vector<Inst> inst;
+    std::vector<double> corner;  // vertices of every element copy, laboratory frame
+    size_t pieces = 0;
     for (size_t q = 0; q < elems.size(); q++) {
         const int64_t j = elems[q];
         const ElemView& v = views[q];
         for (int64_t c = P.copy_off[size_t(j)]; c < P.copy_off[size_t(j) + 1]; c++) {
-            const double* cp = P.copies.data() + kCopySize * c;  // Minv, V, F
+            const double* cp = P.copies.data() + kCopySize * c;
             double Mc[9];
             inv3(cp, Mc);
-            Inst I;
-            I.j = int32_t(j);
-            I.F = cp + 12;
-            I.v = &v;
+            inst.push_back({int32_t(j), cp, &v});
+            for (int f = 0; f < v.nf; f++) pieces += (v.face(nums, f).size() - 1) / 2;
             for (int k = 0; k < v.nv; k++) {
                 const double* x = v.verts + 3 * k;
                 for (int r = 0; r < 3; r++)
                     // + 0.0: a vertex mirrored onto a symmetry plane gets +0, not -0,
                     // so that it keys equal to the original
-                    I.verts.push_back(Mc[3 * r] * x[0] + Mc[3 * r + 1] * x[1] + Mc[3 * r + 2] * x[2] + cp[9 + r] + 0.0);
+                    corner.push_back(Mc[3 * r] * x[0] + Mc[3 * r + 1] * x[1] + Mc[3 * r + 2] * x[2] + cp[9 + r] + 0.0);
             }
-            for (size_t f = 0; f < v.faces.size(); f++) {
-                const double* n = v.face_n[f];
-                double nl[3];
-                for (int r = 0; r < 3; r++) nl[r] = cp[r] * n[0] + cp[3 + r] * n[1] + cp[6 + r] * n[2];
-                const double ln = std::sqrt(nl[0] * nl[0] + nl[1] * nl[1] + nl[2] * nl[2]);
-                for (int r = 0; r < 3; r++) I.normals.push_back(nl[r] / ln);
-            }
-            inst.push_back(std::move(I));
         }
     }
-    std::map<VKey, int32_t> vid;
+    auto lab_normal = [](const Inst& I, int f) {
+        const double* n = I.v->face_n(f);
+        std::array<double, 3> nl;
+        for (size_t r = 0; r < 3; r++) nl[r] = I.cp[r] * n[0] + I.cp[3 + r] * n[1] + I.cp[6 + r] * n[2];
+        const double ln = std::sqrt(nl[0] * nl[0] + nl[1] * nl[1] + nl[2] * nl[2]);
+        for (double& x : nl) x /= ln;
+        return nl;
+    };
+    // unique vertices of every element copy, then the unique faces: the
+    // regrouped sweep pays off only when faces are shared (a face evaluated on
+    // its own recomputes the vertex distances the per-element sweep shares
+    // between the faces of an element), so a model that shares few of them
+    // stops here, before its edges are looked at
+    const size_t corners = corner.size() / 3;
+    IdMap<VKey> vid(corners);
     std::vector<const double*> vpos;
-    std::map<std::pair<int32_t, int32_t>, int64_t> eid;
+    std::vector<int32_t> corner_id(corners);
+    for (size_t k = 0; k < corners; k++) {
+        corner_id[k] = vid.add(vkey(&corner[3 * k]));
+        if (size_t(corner_id[k]) == vpos.size()) vpos.push_back(&corner[3 * k]);
+    }
+    // the pieces of a face: polygons of more than 4 vertices become fan
+    // pieces of at most 4
+    auto face_piece = [](const Loop& loop, size_t t, const int32_t* u) {
+        Piece p{{u[loop[0]], u[loop[t + 1]], u[loop[t + 2]], -1}, 3};
+        if (t + 3 < loop.size()) p.v[p.n++] = u[loop[t + 3]];
+        return p;
+    };
+    IdMap<FKey> fid(pieces);
+    std::vector<int32_t> piece_id;  // of every face piece, in the order walked
+    piece_id.reserve(pieces);
+    {
+        const int32_t* u = corner_id.data();
+        for (const Inst& I : inst) {
+            for (int f = 0; f < I.v->nf; f++) {
+                const Loop loop = I.v->face(nums, f);
+                for (size_t t = 0; t + 2 < loop.size(); t += 2)
+                    piece_id.push_back(fid.add(face_piece(loop, t, u).key()));
+            }
+            u += I.v->nv;
+        }
+    }
+    if (double(fid.size()) > 0.8 * double(pieces)) return;
+    IdMap<EKey> eid(2 * fid.size());
     std::vector<std::vector<std::pair<int32_t, std::array<double, 9>>>> einc;
-    std::map<std::vector<int32_t>, int64_t> fid;
-    std::vector<std::vector<std::pair<int32_t, std::array<double, 3>>>> finc;
-    std::vector<std::vector<int32_t>> floop;  // unique-vertex loop of the first incidence
-    std::vector<const double*> fnorm;
+    std::vector<std::vector<std::pair<int32_t, std::array<double, 3>>>> finc(fid.size());
+    std::vector<Piece> floop(fid.size(), Piece{{0, 0, 0, 0}, 0});  // loop of the first incidence
+    std::vector<std::array<double, 3>> fnorm(fid.size());
+    const int32_t* u = corner_id.data();
+    const int32_t* pid = piece_id.data();
     for (const Inst& I : inst) {
         const ElemView& v = *I.v;
-        const double* F = I.F;
-        std::vector<int32_t> u(size_t(v.nv));
-        for (int k = 0; k < v.nv; k++) {
-            const double* x = I.verts.data() + 3 * k;
-            auto it = vid.find(vkey(x));
-            if (it == vid.end()) {
-                it = vid.emplace(vkey(x), int32_t(vpos.size())).first;
-                vpos.push_back(x);
-            }
-            u[size_t(k)] = it->second;
-        }
-        for (size_t e = 0; e < v.edges.size(); e++) {
-            int32_t a = u[size_t(v.edges[e][0])], b = u[size_t(v.edges[e][1])];
-            auto key = std::make_pair(std::min(a, b), std::max(a, b));
-            auto it = eid.find(key);
-            if (it == eid.end()) {
-                it = eid.emplace(key, int64_t(einc.size())).first;
-                einc.emplace_back();
-            }
+        const double* F = I.cp + 12;
+        for (int e = 0; e < v.ne; e++) {
+            const int32_t* ab = v.edge(nums, e);
+            const size_t id = size_t(eid.add(ekey(u[ab[0]], u[ab[1]])));
+            if (id == einc.size()) einc.emplace_back();
             // F W with W symmetric (xx yy zz xy xz yz)
-            const double* w = v.edge_w[e];
+            const double* w = v.edge_w(e);
             const double W[9] = {w[0], w[3], w[4], w[3], w[1], w[5], w[4], w[5], w[2]};
             std::array<double, 9> FW;
             for (int r = 0; r < 3; r++)
                 for (int c = 0; c < 3; c++)
                     FW[size_t(3 * r + c)] = F[3 * r] * W[c] + F[3 * r + 1] * W[3 + c] + F[3 * r + 2] * W[6 + c];
-            einc[size_t(it->second)].push_back({I.j, FW});
+            einc[id].push_back({I.j, FW});
         }
-        for (size_t f = 0; f < v.faces.size(); f++) {
-            const std::vector<int>& loop = v.faces[f];
-            const double* n1 = I.normals.data() + 3 * f;
-            // polygons of more than 4 vertices become fan pieces of at most 4
+        for (int f = 0; f < v.nf; f++) {
+            const Loop loop = v.face(nums, f);
+            const std::array<double, 3> n1 = lab_normal(I, f);
             for (size_t s = 0; s + 2 < loop.size(); s += 2) {
-                std::vector<int32_t> piece{u[size_t(loop[0])], u[size_t(loop[s + 1])],
-                                           u[size_t(loop[s + 2])]};
-                if (s + 3 < loop.size()) piece.push_back(u[size_t(loop[s + 3])]);
-                std::vector<int32_t> key = piece;
-                std::sort(key.begin(), key.end());
-                auto it = fid.find(key);
+                const size_t id = size_t(*pid++);
                 double sign = 1.0;
-                if (it == fid.end()) {
-                    it = fid.emplace(key, int64_t(finc.size())).first;
-                    finc.emplace_back();
-                    floop.push_back(piece);
-                    fnorm.push_back(n1);
+                if (floop[id].n == 0) {
+                    floop[id] = face_piece(loop, s, u);
+                    fnorm[id] = n1;
                 } else {
-                    const double* n0 = fnorm[size_t(it->second)];
+                    const std::array<double, 3>& n0 = fnorm[id];
                     sign = (n0[0] * n1[0] + n0[1] * n1[1] + n0[2] * n1[2] > 0) ? 1.0 : -1.0;
                 }
                 // sign F^T n of the unique face's normal n
-                const double* n = fnorm[size_t(it->second)];
+                const std::array<double, 3>& n = fnorm[id];
                 std::array<double, 3> gv;
                 for (int c = 0; c < 3; c++) gv[size_t(c)] = sign * (F[c] * n[0] + F[3 + c] * n[1] + F[6 + c] * n[2]);
-                finc[size_t(it->second)].push_back({I.j, gv});
+                finc[id].push_back({I.j, gv});
             }
         }
+        u += v.nv;
     }
-    // the regrouped sweep pays off only when faces are shared: a face
-    // evaluated on its own recomputes the vertex distances the per-element
-    // sweep shares between the faces of an element
-    int64_t face_incidences = 0;
-    for (const auto& f : finc) face_incidences += int64_t(f.size());
-    if (double(finc.size()) > 0.8 * double(face_incidences)) return;
     // Edge paths: each unique edge oriented and ordered so that, where a path
     // continues, its first vertex is the previous edge's second vertex (L_e
     // and W_e do not depend on the orientation).  Triangle strips: where a
@@ -588,58 +669,67 @@ void build_mesh_form(PackedModel& P)
     // the order of its vertices once the normal is fixed).  The sweeps then
     // compute one vertex distance per continued edge or triangle.
     std::vector<int32_t> forder;
-    std::vector<std::vector<int32_t>> fverts;
+    std::vector<Piece> fverts;
     std::vector<char> fcont;
     {
-        std::map<std::pair<int32_t, int32_t>, std::vector<int32_t>> tri_at;
-        for (size_t f = 0; f < floop.size(); f++) {
-            if (floop[f].size() != 3) continue;
-            for (int k = 0; k < 3; k++) {
-                const int32_t a = floop[f][size_t(k)], b = floop[f][size_t((k + 1) % 3)];
-                tri_at[{std::min(a, b), std::max(a, b)}].push_back(int32_t(f));
+        // triangles, or quadrilaterals, on each side of a face piece (a
+        // diagonal of a fanned polygon is a side without being an edge)
+        IdMap<EKey> sid(2 * fid.size());
+        std::vector<std::vector<int32_t>> tri_at, quad_at;
+        auto at = [&](const std::vector<std::vector<int32_t>>& m, int32_t a, int32_t b) -> const std::vector<int32_t>* {
+            const int32_t id = sid.find(ekey(a, b));
+            return id < 0 ? nullptr : &m[size_t(id)];
+        };
+        for (size_t f = 0; f < floop.size(); f++)
+            for (int k = 0; k < floop[f].n; k++) {
+                const size_t id = size_t(sid.add(ekey(floop[f].v[k], floop[f].v[(k + 1) % floop[f].n])));
+                if (id == tri_at.size()) {
+                    tri_at.emplace_back();
+                    quad_at.emplace_back();
+                }
+                (floop[f].n == 3 ? tri_at : quad_at)[id].push_back(int32_t(f));
             }
-        }
         std::vector<char> used(floop.size(), 0);
         auto other = [&](int32_t a, int32_t b) -> int32_t {
-            auto it = tri_at.find({std::min(a, b), std::max(a, b)});
-            if (it == tri_at.end()) return -1;
-            for (int32_t g : it->second)
+            const std::vector<int32_t>* l = at(tri_at, a, b);
+            if (!l) return -1;
+            for (int32_t g : *l)
                 if (!used[size_t(g)]) return g;
             return -1;
         };
         for (size_t f0 = 0; f0 < floop.size(); f0++) {
-            if (used[f0] || floop[f0].size() != 3) continue;
-            std::vector<int32_t> v = floop[f0];
+            if (used[f0] || floop[f0].n != 3) continue;
+            Piece w = floop[f0];
+            int32_t* v = w.v;
             used[f0] = 1;
             // start with the rotation whose last edge continues the strip
             for (int r = 0; r < 3; r++) {
                 if (other(v[1], v[2]) >= 0) break;
-                std::rotate(v.begin(), v.begin() + 1, v.end());
+                std::rotate(v, v + 1, v + 3);
             }
             forder.push_back(int32_t(f0));
-            fverts.push_back(v);
+            fverts.push_back(w);
             fcont.push_back(0);
             // among the triangles on (p, q), take one whose far edge (q, r)
             // still continues the strip, preferring the one with the fewest
             // continuations (strip starts on the C-yoke: 13 % -> 9 %)
             auto third = [&](int32_t g, int32_t a, int32_t b) {
                 int32_t r = -1;
-                for (int32_t x : floop[size_t(g)])
+                for (int32_t x : {floop[size_t(g)].v[0], floop[size_t(g)].v[1], floop[size_t(g)].v[2]})
                     if (x != a && x != b) r = x;
                 return r;
             };
             auto next = [&](int32_t a, int32_t b) -> int32_t {
-                auto it = tri_at.find({std::min(a, b), std::max(a, b)});
-                if (it == tri_at.end()) return -1;
+                const std::vector<int32_t>* l = at(tri_at, a, b);
+                if (!l) return -1;
                 int32_t best = -1;
                 int best_n = 0;
-                for (int32_t g : it->second) {
+                for (int32_t g : *l) {
                     if (used[size_t(g)]) continue;
                     const int32_t r = third(g, a, b);
                     int n = 0;
-                    auto jt = tri_at.find({std::min(b, r), std::max(b, r)});
-                    if (jt != tri_at.end())
-                        for (int32_t h : jt->second)
+                    if (const std::vector<int32_t>* m = at(tri_at, b, r))
+                        for (int32_t h : *m)
                             if (h != g && !used[size_t(h)]) n++;
                     // score: continuing candidates first, then fewer continuations
                     const bool better = best < 0 || (n > 0 && (best_n == 0 || n < best_n));
@@ -655,7 +745,7 @@ void build_mesh_form(PackedModel& P)
                 used[size_t(g)] = 1;
                 const int32_t r = third(g, p, q);
                 forder.push_back(g);
-                fverts.push_back({p, q, r});
+                fverts.push_back({{p, q, r, -1}, 3});
                 fcont.push_back(1);
                 p = q;
                 q = r;
@@ -665,48 +755,41 @@ void build_mesh_form(PackedModel& P)
         // Quadrilateral strips: where a strip continues, a quadrilateral's
         // first two vertices are the previous one's last two, its loop read
         // from there in either direction.
-        std::map<std::pair<int32_t, int32_t>, std::vector<int32_t>> quad_at;
-        for (size_t f = 0; f < floop.size(); f++) {
-            if (floop[f].size() != 4) continue;
-            for (int k = 0; k < 4; k++) {
-                const int32_t a = floop[f][size_t(k)], b = floop[f][size_t((k + 1) % 4)];
-                quad_at[{std::min(a, b), std::max(a, b)}].push_back(int32_t(f));
-            }
-        }
         auto next_quad = [&](int32_t a, int32_t b) -> int32_t {
-            auto it = quad_at.find({std::min(a, b), std::max(a, b)});
-            if (it == quad_at.end()) return -1;
-            for (int32_t g : it->second)
+            const std::vector<int32_t>* l = at(quad_at, a, b);
+            if (!l) return -1;
+            for (int32_t g : *l)
                 if (!used[size_t(g)]) return g;
             return -1;
         };
         for (size_t f0 = 0; f0 < floop.size(); f0++) {
-            if (used[f0] || floop[f0].size() != 4) continue;
-            std::vector<int32_t> v = floop[f0];
+            if (used[f0] || floop[f0].n != 4) continue;
+            Piece w = floop[f0];
+            int32_t* v = w.v;
             used[f0] = 1;
             // start with the rotation whose side (v2, v3) continues the strip
             for (int r = 0; r < 4; r++) {
                 if (next_quad(v[2], v[3]) >= 0) break;
-                std::rotate(v.begin(), v.begin() + 1, v.end());
+                std::rotate(v, v + 1, v + 4);
             }
             forder.push_back(int32_t(f0));
-            fverts.push_back(v);
+            fverts.push_back(w);
             fcont.push_back(2);  // quadrilateral
             int32_t p = v[2], q = v[3];
             for (int32_t g = next_quad(p, q); g >= 0; g = next_quad(p, q)) {
                 used[size_t(g)] = 1;
-                const std::vector<int32_t>& l = floop[size_t(g)];
+                const int32_t* l = floop[size_t(g)].v;
                 int i = 0;
-                while (l[size_t(i)] != p) i++;
+                while (l[i] != p) i++;
                 // around the loop from p through q
-                const int dir = (l[size_t((i + 1) % 4)] == q) ? 1 : 3;
-                std::vector<int32_t> w(4);
-                for (int k = 0; k < 4; k++) w[size_t(k)] = l[size_t((i + dir * k) % 4)];
+                const int dir = (l[(i + 1) % 4] == q) ? 1 : 3;
+                Piece x{{0, 0, 0, 0}, 4};
+                for (int k = 0; k < 4; k++) x.v[k] = l[(i + dir * k) % 4];
                 forder.push_back(g);
-                fverts.push_back(w);
+                fverts.push_back(x);
                 fcont.push_back(3);  // quadrilateral continuing the strip
-                p = w[2];
-                q = w[3];
+                p = x.v[2];
+                q = x.v[3];
             }
         }
         for (size_t f = 0; f < floop.size(); f++)
@@ -720,52 +803,49 @@ void build_mesh_form(PackedModel& P)
     // sweep order that has it (a triangle any of its sides, a quadrilateral
     // its sides (v0,v1), (v1,v2), (v2,v3)): that face's sweep step already
     // holds both vertex offsets, distances and their dot product.
-    std::vector<std::pair<int32_t, int32_t>> ekeys(einc.size());
-    for (const auto& kv : eid) ekeys[size_t(kv.second)] = kv.first;
     std::vector<int64_t> owner(einc.size(), -1);  // 3 * face position + side
     for (size_t o = 0; o < forder.size(); o++) {
-        const size_t nv = fverts[o].size();
+        const Piece& p = fverts[o];
         for (int k = 0; k < 3; k++) {
-            const int32_t a = fverts[o][size_t(k)], b = fverts[o][size_t(k + 1) % nv];
-            const auto it = eid.find({std::min(a, b), std::max(a, b)});
-            if (it == eid.end()) continue;  // a diagonal of a fanned polygon
-            if (owner[size_t(it->second)] < 0) owner[size_t(it->second)] = int64_t(3 * o + k);
+            const int32_t e = eid.find(ekey(p.v[k], p.v[(k + 1) % p.n]));
+            if (e < 0) continue;  // a diagonal of a fanned polygon
+            if (owner[size_t(e)] < 0) owner[size_t(e)] = int64_t(3 * o + k);
         }
     }
     std::vector<int32_t> eorder;
     std::vector<char> eflip, econt;
     {
         std::vector<std::vector<int32_t>> vadj(vpos.size());
-        for (size_t e = 0; e < ekeys.size(); e++) {
-            vadj[size_t(ekeys[e].first)].push_back(int32_t(e));
-            vadj[size_t(ekeys[e].second)].push_back(int32_t(e));
+        for (size_t e = 0; e < eid.size(); e++) {
+            vadj[size_t(eid[e][0])].push_back(int32_t(e));
+            vadj[size_t(eid[e][1])].push_back(int32_t(e));
         }
-        std::vector<char> used(ekeys.size(), 0);
+        std::vector<char> used(eid.size(), 0);
         std::vector<size_t> next(vpos.size(), 0);
         auto take = [&](int32_t v) -> int32_t {
             std::vector<int32_t>& a = vadj[size_t(v)];
             while (next[size_t(v)] < a.size() && used[size_t(a[next[size_t(v)]])]) next[size_t(v)]++;
             return next[size_t(v)] < a.size() ? a[next[size_t(v)]] : -1;
         };
-        for (size_t e = 0; e < ekeys.size(); e++)
+        for (size_t e = 0; e < eid.size(); e++)
             if (owner[e] >= 0) used[e] = 1;  // evaluated by its face
-        for (size_t e0 = 0; e0 < ekeys.size(); e0++) {
+        for (size_t e0 = 0; e0 < eid.size(); e0++) {
             if (used[e0]) continue;
-            int32_t cur = ekeys[e0].first, e = int32_t(e0);
+            int32_t cur = eid[e0][0], e = int32_t(e0);
             bool first = true;
             while (e >= 0) {
                 used[size_t(e)] = 1;
-                const bool flip = ekeys[size_t(e)].first != cur;
+                const bool flip = eid[size_t(e)][0] != cur;
                 eorder.push_back(e);
                 eflip.push_back(flip ? 1 : 0);
                 econt.push_back(first ? 0 : 1);
                 first = false;
-                cur = flip ? ekeys[size_t(e)].first : ekeys[size_t(e)].second;
+                cur = flip ? eid[size_t(e)][0] : eid[size_t(e)][1];
                 e = take(cur);
             }
         }
         M.ne_free = int64_t(eorder.size());
-        for (size_t e = 0; e < ekeys.size(); e++)
+        for (size_t e = 0; e < eid.size(); e++)
             if (owner[e] >= 0) {
                 eorder.push_back(int32_t(e));
                 eflip.push_back(0);
@@ -776,8 +856,8 @@ void build_mesh_form(PackedModel& P)
     M.edge_inc_off.push_back(0);
     for (size_t o = 0; o < eorder.size(); o++) {
         const size_t e = size_t(eorder[o]);
-        const double* a = vpos[size_t(eflip[o] ? ekeys[e].second : ekeys[e].first)];
-        const double* b = vpos[size_t(eflip[o] ? ekeys[e].first : ekeys[e].second)];
+        const double* a = vpos[size_t(eflip[o] ? eid[e][1] : eid[e][0])];
+        const double* b = vpos[size_t(eflip[o] ? eid[e][0] : eid[e][1])];
         double t[3] = {b[0] - a[0], b[1] - a[1], b[2] - a[2]};
         const double len = std::sqrt(t[0] * t[0] + t[1] * t[1] + t[2] * t[2]);
         for (int k = 0; k < 3; k++) t[k] /= len;
@@ -802,11 +882,11 @@ void build_mesh_form(PackedModel& P)
     M.face_inc_off.push_back(0);
     for (size_t o = 0; o < forder.size(); o++) {
         const size_t f = size_t(forder[o]);
-        const std::vector<int32_t>& loop = fverts[o];
-        const double* n = fnorm[f];
+        const Piece& loop = fverts[o];
+        const std::array<double, 3>& n = fnorm[f];
         double vv[4][3] = {{0}};
-        for (size_t k = 0; k < loop.size(); k++)
-            for (int c = 0; c < 3; c++) vv[k][c] = vpos[size_t(loop[k])][c];
+        for (int k = 0; k < loop.n; k++)
+            for (int c = 0; c < 3; c++) vv[k][c] = vpos[size_t(loop.v[k])][c];
         auto area2 = [&](int i0, int i1, int i2) {
             const double e1[3] = {vv[i1][0] - vv[i0][0], vv[i1][1] - vv[i0][1], vv[i1][2] - vv[i0][2]};
             const double e2[3] = {vv[i2][0] - vv[i0][0], vv[i2][1] - vv[i0][1], vv[i2][2] - vv[i0][2]};
@@ -816,10 +896,10 @@ void build_mesh_form(PackedModel& P)
         };
         for (int k = 0; k < 4; k++)
             for (int c = 0; c < 3; c++) M.face_geo.push_back(vv[k][c]);
-        for (int c = 0; c < 3; c++) M.face_geo.push_back(n[c]);
+        for (int c = 0; c < 3; c++) M.face_geo.push_back(n[size_t(c)]);
         M.face_geo.push_back(area2(0, 1, 2));
-        M.face_geo.push_back(loop.size() > 3 ? area2(0, 2, 3) : 0.0);
-        M.face_geo.push_back(double(loop.size()));
+        M.face_geo.push_back(loop.n > 3 ? area2(0, 2, 3) : 0.0);
+        M.face_geo.push_back(double(loop.n));
         M.face_cont.push_back(double(fcont[o]));
         for (const auto& inc : finc[f]) {
             M.face_inc_elem.push_back(inc.first);
@@ -828,32 +908,38 @@ void build_mesh_form(PackedModel& P)
         M.face_inc_off.push_back(int64_t(M.face_inc_elem.size()));
     }
     // inside records (one per element copy, with its field transform) and tile boxes
-    for (const Inst& I : inst) {
+    const double* x = corner.data();
+    double lo[3], hi[3];
+    for (size_t q = 0; q < inst.size(); q++) {
+        const Inst& I = inst[q];
         const ElemView& v = *I.v;
         M.in_elem.push_back(I.j);
-        for (int k = 0; k < 9; k++) M.in_F.push_back(I.F[k]);
-        M.in_geo.push_back(double(v.faces.size()));
+        for (int k = 0; k < 9; k++) M.in_F.push_back(I.cp[12 + k]);
+        M.in_geo.push_back(double(v.nf));
         for (int f = 0; f < kMeshPlanes; f++) {
-            if (f < int(v.faces.size())) {
-                const double* n = I.normals.data() + 3 * f;
-                const double* p0 = I.verts.data() + 3 * v.faces[size_t(f)][0];
-                for (int c = 0; c < 3; c++) M.in_geo.push_back(n[c]);
+            if (f < v.nf) {
+                const std::array<double, 3> n = lab_normal(I, f);
+                const double* p0 = x + 3 * v.face(nums, f)[0];
+                M.in_geo.insert(M.in_geo.end(), n.begin(), n.end());
                 M.in_geo.push_back(n[0] * p0[0] + n[1] * p0[1] + n[2] * p0[2]);
             } else {
                 for (int c = 0; c < 4; c++) M.in_geo.push_back(0.0);
             }
         }
-    }
-    for (size_t t0 = 0; t0 < inst.size(); t0 += kMeshTile) {
-        double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-        for (size_t q = t0; q < std::min(inst.size(), t0 + kMeshTile); q++)
-            for (int k = 0; k < inst[q].v->nv; k++)
-                for (int c = 0; c < 3; c++) {
-                    lo[c] = std::min(lo[c], inst[q].verts[size_t(3 * k + c)]);
-                    hi[c] = std::max(hi[c], inst[q].verts[size_t(3 * k + c)]);
-                }
-        for (int c = 0; c < 3; c++) M.tile_box.push_back(lo[c]);
-        for (int c = 0; c < 3; c++) M.tile_box.push_back(hi[c]);
+        if (q % kMeshTile == 0)
+            for (int c = 0; c < 3; c++) {
+                lo[c] = INFINITY;
+                hi[c] = -INFINITY;
+            }
+        for (int k = 0; k < v.nv; k++, x += 3)
+            for (int c = 0; c < 3; c++) {
+                lo[c] = std::min(lo[c], x[c]);
+                hi[c] = std::max(hi[c], x[c]);
+            }
+        if (q % kMeshTile == kMeshTile - 1 || q + 1 == inst.size()) {
+            M.tile_box.insert(M.tile_box.end(), lo, lo + 3);
+            M.tile_box.insert(M.tile_box.end(), hi, hi + 3);
+        }
     }
     M.active = true;
 }
