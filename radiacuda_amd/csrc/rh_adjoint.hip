@@ -3,13 +3,14 @@
 // matrix pass and the per-element update of the linear-material adjoint
 // relaxation.
 //
-// Mapping: as in the forward field sweep, each lane owns one observation
-// point and every lane of the workgroup visits the same source elements
-// (wave-uniform records).  A lane's contribution to an element (or vertex)
-// gradient is summed over the wavefront with cross-lane shuffles and
-// accumulated per wave in LDS; each workgroup writes one partial per element
-// slot and a second kernel sums the partials in a fixed order, so gradients
-// are deterministic.
+// Mapping of dL/dM: as in the forward field sweep, each lane owns one
+// observation point and every lane of the workgroup visits the same source
+// elements (wave-uniform records); a lane's contribution to an element is
+// summed over the wavefront with cross-lane shuffles and accumulated per wave
+// in LDS.  dL/d(vertex) has it the other way round: a lane owns a triangle and
+// visits the block's points.  In both, each workgroup writes one partial per
+// element or vertex and a second kernel sums the partials in a fixed order, so
+// gradients are deterministic.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,21 +32,24 @@ __device__ __forceinline__ double wsum(double v)
     return v;
 }
 
-constexpr int kAdjSliceE = 64;   // elements per workgroup slice (dL/dM)
+constexpr int kAdjSliceE = 64;   // elements per workgroup slice (dL/dM), at most
 constexpr int kAdjSliceV = 128;  // vertices per workgroup slice (dL/dvertex)
 
 // dL/dM partials: part[bx][j][3] for the elements of slice blockIdx.y.
+// FP64-issue bound where the blocks fill the chip: 1,000 hexahedra at 2,048
+// points, 8 tiles, 279 us in 1,000 blocks of 8 elements and 816 us in 128
+// blocks of 64.
 template <bool SYM>
 __global__ __launch_bounds__(256) void k_adj_m(DevModel m, const double* __restrict__ pts,
                                                int64_t np, const double* __restrict__ g,
-                                               int addin, double* __restrict__ part)
+                                               int addin, int slice, double* __restrict__ part)
 {
     __shared__ double acc[4][kAdjSliceE * 3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < 4 * kAdjSliceE * 3; i += 256) (&acc[0][0])[i] = 0.0;
     __syncthreads();
-    const int64_t j0 = int64_t(blockIdx.y) * kAdjSliceE;
-    const int64_t j1 = (j0 + kAdjSliceE < m.n) ? (j0 + kAdjSliceE) : m.n;
+    const int64_t j0 = int64_t(blockIdx.y) * slice;
+    const int64_t j1 = (j0 + slice < m.n) ? (j0 + slice) : m.n;
     const int64_t tiles = (np + 255) / 256;
     for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         const int64_t p = tile * 256 + threadIdx.x;
@@ -92,82 +96,282 @@ __global__ __launch_bounds__(256) void k_adj_m(DevModel m, const double* __restr
         part[int64_t(blockIdx.x) * 3 * m.n + 3 * j0 + i] = acc[0][i] + acc[1][i] + acc[2][i] + acc[3][i];
 }
 
+// (1 - asinh(s)/s)/s^2 on s^2 <= 1/100 by powers of s^2: Chebyshev interpolant
+// fitted at 60 digits, within 6e-17 relative
+__constant__ double d_asinh_p[6] = {0.16666666666666666, -0.0749999999999521,   0.04464285708693904,
+                                    -0.030381920556719857, 0.02236754133836989, -0.016940234967509307};
+
+// One triangle's part of dL/dvertex: geometry that does not depend on the
+// observation point, and the sums over points.
+struct TriLane {
+    V3<double> v[3];  // corners, element frame
+    V3<double> n, t[3];
+    double len[3], il[3], ia, sigma;  // side lengths and reciprocals, 1/(2 area), n . M
+    V3<double> M;
+    V3<double> G[3];  // per corner: terms of L and of the solid angle
+    V3<double> N;     // adjoint of the unit normal
+    double al[3];     // per side: adjoint of its direction's own component
+};
+
+__device__ __forceinline__ V3<double> axpy(double a, const V3<double>& x, const V3<double>& y)
+{
+    return V3<double>{fma(a, x.x, y.x), fma(a, x.y, y.y), fma(a, x.z, y.z)};
+}
+
+// Derivatives of f = g . 4 pi H_t at one point, in closed form.  With
+// m = sigma n x g, S = sum_e L_e t_e and u -> w the side e,
+//     f = sigma (S . (n x g) - Omega n . g),
+//     D = Ru Rw + u . w,  L = asinh(len (Ru + Rw)/D),
+//     dL/dlen = (Ru + Rw)/D,  dL/dRu = dL/dRw = -len/D,
+//     dOmega/dw = -(u x w)/(Rw D) per side (both ends alike, by 1/Ru, 1/Rw),
+// the last because the solid angle changes by the area that a moved side
+// sweeps, int s/r^3 = 1/(Rw D) along it.  No term needs a derivative of a
+// logarithm's or an arctangent's argument.  Sums over points are taken of the
+// differences between a corner's two sides, never of the sides' own terms,
+// which are larger by distance over size.  gx: minus the sum of the corner
+// derivatives (the normal's and the directions' parts cancel in it).
+__device__ __forceinline__ void tri_point(TriLane& T, const double x[3], const V3<double>& g, V3<double>& gx)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    V3<double> r[3];
+    double R[3], iR[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        r[k] = V3<double>{T.v[k].x - x[0], T.v[k].y - x[1], T.v[k].z - x[2]};
+        // R and 1/R from one seed y: with q = R^2 y and e = 1 - q y both are
+        // the seed's value times 1 + e/2 + 3 e^2/8
+        const double d = dot(r[k], r[k]);
+        const double y = __builtin_amdgcn_rsq(d);
+        const double q = d * y, e = fma(-q, y, 1.0), c = e * fma(e, 0.375, 0.5);
+        R[k] = fma(q, c, q);
+        iR[k] = fma(y, c, y);
+    }
+    const V3<double> ng = cross(T.n, g);
+    const double gn = dot(T.n, g), sgn = T.sigma * gn;
+    V3<double> X[3], S{0.0, 0.0, 0.0};
+    double uw[3], iD[3], sd[3], s2[3], w1[3], k1[3];
+#pragma unroll
+    for (int e = 0; e < 3; e++) {
+        const int f = (e + 1) % 3;
+        X[e] = cross(r[e], r[f]);
+        uw[e] = dot(r[e], r[f]);
+        const double RR = R[e] * R[f];
+        double D = RR + uw[e];
+        // beyond a right angle the sum cancels: |u x w|^2 = (RR - u.w) D
+        if (uw[e] < 0.0) D = dot(X[e], X[e]) * rh_rcp(RR - uw[e]);
+        iD[e] = rh_rcp(D);
+        sd[e] = (R[e] + R[f]) * iD[e];
+        const double s = T.len[e] * sd[e];
+        s2[e] = s * s;
+    }
+    // w1 = sd - L/len and k1 = L/len: where every lane's sides are short
+    // against their distance by the series, which loses no digits in w1
+    if (rh_all(fmax(fmax(s2[0], s2[1]), s2[2]) <= 0.01)) {
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+            double p = d_asinh_p[5];
+#pragma unroll
+            for (int i = 4; i >= 0; i--) p = fma(p, s2[e], d_asinh_p[i]);
+            w1[e] = sd[e] * s2[e] * p;
+            k1[e] = sd[e] - w1[e];
+        }
+    } else {
+        RH_KEEP_BRANCH();
+        const CoefPtr c = rh_coef_rare(d_log_p);
+#pragma unroll
+        for (int e = 0; e < 3; e++) {
+            // len s = sinh L: e^L = (Ru + Rw + len)^2 / (2 D)
+            const double q = R[e] + R[(e + 1) % 3] + T.len[e];
+            k1[e] = rh_log_ratio_c(q * (0.5 * q) * iD[e], 1.0, c) * T.il[e];
+            w1[e] = sd[e] - k1[e];
+        }
+    }
+    const double re = R[0] * R[1] * R[2] + uw[0] * R[2] + uw[2] * R[1] + uw[1] * R[0];
+    const double om = 2.0 * rh_atan2_wave(dot(r[0], X[1]), re);
+    double kk[3], cc[3];
+#pragma unroll
+    for (int e = 0; e < 3; e++) {
+        S = axpy(k1[e] * T.len[e], T.t[e], S);
+        const double tm = T.sigma * dot(T.t[e], ng);
+        T.al[e] = fma(tm, w1[e], T.al[e]);
+        kk[e] = tm * T.len[e] * iD[e];
+        cc[e] = -sgn * iD[e];
+    }
+    // the normal: f = phi sigma, d sigma = dn . M
+    const double phi = dot(S, ng) - om * gn;
+    const V3<double> gS = cross(g, S);
+    T.N = axpy(phi, T.M, axpy(T.sigma, V3<double>{fma(-om, g.x, gS.x), fma(-om, g.y, gS.y), fma(-om, g.z, gS.z)}, T.N));
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const int in = (k + 2) % 3;  // side ending in corner k; side k starts there
+        const double kr = kk[in] + kk[k];
+        const V3<double> h{iR[k] * fma(kr, r[k].x, fma(cc[in], X[in].x, cc[k] * X[k].x)),
+                           iR[k] * fma(kr, r[k].y, fma(cc[in], X[in].y, cc[k] * X[k].y)),
+                           iR[k] * fma(kr, r[k].z, fma(cc[in], X[in].z, cc[k] * X[k].z))};
+        const double dk = T.sigma * (k1[in] - k1[k]);
+        T.G[k] = V3<double>{T.G[k].x + fma(dk, ng.x, -h.x), T.G[k].y + fma(dk, ng.y, -h.y),
+                            T.G[k].z + fma(dk, ng.z, -h.z)};
+        gx.x += h.x;
+        gx.y += h.y;
+        gx.z += h.z;
+    }
+#endif
+}
+
 // dL/dvertex partials: partv[bx][vertex slot][3] for the vertices of element
 // slice [sl[y], sl[y+1]); optional per-point dL/dx partials partx[y][p][3].
-template <bool SYM>
-__global__ __launch_bounds__(256) void k_adj_geom(DevModel m, const double* __restrict__ adj,
+//
+// FP64-issue bound.  A lane holds one triangle (of one transform copy) of the
+// slice in registers and walks the block's points, which lie in LDS and are the
+// same for all lanes; the four waves take every fourth point.  A triangle's
+// nine sums then cross lanes once per block instead of once per point, and
+// what depends on the triangle alone is computed once per block; dL/dx, three
+// sums, is the one that crosses lanes per point.  About 330 FP64 operations
+// for all nine derivatives (forward-mode duals seeded per corner took some
+// 2,700 and nine wave sums): 1,000 hexahedra at 2,048 points 0.35 ms instead
+// of 5.4 ms, of which 0.3 ms is the operations' issue.
+constexpr int kAdjTile = 128;  // points staged at a time
+template <bool SYM, bool GX>
+__global__ __launch_bounds__(256, 2) void k_adj_geom(DevModel m, const double* __restrict__ adj,
                                                   const int64_t* __restrict__ adj_off,
                                                   const int64_t* __restrict__ vert_off,
                                                   const int64_t* __restrict__ sl, int64_t nvert,
                                                   const double* __restrict__ M,
-                                                  const double* __restrict__ pts, int64_t np,
+                                                  const double* __restrict__ pts, int64_t np, int64_t per_block,
                                                   const double* __restrict__ g,
                                                   double* __restrict__ partv,
                                                   double* __restrict__ partx)
 {
-    __shared__ double acc[4][kAdjSliceV * 3];
+    __shared__ double acc[3 * kAdjSliceV];
+    __shared__ double xs[kAdjTile][6];
+    __shared__ double lanes[4][9][64];
+    __shared__ int corner[3][64];
+    __shared__ double copy[SYM ? 21 : 1][64];  // every lane's transform copy
+    __shared__ int first[kAdjSliceV + 1];  // first triangle of each element
+    __shared__ int owner[kAdjSliceV];      // element of each vertex
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < 4 * kAdjSliceV * 3; i += 256) (&acc[0][0])[i] = 0.0;
-    __syncthreads();
     const int64_t j0 = sl[blockIdx.y], j1 = sl[blockIdx.y + 1];
     const int64_t v0 = vert_off[j0];
-    const int64_t tiles = (np + 255) / 256;
-    for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const int64_t p = tile * 256 + threadIdx.x;
-        const bool live = p < np;
-        const double x[3] = {live ? pts[3 * p] : 0.0, live ? pts[3 * p + 1] : 0.0,
-                             live ? pts[3 * p + 2] : 0.0};
-        const double gp[3] = {live ? g[3 * p] : 0.0, live ? g[3 * p + 1] : 0.0,
-                              live ? g[3 * p + 2] : 0.0};
-        double gx[3] = {0.0, 0.0, 0.0};
-        for (int64_t j = j0; j < j1; j++) {
-            const double* rec = adj + adj_off[j];
-            const int nt = adj_ntri(rec);
-            const double Mj[3] = {M[3 * j], M[3 * j + 1], M[3 * j + 2]};
-            const int64_t slot0 = vert_off[j] - v0;
-            for (int64_t c = m.copy_off[j]; c < m.copy_off[j + 1]; c++) {
-                const double* cp = m.copies + 24 * c;
-                double xl[3], gl[3];
+    const int nel = int(j1 - j0);  // at most kAdjSliceV
+    for (int i = threadIdx.x; i < 3 * kAdjSliceV; i += 256) acc[i] = 0.0;
+    for (int e = threadIdx.x; e < nel; e += 256) {
+        first[e + 1] = adj_ntri(adj + adj_off[j0 + e]) * int(m.copy_off[j0 + e + 1] - m.copy_off[j0 + e]);
+        for (int64_t v = vert_off[j0 + e]; v < vert_off[j0 + e + 1]; v++) owner[v - v0] = e;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        first[0] = 0;
+        for (int e = 0; e < nel; e++) first[e + 1] += first[e];
+    }
+    __syncthreads();
+    const int total = first[nel];
+    const int64_t p0 = int64_t(blockIdx.x) * per_block;
+    const int64_t p1 = (p0 + per_block < np) ? (p0 + per_block) : np;
+    if (GX && total == 0)
+        for (int64_t i = 3 * p0 + threadIdx.x; i < 3 * p1; i += 256) partx[int64_t(blockIdx.y) * 3 * np + i] = 0.0;
+    for (int base = 0; base < total; base += 64) {
+        // lanes past the end repeat the last triangle with M = 0
+        const bool live = base + lane < total;
+        const int item = live ? base + lane : total - 1;
+        int el = 0;
+        while (first[el + 1] <= item) el++;
+        const int64_t j = j0 + el;
+        const double* rec = adj + adj_off[j];
+        const int nt = adj_ntri(rec);
+        const double* tri = rec + 2 + 3 * adj_nv(rec) + 3 * ((item - first[el]) % nt);
+        const double* cp = m.copies + 24 * (m.copy_off[j] + (item - first[el]) / nt);
+        const int slot = int(vert_off[j] - v0);
+        if (SYM && wave == 0)
+            for (int k = 0; k < 21; k++) copy[k][lane] = cp[k];
+        TriLane T;
+        for (int k = 0; k < 3; k++) {
+            const int id = int(tri[k]);
+            if (wave == 0) corner[k][lane] = slot + id;
+            T.v[k] = V3<double>{rec[2 + 3 * id], rec[3 + 3 * id], rec[4 + 3 * id]};
+            T.G[k] = V3<double>{0.0, 0.0, 0.0};
+            T.al[k] = 0.0;
+        }
+        T.N = V3<double>{0.0, 0.0, 0.0};
+        T.M = live ? V3<double>{M[3 * j], M[3 * j + 1], M[3 * j + 2]} : V3<double>{0.0, 0.0, 0.0};
+        const V3<double> e1 = vsub(T.v[1], T.v[0]), e2 = vsub(T.v[2], T.v[0]);
+        const V3<double> nn = cross(e1, e2);
+        T.ia = 1.0 / sqrt(dot(nn, nn));
+        T.n = vscale(nn, T.ia);
+        T.sigma = dot(T.n, T.M);
+        for (int e = 0; e < 3; e++) {
+            const V3<double> d = vsub(T.v[(e + 1) % 3], T.v[e]);
+            T.len[e] = sqrt(dot(d, d));
+            T.il[e] = 1.0 / T.len[e];
+            T.t[e] = vscale(d, T.il[e]);
+        }
+        for (int64_t q0 = p0; q0 < p1; q0 += kAdjTile) {
+            const int cnt = int((p1 - q0 < kAdjTile) ? (p1 - q0) : kAdjTile);
+            __syncthreads();
+            for (int i = threadIdx.x; i < 3 * cnt; i += 256) {
+                xs[i / 3][i % 3] = pts[3 * q0 + i];
+                xs[i / 3][3 + i % 3] = kInv4Pi * g[3 * q0 + i];
+            }
+            __syncthreads();
+            for (int i = wave; i < cnt; i += 4) {
+                const double* z = xs[i];
+                double x[3] = {z[0], z[1], z[2]};
+                V3<double> gl{z[3], z[4], z[5]}, gx{0.0, 0.0, 0.0};
                 if (SYM) {
-                    apply_inv(cp, x, xl);
-                    for (int k = 0; k < 3; k++)
-                        gl[k] = kInv4Pi * (cp[12 + k] * gp[0] + cp[15 + k] * gp[1] + cp[18 + k] * gp[2]);
-                } else {
-                    for (int k = 0; k < 3; k++) {
-                        xl[k] = x[k];
-                        gl[k] = kInv4Pi * gp[k];
-                    }
+                    double cm[21];
+                    for (int k = 0; k < 21; k++) cm[k] = copy[k][lane];
+                    apply_inv(cm, z, x);
+                    gl.x = cm[12] * z[3] + cm[15] * z[4] + cm[18] * z[5];
+                    gl.y = cm[13] * z[3] + cm[16] * z[4] + cm[19] * z[5];
+                    gl.z = cm[14] * z[3] + cm[17] * z[4] + cm[20] * z[5];
                 }
-                const double* tri = rec + 2 + 3 * adj_nv(rec);
-                for (int t = 0; t < nt; t++) {
-                    for (int k = 0; k < 3; k++) {
-                        double d[3] = {0.0, 0.0, 0.0};
-                        const int vid = int(tri[3 * t + k]);  // wave-uniform
-                        int vid_lane = vid;
-                        if (live) adj_tri_corner_grad(rec, t, k, xl, Mj, gl, d, &vid_lane);
-                        // translation invariance: d/dxl = -sum over corners of d/dV
-                        if (SYM) {
-                            for (int a = 0; a < 3; a++)
-                                gx[a] -= cp[a] * d[0] + cp[3 + a] * d[1] + cp[6 + a] * d[2];
-                        } else {
-                            for (int a = 0; a < 3; a++) gx[a] -= d[a];
-                        }
-                        for (int a = 0; a < 3; a++) {
-                            const double s = wsum(d[a]);
-                            if (lane == 0) acc[wave][3 * (slot0 + vid) + a] += s;
-                        }
+                tri_point(T, x, gl, gx);
+                if (GX) {
+                    double d[3] = {gx.x, gx.y, gx.z};
+                    if (SYM)
+                        for (int a = 0; a < 3; a++)
+                            d[a] = copy[a][lane] * gx.x + copy[3 + a][lane] * gx.y + copy[6 + a][lane] * gx.z;
+                    for (int a = 0; a < 3; a++) d[a] = wsum(d[a]);
+                    if (lane < 3) {
+                        // the wave's own point: earlier triangles' sum, then these
+                        double* o = partx + (int64_t(blockIdx.y) * np + q0 + i) * 3 + lane;
+                        const double s = (lane == 0) ? d[0] : (lane == 1 ? d[1] : d[2]);
+                        *o = (base == 0) ? s : *o + s;
                     }
                 }
             }
         }
-        if (partx && live)
-            for (int a = 0; a < 3; a++) partx[(int64_t(blockIdx.y) * np + p) * 3 + a] = gx[a];
+        // side directions: dt = (dd - t (t . dd))/len moved both ends by -+ dd;
+        // the length's part is along t; the unit normal: n = (v1 - v0) x (v2 - v0)/|.|
+        const V3<double> q = vscale(axpy(-dot(T.n, T.N), T.n, T.N), T.ia);
+        const V3<double> g1 = cross(e2, q), g2 = cross(q, e1);
+        T.G[0] = vsub(T.G[0], V3<double>{g1.x + g2.x, g1.y + g2.y, g1.z + g2.z});
+        T.G[1] = V3<double>{T.G[1].x + g1.x, T.G[1].y + g1.y, T.G[1].z + g1.z};
+        T.G[2] = V3<double>{T.G[2].x + g2.x, T.G[2].y + g2.y, T.G[2].z + g2.z};
+        for (int k = 0; k < 3; k++) {
+            const V3<double> G = axpy(T.al[(k + 2) % 3], T.t[(k + 2) % 3], axpy(-T.al[k], T.t[k], T.G[k]));
+            lanes[wave][3 * k][lane] = G.x;
+            lanes[wave][3 * k + 1][lane] = G.y;
+            lanes[wave][3 * k + 2][lane] = G.z;
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < 9 * 64; i += 256)
+            (&lanes[0][0][0])[i] += (&lanes[1][0][0])[i] + (&lanes[2][0][0])[i] + (&lanes[3][0][0])[i];
+        __syncthreads();
+        // each vertex coordinate sums its corners in order
+        for (int i = threadIdx.x; i < 3 * int(vert_off[j1] - v0); i += 256) {
+            const int v = i / 3, a = i % 3;
+            const int l0 = max(0, first[owner[v]] - base), l1 = min(64, first[owner[v] + 1] - base);
+            double s = acc[i];
+            for (int l = l0; l < l1; l++)
+                for (int k = 0; k < 3; k++)
+                    if (corner[k][l] == v) s += lanes[0][3 * k + a][l];
+            acc[i] = s;
+        }
+        __syncthreads();
     }
-    __syncthreads();
     const int64_t cnt = 3 * (vert_off[j1] - v0);
     for (int64_t i = threadIdx.x; i < cnt; i += 256)
-        partv[int64_t(blockIdx.x) * 3 * nvert + 3 * v0 + i] =
-            acc[0][i] + acc[1][i] + acc[2][i] + acc[3][i];
+        partv[int64_t(blockIdx.x) * 3 * nvert + 3 * v0 + i] = acc[i];
 }
 
 // out[i] = sum_k part[k * stride + i], i < len
@@ -345,7 +549,29 @@ int64_t adj_point_groups(int64_t np, int64_t slices)
     return std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(pg, tiles), 64));
 }
 
-int64_t adj_m_slices(int64_t n) { return (n + kAdjSliceE - 1) / kAdjSliceE; }
+// Groups of points of the geometry pass: blocks for four a compute unit, each
+// with at least 16 points (four a wave) to spread the triangles' set-up over.
+int64_t adj_geom_groups(int64_t np, int64_t slices)
+{
+    const int64_t g = std::min<int64_t>((np + 15) / 16, 1024 / std::max<int64_t>(1, slices));
+    return std::max<int64_t>(1, std::min<int64_t>(g, 64));
+}
+
+// Elements per slice of the dL/dM sweep: 64, fewer where the tiles of 256 points
+// do not fill the chip (down to 4, below which the blocks' own reductions show).
+static int adj_m_slice(int64_t n, int64_t np)
+{
+    const int64_t tiles = (np + 255) / 256;
+    int e = kAdjSliceE;
+    while (e > 4 && tiles * ((n + e - 1) / e) < 1000) e /= 2;
+    return e;
+}
+
+int64_t adj_m_slices(int64_t n, int64_t np)
+{
+    const int e = adj_m_slice(n, np);
+    return (n + e - 1) / e;
+}
 
 std::vector<int64_t> adj_geom_slices(const std::vector<int64_t>& vert_off, std::string* err)
 {
@@ -357,7 +583,7 @@ std::vector<int64_t> adj_geom_slices(const std::vector<int64_t>& vert_off, std::
             if (err) *err = "element with more than 128 vertices";
             return {};
         }
-        if (vert_off[j + 1] - vert_off[sl.back()] > kAdjSliceV) sl.push_back(j);
+        if (vert_off[j + 1] - vert_off[sl.back()] > kAdjSliceV || j - sl.back() >= kAdjSliceV) sl.push_back(j);
     }
     sl.push_back(n);
     return sl;
@@ -366,12 +592,13 @@ std::vector<int64_t> adj_geom_slices(const std::vector<int64_t>& vert_off, std::
 hipError_t launch_adj_m(const DevModel& m, const double* pts, int64_t np, const double* g, bool addin,
                         double* part, int64_t groups, double* gM, hipStream_t s)
 {
-    const int64_t ns = adj_m_slices(m.n);
+    const int64_t ns = adj_m_slices(m.n, np);
+    const int slice = adj_m_slice(m.n, np);
     const dim3 grid{unsigned(groups), unsigned(ns), 1u};
     if (m.sym)
-        hipLaunchKernelGGL(k_adj_m<true>, grid, dim3(256), 0, s, m, pts, np, g, addin ? 1 : 0, part);
+        hipLaunchKernelGGL(k_adj_m<true>, grid, dim3(256), 0, s, m, pts, np, g, addin ? 1 : 0, slice, part);
     else
-        hipLaunchKernelGGL(k_adj_m<false>, grid, dim3(256), 0, s, m, pts, np, g, addin ? 1 : 0, part);
+        hipLaunchKernelGGL(k_adj_m<false>, grid, dim3(256), 0, s, m, pts, np, g, addin ? 1 : 0, slice, part);
     const int64_t len = 3 * m.n;
     hipLaunchKernelGGL(k_sum_parts, dim3(unsigned((len + 255) / 256)), dim3(256), 0, s, len, groups,
                        len, part, gM);
@@ -385,12 +612,11 @@ hipError_t launch_adj_geom(const DevModel& m, const double* adj, const int64_t* 
                            double* gV, double* gX, hipStream_t s)
 {
     const dim3 grid{unsigned(groups), unsigned(nslices), 1u};
-    if (m.sym)
-        hipLaunchKernelGGL(k_adj_geom<true>, grid, dim3(256), 0, s, m, adj, adj_off, vert_off, sl,
-                           nvert, M, pts, np, g, partv, gX ? partx : nullptr);
-    else
-        hipLaunchKernelGGL(k_adj_geom<false>, grid, dim3(256), 0, s, m, adj, adj_off, vert_off, sl,
-                           nvert, M, pts, np, g, partv, gX ? partx : nullptr);
+    const int64_t per = (np + groups - 1) / groups;
+    auto k = m.sym ? (gX ? k_adj_geom<true, true> : k_adj_geom<true, false>)
+                   : (gX ? k_adj_geom<false, true> : k_adj_geom<false, false>);
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, s, m, adj, adj_off, vert_off, sl, nvert, M, pts, np, per, g, partv,
+                       partx);
     if (gV) {
         const int64_t len = 3 * nvert;
         hipLaunchKernelGGL(k_sum_parts, dim3(unsigned((len + 255) / 256)), dim3(256), 0, s, len,

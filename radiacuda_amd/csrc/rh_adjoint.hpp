@@ -12,9 +12,11 @@
 // Omega_t the signed solid angle (Van Oosterom & Strackee).  For planar faces
 // the internal fan edges cancel pairwise and this equals the face form used by
 // the forward kernels; for displaced vertices it stays a closed triangulated
-// surface, so its derivative is that of a well-defined field.  Derivatives are
+// surface, so its derivative is that of a well-defined field.  The device
+// sweep (rh_adjoint.hip) has the derivatives in closed form; here they are
 // forward-mode (dual numbers) with the three coordinates of one triangle
-// corner seeded at a time: a triangle depends only on its own corners.
+// corner seeded at a time, the independent form that the host build checks it
+// with.
 #pragma once
 
 #include "rh_math.hpp"

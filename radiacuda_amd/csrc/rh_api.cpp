@@ -1797,7 +1797,7 @@ rh_status rh_field_adjoint_dev(rh_model* m, const double* d_M, const double* d_p
     }
     Timer t("adjoint", s);
     if (d_gM) {
-        const int64_t groups = rh::adj_point_groups(np, rh::adj_m_slices(n));
+        const int64_t groups = rh::adj_point_groups(np, rh::adj_m_slices(n, np));
         RH_HIP(grow(m, size_t(groups * 3 * n)));
         t.begin();
         RH_HIP(rh::launch_adj_m(m->dev, d_pts, np, d_gB, field == 0, m->d_work, groups, d_gM, s));
@@ -1806,7 +1806,7 @@ rh_status rh_field_adjoint_dev(rh_model* m, const double* d_M, const double* d_p
     if (d_gV || d_gX) {
         rh_status st = adj_geometry(m);
         if (st != RH_OK) return st;
-        const int64_t groups = rh::adj_point_groups(np, m->n_slices);
+        const int64_t groups = rh::adj_geom_groups(np, m->n_slices);
         const size_t nv_part = size_t(groups * 3 * nvert);
         const size_t nx_part = d_gX ? size_t(m->n_slices * 3 * np) : 0;
         RH_HIP(grow(m, nv_part + nx_part));

@@ -228,9 +228,12 @@ hipError_t launch_current(int64_t ns, const int32_t* kind, const double* par, co
 // Point groups (workgroups along the point axis, each striding over tiles of
 // 256 points) for `slices` element slices.
 int64_t adj_point_groups(int64_t np, int64_t slices);
+// The same for the geometry sweep, whose groups are contiguous ranges of points.
+int64_t adj_geom_groups(int64_t np, int64_t slices);
 // Element slices of the dL/dM sweep.
-int64_t adj_m_slices(int64_t n);
-// Element slice bounds of the dL/dvertex sweep (<= 128 vertices per slice);
+int64_t adj_m_slices(int64_t n, int64_t np);
+// Element slice bounds of the dL/dvertex sweep (<= 128 vertices and elements
+// per slice);
 // empty with *err set if an element has more vertices.
 std::vector<int64_t> adj_geom_slices(const std::vector<int64_t>& vert_off, std::string* err);
 // gM [3n] = sum_p sum_c (Q_j(x'_pc) + [addin and inside] I) F_c^T g_p.
