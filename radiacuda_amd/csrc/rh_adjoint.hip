@@ -20,17 +20,11 @@
 #include "rh_adjoint.hpp"
 #include "rh_eval.hpp"
 #include "rh_kernels.hpp"
+#include "rh_relax_step.hpp"
 
 namespace rh {
 
 namespace {
-
-__device__ __forceinline__ double wsum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
 
 constexpr int kAdjSliceE = 64;   // elements per workgroup slice (dL/dM), at most
 constexpr int kAdjSliceV = 128;  // vertices per workgroup slice (dL/dvertex)
@@ -85,7 +79,7 @@ __global__ __launch_bounds__(256) void k_adj_m(DevModel m, const double* __restr
                 }
             }
             for (int k = 0; k < 3; k++) {
-                const double s = wsum(v[k]);
+                const double s = wave_sum(v[k]);
                 if (lane == 0) acc[wave][3 * (j - j0) + k] += s;
             }
         }
@@ -330,7 +324,7 @@ __global__ __launch_bounds__(256, 2) void k_adj_geom(DevModel m, const double* _
                     if (SYM)
                         for (int a = 0; a < 3; a++)
                             d[a] = copy[a][lane] * gx.x + copy[3 + a][lane] * gx.y + copy[6 + a][lane] * gx.z;
-                    for (int a = 0; a < 3; a++) d[a] = wsum(d[a]);
+                    for (int a = 0; a < 3; a++) d[a] = wave_sum(d[a]);
                     if (lane < 3) {
                         // the wave's own point: earlier triangles' sum, then these
                         double* o = partx + (int64_t(blockIdx.y) * np + q0 + i) * 3 + lane;
@@ -374,16 +368,47 @@ __global__ __launch_bounds__(256, 2) void k_adj_geom(DevModel m, const double* _
         partv[int64_t(blockIdx.x) * 3 * nvert + 3 * v0 + i] = acc[i];
 }
 
-// out[i] = sum_k part[k * stride + i], i < len
+// out[i] = sum_k part[k * stride + i], i < len: 256 / G columns to a block, G
+// threads to a column, each summing every G-th row, then in order over the
+// threads.  93 rows of 1,500 columns: 21 us with a thread per column (a chain
+// of 93 loads in 6 blocks), 3.6 us with 16.
+template <int G>
 __global__ __launch_bounds__(256) void k_sum_parts(int64_t len, int64_t ns, int64_t stride,
                                                    const double* __restrict__ part,
-                                                   double* __restrict__ out)
+                                                   double* __restrict__ out, const int32_t* __restrict__ skip)
 {
-    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (i >= len) return;
+    if (skip && *skip) return;
+    constexpr int C = 256 / G;
+    __shared__ double red[G][C];
+    const int c = threadIdx.x % C, r = threadIdx.x / C;
+    const int64_t i = int64_t(blockIdx.x) * C + c;
     double s = 0.0;
-    for (int64_t k = 0; k < ns; k++) s += part[k * stride + i];
-    out[i] = s;
+    if (i < len) {
+#pragma unroll 8
+        for (int64_t k = r; k < ns; k += G) s += part[k * stride + i];
+    }
+    if (G > 1) {
+        red[r][c] = s;
+        __syncthreads();
+        if (r > 0) return;
+#pragma unroll
+        for (int k = 1; k < G; k++) s += red[k][c];
+    }
+    if (i < len) out[i] = s;
+}
+
+void sum_parts(int64_t len, int64_t ns, int64_t stride, const double* part, double* out, hipStream_t s,
+               const int32_t* skip = nullptr)
+{
+    auto go = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        const int64_t cols = 256 / G;
+        hipLaunchKernelGGL(k_sum_parts<G>, dim3(unsigned((len + cols - 1) / cols)), dim3(256), 0, s, len, ns, stride,
+                           part, out, skip);
+    };
+    // up to 16 rows a thread's chain is one round of loads
+    if (ns <= 16) go(std::integral_constant<int, 1>{});
+    else go(std::integral_constant<int, 16>{});
 }
 
 // Transposed matrix pass: part[rc][col] = sum over rows of chunk rc of
@@ -392,8 +417,9 @@ __global__ __launch_bounds__(256) void k_sum_parts(int64_t len, int64_t ns, int6
 template <class T>
 __global__ __launch_bounds__(256) void k_matvec_t(const T* __restrict__ Q, int64_t nrows, int64_t ld,
                                                   int64_t rows_per_chunk, const double* __restrict__ x,
-                                                  double* __restrict__ part)
+                                                  double* __restrict__ part, const int32_t* __restrict__ skip)
 {
+    if (skip && *skip) return;
     const int64_t c0 = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
     const int64_t r0 = int64_t(blockIdx.y) * rows_per_chunk;
     const int64_t r1 = (r0 + rows_per_chunk < nrows) ? (r0 + rows_per_chunk) : nrows;
@@ -417,8 +443,10 @@ __global__ __launch_bounds__(256) void k_matvec_t(const T* __restrict__ Q, int64
 template <class T, int P>
 __global__ __launch_bounds__(256) void k_matvec_t_sym(const T* __restrict__ Q, int64_t nel, int64_t ldp,
                                                       int64_t el_per_chunk, const double* __restrict__ x,
-                                                      double* __restrict__ part, int64_t ld)
+                                                      double* __restrict__ part, int64_t ld,
+                                                      const int32_t* __restrict__ skip)
 {
+    if (skip && *skip) return;
     const int64_t j0 = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 2;
     const int64_t i0 = int64_t(blockIdx.y) * el_per_chunk;
     const int64_t i1 = (i0 + el_per_chunk < nel) ? (i0 + el_per_chunk) : nel;
@@ -442,8 +470,7 @@ __global__ __launch_bounds__(256) void k_matvec_t_sym(const T* __restrict__ Q, i
     for (int k = 0; k < 6; k++) o[k] = acc[k];
 }
 
-// mu_i = K_i^T lam_i (linear susceptibility tensor of element i, element frame)
-// followed by rowT_i^T when the rows carry a transform.
+// Linear susceptibility tensor of an element (element frame).
 __device__ __forceinline__ void lin_tensor(const double* mat, double K[9])
 {
     if (int(mat[0]) == 0) {
@@ -454,42 +481,30 @@ __device__ __forceinline__ void lin_tensor(const double* mat, double K[9])
     }
 }
 
+// mu = K^T lam
+__device__ __forceinline__ void adj_scale(const double* mat, const double l[3], double* mu)
+{
+    double K[9];
+    lin_tensor(mat, K);
+    for (int a = 0; a < 3; a++) mu[a] = K[a] * l[0] + K[3 + a] * l[1] + K[6 + a] * l[2];
+}
+
 __global__ __launch_bounds__(256) void k_adj_scale(int64_t n, const double* __restrict__ mats,
-                                                   const double* __restrict__ rowt,
                                                    const double* __restrict__ lam,
                                                    double* __restrict__ mu)
 {
     const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (i >= n) return;
-    double K[9];
-    lin_tensor(mats + 16 * i, K);
     const double l[3] = {lam[3 * i], lam[3 * i + 1], lam[3 * i + 2]};
-    double u[3];
-    for (int a = 0; a < 3; a++) u[a] = K[a] * l[0] + K[3 + a] * l[1] + K[6 + a] * l[2];
-    if (rowt) {
-        const double* t = rowt + 9 * i;
-        double w[3];
-        for (int a = 0; a < 3; a++) w[a] = t[a] * u[0] + t[3 + a] * u[1] + t[6 + a] * u[2];
-        for (int a = 0; a < 3; a++) u[a] = w[a];
-    }
-    for (int a = 0; a < 3; a++) mu[3 * i + a] = u[a];
+    adj_scale(mats + 16 * i, l, mu + 3 * i);
 }
 
 // Block-Jacobi update of the transposed system (I - Q^T K^T) lam = rhs:
-// lam_new_i = (I - Qii^T K_i^T)^{-1} (rhs_i + y_i), y = offdiag(Q)^T K^T lam;
-// F = lam_new - lam, per-block [sum |F|^2, max |lam_new|, 0].
-__global__ __launch_bounds__(kRelaxLanes) void k_adj_update(int64_t n, const double* __restrict__ mats,
-                                                    const double* __restrict__ rhs,
-                                                    const double* __restrict__ qdiag,
-                                                    const double* __restrict__ y,
-                                                    const double* __restrict__ lam,
-                                                    double* __restrict__ F,
-                                                    double* __restrict__ partials)
-{
-    __shared__ double red[2][kRelaxLanes];
-    const int64_t i = int64_t(blockIdx.x) * kRelaxLanes + threadIdx.x;
-    double f2 = 0.0, mm = 0.0;
-    if (i < n) {
+// lam_new_i = (I - Qii^T K_i^T)^{-1} (rhs_i + y_i), y = offdiag(Q)^T K^T lam.
+struct TransposedLaw {
+    const double *mats, *rhs, *qdiag, *y;
+    __device__ __forceinline__ void operator()(int64_t i, double* nl, double&) const
+    {
         double K[9];
         lin_tensor(mats + 16 * i, K);
         const double* D = qdiag + 9 * i;
@@ -514,30 +529,41 @@ __global__ __launch_bounds__(kRelaxLanes) void k_adj_update(int64_t n, const dou
         Ai[8] = (A[0] * A[4] - A[1] * A[3]) * id;
         const double r[3] = {rhs[3 * i] + y[3 * i], rhs[3 * i + 1] + y[3 * i + 1],
                              rhs[3 * i + 2] + y[3 * i + 2]};
-        double nl[3];
         for (int a = 0; a < 3; a++) nl[a] = Ai[3 * a] * r[0] + Ai[3 * a + 1] * r[1] + Ai[3 * a + 2] * r[2];
-        for (int a = 0; a < 3; a++) {
-            const double d = nl[a] - lam[3 * i + a];
-            F[3 * i + a] = d;
-            f2 += d * d;
-        }
-        mm = sqrt(nl[0] * nl[0] + nl[1] * nl[1] + nl[2] * nl[2]);
     }
-    red[0][threadIdx.x] = f2;
-    red[1][threadIdx.x] = mm;
-    __syncthreads();
-    for (int s = kRelaxLanes / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            red[0][threadIdx.x] += red[0][threadIdx.x + s];
-            red[1][threadIdx.x] = fmax(red[1][threadIdx.x], red[1][threadIdx.x + s]);
-        }
-        __syncthreads();
+};
+
+__global__ __launch_bounds__(kRelaxLanes) void k_adj_step_dev(int64_t n, TransposedLaw law,
+                                                              const double* __restrict__ lam,
+                                                              double* __restrict__ F,
+                                                              double* __restrict__ partials, HistBufs hb,
+                                                              RelaxDevState* __restrict__ st)
+{
+    relax_step_dev(n, law, lam, F, partials, hb, st);
+}
+
+// The update of lam and the next matrix pass's input mu = K^T lam.
+__global__ __launch_bounds__(kRelaxLanes) void k_adj_update_dev(int64_t n, const double* __restrict__ mats,
+                                                                double* __restrict__ lam, double* __restrict__ mu,
+                                                                const double* __restrict__ F, HistBufs hb,
+                                                                double* __restrict__ lam_out,
+                                                                const RelaxDevState* __restrict__ st)
+{
+    const int done = st->done;
+    if (done == 2) return;
+    const int64_t i = int64_t(blockIdx.x) * kRelaxLanes + threadIdx.x;
+    if (i >= n) return;
+    if (done == 1) {
+        for (int k = 0; k < 3; k++) lam_out[3 * i + k] = lam[3 * i + k] + F[3 * i + k];
+        return;
     }
-    if (threadIdx.x == 0) {
-        partials[3 * blockIdx.x] = red[0][0];
-        partials[3 * blockIdx.x + 1] = red[1][0];
-        partials[3 * blockIdx.x + 2] = 0.0;
+    const UpdateCoef c(st);
+    double l[3];
+    for (int k = 0; k < 3; k++) {
+        l[k] = c.apply(lam[3 * i + k], F, hb, 3 * i + k);
+        lam[3 * i + k] = l[k];
     }
+    adj_scale(mats + 16 * i, l, mu + 3 * i);
 }
 
 }  // namespace
@@ -600,8 +626,7 @@ hipError_t launch_adj_m(const DevModel& m, const double* pts, int64_t np, const 
     else
         hipLaunchKernelGGL(k_adj_m<false>, grid, dim3(256), 0, s, m, pts, np, g, addin ? 1 : 0, slice, part);
     const int64_t len = 3 * m.n;
-    hipLaunchKernelGGL(k_sum_parts, dim3(unsigned((len + 255) / 256)), dim3(256), 0, s, len, groups,
-                       len, part, gM);
+    sum_parts(len, groups, len, part, gM, s);
     return hipGetLastError();
 }
 
@@ -619,13 +644,11 @@ hipError_t launch_adj_geom(const DevModel& m, const double* adj, const int64_t* 
                        partx);
     if (gV) {
         const int64_t len = 3 * nvert;
-        hipLaunchKernelGGL(k_sum_parts, dim3(unsigned((len + 255) / 256)), dim3(256), 0, s, len,
-                           groups, len, partv, gV);
+        sum_parts(len, groups, len, partv, gV, s);
     }
     if (gX) {
         const int64_t len = 3 * np;
-        hipLaunchKernelGGL(k_sum_parts, dim3(unsigned((len + 255) / 256)), dim3(256), 0, s, len,
-                           nslices, len, partx, gX);
+        sum_parts(len, nslices, len, partx, gX, s);
     }
     return hipGetLastError();
 }
@@ -639,23 +662,23 @@ int64_t matvec_t_chunks(int64_t nrows, int64_t ld)
 }
 
 hipError_t launch_matvec_t(const void* Q, int elem_bytes, int64_t nrows, int64_t ld, const double* x,
-                           double* part, int64_t chunks, double* y, hipStream_t s)
+                           double* part, int64_t chunks, double* y, hipStream_t s, const int32_t* skip)
 {
     const int64_t rpc = (nrows + chunks - 1) / chunks;
     const dim3 grid{unsigned((ld + 1023) / 1024), unsigned(chunks), 1u};
     if (elem_bytes == 4)
         hipLaunchKernelGGL(k_matvec_t<float>, grid, dim3(256), 0, s, static_cast<const float*>(Q),
-                           nrows, ld, rpc, x, part);
+                           nrows, ld, rpc, x, part, skip);
     else
         hipLaunchKernelGGL(k_matvec_t<double>, grid, dim3(256), 0, s, static_cast<const double*>(Q),
-                           nrows, ld, rpc, x, part);
-    hipLaunchKernelGGL(k_sum_parts, dim3(unsigned((nrows + 255) / 256)), dim3(256), 0, s, nrows,
-                       chunks, ld, part, y);
+                           nrows, ld, rpc, x, part, skip);
+    sum_parts(nrows, chunks, ld, part, y, s, skip);
     return hipGetLastError();
 }
 
 hipError_t launch_matvec_t_sym(const void* Q, int elem_bytes, int planes, int64_t nel, int64_t ldp,
-                               const double* x, double* part, int64_t chunks, double* y, hipStream_t s)
+                               const double* x, double* part, int64_t chunks, double* y, hipStream_t s,
+                               const int32_t* skip)
 {
     if ((planes != 5 && planes != 6) || ldp % 256 != 0 || chunks < 1) return hipErrorInvalidValue;
     const int64_t epc = (nel + chunks - 1) / chunks;
@@ -664,35 +687,40 @@ hipError_t launch_matvec_t_sym(const void* Q, int elem_bytes, int planes, int64_
     if (elem_bytes == 4) {
         const float* q = static_cast<const float*>(Q);
         if (planes == 5)
-            hipLaunchKernelGGL((k_matvec_t_sym<float, 5>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld);
+            hipLaunchKernelGGL((k_matvec_t_sym<float, 5>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld, skip);
         else
-            hipLaunchKernelGGL((k_matvec_t_sym<float, 6>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld);
+            hipLaunchKernelGGL((k_matvec_t_sym<float, 6>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld, skip);
     } else {
         const double* q = static_cast<const double*>(Q);
         if (planes == 5)
-            hipLaunchKernelGGL((k_matvec_t_sym<double, 5>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld);
+            hipLaunchKernelGGL((k_matvec_t_sym<double, 5>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld, skip);
         else
-            hipLaunchKernelGGL((k_matvec_t_sym<double, 6>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld);
+            hipLaunchKernelGGL((k_matvec_t_sym<double, 6>), grid, dim3(256), 0, s, q, nel, ldp, epc, x, part, ld, skip);
     }
-    hipLaunchKernelGGL(k_sum_parts, dim3(unsigned((3 * nel + 255) / 256)), dim3(256), 0, s, 3 * nel,
-                       chunks, ld, part, y);
+    sum_parts(3 * nel, chunks, ld, part, y, s, skip);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_scale(int64_t n, const double* mats, const double* rowt, const double* lam,
-                            double* mu, hipStream_t s)
+hipError_t launch_adj_scale(int64_t n, const double* mats, const double* lam, double* mu, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_adj_scale, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, n, mats, rowt,
-                       lam, mu);
+    hipLaunchKernelGGL(k_adj_scale, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, n, mats, lam, mu);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_update(int64_t n, const double* mats, const double* rhs, const double* qdiag,
-                             const double* y, const double* lam, double* F, double* partials,
-                             hipStream_t s)
+hipError_t launch_adj_step_dev(int64_t n, const double* mats, const double* rhs, const double* qdiag, const double* y,
+                               const double* lam, double* F, double* partials, const HistBufs& hb,
+                               RelaxDevState* st, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_adj_update, dim3(unsigned(relax_blocks(n))), dim3(kRelaxLanes), 0, s, n, mats, rhs,
-                       qdiag, y, lam, F, partials);
+    hipLaunchKernelGGL(k_adj_step_dev, dim3(unsigned(relax_blocks(n))), dim3(kRelaxLanes), 0, s, n,
+                       TransposedLaw{mats, rhs, qdiag, y}, lam, F, partials, hb, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_adj_update_dev(int64_t n, const double* mats, double* lam, double* mu, const double* F,
+                                 const HistBufs& hb, double* lam_out, const RelaxDevState* st, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_adj_update_dev, dim3(unsigned(relax_blocks(n))), dim3(kRelaxLanes), 0, s, n, mats, lam, mu, F,
+                       hb, lam_out, st);
     return hipGetLastError();
 }
 

@@ -154,61 +154,67 @@ struct RelaxWork {
     double* F = nullptr;   // [n3]
     double* Fp = nullptr;  // [n3] previous F
     double* xp = nullptr;  // [n3] previous x
-    double* dX[kHist] = {nullptr};
-    double* dF[kHist] = {nullptr};
+    double* dX = nullptr;  // kHist differences each, one every `stride` doubles
+    double* dF = nullptr;
+    int64_t stride = 0;
     double* part = nullptr;
-    double* dots = nullptr;
     rh::RelaxDevState* st = nullptr;   // state of the device-driven loop
     rh::RelaxDevState* hst = nullptr;  // pinned: two read-back slots and an upload slot
     hipEvent_t ev[2] = {nullptr, nullptr};
     double* hbuf = nullptr;            // pinned read-back of the host-driven loops
     double* H64 = nullptr;             // [n3] FP64 refinement: field at the collocation points
     double* hx = nullptr;              // [n3] FP64 refinement: corrected external field
+    double* mu = nullptr;              // adjoint: [n3] K^T lam
+    double* tpart = nullptr;           // adjoint: [chunks * ld] transposed-pass partials
+    int64_t chunks = 0;
+    double* arena = nullptr;           // the device arrays above, one allocation
     ~RelaxWork()
     {
-        dfree(x);
-        dfree(y);
-        dfree(F);
-        dfree(Fp);
-        dfree(xp);
-        for (int k = 0; k < kHist; k++) {
-            dfree(dX[k]);
-            dfree(dF[k]);
-        }
-        dfree(part);
-        dfree(dots);
-        dfree(st);
-        dfree(H64);
-        dfree(hx);
+        dfree(arena);
         if (hst) (void)hipHostFree(hst);
         if (hbuf) (void)hipHostFree(hbuf);
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
     }
-    // All arrays of a solve on n elements (3n rows, leading dimension ld).
-    hipError_t alloc(int64_t n, int64_t n3_, int64_t ld_)
+    // All arrays of a solve on n elements (3n rows, leading dimension ld); of an
+    // adjoint solve where chunks > 0.
+    hipError_t alloc(int64_t n, int64_t n3_, int64_t ld_, int64_t chunks_ = 0)
     {
         n3 = n3_;
         ld = ld_;
+        chunks = chunks_;
+        stride = (n3 + 31) / 32 * 32;
         nb = rh::relax_blocks(n);
         db = rh::dot_blocks(n3);
-        hipError_t e = dalloc(&x, size_t(ld));
-        if (e == hipSuccess) e = dalloc(&y, size_t(n3));
-        if (e == hipSuccess) e = dalloc(&F, size_t(n3));
-        if (e == hipSuccess) e = dalloc(&Fp, size_t(n3));
-        if (e == hipSuccess) e = dalloc(&xp, size_t(n3));
-        for (int k = 0; k < kHist && e == hipSuccess; k++) {
-            e = dalloc(&dX[k], size_t(n3));
-            if (e == hipSuccess) e = dalloc(&dF[k], size_t(n3));
-        }
-        if (e == hipSuccess) e = dalloc(&part, size_t(rh::kRelaxPart * nb));
-        if (e == hipSuccess) e = dalloc(&dots, size_t(rh::kDotMax * db));
-        if (e == hipSuccess) e = dalloc(&st, 1);
-        if (e == hipSuccess) e = dalloc(&H64, size_t(n3));
-        if (e == hipSuccess) e = dalloc(&hx, size_t(n3));
+        // two passes over the arrays: their places, then their addresses
+        size_t at = 0;
+        auto place = [&](auto** p, size_t count) {
+            using T = std::remove_pointer_t<std::remove_pointer_t<decltype(p)>>;
+            if (arena) *p = reinterpret_cast<T*>(reinterpret_cast<char*>(arena) + at);
+            at += (count * sizeof(T) + 255) / 256 * 256;
+        };
+        auto places = [&]() {
+            at = 0;
+            place(&x, size_t(ld));
+            for (double** p : {&y, &F, &Fp, &xp}) place(p, size_t(n3));
+            place(&dX, size_t(kHist * stride));
+            place(&dF, size_t(kHist * stride));
+            place(&part, size_t(rh::kRelaxPart * nb));
+            place(&st, 1);
+            if (chunks > 0) {
+                place(&mu, size_t(n3));
+                place(&tpart, size_t(chunks * ld));
+            } else {
+                place(&H64, size_t(n3));
+                place(&hx, size_t(n3));
+            }
+        };
+        places();
+        hipError_t e = dalloc(&arena, at / sizeof(double));
+        if (e == hipSuccess) places();
         if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&hst), 3 * sizeof(rh::RelaxDevState));
-        if (e == hipSuccess)
-            e = hipHostMalloc(reinterpret_cast<void**>(&hbuf), size_t(rh::kRelaxPart * nb + rh::kDotMax * db) * sizeof(double));
+        if (e == hipSuccess && chunks == 0)
+            e = hipHostMalloc(reinterpret_cast<void**>(&hbuf), size_t(rh::kRelaxPart * nb) * sizeof(double));
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[0], hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&ev[1], hipEventDisableTiming);
         return e;
@@ -905,15 +911,7 @@ namespace {
 // Anderson-accelerated block-Jacobi iterations from the iterate in w.x until
 // misfit <= prec or max_iter; writes the final magnetization to d_M and the
 // element fields to d_H.
-// Transposed (adjoint) iteration of a linear-material system: the matrix pass
-// becomes y = offdiag(Q)^T K^T lam and the update the transposed local solve.
-struct AdjointPass {
-    double* mu = nullptr;    // [n3] K^T lam
-    double* tpart = nullptr; // [chunks * ld] transposed-pass partials
-    int64_t chunks = 0;
-};
-
-// Device-driven form of the forward iteration below: the matrix pass, the
+// Device-driven form of the iteration below: the matrix pass, the
 // relaxation step (whose last block runs the Anderson step) and the update
 // all read the loop state on the device.  For a resident matrix the host enqueues iterations in
 // batches without waiting for any of them, copies the state back after each
@@ -923,9 +921,13 @@ struct AdjointPass {
 // memory) runs one iteration per batch and is looked at after each, so no
 // pass is enqueued beyond the last; its iterates are the resident matrix's,
 // bit for bit.
+//
+// adjoint: the transposed iteration of a linear-material system, y =
+// offdiag(Q)^T K^T lam with the transposed local solve (d_hext: right-hand
+// side, d_M: lam; a resident matrix).
 rh_status relax_run_dev(rh_matrix* q, const double* d_mats, const double* d_tab, const double* d_hext,
                         double* d_M, double* d_H, const rh_relax_opts* opts, RelaxWork& w, rh_relax_result* res,
-                        bool keep_if_converged)
+                        bool keep_if_converged, bool adjoint = false)
 {
     const bool lagged = !q->streamed();
     rh_model* m = q->m;
@@ -944,10 +946,10 @@ rh_status relax_run_dev(rh_matrix* q, const double* d_mats, const double* d_tab,
     rh::HistBufs hb{};
     hb.Fp = w.Fp;
     hb.xp = w.xp;
-    for (int k = 0; k < kHist; k++) {
-        hb.dF[k] = w.dF[k];
-        hb.dX[k] = w.dX[k];
-    }
+    hb.dF = w.dF;
+    hb.dX = w.dX;
+    hb.stride = w.stride;
+    if (adjoint) RH_HIP(rh::launch_adj_scale(n, d_mats, w.x, w.mu, s));
     Timer tm("matvec", s);
     int enq = 0, batch = 0, cur = 0, want = lagged ? 4 : 1;
     int it_prev = 0;
@@ -956,6 +958,18 @@ rh_status relax_run_dev(rh_matrix* q, const double* d_mats, const double* d_tab,
         const int cnt = std::min(want, max_iter - enq);
         for (int j = 0; j < cnt; j++) {
             tm.begin();
+            if (adjoint) {
+                if (q->planes)
+                    RH_HIP(rh::launch_matvec_t_sym(q->d_Q, q->elem_bytes, q->planes, n, q->ldp, w.mu, w.tpart, w.chunks,
+                                                   w.y, s, &w.st->done));
+                else
+                    RH_HIP(rh::launch_matvec_t(q->d_Q, q->elem_bytes, n3, q->ld, w.mu, w.tpart, w.chunks, w.y, s,
+                                               &w.st->done));
+                tm.end();
+                RH_HIP(rh::launch_adj_step_dev(n, d_mats, d_hext, q->d_qdiag, w.y, w.x, w.F, w.part, hb, w.st, s));
+                RH_HIP(rh::launch_adj_update_dev(n, d_mats, w.x, w.mu, w.F, hb, d_M, w.st, s));
+                continue;
+            }
             if (lagged)
                 RH_HIP(matvec_rows(q, q->d_Q, 0, n, w.x, w.y, s, &w.st->done));
             else
@@ -1007,15 +1021,15 @@ rh_status relax_run_dev(rh_matrix* q, const double* d_mats, const double* d_tab,
 }
 
 rh_status relax_run(rh_matrix* q, const double* d_mats, const double* d_tab, const double* d_hext,
-                    double* d_M, double* d_H, const rh_relax_opts* opts, RelaxWork& w, double* hbuf,
-                    int64_t nb, int64_t db, rh_relax_result* res,
-                    const AdjointPass* adj = nullptr, bool keep_if_converged = false)
+                    double* d_M, double* d_H, const rh_relax_opts* opts, RelaxWork& w, rh_relax_result* res,
+                    bool keep_if_converged = false)
 {
-    if (!adj && !std::getenv("RADHIP_RELAX_HOST_LOOP"))
+    if (!std::getenv("RADHIP_RELAX_HOST_LOOP"))
         return relax_run_dev(q, d_mats, d_tab, d_hext, d_M, d_H, opts, w, res, keep_if_converged);
     rh_model* m = q->m;
     hipStream_t s = m->stream;
-    const int64_t n = m->host.n, n3 = q->n3;
+    const int64_t n = m->host.n, n3 = q->n3, nb = w.nb;
+    double* hbuf = w.hbuf;
     const double prec = opts->prec;
     const int max_iter = std::max(1, int(opts->max_iter));
     double beta = (opts->omega0 > 0.0) ? opts->omega0 : 0.5;
@@ -1028,17 +1042,7 @@ rh_status relax_run(rh_matrix* q, const double* d_mats, const double* d_tab, con
     while (true) {
         it++;
         tm.begin();
-        if (adj) {
-            RH_HIP(rh::launch_adj_scale(n, d_mats, nullptr, w.x, adj->mu, s));
-            if (q->planes)
-                RH_HIP(rh::launch_matvec_t_sym(q->d_Q, q->elem_bytes, q->planes, n, q->ldp, adj->mu, adj->tpart,
-                                               adj->chunks, w.y, s));
-            else
-                RH_HIP(rh::launch_matvec_t(q->d_Q, q->elem_bytes, n3, q->ld, adj->mu, adj->tpart,
-                                           adj->chunks, w.y, s));
-        } else {
-            RH_HIP(matrix_pass(q, w.x, w.y, s));
-        }
+        RH_HIP(matrix_pass(q, w.x, w.y, s));
         tm.end();
         // dv: the dot products of the newest difference with every stored
         // one, then of every stored difference with F (oldest first)
@@ -1047,82 +1051,34 @@ rh_status relax_run(rh_matrix* q, const double* d_mats, const double* d_tab, con
         double f2 = 0.0;
         maxM = 1e-17;
         maxH = 1e-17;
-        if (adj) {
-            RH_HIP(rh::launch_adj_update(n, d_mats, d_hext, q->d_qdiag, w.y, w.x, w.F, w.part, s));
-            // tentatively extend the history with the newest differences
-            if (it > 1) {
-                const double* v1[2] = {w.F, w.Fp};
-                const double c1[2] = {1.0, -1.0};
-                RH_HIP(rh::launch_lincomb(2, v1, c1, n3, w.dF[head], s));
-                const double* v2[2] = {w.x, w.xp};
-                RH_HIP(rh::launch_lincomb(2, v2, c1, n3, w.dX[head], s));
-                head = (head + 1) % kHist;
-                hist = std::min(hist + 1, kHist);
-            }
-            RH_HIP(hipMemcpyAsync(w.Fp, w.F, size_t(n3) * sizeof(double), hipMemcpyDeviceToDevice, s));
-            RH_HIP(hipMemcpyAsync(w.xp, w.x, size_t(n3) * sizeof(double), hipMemcpyDeviceToDevice, s));
-            for (int k = 0; k < hist; k++) slot[k] = (head - hist + k + kHist) % kHist;
-            int nd = 0;
-            if (hist > 0) {
-                const double* a[rh::kDotMax];
-                const double* b[rh::kDotMax];
-                const int newest = slot[hist - 1];
-                for (int k = 0; k < hist; k++) {
-                    a[nd] = w.dF[newest];
-                    b[nd] = w.dF[slot[k]];
-                    nd++;
-                }
-                for (int k = 0; k < hist; k++) {
-                    a[nd] = w.dF[slot[k]];
-                    b[nd] = w.F;
-                    nd++;
-                }
-                RH_HIP(rh::launch_dots(nd, a, b, n3, w.dots, s));
-                RH_HIP(hipMemcpyAsync(hbuf + 3 * nb, w.dots, size_t(nd * db) * sizeof(double),
-                                      hipMemcpyDeviceToHost, s));
-            }
-            RH_HIP(hipMemcpyAsync(hbuf, w.part, size_t(3 * nb) * sizeof(double), hipMemcpyDeviceToHost, s));
-            RH_HIP(hipStreamSynchronize(s));
-            for (int64_t bb = 0; bb < nb; bb++) {
-                f2 += hbuf[3 * bb];
-                maxM = std::max(maxM, hbuf[3 * bb + 1]);
-                maxH = std::max(maxH, hbuf[3 * bb + 2]);
-            }
-            dv.assign(size_t(nd), 0.0);
-            for (int d = 0; d < nd; d++)
-                for (int64_t bb = 0; bb < db; bb++) dv[size_t(d)] += hbuf[3 * nb + d * db + bb];
-        } else {
-            // the update, the history differences, the copies and the dot
-            // products in one pass
-            rh::HistPack hp;
-            hp.Fp = w.Fp;
-            hp.xp = w.xp;
-            if (it > 1) {
-                hp.dFw = w.dF[head];
-                hp.dXw = w.dX[head];
-                head = (head + 1) % kHist;
-                hist = std::min(hist + 1, kHist);
-            }
+        // the update, the history differences, the copies and the dot
+        // products in one pass
+        rh::HistPack hp;
+        hp.Fp = w.Fp;
+        hp.xp = w.xp;
+        if (it > 1) {
+            hp.dFw = w.dF + head * w.stride;
+            hp.dXw = w.dX + head * w.stride;
+            head = (head + 1) % kHist;
+            hist = std::min(hist + 1, kHist);
+        }
+        for (int k = 0; k < hist; k++) {
+            slot[k] = (head - hist + k + kHist) % kHist;
+            hp.dF[k] = w.dF + slot[k] * w.stride;
+        }
+        hp.nh = hist;
+        RH_HIP(rh::launch_relax_step(n, d_mats, d_tab, d_hext, q->d_qdiag, w.y, w.x, w.F, d_H, w.part, hp, s));
+        RH_HIP(hipMemcpyAsync(hbuf, w.part, size_t(rh::kRelaxPart * nb) * sizeof(double), hipMemcpyDeviceToHost, s));
+        RH_HIP(hipStreamSynchronize(s));
+        dv.assign(size_t(2 * hist), 0.0);
+        for (int64_t bb = 0; bb < nb; bb++) {
+            const double* o = hbuf + rh::kRelaxPart * bb;
+            f2 += o[0];
+            maxM = std::max(maxM, o[1]);
+            maxH = std::max(maxH, o[2]);
             for (int k = 0; k < hist; k++) {
-                slot[k] = (head - hist + k + kHist) % kHist;
-                hp.dF[k] = w.dF[slot[k]];
-            }
-            hp.nh = hist;
-            RH_HIP(rh::launch_relax_step(n, d_mats, d_tab, d_hext, q->d_qdiag, w.y, w.x, w.F, d_H, w.part, hp,
-                                         s));
-            RH_HIP(hipMemcpyAsync(hbuf, w.part, size_t(rh::kRelaxPart * nb) * sizeof(double),
-                                  hipMemcpyDeviceToHost, s));
-            RH_HIP(hipStreamSynchronize(s));
-            dv.assign(size_t(2 * hist), 0.0);
-            for (int64_t bb = 0; bb < nb; bb++) {
-                const double* o = hbuf + rh::kRelaxPart * bb;
-                f2 += o[0];
-                maxM = std::max(maxM, o[1]);
-                maxH = std::max(maxH, o[2]);
-                for (int k = 0; k < hist; k++) {
-                    dv[size_t(k)] += o[3 + k];
-                    dv[size_t(hist + k)] += o[3 + rh::kHistMax + k];
-                }
+                dv[size_t(k)] += o[3 + k];
+                dv[size_t(hist + k)] += o[3 + rh::kHistMax + k];
             }
         }
         misfit = std::sqrt(f2 / double(n));
@@ -1178,9 +1134,9 @@ rh_status relax_run(rh_matrix* q, const double* d_mats, const double* d_tab, con
         v[nv] = w.F;
         c[nv++] = beta;
         for (int k = 0; k < hist; k++) {
-            v[nv] = w.dX[slot[k]];
+            v[nv] = w.dX + slot[k] * w.stride;
             c[nv++] = -gam[size_t(k)];
-            v[nv] = w.dF[slot[k]];
+            v[nv] = w.dF + slot[k] * w.stride;
             c[nv++] = -beta * gam[size_t(k)];
         }
         RH_HIP(rh::launch_lincomb(nv, v, c, n3, w.x, s));
@@ -1257,11 +1213,12 @@ struct NKWork {
 };
 
 rh_status nk_run(rh_matrix* q, const double* d_mats, const double* d_tab, const double* d_hext, double* d_M,
-                 double* d_H, const rh_relax_opts* opts, NKWork& k, RelaxWork& rw, double* hbuf, int64_t nb,
-                 int64_t db, rh_relax_result* res)
+                 double* d_H, const rh_relax_opts* opts, NKWork& k, RelaxWork& rw,
+                 rh_relax_result* res)
 {
     rh_model* m = q->m;
     hipStream_t s = m->stream;
+    const int64_t nb = rw.nb, db = rw.db;
     const int64_t n = m->host.n, n3 = q->n3;
     const double prec = opts->prec;
     const int max_mv = std::max(1, int(opts->max_iter));
@@ -1323,7 +1280,7 @@ rh_status nk_run(rh_matrix* q, const double* d_mats, const double* d_tab, const 
         o2.prec = 100.0 * prec;
         o2.max_iter = std::min(presmooth, max_mv);
         rh_relax_result r2{};
-        if ((st = relax_run(q, d_mats, d_tab, d_hext, d_M, d_H, &o2, rw, hbuf, nb, db, &r2)) != RH_OK) return st;
+        if ((st = relax_run(q, d_mats, d_tab, d_hext, d_M, d_H, &o2, rw, &r2)) != RH_OK) return st;
         mv += r2.matvecs;
         RH_HIP(hipMemcpyAsync(k.Mc, d_M, size_t(n3) * sizeof(double), hipMemcpyDeviceToDevice, s));
     } else {
@@ -1454,7 +1411,7 @@ rh_status nk_run(rh_matrix* q, const double* d_mats, const double* d_tab, const 
         o2.max_iter = std::min(50, max_mv - mv);
         rh_relax_result r2{};
         RH_HIP(hipMemcpyAsync(rw.x, k.Mc, size_t(n3) * sizeof(double), hipMemcpyDeviceToDevice, s));
-        if ((st = relax_run(q, d_mats, d_tab, d_hext, d_M, d_H, &o2, rw, hbuf, nb, db, &r2)) != RH_OK) return st;
+        if ((st = relax_run(q, d_mats, d_tab, d_hext, d_M, d_H, &o2, rw, &r2)) != RH_OK) return st;
         mv += r2.matvecs;
         RH_HIP(hipMemcpyAsync(k.Mc, d_M, size_t(n3) * sizeof(double), hipMemcpyDeviceToDevice, s));
         if ((st = evaluate(k.Mc, k.F, k.D, k.P, k.H, f2)) != RH_OK) return st;
@@ -1530,8 +1487,6 @@ rh_status rh_relax_tab_dev(rh_matrix* q, const double* d_mats, const double* d_t
         q->rw = rw;
     }
     RelaxWork& w = *q->rw;
-    const int64_t nb = w.nb;
-    const int64_t db = w.db;
     RH_HIP(hipMemsetAsync(w.x, 0, size_t(q->ld) * sizeof(double), s));
     // d_H starts the per-element nonlinear solves (previous local field); a
     // zero start keeps repeated solves bit-identical
@@ -1544,18 +1499,16 @@ rh_status rh_relax_tab_dev(rh_matrix* q, const double* d_mats, const double* d_t
             RH_HIP(hipMemcpy2DAsync(w.x + k, 3 * sizeof(double), d_mats + 13 + k, 16 * sizeof(double),
                                     sizeof(double), size_t(n), hipMemcpyDeviceToDevice, s));
     }
-    // pinned read-back of the host-driven loops: residual partials, then dot partials
-    double* hbuf = w.hbuf;
     const bool nk_method = (opts->method == 11);
     NKWork nk;
     if (nk_method) {
         const int km = opts->krylov_m > 0 ? std::max(2, int(opts->krylov_m)) : kKrylovDefault;
-        hipError_t e = nk.alloc(n, q->ld, km, nb, db, s);
+        hipError_t e = nk.alloc(n, q->ld, km, w.nb, w.db, s);
         if (e != hipSuccess) return fail(RH_ERR_NOMEM, std::string("Newton-Krylov work: ") + hipGetErrorString(e));
     }
     auto run = [&](const double* hx, const rh_relax_opts* o, bool keep) -> rh_status {
-        if (nk_method) return nk_run(q, d_mats, d_tab, hx, d_M, d_H, o, nk, w, hbuf, nb, db, res);
-        return relax_run(q, d_mats, d_tab, hx, d_M, d_H, o, w, hbuf, nb, db, res, nullptr, keep);
+        if (nk_method) return nk_run(q, d_mats, d_tab, hx, d_M, d_H, o, nk, w, res);
+        return relax_run(q, d_mats, d_tab, hx, d_M, d_H, o, w, res, keep);
     };
     rh_status st = run(d_hext, opts, false);
     if (st != RH_OK) return st;
@@ -1891,43 +1844,11 @@ rh_status rh_relax_adjoint_dev(rh_matrix* q, const double* d_mats, const double*
                 return fail(RH_ERR_UNSUPPORTED, "relaxation adjoint needs linear materials (kinds 0, 1)");
     }
     RelaxWork w;
-    RH_HIP(dalloc(&w.x, size_t(q->ld)));
-    RH_HIP(dalloc(&w.y, size_t(n3)));
-    RH_HIP(dalloc(&w.F, size_t(n3)));
-    RH_HIP(dalloc(&w.Fp, size_t(n3)));
-    RH_HIP(dalloc(&w.xp, size_t(n3)));
-    for (int k = 0; k < kHist; k++) {
-        RH_HIP(dalloc(&w.dX[k], size_t(n3)));
-        RH_HIP(dalloc(&w.dF[k], size_t(n3)));
-    }
-    const int64_t nb = rh::relax_blocks(n);
-    const int64_t db = rh::dot_blocks(n3);
-    RH_HIP(dalloc(&w.part, size_t(rh::kRelaxPart * nb)));
-    RH_HIP(dalloc(&w.dots, size_t(rh::kDotMax * db)));
-    AdjointPass ap;
-    ap.chunks = rh::matvec_t_chunks(n3, q->ld);
-    struct Free2 {
-        double** a;
-        double** b;
-        ~Free2()
-        {
-            dfree(*a);
-            dfree(*b);
-        }
-    } free2{&ap.mu, &ap.tpart};
-    RH_HIP(dalloc(&ap.mu, size_t(n3)));
-    RH_HIP(dalloc(&ap.tpart, size_t(ap.chunks * q->ld)));
+    RH_HIP(w.alloc(n, n3, q->ld, rh::matvec_t_chunks(n3, q->ld)));
     RH_HIP(hipMemsetAsync(w.x, 0, size_t(q->ld) * sizeof(double), s));
     if (opts->keep_m)
         RH_HIP(hipMemcpyAsync(w.x, d_lam, size_t(n3) * sizeof(double), hipMemcpyDeviceToDevice, s));
-    double* hbuf = nullptr;
-    RH_HIP(hipHostMalloc(reinterpret_cast<void**>(&hbuf), size_t(rh::kRelaxPart * nb + rh::kDotMax * db) * sizeof(double)));
-    struct PinnedFree {
-        double* p;
-        ~PinnedFree() { (void)hipHostFree(p); }
-    } pinned_guard{hbuf};
-    return relax_run(q, d_mats, nullptr, d_rhs, d_lam, w.y /* unused field output */, opts, w, hbuf, nb,
-                     db, res, &ap);
+    return relax_run_dev(q, d_mats, nullptr, d_rhs, d_lam, nullptr, opts, w, res, false, true);
 }
 
 rh_status rh_relax_adjoint(rh_matrix* q, const double* mats, const double* rhs, double* lam,

@@ -20,6 +20,7 @@
 #include "rh_far.hpp"
 #include "rh_geom.hpp"
 #include "rh_kernels.hpp"
+#include "rh_relax_step.hpp"
 #include "rh_mesh.hpp"
 
 namespace rh {
@@ -1058,13 +1059,6 @@ __global__ __launch_bounds__(256) void k_field_reduce(int64_t np, int64_t splits
 // ---------------------------------------------------------------- matrix pass
 typedef float nf4 __attribute__((ext_vector_type(4)));
 typedef double nd2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
 template <int RW>
 __global__ __launch_bounds__(256) void k_matvec_f32(const float* __restrict__ Q, int64_t nrows,
                                                     int64_t ld, const double* __restrict__ x,
@@ -1297,6 +1291,29 @@ __device__ __forceinline__ void solve_IminusA(const double* A, const double* b, 
     mat3_vec(inv, b, H);
 }
 
+// e^x - 1 for x <= 0, to about 1 ulp: x = k ln 2 + r, e^r - 1 = r + r^2 P(r)
+// with P a degree-10 Chebyshev interpolant on |r| <= ln(2)/2 (8.6e-19,
+// relative), then 2^k (e^r - 1) + (2^k - 1), whose second part is exact.
+__device__ __forceinline__ double expm1_neg(double x)
+{
+    x = (x < -40.0) ? -40.0 : x;  // e^-40 is below half an ulp of 1
+    const double k = rint(x * 1.4426950408889634);
+    const double r = fma(-k, kLn2Lo, fma(-k, kLn2Hi, x));
+    double p = 2.0914686968086876e-09;
+    p = fma(p, r, 2.5105217004720745e-08);
+    p = fma(p, r, 2.75572736431103e-07);
+    p = fma(p, r, 2.7557255400206422e-06);
+    p = fma(p, r, 2.4801587325547743e-05);
+    p = fma(p, r, 0.00019841269874820627);
+    p = fma(p, r, 0.0013888888888883748);
+    p = fma(p, r, 0.008333333333326136);
+    p = fma(p, r, 0.04166666666666667);
+    p = fma(p, r, 0.1666666666666667);
+    p = fma(p, r, 0.5);
+    const double e = fma(r * r, p, r), s = ldexp(1.0, int(k));
+    return fma(s, e, s - 1.0);
+}
+
 // secant susceptibility f(h)/h of the tanh-sum law (radmater.h:644-657), h >= 0
 __device__ __forceinline__ double frm_chi(const double* mat, double h)
 {
@@ -1306,8 +1323,9 @@ __device__ __forceinline__ double frm_chi(const double* mat, double h)
         const double ms = mat[2 + t], ks = mat[5 + t];
         if (ms == 0.0) continue;
         if (h > 0.0) {
-            const double u = ks * h / ms;
-            chi += (u < 1e-8) ? ks : ms * tanh(u) / h;
+            const double u = rh_div(ks * h, ms);
+            const double e = expm1_neg(-2.0 * fabs(u));
+            chi += (u < 1e-8) ? ks : ms * copysign(rh_div(-e, 2.0 + e), u) / h;
         } else {
             chi += ks;
         }
@@ -1380,19 +1398,25 @@ __device__ __forceinline__ void law_f_df(const double* mat, const double* tab, d
         df = a[2] + u * (2.0 * c2 + 3.0 * c3 * u);
         return;
     }
+    // The three terms side by side (an absent one has ks = 0 and adds 0).  An
+    // element's solve is a chain of about nine evaluations on one lane, so
+    // their length is the relaxation step's time: with the library's expm1 and
+    // four IEEE divisions a term a step of 8,000 elements took 38 us, with
+    // these 31.
     const int nt = int(mat[1]);
     f = 0.0;
     df = 0.0;
-    for (int t = 0; t < nt; t++) {
-        const double ms = mat[2 + t], ks = mat[5 + t];
-        if (ms == 0.0) continue;
-        const double u = ks * h / ms;
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        const bool on = t < nt && mat[2 + t] != 0.0;
+        const double ms = on ? mat[2 + t] : 1.0, ks = on ? mat[5 + t] : 0.0;
+        const double u = rh_div(ks * h, ms);
         // tanh u and sech^2 u from one expm1: with e = exp(-2|u|) - 1,
         // tanh|u| = -e / (2 + e) and sech^2 u = 4 (1 + e) / (2 + e)^2
-        const double e = expm1(-2.0 * fabs(u));
-        const double d = 2.0 + e;
-        f += ms * copysign(-e / d, u);
-        df += ks * (4.0 * (1.0 + e) / (d * d));
+        const double e = expm1_neg(-2.0 * fabs(u));
+        const double q = rh_rcp(2.0 + e);
+        f = fma(ms, copysign(-e * q, u), f);
+        df = fma(ks, 4.0 * (1.0 + e) * (q * q), df);
     }
 }
 
@@ -1738,40 +1762,6 @@ __global__ __launch_bounds__(256) void k_vcomb(int nv, const double* __restrict_
 }
 
 // ---------------------------------------------------------------- vector helpers
-struct DotPack {
-    const double* a[kDotMax];
-    const double* b[kDotMax];
-};
-
-// All nd dot products in one pass: every lane keeps nd running sums, waves
-// reduce by shuffles, the workgroup writes one partial per dot.
-__global__ __launch_bounds__(256) void k_dots(int nd, DotPack pk, int64_t len,
-                                              double* __restrict__ partials)
-{
-    __shared__ double red[4][kDotMax];
-    double acc[kDotMax];
-#pragma unroll
-    for (int d = 0; d < kDotMax; d++) acc[d] = 0.0;
-    for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < len;
-         i += int64_t(gridDim.x) * 256) {
-#pragma unroll
-        for (int d = 0; d < kDotMax; d++)
-            if (d < nd) acc[d] += pk.a[d][i] * pk.b[d][i];
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int d = 0; d < kDotMax; d++) {
-        if (d < nd) {
-            const double v = wave_sum(acc[d]);
-            if (lane == 0) red[wave][d] = v;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x < nd)
-        partials[threadIdx.x * gridDim.x + blockIdx.x] =
-            red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
-}
-
 struct CombPack {
     const double* v[kCombMax];
     double c[kCombMax];
@@ -1788,87 +1778,23 @@ __global__ __launch_bounds__(256) void k_lincomb(int nv, CombPack pk, int64_t le
     }
 }
 
-__device__ __forceinline__ double wave_max(double v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
-// One relaxation step with its Anderson bookkeeping (one wave per block):
-// lane i updates element i; dF[k] (k < nh, oldest first) are the stored
-// differences, the newest of which (dF[nh - 1]) is the one written here when
-// dFw is set.
-static_assert(kRelaxLanes == 64, "k_relax_step reduces over one wave per block");
-__device__ __forceinline__ void relax_step_block(int64_t n, const double* __restrict__ mats,
-                                                 const double* __restrict__ tab,
-                                                 const double* __restrict__ hext,
-                                                 const double* __restrict__ qdiag,
-                                                 const double* __restrict__ y, const double* __restrict__ M,
-                                                 double* __restrict__ F, double* __restrict__ Hout,
-                                                 double* __restrict__ partials, double* Fp, double* xp,
-                                                 double* dFw, double* dXw, const double* const* dF, int nh)
-{
-    const int64_t i = int64_t(blockIdx.x) * kRelaxLanes + threadIdx.x;
-    double f2 = 0.0, mm = 0.0, hh = 0.0;
-    double dd[2 * kHistMax];
-#pragma unroll
-    for (int k = 0; k < 2 * kHistMax; k++) dd[k] = 0.0;
-    if (i < n) {
+// The element update of the relaxation: H_i = (I - Q_ii K)^{-1} (y + hext + ...)
+// by the element's material law, started from the previous local field.
+struct MaterialLaw {
+    const double *mats, *tab, *hext, *qdiag, *y;
+    double* Hout;
+    __device__ __forceinline__ void operator()(int64_t i, double* mp, double& hh) const
+    {
+        double hl[3];
         const double heff[3] = {y[3 * i] + hext[3 * i], y[3 * i + 1] + hext[3 * i + 1],
                                 y[3 * i + 2] + hext[3 * i + 2]};
         const double warm = sqrt(Hout[3 * i] * Hout[3 * i] + Hout[3 * i + 1] * Hout[3 * i + 1] +
                                  Hout[3 * i + 2] * Hout[3 * i + 2]);
-        double mp[3], hl[3];
         local_solve(mats + 16 * i, qdiag + 9 * i, heff, mp, hl, tab, warm);
-        double fi[3], dfn[3] = {0.0, 0.0, 0.0};
-        for (int k = 0; k < 3; k++) {
-            const int64_t j = 3 * i + k;
-            const double xk = M[j];
-            const double d = mp[k] - xk;
-            fi[k] = d;
-            F[j] = d;
-            Hout[j] = hl[k];
-            f2 += d * d;
-            if (dFw) {
-                dfn[k] = d - Fp[j];
-                dFw[j] = dfn[k];
-                dXw[j] = xk - xp[j];
-            }
-            Fp[j] = d;
-            xp[j] = xk;
-        }
-        mm = sqrt(mp[0] * mp[0] + mp[1] * mp[1] + mp[2] * mp[2]);
+        for (int k = 0; k < 3; k++) Hout[3 * i + k] = hl[k];
         hh = sqrt(hl[0] * hl[0] + hl[1] * hl[1] + hl[2] * hl[2]);
-#pragma unroll
-        for (int h = 0; h < kHistMax; h++) {
-            if (h < nh) {
-                double a = 0.0, b = 0.0;
-                for (int k = 0; k < 3; k++) {
-                    const double v = (h == nh - 1) ? dfn[k] : dF[h][3 * i + k];
-                    a += dfn[k] * v;
-                    b += v * fi[k];
-                }
-                dd[h] = a;
-                dd[kHistMax + h] = b;
-            }
-        }
     }
-    f2 = wave_sum(f2);
-    mm = wave_max(mm);
-    hh = wave_max(hh);
-#pragma unroll
-    for (int k = 0; k < 2 * kHistMax; k++)
-        if ((k % kHistMax) < nh) dd[k] = wave_sum(dd[k]);
-    if (threadIdx.x == 0) {
-        double* o = partials + int64_t(kRelaxPart) * blockIdx.x;
-        o[0] = f2;
-        o[1] = mm;
-        o[2] = hh;
-#pragma unroll
-        for (int k = 0; k < 2 * kHistMax; k++) o[3 + k] = dd[k];
-    }
-}
+};
 
 __global__ __launch_bounds__(kRelaxLanes) void k_relax_step(int64_t n, const double* __restrict__ mats,
                                                             const double* __restrict__ tab,
@@ -1880,164 +1806,8 @@ __global__ __launch_bounds__(kRelaxLanes) void k_relax_step(int64_t n, const dou
                                                             double* __restrict__ Hout,
                                                             double* __restrict__ partials, HistPack hp)
 {
-    relax_step_block(n, mats, tab, hext, qdiag, y, M, F, Hout, partials, hp.Fp, hp.xp, hp.dFw, hp.dXw, hp.dF,
-                     hp.nh);
-}
-
-// The Anderson step of the device-driven loop on one wave: the step partials
-// reduced across the wave in a fixed order, then the residual and convergence
-// test, the restart safeguard, the Gram matrix of the differences in use
-// (kept oldest first, the newest row from this step), the regularized
-// Cholesky solve of the least-squares problem and the update coefficients,
-// and the history extension for the next iteration.  The Gram matrix lives in
-// LDS; the factorization runs column by column with the lanes updating the
-// trailing entries (the same operations in the same order as a row-by-row
-// factorization), and the two triangular solves column by column.
-__device__ void anderson_wave(int64_t nb, const double* __restrict__ partials, RelaxDevState* __restrict__ st)
-{
-    constexpr int H = kHistMax, HP = kHistMax + 1;  // LDS row stride
-    __shared__ double sA[H * HP], sL[H * HP], sz[H], sv[kRelaxPart];
-    const int lane = threadIdx.x & 63;
-    double v[kRelaxPart];
-#pragma unroll
-    for (int k = 0; k < kRelaxPart; k++) v[k] = 0.0;
-    for (int64_t b = lane; b < nb; b += 64) {
-        const double* o = partials + int64_t(kRelaxPart) * b;
-        v[0] += o[0];
-        v[1] = fmax(v[1], o[1]);
-        v[2] = fmax(v[2], o[2]);
-#pragma unroll
-        for (int k = 3; k < kRelaxPart; k++) v[k] += o[k];
-    }
-    v[0] = wave_sum(v[0]);
-    v[1] = wave_max(v[1]);
-    v[2] = wave_max(v[2]);
-#pragma unroll
-    for (int k = 3; k < kRelaxPart; k++) v[k] = wave_sum(v[k]);
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < kRelaxPart; k++) sv[k] = v[k];
-    }
-    __syncthreads();
-    // wave-uniform decisions (every lane reads the same state)
-    const int hist = st->hist;
-    const int head = st->head;
-    const int it = st->it + 1;
-    const double misfit = sqrt(v[0] / st->n);
-    const bool finite = isfinite(misfit);
-    const bool finish = !finite || misfit <= st->prec || it >= st->max_iter;
-    const bool restart = !finish && misfit > 1e4 * st->best;
-    const double best = fmin(st->best, misfit);
-    const double beta = restart ? fmax(0.05, 0.5 * st->beta) : st->beta;
-    bool ok = !finish && !restart && hist > 0;
-    if (ok) {
-        // Gram matrix: live part from the state with the newest row and
-        // column from this step; its regularized copy to factor in sL
-        for (int e = lane; e < H * H; e += 64) {
-            const int a = e / H, c = e - H * (e / H);
-            double g = 0.0;
-            if (a < hist && c < hist) {
-                if (a == hist - 1) g = sv[3 + c];
-                else if (c == hist - 1) g = sv[3 + a];
-                else g = st->G[a * H + c];
-            }
-            sA[a * HP + c] = g;
-        }
-        __syncthreads();
-        double tr = 0.0;
-        for (int a = 0; a < hist; a++) tr += sA[a * HP + a];
-        const double lam = 1e-10 * (tr > 0 ? tr / hist : 1.0);
-        for (int e = lane; e < H * H; e += 64) {
-            const int a = e / H, c = e - H * (e / H);
-            sL[a * HP + c] = sA[a * HP + c] + ((a == c && a < hist) ? lam : 0.0);
-        }
-        __syncthreads();
-        // Cholesky, column k at a time: pivot, the column below it, then the
-        // trailing entries (i, j), k < j <= i, lose L_ik L_jk
-        for (int k = 0; k < hist && ok; k++) {
-            const double dkk = sL[k * HP + k];
-            if (!(dkk > 0.0)) {
-                ok = false;
-                break;
-            }
-            const double lkk = sqrt(dkk);
-            __syncthreads();
-            if (lane == k) sL[k * HP + k] = lkk;
-            if (lane > k && lane < hist) sL[lane * HP + k] = sL[lane * HP + k] / lkk;
-            __syncthreads();
-            for (int e = lane; e < H * H; e += 64) {
-                const int i = e / H, j = e - H * (e / H);
-                if (j > k && i >= j && i < hist) sL[i * HP + j] -= sL[i * HP + k] * sL[j * HP + k];
-            }
-            __syncthreads();
-        }
-    }
-    if (ok) {
-        // L z = r, then L^T gam = z, column by column (gam overwrites z)
-        if (lane < hist) sz[lane] = sv[3 + kHistMax + lane];
-        __syncthreads();
-        for (int k = 0; k < hist; k++) {
-            const double zk = sz[k] / sL[k * HP + k];
-            __syncthreads();
-            if (lane == k) sz[k] = zk;
-            if (lane > k && lane < hist) sz[lane] -= sL[lane * HP + k] * zk;
-            __syncthreads();
-        }
-        for (int k = hist - 1; k >= 0; k--) {
-            const double gk = sz[k] / sL[k * HP + k];
-            __syncthreads();
-            if (lane == k) sz[k] = gk;
-            if (lane < k) sz[lane] -= sL[k * HP + lane] * gk;
-            __syncthreads();
-        }
-    }
-    // state of the next iteration
-    if (lane == 0) {
-        st->arrive = 0;  // every block of this step has arrived
-        st->it = it;
-        st->misfit = misfit;
-        st->maxM = fmax(1e-17, v[1]);
-        st->maxH = fmax(1e-17, v[2]);
-        if (!finite) {
-            st->fail = 1;
-            st->done = 2;
-        } else if (misfit <= st->prec && it == 1 && st->keep_if_converged) {
-            st->done = 2;
-        } else if (finish) {
-            st->done = 1;
-        } else {
-            st->best = best;
-            st->beta = beta;
-            const int nh = ok ? hist : 0, hd = ok ? head : 0;
-            st->cF = beta;
-            for (int c = 0; c < H; c++) {
-                st->cdX[c] = 0.0;
-                st->cdF[c] = 0.0;
-            }
-            if (ok) {
-                const int r0 = (head - hist + 2 * H) % H;  // buffer slot of the oldest difference
-                for (int k = 0; k < hist; k++) {
-                    const int p = (r0 + k) % H;
-                    st->cdX[p] = -sz[k];
-                    st->cdF[p] = -beta * sz[k];
-                }
-            }
-            // the next iteration writes a new difference into slot hd
-            st->ext = 1;
-            st->head = (hd + 1) % H;
-            st->hist = nh + 1 < H ? nh + 1 : H;
-        }
-    }
-    // the Gram matrix of the next iteration: the oldest difference drops out
-    // when the history is full
-    if (ok) {
-        const int sh = (hist == H) ? 1 : 0;
-        for (int e = lane; e < H * H; e += 64) {
-            const int a = e / H, c = e - H * (e / H);
-            const int a2 = a + sh, c2 = c + sh;
-            st->G[e] = (a2 < H && c2 < H) ? sA[a2 * HP + c2] : 0.0;
-        }
-    }
+    relax_step_block(n, MaterialLaw{mats, tab, hext, qdiag, y, Hout}, M, F, partials, hp.Fp, hp.xp, hp.dFw, hp.dXw,
+                     hp.dF, hp.nh);
 }
 
 // The same step in the device-driven loop (history slots from the state); the
@@ -2053,24 +1823,7 @@ __global__ __launch_bounds__(kRelaxLanes) void k_relax_step_dev(int64_t n, const
                                                                 double* __restrict__ partials, HistBufs hb,
                                                                 RelaxDevState* __restrict__ st)
 {
-    if (st->done) return;
-    const int nh = st->hist, head = st->head;
-    const double* dF[kHistMax];
-#pragma unroll
-    for (int k = 0; k < kHistMax; k++) dF[k] = hb.dF[(head - nh + k + 2 * kHistMax) % kHistMax];
-    const int w = (head - 1 + kHistMax) % kHistMax;
-    relax_step_block(n, mats, tab, hext, qdiag, y, M, F, Hout, partials, hb.Fp, hb.xp,
-                     st->ext ? hb.dF[w] : nullptr, st->ext ? hb.dX[w] : nullptr, dF, nh);
-    // release this block's partials, then count it in
-    int arrived = 0;
-    if (threadIdx.x == 0) {
-        __threadfence();
-        arrived = atomicAdd(&st->arrive, 1);
-    }
-    arrived = __shfl(arrived, 0, 64);
-    if (arrived != int(gridDim.x) - 1) return;
-    __threadfence();  // the other blocks' partials are visible to the last one
-    anderson_wave(int64_t(gridDim.x), partials, st);
+    relax_step_dev(n, MaterialLaw{mats, tab, hext, qdiag, y, Hout}, M, F, partials, hb, st);
 }
 
 // The update of the device-driven loop (grid-stride over the 3n components).
@@ -2081,24 +1834,10 @@ __global__ __launch_bounds__(256) void k_update_dev(int64_t n3, double* __restri
 {
     const int done = st->done;
     if (done == 2) return;
-    if (done == 1) {
-        for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n3; i += int64_t(gridDim.x) * 256)
-            M_out[i] = x[i] + F[i];
-        return;
-    }
-    const double cF = st->cF;
-    double cX[kHistMax], cD[kHistMax];
-#pragma unroll
-    for (int b = 0; b < kHistMax; b++) {
-        cX[b] = st->cdX[b];
-        cD[b] = st->cdF[b];
-    }
+    const UpdateCoef c(st);
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < n3; i += int64_t(gridDim.x) * 256) {
-        double acc = x[i] + cF * F[i];
-#pragma unroll
-        for (int b = 0; b < kHistMax; b++)
-            if (cX[b] != 0.0 || cD[b] != 0.0) acc += cX[b] * hb.dX[b][i] + cD[b] * hb.dF[b][i];
-        x[i] = acc;
+        if (done == 1) M_out[i] = x[i] + F[i];
+        else x[i] = c.apply(x[i], F, hb, i);
     }
 }
 
@@ -2458,19 +2197,6 @@ hipError_t launch_vcomb(int nv, const double* V, int64_t ldv, const double* c, c
 }
 
 int64_t dot_blocks(int64_t len) { return std::max<int64_t>(1, std::min<int64_t>(128, (len + 511) / 512)); }
-
-hipError_t launch_dots(int nd, const double* const* a, const double* const* b, int64_t len,
-                       double* partials, hipStream_t s)
-{
-    if (nd < 1 || nd > kDotMax) return hipErrorInvalidValue;
-    DotPack pk;
-    for (int d = 0; d < nd; d++) {
-        pk.a[d] = a[d];
-        pk.b[d] = b[d];
-    }
-    hipLaunchKernelGGL(k_dots, dim3(unsigned(dot_blocks(len))), dim3(256), 0, s, nd, pk, len, partials);
-    return hipGetLastError();
-}
 
 hipError_t launch_lincomb(int nv, const double* const* v, const double* c, int64_t len, double* y,
                           hipStream_t s)

@@ -120,14 +120,9 @@ hipError_t launch_relax_update(int64_t n, const double* mats, const double* tab,
 // with the newest difference, padding to kHistMax, nh dots with F, padding].
 // Anderson depth: on the 40,000-tetrahedron yoke (prec 1e-5) 16 differences
 // took 55-59 iterations where 8 took 60-85 (over mixing factors 0.3-0.9)
-#ifndef RH_HIST
-#define RH_HIST 16
-#endif
-constexpr int kHistMax = RH_HIST;
+constexpr int kHistMax = 16;
 constexpr int kRelaxPart = 3 + 2 * kHistMax;
-// dot products and combined vectors of one host-driven Anderson iteration
-// (launch_dots, launch_lincomb)
-constexpr int kDotMax = 2 * kHistMax + 1;
+// combined vectors of one host-driven Anderson iteration (launch_lincomb)
 constexpr int kCombMax = 2 * kHistMax + 2;
 struct HistPack {
     double* Fp = nullptr;
@@ -168,8 +163,9 @@ struct RelaxDevState {
 struct HistBufs {
     double* Fp;
     double* xp;
-    double* dF[kHistMax];
-    double* dX[kHistMax];
+    double* dF;      // slot b at dF + b * stride, dX likewise
+    double* dX;
+    int64_t stride;
 };
 // relaxation step of the device-driven loop (slots and history from st); the
 // last of its blocks to finish runs the Anderson step (reduction of the nb
@@ -211,11 +207,7 @@ hipError_t launch_mdot(int nv, const double* V, int64_t ldv, const double* w, in
 hipError_t launch_vcomb(int nv, const double* V, int64_t ldv, const double* c, const double* base, double cb,
                         int64_t len, double* out, hipStream_t s);
 
-// Batched dot products: out[k*nb + b] = partial of sum_i a_k[i]*b_k[i] over block b.
 int64_t dot_blocks(int64_t len);
-hipError_t launch_dots(int nd, const double* const* a, const double* const* b, int64_t len,
-                       double* partials, hipStream_t s);
-
 // y = sum_k c_k v_k (k < nv <= 34); y may alias v_0.
 hipError_t launch_lincomb(int nv, const double* const* v, const double* c, int64_t len, double* y,
                           hipStream_t s);
@@ -251,17 +243,20 @@ hipError_t launch_adj_geom(const DevModel& m, const double* adj, const int64_t* 
 // part: chunks * ld doubles.
 int64_t matvec_t_chunks(int64_t nrows, int64_t ld);
 hipError_t launch_matvec_t(const void* Q, int elem_bytes, int64_t nrows, int64_t ld, const double* x,
-                           double* part, int64_t chunks, double* y, hipStream_t s);
+                           double* part, int64_t chunks, double* y, hipStream_t s, const int32_t* skip);
 // The same over nel element rows of the symmetric-block layout (part: chunks *
-// 3*ldp doubles).
+// 3*ldp doubles).  Both return at once where *skip is set.
 hipError_t launch_matvec_t_sym(const void* Q, int elem_bytes, int planes, int64_t nel, int64_t ldp,
-                               const double* x, double* part, int64_t chunks, double* y, hipStream_t s);
-// mu_i = rowT_i^T K_i^T lam_i (rowt may be null).
-hipError_t launch_adj_scale(int64_t n, const double* mats, const double* rowt, const double* lam,
-                            double* mu, hipStream_t s);
-// Block-Jacobi update of (I - Q^T K^T) lam = rhs (linear materials).
-hipError_t launch_adj_update(int64_t n, const double* mats, const double* rhs, const double* qdiag,
-                             const double* y, const double* lam, double* F, double* partials,
-                             hipStream_t s);
+                               const double* x, double* part, int64_t chunks, double* y, hipStream_t s,
+                               const int32_t* skip);
+// mu_i = K_i^T lam_i.
+hipError_t launch_adj_scale(int64_t n, const double* mats, const double* lam, double* mu, hipStream_t s);
+// Block-Jacobi step and update of (I - Q^T K^T) lam = rhs (linear materials) in
+// the device-driven loop; the update also refreshes mu_i = K_i^T lam_i.
+hipError_t launch_adj_step_dev(int64_t n, const double* mats, const double* rhs, const double* qdiag, const double* y,
+                               const double* lam, double* F, double* partials, const HistBufs& hb,
+                               RelaxDevState* st, hipStream_t s);
+hipError_t launch_adj_update_dev(int64_t n, const double* mats, double* lam, double* mu, const double* F,
+                                 const HistBufs& hb, double* lam_out, const RelaxDevState* st, hipStream_t s);
 
 }  // namespace rh
