@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void k_adj_m(DevModel m, const double* __restr
                             gl[k] = gp[k];
                         }
                     }
-                    const bool in = eval_elem<double>(kind, rec, xl, q6);
+                    const bool in = eval_k<double, -1>(kind, rec, xl, q6);
                     const double e = (in && addin) ? 1.0 : 0.0;
                     v[0] += (q6[0] + e) * gl[0] + q6[3] * gl[1] + q6[4] * gl[2];
                     v[1] += q6[3] * gl[0] + (q6[1] + e) * gl[1] + q6[5] * gl[2];

@@ -9,6 +9,7 @@
 
 #include <type_traits>
 
+#include "rh_far.hpp"
 #include "rh_math.hpp"
 
 namespace rh {
@@ -45,10 +46,15 @@ RH_HD void mat3_vec(const double* m, const double v[3], double o[3])
 template <class R, int KIND>
 RH_HD bool eval_k(int kind, const double* __restrict__ rec, const double p[3], double q6[6])
 {
-    if (KIND == 0) return eval_rec<R>(rec, p, q6);
-    if (KIND == 1) return eval_tet<R>(rec, p, q6);
-    if (KIND == 2) return eval_gen<R>(rec, p, q6);
-    return eval_elem<R>(kind, rec, p, q6);
+    if (KIND == 0 || (KIND < 0 && kind == EK_REC)) {
+#ifdef __HIP_DEVICE_COMPILE__
+        return rec_block<R>(rec, p, q6);
+#else
+        return eval_rec<R>(rec, p, q6);
+#endif
+    }
+    if (KIND == 1 || (KIND < 0 && kind == EK_TET)) return eval_tet<R>(rec, p, q6);
+    return eval_gen<R>(rec, p, q6);
 }
 
 // Sum over copies of F_c Q_j(x'), without the row transform.

@@ -485,6 +485,14 @@ __device__ __forceinline__ void field_store(double* __restrict__ B, double* __re
     }
 }
 
+// Blocks without transform copies: the workgroup copies kRecTile records and
+// magnetizations to LDS first.  Read from memory they are a chain of three
+// scalar loads (list, offset, record) per element, which two waves a SIMD do
+// not hide: a host call of 10,000 points on 512 blocks 167 us by that chain,
+// 163 from LDS.  More waves a SIMD (3 or 4, the near form spilling) 171 and 184.
+constexpr int kRecTile = 64;
+constexpr int kRecStage = 6 + 3;
+
 template <class R, bool SYM, int KIND, int PASS>
 __global__ __launch_bounds__(256) void k_field(DevModel m, const double* __restrict__ M,
                                                const double* __restrict__ pts, int64_t np,
@@ -492,13 +500,49 @@ __global__ __launch_bounds__(256) void k_field(DevModel m, const double* __restr
                                                double* __restrict__ H, double* __restrict__ part)
 {
     const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (p >= np) return;
+    const bool live = p < np;
     const int64_t kend = m.koff[KIND + 1];
     const int64_t k0 = m.koff[KIND] + int64_t(blockIdx.y) * js;
     const int64_t k1 = (k0 + js < kend) ? (k0 + js) : kend;
-    const double x[3] = {pts[3 * p], pts[3 * p + 1], pts[3 * p + 2]};
+    double x[3] = {0, 0, 0};
+    if (live) {
+        x[0] = pts[3 * p];
+        x[1] = pts[3 * p + 1];
+        x[2] = pts[3 * p + 2];
+    }
     double b[3] = {0, 0, 0}, h[3] = {0, 0, 0};
-    field_add<R, SYM, KIND, PASS>(view(m), M, m.kidx, k0, k1, x, b, h);
+    if constexpr (KIND == 0 && !SYM) {
+        __shared__ double tile[kRecTile * kRecStage];
+        for (int64_t base = k0; base < k1; base += kRecTile) {
+            const int cnt = int((k1 - base < kRecTile) ? (k1 - base) : kRecTile);
+            __syncthreads();  // the previous tile has been consumed
+            if (int(threadIdx.x) < cnt) {
+                const int64_t j = m.kidx[base + threadIdx.x];
+                const double* rec = m.data + m.off[j];
+                double* o = tile + kRecStage * threadIdx.x;
+                for (int k = 0; k < 6; k++) o[k] = rec[k];
+                for (int k = 0; k < 3; k++) o[6 + k] = M[3 * j + k];
+            }
+            __syncthreads();
+            if (!live) continue;
+#pragma unroll 1
+            for (int q = 0; q < cnt; q++) {
+                const double* rec = tile + kRecStage * q;
+                const double mm[3] = {rec[6], rec[7], rec[8]};
+                double hl[3];
+                bool in;
+                if (!elem_H<R, KIND, PASS>(EK_REC, rec, nullptr, mm, x, hl, in)) continue;
+                for (int k = 0; k < 3; k++) {
+                    h[k] += hl[k];
+                    b[k] += hl[k] + (in ? mm[k] : 0.0);
+                }
+            }
+        }
+        if (!live) return;
+    } else {
+        if (!live) return;
+        field_add<R, SYM, KIND, PASS>(view(m), M, m.kidx, k0, k1, x, b, h);
+    }
     if (part)
         field_store<PASS>(part + ((slice0 + int64_t(blockIdx.y)) * np + p) * 6, b, h);
     else

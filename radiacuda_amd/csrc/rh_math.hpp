@@ -1044,12 +1044,4 @@ RH_HD bool eval_gen(const double* __restrict__ rec, const double p[3], double q6
     return inside;
 }
 
-template <class R>
-RH_HD bool eval_elem(int kind, const double* __restrict__ rec, const double p[3], double q6[6])
-{
-    if (kind == EK_TET) return eval_tet<R>(rec, p, q6);
-    if (kind == EK_REC) return eval_rec<R>(rec, p, q6);
-    return eval_gen<R>(rec, p, q6);
-}
-
 }  // namespace rh
