@@ -27,21 +27,22 @@ namespace rh {
 namespace {
 
 constexpr int kAdjSliceE = 64;   // elements per workgroup slice (dL/dM), at most
+constexpr int kAdjHex = 8;       // hexahedron records staged at a time (dL/dM)
 constexpr int kAdjSliceV = 128;  // vertices per workgroup slice (dL/dvertex)
 
 // dL/dM partials: part[bx][j][3] for the elements of slice blockIdx.y.
 // FP64-issue bound where the blocks fill the chip: 1,000 hexahedra at 2,048
 // points, 8 tiles, 279 us in 1,000 blocks of 8 elements and 816 us in 128
-// blocks of 64.
+// blocks of 64; 165 us with hexahedron records from LDS (gen_block).
 template <bool SYM>
-__global__ __launch_bounds__(256) void k_adj_m(DevModel m, const double* __restrict__ pts,
+__global__ __launch_bounds__(256, 2) void k_adj_m(DevModel m, const double* __restrict__ pts,
                                                int64_t np, const double* __restrict__ g,
                                                int addin, int slice, double* __restrict__ part)
 {
     __shared__ double acc[4][kAdjSliceE * 3];
+    __shared__ double hexes[kAdjHex * kHex];  // hexahedron records
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < 4 * kAdjSliceE * 3; i += 256) (&acc[0][0])[i] = 0.0;
-    __syncthreads();
     const int64_t j0 = int64_t(blockIdx.y) * slice;
     const int64_t j1 = (j0 + slice < m.n) ? (j0 + slice) : m.n;
     const int64_t tiles = (np + 255) / 256;
@@ -53,8 +54,19 @@ __global__ __launch_bounds__(256) void k_adj_m(DevModel m, const double* __restr
         const double gp[3] = {live ? g[3 * p] : 0.0, live ? g[3 * p + 1] : 0.0,
                               live ? g[3 * p + 2] : 0.0};
         for (int64_t j = j0; j < j1; j++) {
+            const int r = int(j - j0) % kAdjHex;
+            if (r == 0) {
+                __syncthreads();  // the previous records have been consumed
+                const int cnt = int((j1 - j < kAdjHex) ? (j1 - j) : kAdjHex);
+                for (int i = threadIdx.x; i < cnt * kHex; i += 256) {
+                    const int q = i / kHex, at = m.hex_at[j + q];
+                    if (at >= 0) hexes[i] = m.hex[int64_t(kHex) * at + i - kHex * q];
+                }
+                __syncthreads();
+            }
             const int kind = m.kind[j];
             const double* rec = m.data + m.off[j];
+            const double* hex = (m.hex_at[j] >= 0) ? hexes + kHex * r : nullptr;
             double v[3] = {0.0, 0.0, 0.0};
             if (live) {
                 for (int64_t c = m.copy_off[j]; c < m.copy_off[j + 1]; c++) {
@@ -71,7 +83,7 @@ __global__ __launch_bounds__(256) void k_adj_m(DevModel m, const double* __restr
                             gl[k] = gp[k];
                         }
                     }
-                    const bool in = eval_k<double, -1>(kind, rec, xl, q6);
+                    const bool in = hex ? gen_block(hex, rec, xl, q6) : eval_k<double, -1>(kind, rec, xl, q6);
                     const double e = (in && addin) ? 1.0 : 0.0;
                     v[0] += (q6[0] + e) * gl[0] + q6[3] * gl[1] + q6[4] * gl[2];
                     v[1] += q6[3] * gl[0] + (q6[1] + e) * gl[1] + q6[5] * gl[2];

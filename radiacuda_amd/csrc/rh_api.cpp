@@ -239,6 +239,8 @@ struct rh_model {
     int32_t* d_kidx = nullptr;
     double* d_charged = nullptr;  // field-only tetrahedron records, rebuilt per field call
     double* d_far = nullptr;      // far-form tetrahedron records of the assembly
+    double* d_hex = nullptr;      // far-form hexahedron records
+    int32_t* d_hex_at = nullptr;  // an element's hexahedron record
     // adjoint geometry, uploaded on the first adjoint call
     double* d_adj = nullptr;
     int64_t* d_adj_off = nullptr;
@@ -313,6 +315,8 @@ void free_model(rh_model* m)
     dfree(m->d_kidx);
     dfree(m->d_charged);
     dfree(m->d_far);
+    dfree(m->d_hex);
+    dfree(m->d_hex_at);
     dfree(m->d_adj);
     dfree(m->d_adj_off);
     dfree(m->d_vert_off);
@@ -406,6 +410,9 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
     if (e == hipSuccess)
         e = dalloc(&m->d_charged, size_t(rh::kChargedTet * (P.kind_off[2] - P.kind_off[1])));
     if (e == hipSuccess) e = dalloc(&m->d_far, size_t(rh::far_tet_doubles(P.kind_off[2] - P.kind_off[1])));
+    const int64_t ngen = P.kind_off[3] - P.kind_off[2];
+    if (e == hipSuccess) e = dalloc(&m->d_hex, size_t(rh::hex_doubles(ngen)));
+    if (e == hipSuccess) e = dalloc(&m->d_hex_at, size_t(P.n));
     rh::DevModel& d = m->dev;
     d.n = P.n;
     d.kind = m->d_kind;
@@ -417,10 +424,12 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
     d.rowt = m->d_rowt;
     d.kidx = m->d_kidx;
     d.far_tet = m->d_far;
+    d.hex = m->d_hex;
+    d.hex_at = m->d_hex_at;
     for (int k = 0; k < 4; k++) d.koff[k] = P.kind_off[k];
     d.sym = P.sym;
     d.rowt_identity = P.rowt_identity;
-    if (e == hipSuccess) e = rh::launch_far_records(d, m->d_far, s);
+    if (e == hipSuccess) e = rh::launch_far_records(d, m->d_far, m->d_hex, m->d_hex_at, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         std::string msg = std::string("model upload: ") + hipGetErrorString(e);

@@ -36,7 +36,114 @@ constexpr int kFarG32 = kFarG + kFarGeo;                    // 78
 constexpr int kFarN3 = kFarG32 + (kFarGeo + 1) / 2;         // 89
 constexpr int kFarTet = kFarN3 + 3;                         // 92 doubles
 
+// Record of a hexahedron (a general polyhedron of six quadrilaterals) for the
+// far form, its vertices renumbered to one topology: 0-3 around a face, 4 + i
+// across from i.  Vertices (24), W xx xy xz yy yz of the 12 edges (60), 2 len
+// (12), len^2 (12), -2 (n_f n_f^T - n_5 n_5^T) of faces 0-4 (25), for each of
+// these n and four times the areas of its two triangles (25) and the squared
+// diagonal between them (5), the squared limit distance and n_5.
+constexpr int kHexW = 24, kHexL = 84, kHexL2 = 96, kHexT = 108, kHexF = 133, kHexD2 = 158, kHexR2 = 163, kHexN5 = 164,
+              kHex = 168;
+
 #ifdef __HIPCC__
+// vertex k of face f, edges' ends, edges and their order around a face
+constexpr int kHexFace[6][4] = {{0, 1, 2, 3}, {0, 1, 5, 4}, {1, 2, 6, 5}, {2, 3, 7, 6}, {3, 0, 4, 7}, {4, 5, 6, 7}};
+constexpr int kHexEdgeA[12] = {0, 1, 2, 3, 4, 5, 6, 7, 0, 1, 2, 3};
+constexpr int kHexEdgeB[12] = {1, 2, 3, 0, 5, 6, 7, 4, 4, 5, 6, 7};
+constexpr int kHexFaceEdge[5][4] = {{0, 1, 2, 3}, {0, 9, 4, 8}, {1, 10, 5, 9}, {2, 11, 6, 10}, {3, 8, 7, 11}};
+
+// Its parts from an element record of 8 vertices, 12 edges, 6 faces and 24
+// face corners; false if they are not a hexahedron's.
+constexpr int kHexIn = kGenHdr + 24 + 12 * kGenEdge + 6 * kGenFace + 24;
+constexpr int kHexInE = kGenHdr + 24, kHexInF = kHexInE + 12 * kGenEdge, kHexInV = kHexInF + 6 * kGenFace;
+__device__ inline bool hex_vertices(const double* rec, int* id)
+{
+    const double *ed = rec + kHexInE, *fc = rec + kHexInF, *fv = rec + kHexInV;
+    for (int f = 0; f < 6; f++)
+        if (int(fc[kGenFace * f + 4]) != 4) return false;
+    for (int i = 0; i < 4; i++) id[i] = int(fv[int(fc[3]) + i]);
+    for (int i = 0; i < 4; i++) {
+        id[4 + i] = -1;
+        for (int e = 0; e < 12; e++) {
+            const int a = int(ed[kGenEdge * e]), b = int(ed[kGenEdge * e + 1]);
+            const int c = (a == id[i]) ? b : (b == id[i] ? a : -1);
+            if (c >= 0 && c != id[0] && c != id[1] && c != id[2] && c != id[3]) id[4 + i] = c;
+        }
+        if (id[4 + i] < 0) return false;
+    }
+    return true;
+}
+__device__ inline bool hex_edge_record(const double* rec, const int* id, int e, double* o)
+{
+    const double *vt = rec + kGenHdr, *ed = rec + kHexInE;
+    const int a = id[e < 8 ? e : e - 8], b = id[e < 8 ? (e & 4) + ((e + 1) & 3) : e - 4];
+    int q = 0;
+    for (; q < 12; q++) {
+        const int c = int(ed[kGenEdge * q]), d = int(ed[kGenEdge * q + 1]);
+        if ((c == a && d == b) || (c == b && d == a)) break;
+    }
+    if (q == 12) return false;
+    const double* E = ed + kGenEdge * q;
+    double* w = o + kHexW + 5 * e;  // stored xx yy zz xy xz yz
+    w[0] = E[6];
+    w[1] = E[9];
+    w[2] = E[10];
+    w[3] = E[7];
+    w[4] = E[11];
+    o[kHexL + e] = 2.0 * E[5];
+    o[kHexL2 + e] = sq3(vt[3 * b] - vt[3 * a], vt[3 * b + 1] - vt[3 * a + 1], vt[3 * b + 2] - vt[3 * a + 2]);
+    return true;
+}
+// the normal of face f in the order of kHexFace, null if it is no face
+__device__ inline const double* hex_normal(const double* rec, const int* id, int f)
+{
+    const double *fc = rec + kHexInF, *fv = rec + kHexInV;
+    const int i = f - 1, j = f & 3;
+    unsigned want;
+    if (f == 0 || f == 5) want = (1u << id[f ? 4 : 0]) | (1u << id[f ? 5 : 1]) | (1u << id[f ? 6 : 2]) | (1u << id[f ? 7 : 3]);
+    else want = (1u << id[i]) | (1u << id[j]) | (1u << id[4 + i]) | (1u << id[4 + j]);
+    for (int q = 0; q < 6; q++) {
+        unsigned got = 0;
+        for (int k = 0; k < 4; k++) got |= 1u << int(fv[int(fc[kGenFace * q + 3]) + k]);
+        if (got == want) return fc + kGenFace * q;
+    }
+    return nullptr;
+}
+__device__ inline bool hex_face_record(const double* rec, const int* id, int f, double* o)
+{
+    const double* vt = rec + kGenHdr;
+    const double *n = hex_normal(rec, id, f), *m = hex_normal(rec, id, 5);
+    if (!n || !m) return false;
+    double* t = o + kHexT + 5 * f;
+    t[0] = -2.0 * (n[0] * n[0] - m[0] * m[0]);
+    t[1] = -2.0 * (n[0] * n[1] - m[0] * m[1]);
+    t[2] = -2.0 * (n[0] * n[2] - m[0] * m[2]);
+    t[3] = -2.0 * (n[1] * n[1] - m[1] * m[1]);
+    t[4] = -2.0 * (n[1] * n[2] - m[1] * m[2]);
+    const int i = f - 1, j = f & 3;
+    const double* a = vt + 3 * id[f == 0 ? 0 : i];
+    auto side = [&](int k) { return v3(vt[3 * k] - a[0], vt[3 * k + 1] - a[1], vt[3 * k + 2] - a[2]); };
+    const V3<double> e1 = side(id[f == 0 ? 1 : j]), e2 = side(id[f == 0 ? 2 : 4 + j]), e3 = side(id[f == 0 ? 3 : 4 + i]);
+    const V3<double> c1 = cross(e1, e2), c2 = cross(e2, e3);
+    double* g = o + kHexF + 5 * f;
+    for (int c = 0; c < 3; c++) g[c] = n[c];
+    g[3] = 2.0 * sqrt(dot(c1, c1));
+    g[4] = 2.0 * sqrt(dot(c2, c2));
+    o[kHexD2 + f] = dot(e2, e2);
+    return true;
+}
+__device__ inline void hex_close_record(const double* rec, const int* id, double* o)
+{
+    for (int k = 0; k < 8; k++)
+        for (int c = 0; c < 3; c++) o[3 * k + c] = rec[kGenHdr + 3 * id[k] + c];
+    double l2 = 0.0;
+    for (int e = 0; e < 12; e++) l2 = fmax(l2, o[kHexL2 + e]);
+    o[kHexR2] = 4.0 * l2;
+    const double* n = hex_normal(rec, id, 5);
+    for (int c = 0; c < 3; c++) o[kHexN5 + c] = n[c];
+    o[kHex - 1] = 0.0;
+}
+
 __device__ __forceinline__ void far_tet_record(const double* __restrict__ rec, double* __restrict__ o)
 {
     for (int k = 0; k < 12; k++) o[k] = rec[k];
@@ -363,6 +470,144 @@ __device__ __forceinline__ bool rec_block(const double* __restrict__ rec, const 
 #pragma unroll
         for (int k = 0; k < 6; k++) q6[k] = far ? q6[k] : qn[k];
     }
+    return in;
+}
+
+// Keeps a record's reads from being hoisted past here: in one block of code the
+// scheduler would load all 164 values first, into registers that it then spills.
+#ifdef __HIP_DEVICE_COMPILE__
+#define FAR_GROUP()                   \
+    do {                              \
+        asm volatile("" ::: "memory"); \
+        __builtin_amdgcn_sched_barrier(0); \
+    } while (0)
+#else
+#define FAR_GROUP()
+#endif
+
+// The block at points near a hexahedron: one edge and one face at a time from
+// the record, each with the tier its wave needs, as near_tet_block.
+__device__ inline bool near_hex_block(const double* __restrict__ h, const double p[3], double q5[5])
+{
+    auto vtx = [&](int k, V3<double>& r, double& d) {
+        r = rel<double>(h + 3 * k, p);
+        d = rh_sqrt(dot(r, r));
+    };
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int e = 0; e < 12; e++) {
+        const int a = e & 7, top = e & 4;
+        const int b = (e < 8) ? top + ((e + 1) & 3) : e - 4;
+        V3<double> ra[1], rb[1];
+        double da[1], db[1], S[1], L[1];
+        vtx(e < 8 ? a : e - 8, ra[0], da[0]);
+        vtx(b, rb[0], db[0]);
+        S[0] = da[0] + db[0];
+        edge_L2(ra, da, rb, db, S, h[kHexL + e], kEdge6Top, L);
+        for (int k = 0; k < 5; k++) acc[k] += L[0] * h[kHexW + 5 * e + k];
+    }
+    bool inside = true;
+#pragma unroll 1
+    for (int f = 0; f < 5; f++) {
+        // corners and edges as in kHexFace and kHexFaceEdge
+        const int i = f - 1, j = f & 3;
+        const int b = (f == 0) ? 1 : j, c = (f == 0) ? 2 : 4 + j, e = (f == 0) ? 3 : 4 + i, a = (f == 0) ? 0 : i;
+        const int ab = (f == 0) ? 0 : i, bc = (f == 0) ? 1 : 8 + j, ce = (f == 0) ? 2 : 4 + i, ea = (f == 0) ? 3 : 8 + i;
+        V3<double> ra, rb, rc, re;
+        double da, db, dc, de, om[1];
+        vtx(a, ra, da);
+        vtx(b, rb, db);
+        vtx(c, rc, dc);
+        vtx(e, re, de);
+        const double* g = h + kHexF + 5 * f;
+        const double D = da + dc, D2 = h[kHexD2 + f], z = dot(ra, v3(g[0], g[1], g[2]));
+        const double r1 = ((da + db) * (db + dc)) * D - (dc * h[kHexL2 + ab] + db * D2 + da * h[kHexL2 + bc]);
+        const double r2 = ((de + da) * (dc + de)) * D - (da * h[kHexL2 + ce] + de * D2 + dc * h[kHexL2 + ea]);
+        const double i1 = z * g[3], i2 = z * g[4];
+        inside = inside && (z > 0.0);
+        const double im[1] = {r1 * i2 + r2 * i1}, rr[1] = {r1 * r2 - i1 * i2};
+        rh_atan2_wave(im, rr, kAtan32Top, om);
+        for (int k = 0; k < 5; k++) acc[k] += om[0] * h[kHexT + 5 * f + k];
+    }
+    const double* n = h + kHexN5;
+    {
+        const V3<double> r4 = rel<double>(h + 12, p);  // face 5 holds vertex 4
+        inside = inside && (dot(r4, v3(n[0], n[1], n[2])) > 0.0);
+    }
+    // the solid angles sum to 4 pi inside: the sixth face's share of it
+    const double in4 = inside ? 4.0 * kPi : 0.0;
+    acc[0] -= in4 * n[0] * n[0];
+    acc[1] -= in4 * n[0] * n[1];
+    acc[2] -= in4 * n[0] * n[2];
+    acc[3] -= in4 * n[1] * n[1];
+    acc[4] -= in4 * n[1] * n[2];
+    far_scale(acc, q5);
+    return inside;
+}
+
+// General polyhedron at p (element frame); h: its hexahedron record, null if it
+// is none (then by eval_gen).  Points whose distances from all corners are at
+// least two longest edges take the far form: 8 offsets and roots, 12 short edge
+// integrals, and for each of five faces two triangle denominators and one short
+// arctangent, about 600 issue slots against 3,000 for eval_gen, which forms
+// both ends of every edge and every face's corners anew and reads its record
+// through chains of scalar loads (36,000 cycles where few waves hide them).
+// The far test is each lane's own, as for blocks.
+__device__ __forceinline__ bool gen_block(const double* __restrict__ h, const double* __restrict__ rec,
+                                          const double p[3], double q6[6])
+{
+    if (!h) return eval_gen<double>(rec, p, q6);
+    V3<double> r[8];
+    double d[8], least = INFINITY;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        r[k] = rel<double>(h + 3 * k, p);
+        const double d2 = dot(r[k], r[k]);
+        least = fmin(least, d2);
+        d[k] = rh_sqrt(d2);
+    }
+    const bool far = least >= h[kHexR2];
+    FAR_GROUP();
+    double q5[5];
+    if (rh_any(far)) {
+        double S[12], acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 12; e++) {
+            S[e] = d[kHexEdgeA[e]] + d[kHexEdgeB[e]];
+            const double L = far_atanh2(rh_div(h[kHexL + e], S[e]));
+#pragma unroll
+            for (int k = 0; k < 5; k++) acc[k] += L * h[kHexW + 5 * e + k];
+            if ((e & 1) == 1) FAR_GROUP();
+        }
+#pragma unroll
+        for (int f = 0; f < 5; f++) {
+            const int a = kHexFace[f][0], b = kHexFace[f][1], c = kHexFace[f][2], e = kHexFace[f][3];
+            const int ab = kHexFaceEdge[f][0], bc = kHexFaceEdge[f][1], ce = kHexFaceEdge[f][2], ea = kHexFaceEdge[f][3];
+            const double* g = h + kHexF + 5 * f;
+            const double D = d[a] + d[c], D2 = h[kHexD2 + f], z = dot(r[a], v3(g[0], g[1], g[2]));
+            const double r1 = (S[ab] * S[bc]) * D - (d[c] * h[kHexL2 + ab] + d[b] * D2 + d[a] * h[kHexL2 + bc]);
+            const double r2 = (S[ea] * S[ce]) * D - (d[a] * h[kHexL2 + ce] + d[e] * D2 + d[c] * h[kHexL2 + ea]);
+            const double i1 = z * g[3], i2 = z * g[4];
+            const double om = far_atan(rh_div(r1 * i2 + r2 * i1, r1 * r2 - i1 * i2));
+#pragma unroll
+            for (int k = 0; k < 5; k++) acc[k] += om * h[kHexT + 5 * f + k];
+            FAR_GROUP();
+        }
+        far_scale(acc, q5);
+    }
+    bool in = false;
+    if (rh_any(!far)) {
+        double qn[5];
+        in = near_hex_block(h, p, qn) && !far;
+#pragma unroll
+        for (int k = 0; k < 5; k++) q5[k] = far ? q5[k] : qn[k];
+    }
+    q6[0] = q5[0];
+    q6[1] = q5[3];
+    q6[2] = -(q5[0] + q5[3]) - (in ? 1.0 : 0.0);
+    q6[3] = q5[1];
+    q6[4] = q5[2];
+    q6[5] = q5[4];
     return in;
 }
 #endif

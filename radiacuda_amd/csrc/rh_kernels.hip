@@ -51,6 +51,50 @@ __global__ __launch_bounds__(256) void k_far_records(DevModel m, double* __restr
     far_tet_record(m.data + m.off[m.kidx[k]], out + kFarTet * (k - m.koff[1]));
 }
 
+// Far-form records of the hexahedra among the general polyhedra, one wave each;
+// elements of the other kinds have none.
+__global__ __launch_bounds__(64) void k_hex_records(DevModel m, double* __restrict__ out, int32_t* __restrict__ at)
+{
+    __shared__ double rec[kHexIn], o[kHex];
+    __shared__ int id[8];
+    __shared__ int ok;
+    const int64_t q = blockIdx.x, j = m.kidx[m.koff[2] + q];
+    const double* src = m.data + m.off[j];
+    const bool hex = int(src[0]) == 8 && int(src[1]) == 12 && int(src[2]) == 6 && int(src[3]) == 24;
+    if (!hex) {
+        if (threadIdx.x == 0) at[j] = -1;
+        return;
+    }
+    for (int i = threadIdx.x; i < kHexIn; i += 64) rec[i] = src[i];
+    __syncthreads();
+    if (threadIdx.x == 0) ok = hex_vertices(rec, id) ? 1 : 0;
+    __syncthreads();
+    if (!ok) {
+        if (threadIdx.x == 0) at[j] = -1;
+        return;
+    }
+    bool fits = true;
+    if (threadIdx.x < 12) fits = hex_edge_record(rec, id, threadIdx.x, o);
+    else if (threadIdx.x < 17) fits = hex_face_record(rec, id, threadIdx.x - 12, o);
+    if (__any(!fits)) {
+        if (threadIdx.x == 0) at[j] = -1;
+        return;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        hex_close_record(rec, id, o);
+        at[j] = int32_t(q);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < kHex; i += 64) out[kHex * q + i] = o[i];
+}
+
+__global__ __launch_bounds__(256) void k_no_hex(int64_t n, const int32_t* __restrict__ kidx, int32_t* __restrict__ at)
+{
+    const int64_t k = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (k < n) at[kidx[k]] = -1;
+}
+
 // The far form of a tetrahedron's block at x when every lane of the wave is
 // far (else false).  FAR32: FP32 integrals beyond two circumradii of the
 // vertex mean, as block_Q_mixed takes them (vertices come first in the far
@@ -492,6 +536,10 @@ __device__ __forceinline__ void field_store(double* __restrict__ B, double* __re
 // 163 from LDS.  More waves a SIMD (3 or 4, the near form spilling) 171 and 184.
 constexpr int kRecTile = 64;
 constexpr int kRecStage = 6 + 3;
+// General polyhedra (FP64): hexahedron records and magnetizations likewise.
+// 2,048 points and 1,000 hexahedra 329 us by eval_gen, 128 now.
+constexpr int kHexTile = 16;
+constexpr int kHexStage = kHex + 3;
 
 template <class R, bool SYM, int KIND, int PASS>
 __global__ __launch_bounds__(256) void k_field(DevModel m, const double* __restrict__ M,
@@ -535,6 +583,66 @@ __global__ __launch_bounds__(256) void k_field(DevModel m, const double* __restr
                 for (int k = 0; k < 3; k++) {
                     h[k] += hl[k];
                     b[k] += hl[k] + (in ? mm[k] : 0.0);
+                }
+            }
+        }
+        if (!live) return;
+    } else if constexpr (KIND == 2 && PASS == kPassAll) {
+        static_assert(sizeof(R) == 8, "the single-precision sweep is two passes");
+        __shared__ double tile[kHexTile * kHexStage];
+        __shared__ int32_t elem[kHexTile], at[kHexTile];
+        for (int64_t base = k0; base < k1; base += kHexTile) {
+            const int cnt = int((k1 - base < kHexTile) ? (k1 - base) : kHexTile);
+            __syncthreads();  // the previous tile has been consumed
+            if (int(threadIdx.x) < cnt) {
+                const int32_t j = m.kidx[base + threadIdx.x];
+                elem[threadIdx.x] = j;
+                at[threadIdx.x] = m.hex_at[j];
+                for (int k = 0; k < 3; k++) tile[kHexStage * threadIdx.x + kHex + k] = M[3 * int64_t(j) + k];
+            }
+            __syncthreads();
+            for (int i = threadIdx.x; i < cnt * kHex; i += 256) {
+                const int q = i / kHex, k = i - kHex * q;
+                if (at[q] >= 0) tile[kHexStage * q + k] = m.hex[int64_t(kHex) * at[q] + k];
+            }
+            __syncthreads();
+            if (!live) continue;
+#pragma unroll 1
+            for (int q = 0; q < cnt; q++) {
+                const double* rec = tile + kHexStage * q;
+                const double mm[3] = {rec[kHex], rec[kHex + 1], rec[kHex + 2]};
+                const int64_t j = __builtin_amdgcn_readfirstlane(elem[q]);
+                const double* er = m.data + m.off[j];
+                auto H_at = [&](const double* xl, double* hl) {
+                    double q6[6];
+                    const bool in = gen_block(at[q] >= 0 ? rec : nullptr, er, xl, q6);
+                    hl[0] = q6[0] * mm[0] + q6[3] * mm[1] + q6[4] * mm[2];
+                    hl[1] = q6[3] * mm[0] + q6[1] * mm[1] + q6[5] * mm[2];
+                    hl[2] = q6[4] * mm[0] + q6[5] * mm[1] + q6[2] * mm[2];
+                    return in;
+                };
+                double hl[3];
+                if (!SYM) {
+                    const bool in = H_at(x, hl);
+                    for (int k = 0; k < 3; k++) {
+                        h[k] += hl[k];
+                        b[k] += hl[k] + (in ? mm[k] : 0.0);
+                    }
+                    continue;
+                }
+                for (int64_t c = m.copy_off[j]; c < m.copy_off[j + 1]; c++) {
+                    const double* cp = m.copies + 24 * c;
+                    double xl[3], hg[3], bg[3];
+                    apply_inv(cp, x, xl);
+                    const bool in = H_at(xl, hl);
+                    const double bl[3] = {hl[0] + (in ? mm[0] : 0.0), hl[1] + (in ? mm[1] : 0.0),
+                                          hl[2] + (in ? mm[2] : 0.0)};
+                    mat3_vec(cp + 12, hl, hg);
+                    mat3_vec(cp + 12, bl, bg);
+                    for (int k = 0; k < 3; k++) {
+                        h[k] += hg[k];
+                        b[k] += bg[k];
+                    }
                 }
             }
         }
@@ -1904,12 +2012,17 @@ __global__ __launch_bounds__(256) void k_current(int64_t ns, const int32_t* __re
 
 // ---------------------------------------------------------------- launchers
 int64_t far_tet_doubles(int64_t ntet) { return kFarTet * ntet; }
+int64_t hex_doubles(int64_t ngen) { return kHex * ngen; }
 
-hipError_t launch_far_records(const DevModel& m, double* out, hipStream_t s)
+hipError_t launch_far_records(const DevModel& m, double* tet, double* hex, int32_t* hex_at, hipStream_t s)
 {
     const int64_t ntet = m.koff[2] - m.koff[1];
-    if (ntet == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_far_records, dim3(unsigned((ntet + 255) / 256)), dim3(256), 0, s, m, out);
+    if (ntet > 0) hipLaunchKernelGGL(k_far_records, dim3(unsigned((ntet + 255) / 256)), dim3(256), 0, s, m, tet);
+    const int64_t ngen = m.koff[3] - m.koff[2];
+    if (m.koff[2] > 0)
+        hipLaunchKernelGGL(k_no_hex, dim3(unsigned((m.koff[2] + 255) / 256)), dim3(256), 0, s, m.koff[2], m.kidx,
+                           hex_at);
+    if (ngen > 0) hipLaunchKernelGGL(k_hex_records, dim3(unsigned(ngen)), dim3(64), 0, s, m, hex, hex_at);
     return hipGetLastError();
 }
 
@@ -1937,13 +2050,13 @@ hipError_t launch_assemble(const DevModel& m, void* Q, int elem_bytes, int64_t l
 
 namespace {
 // element splits for one kind slot: enough workgroups to fill the chip
-int64_t slot_splits(int64_t np, int64_t cnt, int64_t per_block = 256)
+int64_t slot_splits(int64_t np, int64_t cnt, int64_t per_block = 256, int64_t least = 16)
 {
     if (cnt == 0) return 0;
     const int64_t blocks = (np + per_block - 1) / per_block;
     if (blocks >= 2048 || cnt < 64) return 1;
     int64_t sp = (2048 + blocks - 1) / blocks;
-    sp = std::min<int64_t>(sp, std::max<int64_t>(1, cnt / 16));
+    sp = std::min<int64_t>(sp, std::max<int64_t>(1, cnt / least));
     return std::max<int64_t>(1, sp);
 }
 
@@ -2003,7 +2116,10 @@ void slot_plan(const DevModel& m, int64_t np, int64_t sp[3], int64_t work_cap)
         sp[2] = 0;
     } else {
         sp[1] = slot_splits(np, m.koff[2] - m.koff[1]);
-        sp[2] = slot_splits(np, m.koff[3] - m.koff[2]);
+        // slices of 8: the near elements of a point lie side by side, and a slice
+        // of 16 of them is the sweep's longest wave (2,048 points, 1,000
+        // hexahedra: 191 us with 16, 128 with 8)
+        sp[2] = slot_splits(np, m.koff[3] - m.koff[2], 256, 8);
     }
     if (work_cap < 0) return;
     // halve the largest split count until the partials fit or every slot is

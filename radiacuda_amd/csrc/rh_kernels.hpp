@@ -49,16 +49,20 @@ struct DevModel {
     int64_t koff[4] = {0, 0, 0, 0};  // slot ranges in kidx (block, tet, general)
     const double* charged = nullptr;  // field-only tetrahedron records (per call)
     const double* far_tet = nullptr;  // far-form tetrahedron records (rh_far.hpp), kidx order
+    const double* hex = nullptr;      // far-form hexahedron records
+    const int32_t* hex_at = nullptr;  // [n] an element's record in hex, -1 if it has none
     bool sym = false;
     bool rowt_identity = true;
     MeshDev mesh;
     bool use_mesh = false;  // field sweeps use the mesh form (when active)
 };
 
-// Doubles of the far-form records of ntet tetrahedra, and the kernel that
-// builds them from the element records (once per model).
+// Doubles of the far-form records of ntet tetrahedra and of ngen general
+// polyhedra (the hexahedra among them), and the kernels that build them from
+// the element records (once per model).
 int64_t far_tet_doubles(int64_t ntet);
-hipError_t launch_far_records(const DevModel& m, double* out, hipStream_t s);
+int64_t hex_doubles(int64_t ngen);
+hipError_t launch_far_records(const DevModel& m, double* tet, double* hex, int32_t* hex_at, hipStream_t s);
 
 // Interaction-matrix rows of elements [r0, r1) into Q (row-major, leading
 // dimension ld elements of elem_bytes = 4 or 8; Q points at row 3*r0); the
