@@ -5,7 +5,8 @@
 // Mapping (wave64): in the assembly and field kernels each lane owns one
 // observation point (a matrix row's collocation point, or a field point) and
 // every lane of the workgroup sweeps the same source elements, so element
-// records are read with wave-uniform addresses (scalar-cache loads, no
+// records are read at wave-uniform addresses (from LDS where a sweep is long
+// enough to stage them, otherwise through the scalar cache; no
 // per-lane gathers) and the per-element branches are uniform.  These kernels
 // are bound by FP64 transcendental/VALU throughput.  The matrix pass streams
 // the matrix once per iteration with 16-byte non-temporal loads and FP64

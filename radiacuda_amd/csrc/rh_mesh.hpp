@@ -17,14 +17,14 @@
 
 namespace rh {
 
-// Charged edge record: a(3), b(3), t(3), 2 len, w(3), cont (1: a is the
-// previous record's b).  The FP32 sweep's records hold 2 len and the near
+// Charged edge record: a(3), b(3), t(3), 2 len, w(3), 0 (edge_flag, an array
+// beside the records, tells whether a is the previous record's b).  The FP32 sweep's records hold 2 len and the near
 // distance as floats in slot 6 (the near pass reads slot 9).
 constexpr int kMeshEdge = 14;
 // Charged face record: v0..v3 (12), n(3), 4*area(v0,v1,v2), 4*area(v0,v2,v3),
-// nv, -2 g(3), code (0 triangle, 1 triangle whose v0, v1 are the previous
-// record's v1, v2, 2 quadrilateral, 3 quadrilateral whose v0, v1 are the
-// previous record's v2, v3), then the edges the face owns: for the sides
+// nv, -2 g(3), 0 (face_flag tells the owned sides and whether a triangle's v0,
+// v1 are the previous record's v1, v2, or a quadrilateral's the previous
+// record's v2, v3), then the edges the face owns: for the sides
 // (v0,v1), (v1,v2), (v2,v0) of a triangle or (v0,v1), (v1,v2), (v2,v3) of a
 // quadrilateral in turn 2 len and w(3) (slots 22-33); slot 35: the FP32
 // sweep's near distance (a float); slots 36-40: the squared distances of
