@@ -102,128 +102,6 @@ __global__ __launch_bounds__(256, 2) void k_adj_m(DevModel m, const double* __re
         part[int64_t(blockIdx.x) * 3 * m.n + 3 * j0 + i] = acc[0][i] + acc[1][i] + acc[2][i] + acc[3][i];
 }
 
-// (1 - asinh(s)/s)/s^2 on s^2 <= 1/100 by powers of s^2: Chebyshev interpolant
-// fitted at 60 digits, within 6e-17 relative
-__constant__ double d_asinh_p[6] = {0.16666666666666666, -0.0749999999999521,   0.04464285708693904,
-                                    -0.030381920556719857, 0.02236754133836989, -0.016940234967509307};
-
-// One triangle's part of dL/dvertex: geometry that does not depend on the
-// observation point, and the sums over points.
-struct TriLane {
-    V3<double> v[3];  // corners, element frame
-    V3<double> n, t[3];
-    double len[3], il[3], ia, sigma;  // side lengths and reciprocals, 1/(2 area), n . M
-    V3<double> M;
-    V3<double> G[3];  // per corner: terms of L and of the solid angle
-    V3<double> N;     // adjoint of the unit normal
-    double al[3];     // per side: adjoint of its direction's own component
-};
-
-__device__ __forceinline__ V3<double> axpy(double a, const V3<double>& x, const V3<double>& y)
-{
-    return V3<double>{fma(a, x.x, y.x), fma(a, x.y, y.y), fma(a, x.z, y.z)};
-}
-
-// Derivatives of f = g . 4 pi H_t at one point, in closed form.  With
-// m = sigma n x g, S = sum_e L_e t_e and u -> w the side e,
-//     f = sigma (S . (n x g) - Omega n . g),
-//     D = Ru Rw + u . w,  L = asinh(len (Ru + Rw)/D),
-//     dL/dlen = (Ru + Rw)/D,  dL/dRu = dL/dRw = -len/D,
-//     dOmega/dw = -(u x w)/(Rw D) per side (both ends alike, by 1/Ru, 1/Rw),
-// the last because the solid angle changes by the area that a moved side
-// sweeps, int s/r^3 = 1/(Rw D) along it.  No term needs a derivative of a
-// logarithm's or an arctangent's argument.  Sums over points are taken of the
-// differences between a corner's two sides, never of the sides' own terms,
-// which are larger by distance over size.  gx: minus the sum of the corner
-// derivatives (the normal's and the directions' parts cancel in it).
-__device__ __forceinline__ void tri_point(TriLane& T, const double x[3], const V3<double>& g, V3<double>& gx)
-{
-#ifdef __HIP_DEVICE_COMPILE__
-    V3<double> r[3];
-    double R[3], iR[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        r[k] = V3<double>{T.v[k].x - x[0], T.v[k].y - x[1], T.v[k].z - x[2]};
-        // R and 1/R from one seed y: with q = R^2 y and e = 1 - q y both are
-        // the seed's value times 1 + e/2 + 3 e^2/8
-        const double d = dot(r[k], r[k]);
-        const double y = __builtin_amdgcn_rsq(d);
-        const double q = d * y, e = fma(-q, y, 1.0), c = e * fma(e, 0.375, 0.5);
-        R[k] = fma(q, c, q);
-        iR[k] = fma(y, c, y);
-    }
-    const V3<double> ng = cross(T.n, g);
-    const double gn = dot(T.n, g), sgn = T.sigma * gn;
-    V3<double> X[3], S{0.0, 0.0, 0.0};
-    double uw[3], iD[3], sd[3], s2[3], w1[3], k1[3];
-#pragma unroll
-    for (int e = 0; e < 3; e++) {
-        const int f = (e + 1) % 3;
-        X[e] = cross(r[e], r[f]);
-        uw[e] = dot(r[e], r[f]);
-        const double RR = R[e] * R[f];
-        double D = RR + uw[e];
-        // beyond a right angle the sum cancels: |u x w|^2 = (RR - u.w) D
-        if (uw[e] < 0.0) D = dot(X[e], X[e]) * rh_rcp(RR - uw[e]);
-        iD[e] = rh_rcp(D);
-        sd[e] = (R[e] + R[f]) * iD[e];
-        const double s = T.len[e] * sd[e];
-        s2[e] = s * s;
-    }
-    // w1 = sd - L/len and k1 = L/len: where every lane's sides are short
-    // against their distance by the series, which loses no digits in w1
-    if (rh_all(fmax(fmax(s2[0], s2[1]), s2[2]) <= 0.01)) {
-#pragma unroll
-        for (int e = 0; e < 3; e++) {
-            double p = d_asinh_p[5];
-#pragma unroll
-            for (int i = 4; i >= 0; i--) p = fma(p, s2[e], d_asinh_p[i]);
-            w1[e] = sd[e] * s2[e] * p;
-            k1[e] = sd[e] - w1[e];
-        }
-    } else {
-        RH_KEEP_BRANCH();
-        const CoefPtr c = rh_coef_rare(d_log_p);
-#pragma unroll
-        for (int e = 0; e < 3; e++) {
-            // len s = sinh L: e^L = (Ru + Rw + len)^2 / (2 D)
-            const double q = R[e] + R[(e + 1) % 3] + T.len[e];
-            k1[e] = rh_log_ratio_c(q * (0.5 * q) * iD[e], 1.0, c) * T.il[e];
-            w1[e] = sd[e] - k1[e];
-        }
-    }
-    const double re = R[0] * R[1] * R[2] + uw[0] * R[2] + uw[2] * R[1] + uw[1] * R[0];
-    const double om = 2.0 * rh_atan2_wave(dot(r[0], X[1]), re);
-    double kk[3], cc[3];
-#pragma unroll
-    for (int e = 0; e < 3; e++) {
-        S = axpy(k1[e] * T.len[e], T.t[e], S);
-        const double tm = T.sigma * dot(T.t[e], ng);
-        T.al[e] = fma(tm, w1[e], T.al[e]);
-        kk[e] = tm * T.len[e] * iD[e];
-        cc[e] = -sgn * iD[e];
-    }
-    // the normal: f = phi sigma, d sigma = dn . M
-    const double phi = dot(S, ng) - om * gn;
-    const V3<double> gS = cross(g, S);
-    T.N = axpy(phi, T.M, axpy(T.sigma, V3<double>{fma(-om, g.x, gS.x), fma(-om, g.y, gS.y), fma(-om, g.z, gS.z)}, T.N));
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const int in = (k + 2) % 3;  // side ending in corner k; side k starts there
-        const double kr = kk[in] + kk[k];
-        const V3<double> h{iR[k] * fma(kr, r[k].x, fma(cc[in], X[in].x, cc[k] * X[k].x)),
-                           iR[k] * fma(kr, r[k].y, fma(cc[in], X[in].y, cc[k] * X[k].y)),
-                           iR[k] * fma(kr, r[k].z, fma(cc[in], X[in].z, cc[k] * X[k].z))};
-        const double dk = T.sigma * (k1[in] - k1[k]);
-        T.G[k] = V3<double>{T.G[k].x + fma(dk, ng.x, -h.x), T.G[k].y + fma(dk, ng.y, -h.y),
-                            T.G[k].z + fma(dk, ng.z, -h.z)};
-        gx.x += h.x;
-        gx.y += h.y;
-        gx.z += h.z;
-    }
-#endif
-}
-
 // dL/dvertex partials: partv[bx][vertex slot][3] for the vertices of element
 // slice [sl[y], sl[y+1]); optional per-point dL/dx partials partx[y][p][3].
 //
@@ -294,22 +172,8 @@ __global__ __launch_bounds__(256, 2) void k_adj_geom(DevModel m, const double* _
             const int id = int(tri[k]);
             if (wave == 0) corner[k][lane] = slot + id;
             T.v[k] = V3<double>{rec[2 + 3 * id], rec[3 + 3 * id], rec[4 + 3 * id]};
-            T.G[k] = V3<double>{0.0, 0.0, 0.0};
-            T.al[k] = 0.0;
         }
-        T.N = V3<double>{0.0, 0.0, 0.0};
-        T.M = live ? V3<double>{M[3 * j], M[3 * j + 1], M[3 * j + 2]} : V3<double>{0.0, 0.0, 0.0};
-        const V3<double> e1 = vsub(T.v[1], T.v[0]), e2 = vsub(T.v[2], T.v[0]);
-        const V3<double> nn = cross(e1, e2);
-        T.ia = 1.0 / sqrt(dot(nn, nn));
-        T.n = vscale(nn, T.ia);
-        T.sigma = dot(T.n, T.M);
-        for (int e = 0; e < 3; e++) {
-            const V3<double> d = vsub(T.v[(e + 1) % 3], T.v[e]);
-            T.len[e] = sqrt(dot(d, d));
-            T.il[e] = 1.0 / T.len[e];
-            T.t[e] = vscale(d, T.il[e]);
-        }
+        tri_open(T, live ? V3<double>{M[3 * j], M[3 * j + 1], M[3 * j + 2]} : V3<double>{0.0, 0.0, 0.0});
         for (int64_t q0 = p0; q0 < p1; q0 += kAdjTile) {
             const int cnt = int((p1 - q0 < kAdjTile) ? (p1 - q0) : kAdjTile);
             __syncthreads();
@@ -346,18 +210,12 @@ __global__ __launch_bounds__(256, 2) void k_adj_geom(DevModel m, const double* _
                 }
             }
         }
-        // side directions: dt = (dd - t (t . dd))/len moved both ends by -+ dd;
-        // the length's part is along t; the unit normal: n = (v1 - v0) x (v2 - v0)/|.|
-        const V3<double> q = vscale(axpy(-dot(T.n, T.N), T.n, T.N), T.ia);
-        const V3<double> g1 = cross(e2, q), g2 = cross(q, e1);
-        T.G[0] = vsub(T.G[0], V3<double>{g1.x + g2.x, g1.y + g2.y, g1.z + g2.z});
-        T.G[1] = V3<double>{T.G[1].x + g1.x, T.G[1].y + g1.y, T.G[1].z + g1.z};
-        T.G[2] = V3<double>{T.G[2].x + g2.x, T.G[2].y + g2.y, T.G[2].z + g2.z};
+        V3<double> G[3];
+        tri_close(T, G);
         for (int k = 0; k < 3; k++) {
-            const V3<double> G = axpy(T.al[(k + 2) % 3], T.t[(k + 2) % 3], axpy(-T.al[k], T.t[k], T.G[k]));
-            lanes[wave][3 * k][lane] = G.x;
-            lanes[wave][3 * k + 1][lane] = G.y;
-            lanes[wave][3 * k + 2][lane] = G.z;
+            lanes[wave][3 * k][lane] = G[k].x;
+            lanes[wave][3 * k + 1][lane] = G[k].y;
+            lanes[wave][3 * k + 2][lane] = G[k].z;
         }
         __syncthreads();
         for (int i = threadIdx.x; i < 9 * 64; i += 256)

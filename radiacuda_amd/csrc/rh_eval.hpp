@@ -120,11 +120,7 @@ RH_HD bool near_element(int kind, const double* __restrict__ rec, const double x
 template <int KIND>
 RH_HD void eval_mixed(int kind, const double* __restrict__ rec, const double xl[3], double q6[6])
 {
-    bool near = near_element<KIND>(kind, rec, xl);
-#ifdef __HIP_DEVICE_COMPILE__
-    near = rh_any(near);
-#endif
-    if (near)
+    if (rh_any(near_element<KIND>(kind, rec, xl)))
         eval_k<double, KIND>(kind, rec, xl, q6);
     else
         eval_k<float, KIND>(kind, rec, xl, q6);
@@ -155,6 +151,40 @@ RH_HD void block_Q_mixed(const ModelView& mv, int64_t j, const double x[3], doub
             for (int b = 0; b < 3; b++)
                 q9[3 * a + b] += F[3 * a] * ql[b] + F[3 * a + 1] * ql[3 + b] + F[3 * a + 2] * ql[6 + b];
     }
+}
+
+// The far form of a tetrahedron's block at x when every lane of the wave is
+// far (else false).  FAR32: FP32 integrals beyond two circumradii of the
+// vertex mean, as block_Q_mixed takes them (vertices come first in the far
+// record, as in the element record).
+template <bool FAR32>
+RH_HD bool tet_fp32(const double* __restrict__ far, const double x[3])
+{
+    if constexpr (FAR32) return !rh_any(near_element<1>(EK_TET, far, x));
+    else return false;
+}
+template <bool FAR32>
+RH_HD bool far_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
+{
+    auto eval = [&](auto zero) {
+        using R = decltype(zero);
+        FarTet<R> t;
+        if (!far_tet_open<R>(far, x, t)) return false;
+        far_tet_block<R>(far, t, q5);
+        return true;
+    };
+    if constexpr (FAR32) {
+        if (tet_fp32<FAR32>(far, x)) return eval(float(0));
+    }
+    return eval(double(0));
+}
+template <bool FAR32>
+RH_HD bool near_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
+{
+    if constexpr (FAR32) {
+        if (tet_fp32<FAR32>(far, x)) return near_tet_block<float>(far, x, q5);
+    }
+    return near_tet_block<double>(far, x, q5);
 }
 
 // Near test of the FP32 field sweeps (element frame): blocks and tetrahedra
@@ -190,11 +220,7 @@ RH_HD bool near32(int kind, const double* __restrict__ rec, const double* __rest
                   const double x[3])
 {
     if (crec) return tet_near32(crec, x);
-    bool near = near_field<KIND>(kind, rec, x);
-#ifdef __HIP_DEVICE_COMPILE__
-    near = rh_any(near);
-#endif
-    return near;
+    return rh_any(near_field<KIND>(kind, rec, x));
 }
 
 // One element's H at x (element frame) from its record (or its charged

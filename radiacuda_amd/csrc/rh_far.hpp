@@ -1,5 +1,5 @@
 // rh_far.hpp -- interaction blocks of elements that are far from every point
-// of a wave, or from a lane's own point (blocks) (device only).
+// of a wave, or from a lane's own point (blocks, hexahedra).
 //
 // With S = Ra + Rb the sum of an edge's end distances, its integral is
 // 2 atanh(len / S) and a triangle's half solid angle has the tangent
@@ -45,7 +45,6 @@ constexpr int kFarTet = kFarN3 + 3;                         // 92 doubles
 constexpr int kHexW = 24, kHexL = 84, kHexL2 = 96, kHexT = 108, kHexF = 133, kHexD2 = 158, kHexR2 = 163, kHexN5 = 164,
               kHex = 168;
 
-#ifdef __HIPCC__
 // vertex k of face f, edges' ends, edges and their order around a face
 constexpr int kHexFace[6][4] = {{0, 1, 2, 3}, {0, 1, 5, 4}, {1, 2, 6, 5}, {2, 3, 7, 6}, {3, 0, 4, 7}, {4, 5, 6, 7}};
 constexpr int kHexEdgeA[12] = {0, 1, 2, 3, 4, 5, 6, 7, 0, 1, 2, 3};
@@ -56,7 +55,7 @@ constexpr int kHexFaceEdge[5][4] = {{0, 1, 2, 3}, {0, 9, 4, 8}, {1, 10, 5, 9}, {
 // face corners; false if they are not a hexahedron's.
 constexpr int kHexIn = kGenHdr + 24 + 12 * kGenEdge + 6 * kGenFace + 24;
 constexpr int kHexInE = kGenHdr + 24, kHexInF = kHexInE + 12 * kGenEdge, kHexInV = kHexInF + 6 * kGenFace;
-__device__ inline bool hex_vertices(const double* rec, int* id)
+RH_HD bool hex_vertices(const double* rec, int* id)
 {
     const double *ed = rec + kHexInE, *fc = rec + kHexInF, *fv = rec + kHexInV;
     for (int f = 0; f < 6; f++)
@@ -73,7 +72,7 @@ __device__ inline bool hex_vertices(const double* rec, int* id)
     }
     return true;
 }
-__device__ inline bool hex_edge_record(const double* rec, const int* id, int e, double* o)
+RH_HD bool hex_edge_record(const double* rec, const int* id, int e, double* o)
 {
     const double *vt = rec + kGenHdr, *ed = rec + kHexInE;
     const int a = id[e < 8 ? e : e - 8], b = id[e < 8 ? (e & 4) + ((e + 1) & 3) : e - 4];
@@ -95,7 +94,7 @@ __device__ inline bool hex_edge_record(const double* rec, const int* id, int e, 
     return true;
 }
 // the normal of face f in the order of kHexFace, null if it is no face
-__device__ inline const double* hex_normal(const double* rec, const int* id, int f)
+RH_HD const double* hex_normal(const double* rec, const int* id, int f)
 {
     const double *fc = rec + kHexInF, *fv = rec + kHexInV;
     const int i = f - 1, j = f & 3;
@@ -109,7 +108,7 @@ __device__ inline const double* hex_normal(const double* rec, const int* id, int
     }
     return nullptr;
 }
-__device__ inline bool hex_face_record(const double* rec, const int* id, int f, double* o)
+RH_HD bool hex_face_record(const double* rec, const int* id, int f, double* o)
 {
     const double* vt = rec + kGenHdr;
     const double *n = hex_normal(rec, id, f), *m = hex_normal(rec, id, 5);
@@ -132,7 +131,7 @@ __device__ inline bool hex_face_record(const double* rec, const int* id, int f, 
     o[kHexD2 + f] = dot(e2, e2);
     return true;
 }
-__device__ inline void hex_close_record(const double* rec, const int* id, double* o)
+RH_HD void hex_close_record(const double* rec, const int* id, double* o)
 {
     for (int k = 0; k < 8; k++)
         for (int c = 0; c < 3; c++) o[3 * k + c] = rec[kGenHdr + 3 * id[k] + c];
@@ -144,7 +143,7 @@ __device__ inline void hex_close_record(const double* rec, const int* id, double
     o[kHex - 1] = 0.0;
 }
 
-__device__ __forceinline__ void far_tet_record(const double* __restrict__ rec, double* __restrict__ o)
+RH_HD void far_tet_record(const double* __restrict__ rec, double* __restrict__ o)
 {
     for (int k = 0; k < 12; k++) o[k] = rec[k];
     double* g = o + kFarG;
@@ -180,26 +179,22 @@ __device__ __forceinline__ void far_tet_record(const double* __restrict__ rec, d
     for (int k = 0; k < 3; k++) o[kFarN3 + k] = n3[k];
 }
 template <class R>
-__device__ __forceinline__ const R* far_geo(const double* __restrict__ rec)
+RH_HD const R* far_geo(const double* __restrict__ rec)
 {
     if constexpr (sizeof(R) == 4) return reinterpret_cast<const float*>(rec + kFarG32);
     else return rec + kFarG;
 }
 
 // 2 atanh(X/2) for X <= 1/2 and atan(t) for |t| <= tan(pi/16), no branches.
-__device__ __forceinline__ double far_atanh2(double X)
+RH_HD double far_atanh2(double X)
 {
-#ifdef __HIP_DEVICE_COMPILE__
     const double u = X * X;
     double p = d_edge2_p[7];
 #pragma unroll
     for (int k = 6; k >= 0; k--) p = fma(p, u, d_edge2_p[k]);
     return fma(X * u, p, X);
-#else
-    return X;
-#endif
 }
-__device__ __forceinline__ float far_atanh2(float X)
+RH_HD float far_atanh2(float X)
 {
     // the degree-3 interpolant on X <= 1/2 (8e-10 relative)
     const float u = X * X;
@@ -208,25 +203,21 @@ __device__ __forceinline__ float far_atanh2(float X)
     p = fmaf(p, u, 0.0833333303f);
     return fmaf(X * u, p, X);
 }
-__device__ __forceinline__ double far_atan(double t)
+RH_HD double far_atan(double t)
 {
-#ifdef __HIP_DEVICE_COMPILE__
     const double u = t * t;
     double p = d_atan16_p[6];
 #pragma unroll
     for (int k = 5; k >= 0; k--) p = fma(p, u, d_atan16_p[k]);
     return fma(t * u, p, t);
-#else
-    return t;
-#endif
 }
-__device__ __forceinline__ float far_atan(float t)
+RH_HD float far_atan(float t)
 {
     const float u = t * t;
     const float p = fmaf(fmaf(-0.13649502f, u, 0.19990657f), u, -0.33333313f);
     return fmaf(t * u, p, t);
 }
-__device__ __forceinline__ float rh_div(float y, float d) { return y * rh_rcp(d); }
+RH_HD float rh_div(float y, float d) { return y * rh_rcp(d); }
 
 // Distances of the vertices of a far record from p and their pair sums;
 // whether every lane of the wave is far.
@@ -236,7 +227,7 @@ struct FarTet {
     R d[4], S[6];
 };
 template <class R>
-__device__ __forceinline__ bool far_tet_open(const double* __restrict__ rec, const double p[3], FarTet<R>& t)
+RH_HD bool far_tet_open(const double* __restrict__ rec, const double p[3], FarTet<R>& t)
 {
     const R* g = far_geo<R>(rec);
 #pragma unroll
@@ -256,7 +247,7 @@ __device__ __forceinline__ bool far_tet_open(const double* __restrict__ rec, con
 // q5 = acc / (4 pi), kept as products: what is formed from the entries (zz, in
 // the layouts that store it) is then the same in every kernel, whatever the
 // compiler would contract.
-__device__ __forceinline__ void far_scale(const double (&acc)[5], double q5[5])
+RH_HD void far_scale(const double (&acc)[5], double q5[5])
 {
 #pragma unroll
     for (int k = 0; k < 5; k++) {
@@ -269,7 +260,7 @@ __device__ __forceinline__ void far_scale(const double (&acc)[5], double q5[5])
 
 // The block's xx, xy, xz, yy, yz (zz = -(xx + yy)).
 template <class R>
-__device__ __forceinline__ void far_tet_block(const double* __restrict__ rec, const FarTet<R>& t, double q5[5])
+RH_HD void far_tet_block(const double* __restrict__ rec, const FarTet<R>& t, double q5[5])
 {
     const R* g = far_geo<R>(rec);
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -302,7 +293,7 @@ __device__ __forceinline__ void far_tet_block(const double* __restrict__ rec, co
 // the point is inside (zz is then -(xx + yy) - 1): the signs of the four plane
 // distances, as in eval_tet.
 template <class R>
-__device__ __forceinline__ bool near_tet_block(const double* __restrict__ rec, const double p[3], double q5[5])
+RH_HD bool near_tet_block(const double* __restrict__ rec, const double p[3], double q5[5])
 {
     const R* g = far_geo<R>(rec);
     auto vtx = [&](int k, V3<R>& r, R& d) {
@@ -375,7 +366,7 @@ __device__ __forceinline__ bool near_tet_block(const double* __restrict__ rec, c
 //
 // X, Y, Z: corner coordinates relative to the point, w: edge lengths.
 template <class R>
-__device__ __forceinline__ void far_rec_block(const R (&X)[2], const R (&Y)[2], const R (&Z)[2], const R (&D)[2][2][2],
+RH_HD void far_rec_block(const R (&X)[2], const R (&Y)[2], const R (&Z)[2], const R (&D)[2][2][2],
                                               const R (&w)[3], double q6[6])
 {
     // sums of end distances of the edges along x, y, z
@@ -436,13 +427,18 @@ __device__ __forceinline__ void far_rec_block(const R (&X)[2], const R (&Y)[2], 
 
 // Q of a block at p (element frame); returns whether p is inside.
 template <class R>
-__device__ __forceinline__ bool rec_block(const double* __restrict__ rec, const double p[3], double q6[6])
+RH_HD bool rec_block(const double* __restrict__ rec, const double p[3], double q6[6])
 {
     const double c[3] = {rec[0] - p[0], rec[1] - p[1], rec[2] - p[2]};
     // FP32: lengths in units of a power of two near the distance (exact), since
     // the faces' factors are of the 12th degree in them
     double u = 1.0;
-    if (sizeof(R) == 4) u = ldexp(1.0, -(__builtin_amdgcn_frexp_exp(sq3(c[0], c[1], c[2])) >> 1));
+    if (sizeof(R) == 4) {
+        double mant;
+        int ex;
+        rh_frexp(sq3(c[0], c[1], c[2]), mant, ex);
+        u = ldexp(1.0, -(ex >> 1));
+    }
     R x[3][2], w[3], D[2][2][2];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -487,7 +483,7 @@ __device__ __forceinline__ bool rec_block(const double* __restrict__ rec, const 
 
 // The block at points near a hexahedron: one edge and one face at a time from
 // the record, each with the tier its wave needs, as near_tet_block.
-__device__ inline bool near_hex_block(const double* __restrict__ h, const double p[3], double q5[5])
+RH_HD bool near_hex_block(const double* __restrict__ h, const double p[3], double q5[5])
 {
     auto vtx = [&](int k, V3<double>& r, double& d) {
         r = rel<double>(h + 3 * k, p);
@@ -553,7 +549,7 @@ __device__ inline bool near_hex_block(const double* __restrict__ h, const double
 // both ends of every edge and every face's corners anew and reads its record
 // through chains of scalar loads (36,000 cycles where few waves hide them).
 // The far test is each lane's own, as for blocks.
-__device__ __forceinline__ bool gen_block(const double* __restrict__ h, const double* __restrict__ rec,
+RH_HD bool gen_block(const double* __restrict__ h, const double* __restrict__ rec,
                                           const double p[3], double q6[6])
 {
     if (!h) return eval_gen<double>(rec, p, q6);
@@ -610,6 +606,5 @@ __device__ __forceinline__ bool gen_block(const double* __restrict__ h, const do
     q6[5] = q5[4];
     return in;
 }
-#endif
 
 }  // namespace rh

@@ -411,3 +411,248 @@ int rhc_mesh_stats(const rh_model_desc* d, int64_t* out)
 }
 
 }  // extern "C"
+
+// ---------------------------------------------------------------- device forms
+// The forms that the kernels evaluate (rh_mesh.hpp, rh_far.hpp, rh_adjoint.hpp),
+// each point a wave of its own.
+namespace {
+using rh::V3;
+
+// One charged mesh in the device's layout.
+struct ChargedMesh {
+    std::vector<double> edge, face;
+};
+ChargedMesh charge_sweep(const rh::MeshForm& F, const double* M, bool pack32)
+{
+    std::vector<double> ce, cf, ci;
+    charge_mesh(F, M, ce, cf, ci);
+    ChargedMesh c;
+    c.edge.resize(ce.size());
+    c.face.resize(cf.size());
+    for (int64_t i = 0; i < F.n_edges(); i++)
+        rh::mesh_charge_edge(F.edge_geo.data() + rh::kMeshEdgeGeo * i, &ce[size_t(rh::kMeshEdge * i + 10)], pack32,
+                             &c.edge[size_t(rh::kMeshEdge * i)]);
+    for (int64_t i = 0; i < F.n_faces(); i++) {
+        const double* g = F.face_geo.data() + rh::kMeshFaceGeo * i;
+        // the net charge back from its vector along n
+        const double* v = &cf[size_t(rh::kMeshFace * i + 18)];
+        const double s = v[0] * g[12] + v[1] * g[13] + v[2] * g[14];
+        rh::mesh_charge_face(g, s, F.face_edge.data() + 3 * i, F.edge_geo.data(), c.edge.data(), pack32,
+                             &c.face[size_t(rh::kMeshFace * i)]);
+    }
+    return c;
+}
+
+// An edge swept on its own, and a face with the edges it owns, at x: what
+// k_field_mesh adds to 4 pi H.
+template <class R>
+void sweep_edge(const double* rec, const double x[3], double h[3])
+{
+    const double p[1][3] = {{x[0], x[1], x[2]}};
+    rh::MeshVtxN<R, 1> a, b;
+    rh::mesh_vtx<R, 1>(rec, p, a);
+    rh::mesh_vtx<R, 1>(rec + 3, p, b);
+    R s[1], L[1];
+    rh::mesh_sum<R, 1>(a, b, s);
+    double l;
+    if (sizeof(R) == 4) {
+        const float* f = reinterpret_cast<const float*>(rec + 6);
+        if (rh::mesh32_near(std::fmin(float(a.d[0]), float(b.d[0])), f[1])) {
+            l = rh::mesh_edge_L_near(rec, x);
+        } else {
+            rh::edge_L2(a.r, a.d, b.r, b.d, s, R(f[0]), rh::kEdge6Top, L);
+            l = double(L[0]);
+        }
+    } else {
+        rh::edge_L2(a.r, a.d, b.r, b.d, s, R(rec[9]), rh::kEdge6Top, L);
+        l = double(L[0]);
+    }
+    for (int k = 0; k < 3; k++) h[k] += l * rec[10 + k];
+}
+template <class R>
+void sweep_face(const double* rec, const int64_t* face_edge, const double x[3], double h[3])
+{
+    const int nv = rec[17] > 3.5 ? 4 : 3;
+    const double p[1][3] = {{x[0], x[1], x[2]}};
+    rh::MeshVtxN<R, 1> v[4];
+    float least = INFINITY;
+    for (int k = 0; k < nv; k++) {
+        rh::mesh_vtx<R, 1>(rec + 3 * k, p, v[k]);
+        least = std::fmin(least, float(v[k].d[0]));
+    }
+    int mask = 0;
+    for (int k = 0; k < 3; k++)
+        if (face_edge[k] >= 0) mask |= 1 << k;
+    if (sizeof(R) == 4 && rh::mesh32_near(least, reinterpret_cast<const float*>(rec + rh::kMeshFaceEdges + 13)[0])) {
+        const rh::MeshFace64 f = rh::mesh_face_near(rec, mask, x);
+        h[0] += f.h0 + f.om * rec[18];
+        h[1] += f.h1 + f.om * rec[19];
+        h[2] += f.h2 + f.om * rec[20];
+        return;
+    }
+    R s[4][1], om[1];
+    for (int k = 0; k < nv; k++) rh::mesh_sum<R, 1>(v[k], v[(k + 1) % nv], s[k]);
+    if (nv == 3)
+        rh::mesh_tri_half_omega<R, 1>(v[0], v[1], v[2], s[0], s[1], s[2], rec, rh::kAtan32Top, om);
+    else
+        rh::mesh_quad_half_omega<R, 1>(v[0], v[1], v[2], v[3], s[0], s[1], s[2], rec, rh::kAtan32Top, om);
+    for (int k = 0; k < 3; k++) h[k] += double(om[0]) * rec[18 + k];
+    for (int k = 0; k < 3; k++) {
+        if (!(mask & (1 << k))) continue;
+        const double* e = rec + rh::kMeshFaceEdges + 4 * k;
+        const int q = (k + 1) % nv;
+        R L[1];
+        rh::edge_L2(v[k].r, v[k].d, v[q].r, v[q].d, s[k], R(e[0]), rh::kEdge6Top, L);
+        for (int c = 0; c < 3; c++) h[c] += double(L[0]) * e[1 + c];
+    }
+}
+
+// Far-form record of a general polyhedron if it is a hexahedron.
+bool hex_record(const double* src, double* o)
+{
+    if (int(src[0]) != 8 || int(src[1]) != 12 || int(src[2]) != 6 || int(src[3]) != 24) return false;
+    int id[8];
+    if (!rh::hex_vertices(src, id)) return false;
+    for (int e = 0; e < 12; e++)
+        if (!rh::hex_edge_record(src, id, e, o)) return false;
+    for (int f = 0; f < 5; f++)
+        if (!rh::hex_face_record(src, id, f, o)) return false;
+    rh::hex_close_record(src, id, o);
+    return true;
+}
+
+// Q of one element in its own frame by the kernels' forms; returns whether the
+// point is inside.
+template <bool FAR32>
+bool device_block(int kind, const double* rec, const double* far, const double* hex, const double x[3], double q6[6])
+{
+    if (kind == rh::EK_REC) {
+        if (FAR32 && !rh::near_element<0>(kind, rec, x)) return rh::rec_block<float>(rec, x, q6);
+        return rh::rec_block<double>(rec, x, q6);
+    }
+    if (kind != rh::EK_TET) return rh::gen_block(hex, rec, x, q6);
+    double q5[5];
+    bool in = false;
+    if (!rh::far_tet_eval<FAR32>(far, x, q5)) in = rh::near_tet_eval<FAR32>(far, x, q5);
+    q6[0] = q5[0];
+    q6[1] = q5[3];
+    q6[2] = -(q5[0] + q5[3]) - (in ? 1.0 : 0.0);
+    q6[3] = q5[1];
+    q6[4] = q5[2];
+    q6[5] = q5[4];
+    return in;
+}
+}  // namespace
+
+extern "C" {
+
+// Field of the mesh form by the sweep's forms, other elements as rhc_field_mesh;
+// 2 when the model has no mesh form.
+int rhc_field_sweep(const rh_model_desc* d, const double* M, const double* pts, int64_t np, int32_t fp32, double* B,
+                    double* H)
+{
+    rh::PackedModel P;
+    rh_status st = rh::pack_model(d, &P, &g_err);
+    if (st != RH_OK) return st;
+    const rh::MeshForm& F = P.mesh;
+    if (!F.active) return 2;
+    const ChargedMesh c = charge_sweep(F, M, fp32 != 0);
+    std::vector<double> ce, cf, ci;
+    charge_mesh(F, M, ce, cf, ci);
+    rh::ModelView mv = view(P);
+    for (int64_t p = 0; p < np; p++) {
+        const double* x = pts + 3 * p;
+        double h[3] = {0, 0, 0}, mi[3] = {0, 0, 0}, hb[3] = {0, 0, 0}, bb[3] = {0, 0, 0};
+        for (int64_t i = 0; i < F.ne_free; i++) {
+            const double* rec = &c.edge[size_t(rh::kMeshEdge * i)];
+            if (fp32) sweep_edge<float>(rec, x, h);
+            else sweep_edge<double>(rec, x, h);
+        }
+        for (int64_t i = 0; i < F.n_faces(); i++) {
+            const double* rec = &c.face[size_t(rh::kMeshFace * i)];
+            if (fp32) sweep_face<float>(rec, F.face_edge.data() + 3 * i, x, h);
+            else sweep_face<double>(rec, F.face_edge.data() + 3 * i, x, h);
+        }
+        for (int64_t i = 0; i < F.n_in(); i++) {
+            const double* r = &ci[size_t(rh::kMeshIn * i)];
+            if (rh::mesh_inside(r, x))
+                for (int k = 0; k < 3; k++) mi[k] += r[1 + k];
+        }
+        rh::field_add<double, true, 0>(mv, M, P.kind_idx.data(), P.kind_off[0], P.kind_off[1], x, bb, hb);
+        for (int k = 0; k < 3; k++) {
+            const double hk = h[k] * rh::kInv4Pi;
+            B[3 * p + k] = hk + mi[k] + bb[k];
+            H[3 * p + k] = hk + hb[k];
+        }
+    }
+    return RH_OK;
+}
+
+// Blocks q9 [np][n][9] of every element (its own frame, no transforms) at np
+// points by the kernels' forms (fp32: the mixed assembly's choice), and whether
+// the point is inside [np][n].
+int rhc_device_blocks(const rh_model_desc* d, const double* pts, int64_t np, int32_t fp32, double* q9, int32_t* inside)
+{
+    rh::PackedModel P;
+    rh_status st = rh::pack_model(d, &P, &g_err);
+    if (st != RH_OK) return st;
+    for (int64_t j = 0; j < P.n; j++) {
+        const double* rec = P.data.data() + P.off[j];
+        double far[rh::kFarTet], hex[rh::kHex];
+        const double* hx = nullptr;
+        if (P.kind[j] == rh::EK_TET) rh::far_tet_record(rec, far);
+        else if (P.kind[j] == rh::EK_GEN && hex_record(rec, hex)) hx = hex;
+        for (int64_t p = 0; p < np; p++) {
+            double q6[6];
+            const bool in = fp32 ? device_block<true>(P.kind[j], rec, far, hx, pts + 3 * p, q6)
+                                 : device_block<false>(P.kind[j], rec, far, hx, pts + 3 * p, q6);
+            rh::q6_to_q9(q6, q9 + 9 * (p * P.n + j));
+            inside[p * P.n + j] = in ? 1 : 0;
+        }
+    }
+    return RH_OK;
+}
+
+// rhc_adj_grad by the closed-form derivatives of the kernel.
+int rhc_adj_grad_tri(const rh_model_desc* d, const double* M, const double* pts, int64_t np, const double* g,
+                     double* gV, double* gX)
+{
+    rh::PackedModel P;
+    rh_status st = rh::pack_model(d, &P, &g_err);
+    if (st != RH_OK) return st;
+    const int64_t nvert = P.vert_off.back();
+    for (int64_t k = 0; k < 3 * nvert; k++) gV[k] = 0.0;
+    for (int64_t k = 0; k < 3 * np; k++) gX[k] = 0.0;
+    for (int64_t j = 0; j < P.n; j++) {
+        const double* rec = P.adj.data() + P.adj_off[j];
+        const double* tri = rec + 2 + 3 * rh::adj_nv(rec);
+        for (int t = 0; t < rh::adj_ntri(rec); t++) {
+            rh::TriLane T;
+            for (int k = 0; k < 3; k++) {
+                const double* v = rec + 2 + 3 * int(tri[3 * t + k]);
+                T.v[k] = V3<double>{v[0], v[1], v[2]};
+            }
+            rh::tri_open(T, V3<double>{M[3 * j], M[3 * j + 1], M[3 * j + 2]});
+            for (int64_t p = 0; p < np; p++) {
+                V3<double> gx{0.0, 0.0, 0.0};
+                rh::tri_point(T, pts + 3 * p,
+                              V3<double>{rh::kInv4Pi * g[3 * p], rh::kInv4Pi * g[3 * p + 1], rh::kInv4Pi * g[3 * p + 2]},
+                              gx);
+                gX[3 * p] += gx.x;
+                gX[3 * p + 1] += gx.y;
+                gX[3 * p + 2] += gx.z;
+            }
+            V3<double> G[3];
+            rh::tri_close(T, G);
+            for (int k = 0; k < 3; k++) {
+                double* o = gV + 3 * (P.vert_off[j] + int(tri[3 * t + k]));
+                o[0] += G[k].x;
+                o[1] += G[k].y;
+                o[2] += G[k].z;
+            }
+        }
+    }
+    return RH_OK;
+}
+
+}  // extern "C"

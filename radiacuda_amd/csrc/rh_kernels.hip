@@ -96,40 +96,6 @@ __global__ __launch_bounds__(256) void k_no_hex(int64_t n, const int32_t* __rest
     if (k < n) at[kidx[k]] = -1;
 }
 
-// The far form of a tetrahedron's block at x when every lane of the wave is
-// far (else false).  FAR32: FP32 integrals beyond two circumradii of the
-// vertex mean, as block_Q_mixed takes them (vertices come first in the far
-// record, as in the element record).
-template <bool FAR32>
-__device__ __forceinline__ bool tet_fp32(const double* __restrict__ far, const double x[3])
-{
-    if constexpr (FAR32) return !rh_any(near_element<1>(EK_TET, far, x));
-    else return false;
-}
-template <bool FAR32>
-__device__ __forceinline__ bool far_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
-{
-    auto eval = [&](auto zero) {
-        using R = decltype(zero);
-        FarTet<R> t;
-        if (!far_tet_open<R>(far, x, t)) return false;
-        far_tet_block<R>(far, t, q5);
-        return true;
-    };
-    if constexpr (FAR32) {
-        if (tet_fp32<FAR32>(far, x)) return eval(float(0));
-    }
-    return eval(double(0));
-}
-template <bool FAR32>
-__device__ __forceinline__ bool near_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
-{
-    if constexpr (FAR32) {
-        if (tet_fp32<FAR32>(far, x)) return near_tet_block<float>(far, x, q5);
-    }
-    return near_tet_block<double>(far, x, q5);
-}
-
 template <class T>
 __device__ __forceinline__ void store_out(T* p, double v) { *p = T(v); }
 
@@ -768,21 +734,7 @@ __global__ __launch_bounds__(256) void k_mesh_charge_edges(MeshDev md, const dou
         w[1] += W[3] * m0 + W[4] * m1 + W[5] * m2;
         w[2] += W[6] * m0 + W[7] * m1 + W[8] * m2;
     }
-    const double* g = md.edge_geo + kMeshEdgeGeo * i;
-    double* o = md.ch_edge + kMeshEdge * i;
-    for (int k = 0; k < kMeshEdgeGeo - 1; k++) o[k] = g[k];
-    o[9] = 2.0 * g[9];
-    o[10] = w[0];
-    o[11] = w[1];
-    o[12] = w[2];
-    o[13] = 0.0;
-    if (pack32) {
-        // slot 6: 2 len and the near distance of the FP32 sweep (kNear32 lengths)
-        float* f = reinterpret_cast<float*>(o + 6);
-        const float len = float(g[9]);
-        f[0] = 2.0f * len;
-        f[1] = kNear32 * len;
-    }
+    mesh_charge_edge(md.edge_geo + kMeshEdgeGeo * i, w, pack32, md.ch_edge + kMeshEdge * i);
 }
 
 __global__ __launch_bounds__(256) void k_mesh_charge_faces(MeshDev md, const double* __restrict__ M, bool pack32)
@@ -790,78 +742,14 @@ __global__ __launch_bounds__(256) void k_mesh_charge_faces(MeshDev md, const dou
     const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (i >= md.nf) return;
     const double* g = md.face_geo + kMeshFaceGeo * i;
-    const double n0 = g[12], n1 = g[13], n2 = g[14];
     double s = 0.0;
     for (int64_t k = md.face_inc_off[i]; k < md.face_inc_off[i + 1]; k++) {
         const int64_t j = md.face_inc_elem[k];
         const double* v = md.face_inc_v + 3 * k;
         s += v[0] * M[3 * j] + v[1] * M[3 * j + 1] + v[2] * M[3 * j + 2];
     }
-    double* o = md.ch_face + kMeshFace * i;
-    const bool tri = !(g[17] > 3.5);
-    const double a1 = g[15], a2 = g[16];
-    const double nk = tri ? 2.0 * a1 : 1.0;  // triangles: n scaled by four times the area
-    for (int k = 0; k < 12; k++) o[k] = g[k];
-    o[12] = nk * n0;
-    o[13] = nk * n1;
-    o[14] = nk * n2;
-    o[15] = 2.0 * a1;
-    o[16] = 2.0 * a2;
-    o[17] = g[17];
-    // squared distances of (v0,v1), (v1,v2), (v0,v2), (v2,v3), (v0,v3)
-    const int pa[5] = {0, 1, 0, 2, 0}, pb[5] = {1, 2, 2, 3, 3};
-    double l2[5];
-    for (int k = 0; k < 5; k++) {
-        const double* u = g + 3 * pa[k];
-        const double* v = g + 3 * pb[k];
-        l2[k] = (tri && k > 2) ? 0.0 : sq3(v[0] - u[0], v[1] - u[1], v[2] - u[2]);
-        o[kMeshFaceLen2 + k] = l2[k];
-    }
-    o[kMeshFaceLen2 + 5] = 0.0;
-    o[18] = -2.0 * (s * n0);
-    o[19] = -2.0 * (s * n1);
-    o[20] = -2.0 * (s * n2);
-    o[21] = 0.0;
-    // owned edges: twice the length and the net weight of the charged edge record
-    // (charged before the faces, on the same stream)
-    for (int k = 0; k < 3; k++) {
-        const int64_t e = md.face_edge[3 * i + k];
-        double* d = o + kMeshFaceEdges + 4 * k;
-        if (e >= 0) {
-            const double* ce = md.ch_edge + kMeshEdge * e;
-            d[0] = 2.0 * md.edge_geo[kMeshEdgeGeo * e + 9];
-            d[1] = ce[10];
-            d[2] = ce[11];
-            d[3] = ce[12];
-        } else {
-            d[0] = d[1] = d[2] = d[3] = 0.0;
-        }
-    }
-    o[kMeshFaceEdges + 12] = 0.0;
-    o[kMeshFaceEdges + 13] = 0.0;
-    if (pack32) {
-        // slot 35: the near distance of the FP32 sweep (kNear32 longest sides)
-        const int nv = tri ? 3 : 4;
-        double lmax = 0.0;
-        for (int k = 0; k < nv; k++) {
-            const double* a = g + 3 * k;
-            const double* b = g + 3 * ((k + 1) % nv);
-            const double d0 = b[0] - a[0], d1 = b[1] - a[1], d2 = b[2] - a[2];
-            lmax = fmax(lmax, sqrt(d0 * d0 + d1 * d1 + d2 * d2));
-        }
-        reinterpret_cast<float*>(o + kMeshFaceEdges + 13)[0] = float(double(kNear32) * lmax);
-    }
-    if (pack32) {
-        float* f = reinterpret_cast<float*>(o + 12);
-        f[0] = float(nk * n0);
-        f[1] = float(nk * n1);
-        f[2] = float(nk * n2);
-        f[3] = float(2.0 * a1);
-        f[4] = float(2.0 * a2);
-        f[5] = 0.0f;
-        float* l = reinterpret_cast<float*>(o + kMeshFaceLen2);
-        for (int k = 0; k < 5; k++) l[k] = float(l2[k]);
-    }
+    // owned edges were charged before, on the same stream
+    mesh_charge_face(g, s, md.face_edge + 3 * i, md.edge_geo, md.ch_edge, pack32, md.ch_face + kMeshFace * i);
 }
 
 __global__ __launch_bounds__(256) void k_mesh_charge_in(MeshDev md, const double* __restrict__ M)

@@ -42,11 +42,15 @@
 
 namespace rh {
 
-#ifdef __HIPCC__
 // Votes over the active lanes, straight from the comparison's mask (__all and
 // __any first turn the lane's answer into an integer and compare that again).
+// The host build is a wave of one lane.
+#ifdef __HIP_DEVICE_COMPILE__
 __device__ __forceinline__ bool rh_all(bool c) { return __builtin_amdgcn_ballot_w64(!c) == 0; }
 __device__ __forceinline__ bool rh_any(bool c) { return __builtin_amdgcn_ballot_w64(c) != 0; }
+#else
+RH_HD bool rh_all(bool c) { return c; }
+RH_HD bool rh_any(bool c) { return c; }
 #endif
 
 constexpr double kInv4Pi = 0.079577471545947667884441881686257181;  // 1/(4 pi)
@@ -166,43 +170,39 @@ RH_HD float rh_log1p(float x)
 // (atan(t)/t - 1)/t^2 on those ranges, fitted at 60 digits; evaluated in
 // double they are within 6e-17 absolute of ln(a/b) and 3e-17 of atan t.  The host build
 // runs the same code with exactly rounded seeds.
-constexpr double kLogP[10] = {0.6666666666666666,  0.40000000000014585, 0.2857142856710876,
-                              0.22222222717427864, 0.18181789436132859, 0.15385570064958623,
-                              0.13314144209654935, 0.12001072809590713, 0.08800738486144674,
-                              0.1616404561194353};
-constexpr double kAtanP[11] = {-0.3333333333333333,  0.1999999999999552,   -0.14285714284666542,
-                               0.11111111015256361,  -0.09090904578123903, 0.07692183190826087,
-                               -0.06664511447381948, 0.0585814891280221,   -0.0508544973794026,
-                               0.03923165829558719,  -0.01917688711906226};
-#ifdef __HIP_DEVICE_COMPILE__
-// The same coefficients in constant memory: the kernels then hold them in
+//
+// The coefficients lie in constant memory: the kernels then hold them in
 // scalar registers and the Horner steps take them as the scalar operand of
 // v_fma_f64 (as immediates they are copied into vector registers per step).
-static __constant__ double d_log_p[10] = {0.6666666666666666,  0.40000000000014585, 0.2857142856710876,
+#ifdef __HIP_DEVICE_COMPILE__
+#define RH_TABLE static __constant__ double
+#else
+#define RH_TABLE static constexpr double
+#endif
+RH_TABLE d_log_p[10] = {0.6666666666666666,  0.40000000000014585, 0.2857142856710876,
                                           0.22222222717427864, 0.18181789436132859, 0.15385570064958623,
                                           0.13314144209654935, 0.12001072809590713, 0.08800738486144674,
                                           0.1616404561194353};
-static __constant__ double d_atan_p[11] = {
+RH_TABLE d_atan_p[11] = {
     -0.3333333333333333,  0.1999999999999552,   -0.14285714284666542, 0.11111111015256361,
     -0.09090904578123903, 0.07692183190826087,  -0.06664511447381948, 0.0585814891280221,
     -0.0508544973794026,  0.03923165829558719,  -0.01917688711906226};
 // (atan(t) - t)/t^3 on |t| <= tan(pi/16) in u = t^2: Chebyshev interpolant of
 // degree 6 fitted at 60 digits (within 7.3e-18 of atan t)
-static __constant__ double d_atan16_p[7] = {-0.33333333333333237, 0.19999999999760989, -0.14285714188882722,
+RH_TABLE d_atan16_p[7] = {-0.33333333333333237, 0.19999999999760989, -0.14285714188882722,
                                             0.11111096372965646,  -0.090898379007095286, 0.076521309422432607,
                                             -0.059098572131161474};
 // the same on |t| <= 1/32, degree 3 (within 2e-20 of atan t)
-static __constant__ double d_atan32_p[4] = {-0.3333333333333327, 0.19999999997886797, -0.1428570346460735,
+RH_TABLE d_atan32_p[4] = {-0.3333333333333327, 0.19999999997886797, -0.1428570346460735,
                                             0.11093375583013043};
 // ln((1 + X/2)/(1 - X/2)) = X + X^3 P(X^2): P on X <= 1/6 (degree 4, within
 // 1.7e-17 of the result, relative) and on X <= 1/2 (degree 7, 3.1e-17),
 // Chebyshev interpolants fitted at 60 digits
-static __constant__ double d_edge6_p[5] = {0.08333333333333395, 0.01249999999889163, 0.0022321431761517696,
+RH_TABLE d_edge6_p[5] = {0.08333333333333395, 0.01249999999889163, 0.0022321431761517696,
                                            0.00043399566660258694, 9.009544000788967e-05};
-static __constant__ double d_edge2_p[8] = {0.08333333333333322,   0.012500000000060307,  0.002232142852088486,
+RH_TABLE d_edge2_p[8] = {0.08333333333333322,   0.012500000000060307,  0.002232142852088486,
                                            0.0004340279388094421, 8.877589708906781e-05, 1.8801225959087634e-05,
                                            3.971004714131101e-06, 1.128428632788004e-06};
-#endif
 // Coefficients of a branch that few waves take: read there (the address is
 // hidden from the compiler, which would otherwise load every branch's
 // coefficients ahead of the sweep's loop and spill scalar registers for them).
@@ -214,6 +214,9 @@ __device__ __forceinline__ CoefPtr rh_coef_rare(const double* c)
     asm volatile("" : "+s"(a));
     return (CoefPtr)a;
 }
+#else
+typedef const double* CoefPtr;
+RH_HD CoefPtr rh_coef_rare(const double* c) { return c; }
 #endif
 constexpr double kAtan32Top = 0.11093375583013043, kEdge6Top = 9.009544000788967e-05;
 constexpr double kTanPi16 = 0.19891236737965800;
@@ -247,13 +250,17 @@ RH_HD double rh_div(double y, double d)
     return fma(t, fma(e, e, e), t);
 }
 
-RH_HD double rh_sqrt(double x)
+RH_HD double rh_rsq_seed(double x)
 {
 #ifdef __HIP_DEVICE_COMPILE__
-    const double y = __builtin_amdgcn_rsq(x);
+    return __builtin_amdgcn_rsq(x);
 #else
-    const double y = 1.0 / sqrt(x);
+    return 1.0 / sqrt(x);
 #endif
+}
+RH_HD double rh_sqrt(double x)
+{
+    const double y = rh_rsq_seed(x);
     // the seed is within 2^-24 (measured on gfx950): with g = x y and
     // e = 1 - g y (exact but for its last rounding), sqrt(x) = g / sqrt(1 - e)
     // up to half of g's own rounding error; the series is cut after e^2
@@ -293,11 +300,7 @@ RH_HD double rh_log_ratio_c(double num, double den, C c)
 }
 RH_HD double rh_log_ratio(double num, double den)
 {
-#ifdef __HIP_DEVICE_COMPILE__
     return rh_log_ratio_c(num, den, d_log_p);
-#else
-    return rh_log_ratio_c(num, den, kLogP);
-#endif
 }
 RH_HD float rh_log_ratio(float num, float den) { return logf(num / den); }
 
@@ -321,11 +324,7 @@ RH_HD double rh_atan2_c(double y, double x, C c)
 }
 RH_HD double rh_atan2(double y, double x)
 {
-#ifdef __HIP_DEVICE_COMPILE__
     return rh_atan2_c(y, x, d_atan_p);
-#else
-    return rh_atan2_c(y, x, kAtanP);
-#endif
 }
 
 // atan2 for sweeps in which most angles are small.  Four tiers, chosen per
@@ -345,12 +344,9 @@ RH_HD double rh_atan2(double y, double x)
 // decide, and the two differ by rounding (about 1e-17 absolute).  A sweep's
 // result for one point can change at that level with the order or batching
 // of the points.
-#ifdef __HIPCC__
 template <int N>
-__device__ __forceinline__ void rh_atan2_wave(const double (&y)[N], const double (&x)[N], double top_c,
-                                              double (&a)[N])
+RH_HD void rh_atan2_wave(const double (&y)[N], const double (&x)[N], double top_c, double (&a)[N])
 {
-#ifdef __HIP_DEVICE_COMPILE__
     // waves whose angles are all below 1/32 or pi/16 (distant faces) take a
     // shorter polynomial (same accuracy on that range)
     bool c32 = true;
@@ -398,19 +394,13 @@ __device__ __forceinline__ void rh_atan2_wave(const double (&y)[N], const double
             a[i] = rh_atan2_c(y[i], x[i], c);
         }
     }
-#endif
 }
-#endif
 RH_HD double rh_atan2_wave(double y, double x)
 {
-#ifdef __HIP_DEVICE_COMPILE__
     const double yy[1] = {y}, xx[1] = {x};
     double a[1];
     rh_atan2_wave(yy, xx, kAtan32Top, a);
     return a[0];
-#else
-    return rh_atan2(y, x);
-#endif
 }
 // FP32 counterpart: degree 2 below pi/16 (within 9e-9 of atan t in float
 // arithmetic, 1.6e-9 in exact arithmetic) and degree 4 below pi/8 (1.8e-8);
@@ -418,7 +408,6 @@ RH_HD double rh_atan2_wave(double y, double x)
 // 1e-8 of an angle with the order or batching of the points.
 RH_HD float rh_atan2_wave(float y, float x)
 {
-#ifdef __HIP_DEVICE_COMPILE__
     // below pi/16: degree 2 in t^2 (within 9e-9 of atan t in float arithmetic)
     if (rh_all(fabsf(y) < 0.19891237f * x)) {
         const float t = y * rh_rcp(x);
@@ -434,12 +423,10 @@ RH_HD float rh_atan2_wave(float y, float x)
                              u * (-0.14263956248760223f + u * (0.10743731260299683f + u * -0.06451927870512009f)));
         return fmaf(t * u, p, t);
     }
-#endif
     return rh_atan2(y, x);
 }
-#ifdef __HIPCC__
 template <int N>
-__device__ __forceinline__ void rh_atan2_wave(const float (&y)[N], const float (&x)[N], double, float (&a)[N])
+RH_HD void rh_atan2_wave(const float (&y)[N], const float (&x)[N], double, float (&a)[N])
 {
     bool c16 = true;
 #pragma unroll
@@ -456,7 +443,6 @@ __device__ __forceinline__ void rh_atan2_wave(const float (&y)[N], const float (
 #pragma unroll
     for (int i = 0; i < N; i++) a[i] = rh_atan2_wave(y[i], x[i]);
 }
-#endif
 
 // Vertex relative to the observation point, formed in FP64 then rounded to R.
 template <class R>
@@ -526,10 +512,7 @@ RH_HD void edge_L_ratio(const V3<double>& ra, double Ra, const V3<double>& rb, d
     const double q = len * (len + (Ra + Rb));
     den = fma(Ra, Rb, dab);
     num = den + q;
-#ifdef __HIP_DEVICE_COMPILE__
-    if (!rh_all(dab >= 0.0))
-#endif
-    {
+    if (!rh_all(dab >= 0.0)) {
         RH_KEEP_BRANCH();
         if (dab < 0.0) {
             const V3<double> c = cross(ra, rb);
@@ -550,10 +533,7 @@ RH_HD float edge_L(const V3<float>& ra, float Ra, const V3<float>& rb, float Rb,
 {
     const float q = len * (len + (Ra + Rb));
     float delta = q * rh_rcp(fmaf(Ra, Rb, dab));
-#ifdef __HIP_DEVICE_COMPILE__
-    if (!rh_all(dab >= 0.0f))
-#endif
-    {
+    if (!rh_all(dab >= 0.0f)) {
         RH_KEEP_BRANCH();
         if (dab < 0.0f) {
             const V3<float> c = cross(ra, rb);
@@ -569,7 +549,6 @@ RH_HD R edge_L(const V3<R>& ra, R Ra, const V3<R>& rb, R Rb, R len)
     return edge_L(ra, Ra, rb, Rb, dot(ra, rb), len);
 }
 
-#ifdef __HIPCC__
 // The same integral from twice the length and the sum S = Ra + Rb at N points
 // of a lane, for sweeps in which most edges are short against their distance:
 // with X = 2 len / S, L = 2 atanh(X/2) = X + X^3 P(X^2).  No term cancels, so the error is relative
@@ -581,11 +560,9 @@ RH_HD R edge_L(const V3<R>& ra, R Ra, const V3<R>& rb, R Rb, R len)
 // coefficient (kEdge6Top) in a vector register: an FMA of two scalar operands
 // needs a move first.
 template <int N>
-__device__ __forceinline__ void edge_L2(const V3<double> (&ra)[N], const double (&Ra)[N], const V3<double> (&rb)[N],
-                                        const double (&Rb)[N], const double (&S)[N], double len2, double top_c,
-                                        double (&L)[N])
+RH_HD void edge_L2(const V3<double> (&ra)[N], const double (&Ra)[N], const V3<double> (&rb)[N],
+                   const double (&Rb)[N], const double (&S)[N], double len2, double top_c, double (&L)[N])
 {
-#ifdef __HIP_DEVICE_COMPILE__
     double X[N], u[N], top = 0.0;
 #pragma unroll
     for (int i = 0; i < N; i++) {
@@ -621,13 +598,12 @@ __device__ __forceinline__ void edge_L2(const V3<double> (&ra)[N], const double 
         edge_L_ratio(ra[i], Ra[i], rb[i], Rb[i], dot(ra[i], rb[i]), 0.5 * len2, num, den);
         L[i] = rh_log_ratio_c(num, den, c);
     }
-#endif
 }
 // FP32: degree 2 on X <= 1/4 and degree 5 on X <= 1 (5.4e-9 relative), from
 // the same Chebyshev fits; the quotient carries about 2 ulp.
 template <int N>
-__device__ __forceinline__ void edge_L2(const V3<float> (&ra)[N], const float (&Ra)[N], const V3<float> (&rb)[N],
-                                        const float (&Rb)[N], const float (&S)[N], float len2, double, float (&L)[N])
+RH_HD void edge_L2(const V3<float> (&ra)[N], const float (&Ra)[N], const V3<float> (&rb)[N], const float (&Rb)[N],
+                   const float (&S)[N], float len2, double, float (&L)[N])
 {
     float X[N], u[N], top = 0.0f;
 #pragma unroll
@@ -660,7 +636,6 @@ __device__ __forceinline__ void edge_L2(const V3<float> (&ra)[N], const float (&
 #pragma unroll
     for (int i = 0; i < N; i++) L[i] = edge_L(ra[i], Ra[i], rb[i], Rb[i], 0.5f * len2);
 }
-#endif
 
 // Solid-angle factor of triangle (r1, r2, r3) as a complex number whose
 // argument is half the signed solid angle (Van Oosterom & Strackee 1983).
@@ -916,11 +891,7 @@ RH_HD bool tet_near32(const double* __restrict__ rec, const double p[3])
         const V3<float> r = rel<float>(rec + 3 * v, p);
         d = fminf(d, rh_sqrt(sq3(r.x, r.y, r.z)));
     }
-    bool near = d < kNear32 * float(rec[kChargedM + 3]);
-#ifdef __HIP_DEVICE_COMPILE__
-    near = rh_any(near);
-#endif
-    return near;
+    return rh_any(d < kNear32 * float(rec[kChargedM + 3]));
 }
 
 template <class R>

@@ -111,7 +111,6 @@ struct MeshVtxN {
     R d[N];
 };
 
-#ifdef __HIPCC__
 // FP32 sweep records: the geometry the lanes use in FP32 is stored as floats
 // when the records are charged (edge slot 6: 2 len, near distance; face slots
 // 12-14: n(3), the two doubled areas), so the sweep converts none of it per
@@ -122,7 +121,7 @@ struct MeshGeo {
     R n0, n1, n2, a1, a2, l01, l12, l02, l23, l03;
 };
 template <class R>
-__device__ __forceinline__ MeshGeo<R> mesh_geo(const double* __restrict__ rec)
+RH_HD MeshGeo<R> mesh_geo(const double* __restrict__ rec)
 {
     if constexpr (sizeof(R) == 4) {
         const float* f = reinterpret_cast<const float*>(rec + 12);
@@ -135,7 +134,7 @@ __device__ __forceinline__ MeshGeo<R> mesh_geo(const double* __restrict__ rec)
 }
 
 template <class R, int N>
-__device__ __forceinline__ void mesh_vtx(const double* __restrict__ v, const double (&p)[N][3], MeshVtxN<R, N>& o)
+RH_HD void mesh_vtx(const double* __restrict__ v, const double (&p)[N][3], MeshVtxN<R, N>& o)
 {
 #pragma unroll
     for (int i = 0; i < N; i++) {
@@ -145,7 +144,7 @@ __device__ __forceinline__ void mesh_vtx(const double* __restrict__ v, const dou
 }
 // S = Ra + Rb
 template <class R, int N>
-__device__ __forceinline__ void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b, R (&o)[N])
+RH_HD void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b, R (&o)[N])
 {
 #pragma unroll
     for (int i = 0; i < N; i++) o[i] = a.d[i] + b.d[i];
@@ -159,7 +158,7 @@ __device__ __forceinline__ void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN
 // keeps the error of the dot products' form (a few ulp of R^3), no dot product
 // is formed, and the sums are those that the edges' integrals divide by.
 template <class R, int N>
-__device__ __forceinline__ void mesh_tri_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
+RH_HD void mesh_tri_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
                                                     const MeshVtxN<R, N>& c, const R (&sab)[N], const R (&sbc)[N],
                                                     const R (&sca)[N], const double* __restrict__ rec, double top_c,
                                                     R (&om)[N])
@@ -173,7 +172,6 @@ __device__ __forceinline__ void mesh_tri_half_omega(const MeshVtxN<R, N>& a, con
     }
     rh_atan2_wave(im, re, top_c, om);
 }
-#endif
 
 // FP64 half solid angle of a face of an FP32 sweep record, whose normal and
 // areas are stored as floats: the fan triangles' triple products r0 . (r1 x r2)
@@ -211,11 +209,7 @@ RH_HD double mesh_face_half_omega_near(const double* __restrict__ rec, const dou
 // the record carries it (faces: slot 35, edges: slot 6, second float).
 RH_HD bool mesh32_near(float dmin, float thr)
 {
-    bool near = dmin < thr;
-#ifdef __HIP_DEVICE_COMPILE__
-    near = rh_any(near);
-#endif
-    return near;
+    return rh_any(dmin < thr);
 }
 
 // L_e of an FP32 sweep edge record in FP64 (vertices in slots 0-5, twice the
@@ -248,11 +242,10 @@ RH_HD MeshFace64 mesh_face_near(const double* __restrict__ rec, int mask, const 
     return t;
 }
 
-#ifdef __HIPCC__
 // Half the signed solid angle of a quadrilateral record, likewise: the fans
 // (v0,v1,v2) and (v0,v2,v3) multiplied as complex numbers.
 template <class R, int N>
-__device__ __forceinline__ void mesh_quad_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
+RH_HD void mesh_quad_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
                                                      const MeshVtxN<R, N>& c, const MeshVtxN<R, N>& d,
                                                      const R (&sab)[N], const R (&sbc)[N], const R (&scd)[N],
                                                      const double* __restrict__ rec, double top_c, R (&om)[N])
@@ -271,7 +264,96 @@ __device__ __forceinline__ void mesh_quad_half_omega(const MeshVtxN<R, N>& a, co
     }
     rh_atan2_wave(im, re, top_c, om);
 }
-#endif
+
+// Charged record of an edge with net weight w from its geometry, and of a face
+// with net charge s whose sides are the edges face_edge[k] (-1: not owned) of
+// the geometry edge_geo and the charged records ch_edge; pack32: for the FP32
+// sweep.
+RH_HD void mesh_charge_edge(const double* __restrict__ g, const double w[3], bool pack32, double* __restrict__ o)
+{
+    for (int k = 0; k < kMeshEdgeGeo - 1; k++) o[k] = g[k];
+    o[9] = 2.0 * g[9];
+    o[10] = w[0];
+    o[11] = w[1];
+    o[12] = w[2];
+    o[13] = 0.0;
+    if (pack32) {
+        // slot 6: 2 len and the near distance of the FP32 sweep (kNear32 lengths)
+        float* f = reinterpret_cast<float*>(o + 6);
+        const float len = float(g[9]);
+        f[0] = 2.0f * len;
+        f[1] = kNear32 * len;
+    }
+}
+RH_HD void mesh_charge_face(const double* __restrict__ g, double s, const int64_t* __restrict__ face_edge,
+                            const double* __restrict__ edge_geo, const double* __restrict__ ch_edge, bool pack32,
+                            double* __restrict__ o)
+{
+    const double n0 = g[12], n1 = g[13], n2 = g[14];
+    const bool tri = !(g[17] > 3.5);
+    const double a1 = g[15], a2 = g[16];
+    const double nk = tri ? 2.0 * a1 : 1.0;  // triangles: n scaled by four times the area
+    for (int k = 0; k < 12; k++) o[k] = g[k];
+    o[12] = nk * n0;
+    o[13] = nk * n1;
+    o[14] = nk * n2;
+    o[15] = 2.0 * a1;
+    o[16] = 2.0 * a2;
+    o[17] = g[17];
+    // squared distances of (v0,v1), (v1,v2), (v0,v2), (v2,v3), (v0,v3)
+    const int pa[5] = {0, 1, 0, 2, 0}, pb[5] = {1, 2, 2, 3, 3};
+    double l2[5];
+    for (int k = 0; k < 5; k++) {
+        const double* u = g + 3 * pa[k];
+        const double* v = g + 3 * pb[k];
+        l2[k] = (tri && k > 2) ? 0.0 : sq3(v[0] - u[0], v[1] - u[1], v[2] - u[2]);
+        o[kMeshFaceLen2 + k] = l2[k];
+    }
+    o[kMeshFaceLen2 + 5] = 0.0;
+    o[18] = -2.0 * (s * n0);
+    o[19] = -2.0 * (s * n1);
+    o[20] = -2.0 * (s * n2);
+    o[21] = 0.0;
+    // owned edges: twice the length and the net weight of the charged edge record
+    for (int k = 0; k < 3; k++) {
+        const int64_t e = face_edge[k];
+        double* d = o + kMeshFaceEdges + 4 * k;
+        if (e >= 0) {
+            const double* ce = ch_edge + kMeshEdge * e;
+            d[0] = 2.0 * edge_geo[kMeshEdgeGeo * e + 9];
+            d[1] = ce[10];
+            d[2] = ce[11];
+            d[3] = ce[12];
+        } else {
+            d[0] = d[1] = d[2] = d[3] = 0.0;
+        }
+    }
+    o[kMeshFaceEdges + 12] = 0.0;
+    o[kMeshFaceEdges + 13] = 0.0;
+    if (pack32) {
+        // slot 35: the near distance of the FP32 sweep (kNear32 longest sides)
+        const int nv = tri ? 3 : 4;
+        double lmax = 0.0;
+        for (int k = 0; k < nv; k++) {
+            const double* a = g + 3 * k;
+            const double* b = g + 3 * ((k + 1) % nv);
+            const double d0 = b[0] - a[0], d1 = b[1] - a[1], d2 = b[2] - a[2];
+            lmax = fmax(lmax, sqrt(d0 * d0 + d1 * d1 + d2 * d2));
+        }
+        reinterpret_cast<float*>(o + kMeshFaceEdges + 13)[0] = float(double(kNear32) * lmax);
+    }
+    if (pack32) {
+        float* f = reinterpret_cast<float*>(o + 12);
+        f[0] = float(nk * n0);
+        f[1] = float(nk * n1);
+        f[2] = float(nk * n2);
+        f[3] = float(2.0 * a1);
+        f[4] = float(2.0 * a2);
+        f[5] = 0.0f;
+        float* l = reinterpret_cast<float*>(o + kMeshFaceLen2);
+        for (int k = 0; k < 5; k++) l[k] = float(l2[k]);
+    }
+}
 
 // Plane test of one inside record.
 RH_HD bool mesh_inside(const double* __restrict__ rec, const double p[3])
