@@ -329,7 +329,7 @@ RH_HD double rh_atan2(double y, double x)
 
 // atan2 for sweeps in which most angles are small.  Four tiers, chosen per
 // wave by a vote over its active lanes:
-// - every lane has x > 0 and |y| <= x / 32: a degree-3 polynomial in t^2
+// - every lane has x > 0 and |y| < x / 32: a degree-3 polynomial in t^2
 //   fitted to that range (within 2e-20 of atan t in exact arithmetic);
 // - every lane has x > 0 and |y| < tan(pi/16) x: a degree-6 polynomial in t^2
 //   on t = y/x fitted to that range (within 7.4e-18 of atan t in exact
@@ -339,6 +339,8 @@ RH_HD double rh_atan2(double y, double x)
 //   (its octant reduction is the identity there), so this tier and rh_atan2
 //   give identical results;
 // - any other wave: rh_atan2.
+// The tests are strict, so that (0, 0), a face seen from a point on one of its
+// sides, falls through to rh_atan2, which answers 0.
 // A lane's result therefore depends on which points share its wave: a lane
 // below pi/16 gets the short polynomial or the long one as its wave-mates
 // decide, and the two differ by rounding (about 1e-17 absolute).  A sweep's
@@ -351,7 +353,7 @@ RH_HD void rh_atan2_wave(const double (&y)[N], const double (&x)[N], double top_
     // shorter polynomial (same accuracy on that range)
     bool c32 = true;
 #pragma unroll
-    for (int i = 0; i < N; i++) c32 = c32 && (fabs(y[i]) <= 0.03125 * x[i]);
+    for (int i = 0; i < N; i++) c32 = c32 && (fabs(y[i]) < 0.03125 * x[i]);
     if (rh_all(c32)) {
         const double* c = d_atan32_p;
 #pragma unroll
