@@ -219,13 +219,13 @@ struct TriLane {
     double al[3];     // per side: adjoint of its direction's own component
 };
 
-RH_HD V3<double> axpy(double a, const V3<double>& x, const V3<double>& y)
+RH_FORM V3<double> axpy(double a, const V3<double>& x, const V3<double>& y)
 {
     return V3<double>{fma(a, x.x, y.x), fma(a, x.y, y.y), fma(a, x.z, y.z)};
 }
 
 // Geometry of a triangle whose corners T.v are set, magnetization M, sums zero.
-RH_HD void tri_open(TriLane& T, const V3<double>& M)
+RH_FORM void tri_open(TriLane& T, const V3<double>& M)
 {
     for (int k = 0; k < 3; k++) {
         T.G[k] = V3<double>{0.0, 0.0, 0.0};
@@ -257,7 +257,7 @@ RH_HD void tri_open(TriLane& T, const V3<double>& M)
 // differences between a corner's two sides, never of the sides' own terms,
 // which are larger by distance over size.  gx: minus the sum of the corner
 // derivatives (the normal's and the directions' parts cancel in it).
-RH_HD void tri_point(TriLane& T, const double x[3], const V3<double>& g, V3<double>& gx)
+RH_FORM void tri_point(TriLane& T, const double x[3], const V3<double>& g, V3<double>& gx)
 {
     V3<double> r[3];
     double R[3], iR[3];
@@ -346,7 +346,7 @@ RH_HD void tri_point(TriLane& T, const double x[3], const V3<double>& g, V3<doub
 // Corner gradients from the sums.  Side directions: dt = (dd - t (t . dd))/len
 // moved both ends by -+ dd; the length's part is along t; the unit normal:
 // n = (v1 - v0) x (v2 - v0)/|.|
-RH_HD void tri_close(const TriLane& T, V3<double> (&G)[3])
+RH_FORM void tri_close(const TriLane& T, V3<double> (&G)[3])
 {
     const V3<double> e1 = vsub(T.v[1], T.v[0]), e2 = vsub(T.v[2], T.v[0]);
     const V3<double> q = vscale(axpy(-dot(T.n, T.N), T.n, T.N), T.ia);

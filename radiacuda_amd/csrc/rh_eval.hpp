@@ -158,13 +158,13 @@ RH_HD void block_Q_mixed(const ModelView& mv, int64_t j, const double x[3], doub
 // vertex mean, as block_Q_mixed takes them (vertices come first in the far
 // record, as in the element record).
 template <bool FAR32>
-RH_HD bool tet_fp32(const double* __restrict__ far, const double x[3])
+RH_FORM bool tet_fp32(const double* __restrict__ far, const double x[3])
 {
     if constexpr (FAR32) return !rh_any(near_element<1>(EK_TET, far, x));
     else return false;
 }
 template <bool FAR32>
-RH_HD bool far_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
+RH_FORM bool far_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
 {
     auto eval = [&](auto zero) {
         using R = decltype(zero);
@@ -179,7 +179,7 @@ RH_HD bool far_tet_eval(const double* __restrict__ far, const double x[3], doubl
     return eval(double(0));
 }
 template <bool FAR32>
-RH_HD bool near_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
+RH_FORM bool near_tet_eval(const double* __restrict__ far, const double x[3], double q5[5])
 {
     if constexpr (FAR32) {
         if (tet_fp32<FAR32>(far, x)) return near_tet_block<float>(far, x, q5);

@@ -55,7 +55,7 @@ constexpr int kHexFaceEdge[5][4] = {{0, 1, 2, 3}, {0, 9, 4, 8}, {1, 10, 5, 9}, {
 // face corners; false if they are not a hexahedron's.
 constexpr int kHexIn = kGenHdr + 24 + 12 * kGenEdge + 6 * kGenFace + 24;
 constexpr int kHexInE = kGenHdr + 24, kHexInF = kHexInE + 12 * kGenEdge, kHexInV = kHexInF + 6 * kGenFace;
-RH_HD bool hex_vertices(const double* rec, int* id)
+RH_FORM bool hex_vertices(const double* rec, int* id)
 {
     const double *ed = rec + kHexInE, *fc = rec + kHexInF, *fv = rec + kHexInV;
     for (int f = 0; f < 6; f++)
@@ -72,7 +72,7 @@ RH_HD bool hex_vertices(const double* rec, int* id)
     }
     return true;
 }
-RH_HD bool hex_edge_record(const double* rec, const int* id, int e, double* o)
+RH_FORM bool hex_edge_record(const double* rec, const int* id, int e, double* o)
 {
     const double *vt = rec + kGenHdr, *ed = rec + kHexInE;
     const int a = id[e < 8 ? e : e - 8], b = id[e < 8 ? (e & 4) + ((e + 1) & 3) : e - 4];
@@ -94,7 +94,7 @@ RH_HD bool hex_edge_record(const double* rec, const int* id, int e, double* o)
     return true;
 }
 // the normal of face f in the order of kHexFace, null if it is no face
-RH_HD const double* hex_normal(const double* rec, const int* id, int f)
+RH_FORM const double* hex_normal(const double* rec, const int* id, int f)
 {
     const double *fc = rec + kHexInF, *fv = rec + kHexInV;
     const int i = f - 1, j = f & 3;
@@ -108,7 +108,7 @@ RH_HD const double* hex_normal(const double* rec, const int* id, int f)
     }
     return nullptr;
 }
-RH_HD bool hex_face_record(const double* rec, const int* id, int f, double* o)
+RH_FORM bool hex_face_record(const double* rec, const int* id, int f, double* o)
 {
     const double* vt = rec + kGenHdr;
     const double *n = hex_normal(rec, id, f), *m = hex_normal(rec, id, 5);
@@ -131,7 +131,7 @@ RH_HD bool hex_face_record(const double* rec, const int* id, int f, double* o)
     o[kHexD2 + f] = dot(e2, e2);
     return true;
 }
-RH_HD void hex_close_record(const double* rec, const int* id, double* o)
+RH_FORM void hex_close_record(const double* rec, const int* id, double* o)
 {
     for (int k = 0; k < 8; k++)
         for (int c = 0; c < 3; c++) o[3 * k + c] = rec[kGenHdr + 3 * id[k] + c];
@@ -143,7 +143,7 @@ RH_HD void hex_close_record(const double* rec, const int* id, double* o)
     o[kHex - 1] = 0.0;
 }
 
-RH_HD void far_tet_record(const double* __restrict__ rec, double* __restrict__ o)
+RH_FORM void far_tet_record(const double* __restrict__ rec, double* __restrict__ o)
 {
     for (int k = 0; k < 12; k++) o[k] = rec[k];
     double* g = o + kFarG;
@@ -179,14 +179,14 @@ RH_HD void far_tet_record(const double* __restrict__ rec, double* __restrict__ o
     for (int k = 0; k < 3; k++) o[kFarN3 + k] = n3[k];
 }
 template <class R>
-RH_HD const R* far_geo(const double* __restrict__ rec)
+RH_FORM const R* far_geo(const double* __restrict__ rec)
 {
     if constexpr (sizeof(R) == 4) return reinterpret_cast<const float*>(rec + kFarG32);
     else return rec + kFarG;
 }
 
 // 2 atanh(X/2) for X <= 1/2 and atan(t) for |t| <= tan(pi/16), no branches.
-RH_HD double far_atanh2(double X)
+RH_FORM double far_atanh2(double X)
 {
     const double u = X * X;
     double p = d_edge2_p[7];
@@ -194,7 +194,7 @@ RH_HD double far_atanh2(double X)
     for (int k = 6; k >= 0; k--) p = fma(p, u, d_edge2_p[k]);
     return fma(X * u, p, X);
 }
-RH_HD float far_atanh2(float X)
+RH_FORM float far_atanh2(float X)
 {
     // the degree-3 interpolant on X <= 1/2 (8e-10 relative)
     const float u = X * X;
@@ -203,7 +203,7 @@ RH_HD float far_atanh2(float X)
     p = fmaf(p, u, 0.0833333303f);
     return fmaf(X * u, p, X);
 }
-RH_HD double far_atan(double t)
+RH_FORM double far_atan(double t)
 {
     const double u = t * t;
     double p = d_atan16_p[6];
@@ -211,13 +211,13 @@ RH_HD double far_atan(double t)
     for (int k = 5; k >= 0; k--) p = fma(p, u, d_atan16_p[k]);
     return fma(t * u, p, t);
 }
-RH_HD float far_atan(float t)
+RH_FORM float far_atan(float t)
 {
     const float u = t * t;
     const float p = fmaf(fmaf(-0.13649502f, u, 0.19990657f), u, -0.33333313f);
     return fmaf(t * u, p, t);
 }
-RH_HD float rh_div(float y, float d) { return y * rh_rcp(d); }
+RH_FORM float rh_div(float y, float d) { return y * rh_rcp(d); }
 
 // Distances of the vertices of a far record from p and their pair sums;
 // whether every lane of the wave is far.
@@ -227,7 +227,7 @@ struct FarTet {
     R d[4], S[6];
 };
 template <class R>
-RH_HD bool far_tet_open(const double* __restrict__ rec, const double p[3], FarTet<R>& t)
+RH_FORM bool far_tet_open(const double* __restrict__ rec, const double p[3], FarTet<R>& t)
 {
     const R* g = far_geo<R>(rec);
 #pragma unroll
@@ -247,7 +247,7 @@ RH_HD bool far_tet_open(const double* __restrict__ rec, const double p[3], FarTe
 // q5 = acc / (4 pi), kept as products: what is formed from the entries (zz, in
 // the layouts that store it) is then the same in every kernel, whatever the
 // compiler would contract.
-RH_HD void far_scale(const double (&acc)[5], double q5[5])
+RH_FORM void far_scale(const double (&acc)[5], double q5[5])
 {
 #pragma unroll
     for (int k = 0; k < 5; k++) {
@@ -260,7 +260,7 @@ RH_HD void far_scale(const double (&acc)[5], double q5[5])
 
 // The block's xx, xy, xz, yy, yz (zz = -(xx + yy)).
 template <class R>
-RH_HD void far_tet_block(const double* __restrict__ rec, const FarTet<R>& t, double q5[5])
+RH_FORM void far_tet_block(const double* __restrict__ rec, const FarTet<R>& t, double q5[5])
 {
     const R* g = far_geo<R>(rec);
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -293,7 +293,7 @@ RH_HD void far_tet_block(const double* __restrict__ rec, const FarTet<R>& t, dou
 // the point is inside (zz is then -(xx + yy) - 1): the signs of the four plane
 // distances, as in eval_tet.
 template <class R>
-RH_HD bool near_tet_block(const double* __restrict__ rec, const double p[3], double q5[5])
+RH_FORM bool near_tet_block(const double* __restrict__ rec, const double p[3], double q5[5])
 {
     const R* g = far_geo<R>(rec);
     auto vtx = [&](int k, V3<R>& r, R& d) {
@@ -366,7 +366,7 @@ RH_HD bool near_tet_block(const double* __restrict__ rec, const double p[3], dou
 //
 // X, Y, Z: corner coordinates relative to the point, w: edge lengths.
 template <class R>
-RH_HD void far_rec_block(const R (&X)[2], const R (&Y)[2], const R (&Z)[2], const R (&D)[2][2][2],
+RH_FORM void far_rec_block(const R (&X)[2], const R (&Y)[2], const R (&Z)[2], const R (&D)[2][2][2],
                                               const R (&w)[3], double q6[6])
 {
     // sums of end distances of the edges along x, y, z
@@ -427,7 +427,7 @@ RH_HD void far_rec_block(const R (&X)[2], const R (&Y)[2], const R (&Z)[2], cons
 
 // Q of a block at p (element frame); returns whether p is inside.
 template <class R>
-RH_HD bool rec_block(const double* __restrict__ rec, const double p[3], double q6[6])
+RH_FORM bool rec_block(const double* __restrict__ rec, const double p[3], double q6[6])
 {
     const double c[3] = {rec[0] - p[0], rec[1] - p[1], rec[2] - p[2]};
     // FP32: lengths in units of a power of two near the distance (exact), since
@@ -483,7 +483,7 @@ RH_HD bool rec_block(const double* __restrict__ rec, const double p[3], double q
 
 // The block at points near a hexahedron: one edge and one face at a time from
 // the record, each with the tier its wave needs, as near_tet_block.
-RH_HD bool near_hex_block(const double* __restrict__ h, const double p[3], double q5[5])
+RH_FORM bool near_hex_block(const double* __restrict__ h, const double p[3], double q5[5])
 {
     auto vtx = [&](int k, V3<double>& r, double& d) {
         r = rel<double>(h + 3 * k, p);
@@ -549,7 +549,7 @@ RH_HD bool near_hex_block(const double* __restrict__ h, const double p[3], doubl
 // both ends of every edge and every face's corners anew and reads its record
 // through chains of scalar loads (36,000 cycles where few waves hide them).
 // The far test is each lane's own, as for blocks.
-RH_HD bool gen_block(const double* __restrict__ h, const double* __restrict__ rec,
+RH_FORM bool gen_block(const double* __restrict__ h, const double* __restrict__ rec,
                                           const double p[3], double q6[6])
 {
     if (!h) return eval_gen<double>(rec, p, q6);

@@ -121,7 +121,7 @@ struct MeshGeo {
     R n0, n1, n2, a1, a2, l01, l12, l02, l23, l03;
 };
 template <class R>
-RH_HD MeshGeo<R> mesh_geo(const double* __restrict__ rec)
+RH_FORM MeshGeo<R> mesh_geo(const double* __restrict__ rec)
 {
     if constexpr (sizeof(R) == 4) {
         const float* f = reinterpret_cast<const float*>(rec + 12);
@@ -134,7 +134,7 @@ RH_HD MeshGeo<R> mesh_geo(const double* __restrict__ rec)
 }
 
 template <class R, int N>
-RH_HD void mesh_vtx(const double* __restrict__ v, const double (&p)[N][3], MeshVtxN<R, N>& o)
+RH_FORM void mesh_vtx(const double* __restrict__ v, const double (&p)[N][3], MeshVtxN<R, N>& o)
 {
 #pragma unroll
     for (int i = 0; i < N; i++) {
@@ -144,7 +144,7 @@ RH_HD void mesh_vtx(const double* __restrict__ v, const double (&p)[N][3], MeshV
 }
 // S = Ra + Rb
 template <class R, int N>
-RH_HD void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b, R (&o)[N])
+RH_FORM void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b, R (&o)[N])
 {
 #pragma unroll
     for (int i = 0; i < N; i++) o[i] = a.d[i] + b.d[i];
@@ -158,7 +158,7 @@ RH_HD void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b, R (&o)[N])
 // keeps the error of the dot products' form (a few ulp of R^3), no dot product
 // is formed, and the sums are those that the edges' integrals divide by.
 template <class R, int N>
-RH_HD void mesh_tri_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
+RH_FORM void mesh_tri_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
                                                     const MeshVtxN<R, N>& c, const R (&sab)[N], const R (&sbc)[N],
                                                     const R (&sca)[N], const double* __restrict__ rec, double top_c,
                                                     R (&om)[N])
@@ -245,7 +245,7 @@ RH_HD MeshFace64 mesh_face_near(const double* __restrict__ rec, int mask, const 
 // Half the signed solid angle of a quadrilateral record, likewise: the fans
 // (v0,v1,v2) and (v0,v2,v3) multiplied as complex numbers.
 template <class R, int N>
-RH_HD void mesh_quad_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
+RH_FORM void mesh_quad_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
                                                      const MeshVtxN<R, N>& c, const MeshVtxN<R, N>& d,
                                                      const R (&sab)[N], const R (&sbc)[N], const R (&scd)[N],
                                                      const double* __restrict__ rec, double top_c, R (&om)[N])
