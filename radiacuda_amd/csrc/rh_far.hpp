@@ -316,9 +316,8 @@ RH_FORM bool near_tet_block(const double* __restrict__ rec, const double p[3], d
     bool inside = true;
 #pragma unroll 1
     for (int f = 0; f < 3; f++) {
-        // faces (1,2,3) (0,3,2) (0,1,3): squared edges opposite a, b, c
+        // faces (1,2,3) (0,3,2) (0,1,3)
         const int a = (f == 0) ? 1 : 0, b = (f == 0) ? 2 : (f == 1 ? 3 : 1), c = (f == 1) ? 2 : 3;
-        const int ab = (f == 0) ? 3 : (f == 1 ? 2 : 0), bc = (f == 2) ? 4 : 5, ca = (f == 0) ? 4 : (f == 1 ? 1 : 2);
         V3<R> ra, rb, rc;
         R da, db, dc, om[1];
         vtx(a, ra, da);
@@ -326,7 +325,7 @@ RH_FORM bool near_tet_block(const double* __restrict__ rec, const double p[3], d
         vtx(c, rc, dc);
         const R* n = g + 12 + 3 * f;
         const R im[1] = {dot(ra, v3(n[0], n[1], n[2]))};
-        const R re[1] = {((da + db) * (db + dc)) * (dc + da) - (dc * g[6 + ab] + db * g[6 + ca] + da * g[6 + bc])};
+        const R re[1] = {tri_re2(ra, da, rb, db, rc, dc)};
         inside = inside && (im[0] > R(0));
         rh_atan2_wave(im, re, kAtan32Top, om);
         for (int k = 0; k < 5; k++) acc[k] += double(om[0]) * rec[kFarT + 5 * f + k];
@@ -505,10 +504,9 @@ RH_FORM bool near_hex_block(const double* __restrict__ h, const double p[3], dou
     bool inside = true;
 #pragma unroll 1
     for (int f = 0; f < 5; f++) {
-        // corners and edges as in kHexFace and kHexFaceEdge
+        // corners as in kHexFace
         const int i = f - 1, j = f & 3;
         const int b = (f == 0) ? 1 : j, c = (f == 0) ? 2 : 4 + j, e = (f == 0) ? 3 : 4 + i, a = (f == 0) ? 0 : i;
-        const int ab = (f == 0) ? 0 : i, bc = (f == 0) ? 1 : 8 + j, ce = (f == 0) ? 2 : 4 + i, ea = (f == 0) ? 3 : 8 + i;
         V3<double> ra, rb, rc, re;
         double da, db, dc, de, om[1];
         vtx(a, ra, da);
@@ -516,9 +514,8 @@ RH_FORM bool near_hex_block(const double* __restrict__ h, const double p[3], dou
         vtx(c, rc, dc);
         vtx(e, re, de);
         const double* g = h + kHexF + 5 * f;
-        const double D = da + dc, D2 = h[kHexD2 + f], z = dot(ra, v3(g[0], g[1], g[2]));
-        const double r1 = ((da + db) * (db + dc)) * D - (dc * h[kHexL2 + ab] + db * D2 + da * h[kHexL2 + bc]);
-        const double r2 = ((de + da) * (dc + de)) * D - (da * h[kHexL2 + ce] + de * D2 + dc * h[kHexL2 + ea]);
+        const double z = dot(ra, v3(g[0], g[1], g[2]));
+        const double r1 = tri_re2(ra, da, rb, db, rc, dc), r2 = tri_re2(ra, da, rc, dc, re, de);
         const double i1 = z * g[3], i2 = z * g[4];
         inside = inside && (z > 0.0);
         const double im[1] = {r1 * i2 + r2 * i1}, rr[1] = {r1 * r2 - i1 * i2};

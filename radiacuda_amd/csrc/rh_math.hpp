@@ -355,24 +355,22 @@ RH_HD double rh_atan2(double y, double x)
 // decide, and the two differ by rounding (about 1e-17 absolute).  A sweep's
 // result for one point can change at that level with the order or batching
 // of the points.
+// The first tier's polynomial.
 template <int N>
-RH_FORM void rh_atan2_wave(const double (&y)[N], const double (&x)[N], double top_c, double (&a)[N])
+RH_FORM void rh_atan32(const double (&y)[N], const double (&x)[N], double top_c, double (&a)[N])
 {
-    // waves whose angles are all below 1/32 or pi/16 (distant faces) take a
-    // shorter polynomial (same accuracy on that range)
-    bool c32 = true;
+    const double* c = d_atan32_p;
 #pragma unroll
-    for (int i = 0; i < N; i++) c32 = c32 && (fabs(y[i]) < 0.03125 * x[i]);
-    if (rh_all(c32)) {
-        const double* c = d_atan32_p;
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            const double t = rh_div(y[i], x[i]), u = t * t;
-            const double p = fma(fma(fma(top_c, u, c[2]), u, c[1]), u, c[0]);
-            a[i] = fma(t * u, p, t);
-        }
-        return;
+    for (int i = 0; i < N; i++) {
+        const double t = rh_div(y[i], x[i]), u = t * t;
+        const double p = fma(fma(fma(top_c, u, c[2]), u, c[1]), u, c[0]);
+        a[i] = fma(t * u, p, t);
     }
+}
+// The tiers after the first.
+template <int N>
+RH_FORM void rh_atan2_rest(const double (&y)[N], const double (&x)[N], double (&a)[N])
+{
     bool c16 = true, c8 = true;
 #pragma unroll
     for (int i = 0; i < N; i++) {
@@ -405,6 +403,15 @@ RH_FORM void rh_atan2_wave(const double (&y)[N], const double (&x)[N], double to
             a[i] = rh_atan2_c(y[i], x[i], c);
         }
     }
+}
+template <int N>
+RH_FORM void rh_atan2_wave(const double (&y)[N], const double (&x)[N], double top_c, double (&a)[N])
+{
+    bool c32 = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) c32 = c32 && (fabs(y[i]) < 0.03125 * x[i]);
+    if (rh_all(c32)) rh_atan32(y, x, top_c, a);
+    else rh_atan2_rest(y, x, a);
 }
 RH_HD double rh_atan2_wave(double y, double x)
 {
@@ -656,6 +663,18 @@ RH_HD void tri_factor(const V3<R>& r1, R R1, const V3<R>& r2, R R2, const V3<R>&
 {
     im = dot(r1, cross(r2, r3));
     re = R1 * R2 * R3 + dot(r1, r2) * R3 + dot(r1, r3) * R2 + dot(r2, r3) * R1;
+}
+
+// Twice its real part from the distances, for records whose imaginary part is
+// 4 area n . r (the triple product's double).  Each term carries the distance
+// of every vertex as a factor, so that it keeps its digits next to a vertex,
+// where S01 S12 S20 - R2 l01^2 - R1 l02^2 - R0 l12^2 (S: sums of distances),
+// the same value, is a difference of terms of the edges' size: with a 10 mm
+// triangle 7e-12 of the angle at 1e-3 edges from a vertex against 6e-14 here.
+template <class R>
+RH_HD R tri_re2(const V3<R>& r1, R R1, const V3<R>& r2, R R2, const V3<R>& r3, R R3)
+{
+    return R(2) * ((R1 * R2 + dot(r1, r2)) * R3 + (dot(r1, r3) * R2 + dot(r2, r3) * R1));
 }
 
 // q6 layout: xx, yy, zz, xy, xz, yz.

@@ -53,7 +53,8 @@ def _meshes():
     yield "hexes", W.halbach(n_seg=4, n_az=2, n_rad=2, n_ax=2, n_points=1)[0]
 
 
-@pytest.mark.parametrize("lo", [0.5])
+# from 1e-3 mm of the vertices, elements being some mm
+@pytest.mark.parametrize("lo", [0.5, -3])
 @pytest.mark.parametrize("which", ["tets", "hexes"])
 def test_sweep_forms_equal_per_element(L, which, lo):  # noqa: F811
     top = next(t for w, t in _meshes() if w == which)
@@ -119,4 +120,26 @@ def test_vertex_derivatives_equal_forward_mode(L):  # noqa: F811
     # sums of some 200 x 12 terms, each to about 1e-14 of the largest
     for a, b in zip(out["rhc_adj_grad"], out["rhc_adj_grad_tri"]):
         assert np.abs(a - b).max() <= 1e-11 * np.abs(a).max()
+    rad.UtiDelAll()
+
+
+def test_tetrahedron_block_next_to_a_vertex(L):  # noqa: F811
+    """At 1e-3 edges a plane distance carries 1.1e-16 / 1e-3 of itself, times
+    the few operations of its dot product: 1e-12 of the angles, in either form.
+    (A denominator formed as a difference of terms of the edges' size, not of
+    the vertex distance's, was off by 1e-11.)"""
+    rng = np.random.default_rng(49)
+    rad.UtiDelAll()
+    ids = []
+    for k in range(20):
+        t = 10 * rng.normal(size=(4, 3)) + rng.uniform(-20, 20, 3)
+        ids.append(rad.ObjPolyhdr(t.tolist(), [[1, 2, 3], [1, 2, 4], [1, 3, 4], [2, 3, 4]], [0, 0, 1]))
+    P, items = models.packed(rad.ObjCnt(ids))
+    n = len(items)
+    d = rng.normal(size=(2000, 3))
+    pts = P["verts"][rng.integers(len(P["verts"]), size=2000)] + 1e-2 * d / np.linalg.norm(d, axis=1)[:, None]
+    q, _ins = _blocks(L, P, n, pts)
+    M = np.tile([0.0, 0.0, 1.0], (n, 1))
+    H = _field(L, "rhc_field", P, M, pts)[1]
+    assert np.abs(q[..., 2].sum(axis=1) - H).max() <= 1e-12
     rad.UtiDelAll()
