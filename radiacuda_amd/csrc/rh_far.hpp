@@ -481,8 +481,14 @@ RH_FORM bool rec_block(const double* __restrict__ rec, const double p[3], double
 #endif
 
 // The block at points near a hexahedron: one edge and one face at a time from
-// the record, each with the tier its wave needs, as near_tet_block.
-RH_FORM bool near_hex_block(const double* __restrict__ h, const double p[3], double q5[5])
+// the record, each with the tier its wave needs, as near_tet_block.  All six
+// solid angles are formed, from the corners' triple products (which keep their
+// digits next to a corner, where a plane distance times the area does not), and
+// half[0] is their sum, halved: 2 pi inside, 0 outside.  At a point on a face
+// that face's angle is one of its two limits, by the sign of a rounded or a
+// zero triple product, and the others stand; five angles closed by the plane
+// tests' answer were off by 4 pi there.
+RH_FORM bool near_hex_block(const double* __restrict__ h, const double p[3], double q5[5], double half[1])
 {
     auto vtx = [&](int k, V3<double>& r, double& d) {
         r = rel<double>(h + 3 * k, p);
@@ -502,38 +508,38 @@ RH_FORM bool near_hex_block(const double* __restrict__ h, const double p[3], dou
         for (int k = 0; k < 5; k++) acc[k] += L[0] * h[kHexW + 5 * e + k];
     }
     bool inside = true;
+    const double* n5 = h + kHexN5;
+    half[0] = 0.0;
 #pragma unroll 1
-    for (int f = 0; f < 5; f++) {
-        // corners as in kHexFace
+    for (int f = 0; f < 6; f++) {
+        // corners as in kHexFace: outward for face 0, inward for the others
         const int i = f - 1, j = f & 3;
-        const int b = (f == 0) ? 1 : j, c = (f == 0) ? 2 : 4 + j, e = (f == 0) ? 3 : 4 + i, a = (f == 0) ? 0 : i;
+        const int a = (f == 0) ? 0 : (f == 5 ? 4 : i), b = (f == 0) ? 1 : (f == 5 ? 5 : j);
+        const int c = (f == 0) ? 2 : (f == 5 ? 6 : 4 + j), e = (f == 0) ? 3 : (f == 5 ? 7 : 4 + i);
         V3<double> ra, rb, rc, re;
-        double da, db, dc, de, om[1];
+        double da, db, dc, de, om[1], i1, r1, i2, r2;
         vtx(a, ra, da);
         vtx(b, rb, db);
         vtx(c, rc, dc);
         vtx(e, re, de);
-        const double* g = h + kHexF + 5 * f;
-        const double z = dot(ra, v3(g[0], g[1], g[2]));
-        const double r1 = tri_re2(ra, da, rb, db, rc, dc), r2 = tri_re2(ra, da, rc, dc, re, de);
-        const double i1 = z * g[3], i2 = z * g[4];
-        inside = inside && (z > 0.0);
-        const double im[1] = {r1 * i2 + r2 * i1}, rr[1] = {r1 * r2 - i1 * i2};
+        const double* n = (f == 5) ? n5 : h + kHexF + 5 * f;
+        inside = inside && (dot(ra, v3(n[0], n[1], n[2])) > 0.0);
+        tri_factor(ra, da, rb, db, rc, dc, r1, i1);
+        tri_factor(ra, da, rc, dc, re, de, r2, i2);
+        const double s = (f == 0) ? 1.0 : -1.0;
+        const double im[1] = {s * (r1 * i2 + r2 * i1)}, rr[1] = {r1 * r2 - i1 * i2};
         rh_atan2_wave(im, rr, kAtan32Top, om);
+        half[0] += om[0];
+        if (f == 5) break;
         for (int k = 0; k < 5; k++) acc[k] += om[0] * h[kHexT + 5 * f + k];
     }
-    const double* n = h + kHexN5;
-    {
-        const V3<double> r4 = rel<double>(h + 12, p);  // face 5 holds vertex 4
-        inside = inside && (dot(r4, v3(n[0], n[1], n[2])) > 0.0);
-    }
-    // the solid angles sum to 4 pi inside: the sixth face's share of it
-    const double in4 = inside ? 4.0 * kPi : 0.0;
-    acc[0] -= in4 * n[0] * n[0];
-    acc[1] -= in4 * n[0] * n[1];
-    acc[2] -= in4 * n[0] * n[2];
-    acc[3] -= in4 * n[1] * n[1];
-    acc[4] -= in4 * n[1] * n[2];
+    // the records' weights are the faces' less the sixth's
+    const double w = 2.0 * half[0];
+    acc[0] -= w * n5[0] * n5[0];
+    acc[1] -= w * n5[0] * n5[1];
+    acc[2] -= w * n5[0] * n5[2];
+    acc[3] -= w * n5[1] * n5[1];
+    acc[4] -= w * n5[1] * n5[2];
     far_scale(acc, q5);
     return inside;
 }
@@ -588,16 +594,18 @@ RH_FORM bool gen_block(const double* __restrict__ h, const double* __restrict__ 
         }
         far_scale(acc, q5);
     }
+    double half = 0.0;  // the solid angles' sum, halved
     bool in = false;
     if (rh_any(!far)) {
-        double qn[5];
-        in = near_hex_block(h, p, qn) && !far;
+        double qn[5], hn[1];
+        in = near_hex_block(h, p, qn, hn) && !far;
+        half = far ? 0.0 : hn[0];
 #pragma unroll
         for (int k = 0; k < 5; k++) q5[k] = far ? q5[k] : qn[k];
     }
     q6[0] = q5[0];
     q6[1] = q5[3];
-    q6[2] = -(q5[0] + q5[3]) - (in ? 1.0 : 0.0);
+    q6[2] = -(q5[0] + q5[3]) - 2.0 * kInv4Pi * half;
     q6[3] = q5[1];
     q6[4] = q5[2];
     q6[5] = q5[4];
