@@ -13,6 +13,7 @@
 #include <cstring>
 #include <utility>
 
+#include "rh_idmap.hpp"
 #include "rh_math.hpp"
 #include "rh_mesh.hpp"
 
@@ -152,65 +153,6 @@ void pack_tet(std::vector<Vec> V, std::vector<double>& d)
         d.push_back(nrm(c));  // twice the face area
     }
 }
-
-// Ids of vertices, edges and faces in order of first occurrence:
-// open addressing over a table of ids at most half full, keys stored in id
-// order (no allocation per key).  The key's words are mixed by a multiplication
-// each.  Models are packed on every geometry change, so this is on the path of
-// a gradient step: with ordered maps and a vector per face the 1,000 polyhedra
-// of an undulator took 13 ms of one core here and take 3.4 ms (a step over them
-// 12.8 -> 7.8 ms).
-using VKey = std::array<uint64_t, 3>;   // bits of the coordinates
-using EKey = std::array<int32_t, 2>;    // ascending vertex ids
-using FKey = std::array<int32_t, 4>;    // ascending vertex ids, a triangle's first one -1
-inline uint64_t mix(uint64_t h, uint64_t w)
-{
-    h = (h ^ w) * 0x9E3779B97F4A7C15ull;
-    return h ^ (h >> 29);
-}
-inline uint64_t word2(int32_t a, int32_t b) { return (uint64_t(uint32_t(a)) << 32) | uint32_t(b); }
-inline uint64_t hash_key(const VKey& k) { return mix(mix(mix(1, k[0]), k[1]), k[2]); }
-inline uint64_t hash_key(const EKey& k) { return mix(1, word2(k[0], k[1])); }
-inline uint64_t hash_key(const FKey& k) { return mix(mix(1, word2(k[0], k[1])), word2(k[2], k[3])); }
-
-template <class Key>
-class IdMap {
-public:
-    explicit IdMap(size_t expect)
-    {
-        keys_.reserve(expect);
-        size_t n = 16;
-        while (n < 2 * expect) n *= 2;
-        slot_.assign(n, -1);
-    }
-    // id of the key, a new one if it is not there
-    int32_t add(const Key& k)
-    {
-        size_t i = place(k);
-        if (slot_[i] >= 0) return slot_[i];
-        if (2 * (keys_.size() + 1) > slot_.size()) {
-            slot_.assign(2 * slot_.size(), -1);
-            for (size_t q = 0; q < keys_.size(); q++) slot_[place(keys_[q])] = int32_t(q);
-            i = place(k);
-        }
-        keys_.push_back(k);
-        return slot_[i] = int32_t(keys_.size() - 1);
-    }
-    int32_t find(const Key& k) const { return slot_[place(k)]; }
-    size_t size() const { return keys_.size(); }
-    const Key& operator[](size_t id) const { return keys_[id]; }
-
-private:
-    size_t place(const Key& k) const
-    {
-        const size_t m = slot_.size() - 1;
-        size_t i = size_t(hash_key(k)) & m;
-        while (slot_[i] >= 0 && keys_[size_t(slot_[i])] != k) i = (i + 1) & m;
-        return i;
-    }
-    std::vector<Key> keys_;
-    std::vector<int32_t> slot_;
-};
 
 EKey ekey(int32_t a, int32_t b) { return {std::min(a, b), std::max(a, b)}; }
 void pack_gen(const std::vector<Vec>& V, const std::vector<Face>& F, std::vector<double>& d)
@@ -448,13 +390,6 @@ rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err)
 }
 
 namespace {
-
-VKey vkey(const double* v)
-{
-    VKey k;
-    std::memcpy(k.data(), v, 3 * sizeof(double));
-    return k;
-}
 
 // a face piece: its loop of 3 or 4 unique vertices
 struct Piece {

@@ -8,6 +8,7 @@
 #include "rh_current.hpp"
 #include "rh_eval.hpp"
 #include "rh_geom.hpp"
+#include "rh_idmap.hpp"
 #include "rh_mesh.hpp"
 #include "rh_opcount.hpp"
 
@@ -653,6 +654,16 @@ int rhc_adj_grad_tri(const rh_model_desc* d, const double* M, const double* pts,
         }
     }
     return RH_OK;
+}
+
+// Mean number of slots that the packer's vertex table looks at per vertex, n
+// vertices xyz (repeated ones count once); returns the number of unique ones.
+int64_t rhc_vertex_probes(const double* xyz, int64_t n, double* probes)
+{
+    rh::IdMap<rh::VKey> ids{size_t(n)};
+    for (int64_t k = 0; k < n; k++) ids.add(rh::vkey(xyz + 3 * k));
+    *probes = ids.probes();
+    return int64_t(ids.size());
 }
 
 }  // extern "C"
