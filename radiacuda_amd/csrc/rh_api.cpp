@@ -379,6 +379,31 @@ rh_status rh_kernel_time(const char* family, double* avg_ms, int64_t* count)
     return RH_OK;
 }
 
+namespace {
+// The far-form records of the model's hexahedra, 1.3 KB each, which the field
+// sweeps element by element and the gradient by the magnetization read: built
+// with the model where those sweeps carry its fields, at the first call that
+// reads them where the mesh form does.  Without them (no hexahedron, or no
+// memory left) the sweeps take the general form.
+hipError_t hex_records(rh_model* m)
+{
+    if (m->d_hex) return hipSuccess;
+    int64_t count = 0;
+    const std::vector<int32_t> at = rh::hex_places(m->host, &count);
+    if (count == 0) return hipSuccess;
+    if (dalloc(&m->d_hex, size_t(rh::hex_doubles(count))) != hipSuccess) {
+        (void)hipGetLastError();
+        m->d_hex = nullptr;
+        return hipSuccess;
+    }
+    m->dev.hex = m->d_hex;
+    hipError_t e = hipMemcpyAsync(m->d_hex_at, at.data(), at.size() * sizeof(int32_t), hipMemcpyHostToDevice, m->stream);
+    if (e == hipSuccess) e = rh::launch_hexes(m->dev, m->d_hex, m->d_hex_at, m->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+    return e;
+}
+}  // namespace
+
 rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, rh_model** out)
 {
     if (!desc || !out) return fail(RH_ERR_ARG, "null argument");
@@ -410,9 +435,8 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
     if (e == hipSuccess)
         e = dalloc(&m->d_charged, size_t(rh::kChargedTet * (P.kind_off[2] - P.kind_off[1])));
     if (e == hipSuccess) e = dalloc(&m->d_far, size_t(rh::far_tet_doubles(P.kind_off[2] - P.kind_off[1])));
-    const int64_t ngen = P.kind_off[3] - P.kind_off[2];
-    if (e == hipSuccess) e = dalloc(&m->d_hex, size_t(rh::hex_doubles(ngen)));
     if (e == hipSuccess) e = dalloc(&m->d_hex_at, size_t(P.n));
+    if (e == hipSuccess && P.n > 0) e = hipMemsetAsync(m->d_hex_at, 0xff, size_t(P.n) * sizeof(int32_t), s);
     rh::DevModel& d = m->dev;
     d.n = P.n;
     d.kind = m->d_kind;
@@ -424,12 +448,12 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
     d.rowt = m->d_rowt;
     d.kidx = m->d_kidx;
     d.far_tet = m->d_far;
-    d.hex = m->d_hex;
     d.hex_at = m->d_hex_at;
     for (int k = 0; k < 4; k++) d.koff[k] = P.kind_off[k];
     d.sym = P.sym;
     d.rowt_identity = P.rowt_identity;
-    if (e == hipSuccess) e = rh::launch_far_records(d, m->d_far, m->d_hex, m->d_hex_at, s);
+    if (e == hipSuccess) e = rh::launch_far_tets(d, m->d_far, s);
+    if (e == hipSuccess && !P.mesh.active) e = hex_records(m);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         std::string msg = std::string("model upload: ") + hipGetErrorString(e);
@@ -500,6 +524,10 @@ rh_status rh_model_set_field_form(rh_model* m, int32_t form)
     if (!m) return fail(RH_ERR_ARG, "null argument");
     if (form != 0 && form != 1) return fail(RH_ERR_ARG, "form must be 0 (automatic) or 1 (per element)");
     m->dev.use_mesh = (form == 0) && m->dev.mesh.active;
+    if (form == 1) {
+        RH_HIP(enter_device(m->device));
+        RH_HIP(hex_records(m));
+    }
     return RH_OK;
 }
 
@@ -1759,6 +1787,7 @@ rh_status rh_field_adjoint_dev(rh_model* m, const double* d_M, const double* d_p
     }
     Timer t("adjoint", s);
     if (d_gM) {
+        RH_HIP(hex_records(m));
         const int64_t groups = rh::adj_point_groups(np, rh::adj_m_slices(n, np));
         RH_HIP(grow(m, size_t(groups * 3 * n)));
         t.begin();

@@ -461,6 +461,19 @@ ElemView view_elem(const PackedModel& P, int64_t j, std::vector<int32_t>& a)
 }
 }  // namespace
 
+std::vector<int32_t> hex_places(const PackedModel& P, int64_t* count)
+{
+    std::vector<int32_t> at(size_t(P.n), -1);
+    int32_t q = 0;
+    for (int64_t k = P.kind_off[2]; k < P.kind_off[3]; k++) {
+        const size_t j = size_t(P.kind_idx[size_t(k)]);
+        const double* r = P.data.data() + P.off[j];
+        if (r[0] == 8.0 && r[1] == 12.0 && r[2] == 6.0 && r[3] == 24.0) at[j] = q++;
+    }
+    *count = q;
+    return at;
+}
+
 void build_mesh_form(PackedModel& P)
 {
     MeshForm& M = P.mesh;

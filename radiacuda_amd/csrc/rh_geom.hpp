@@ -76,6 +76,10 @@ struct PackedModel {
 // qualify).
 void build_mesh_form(PackedModel& P);
 
+// Every element's place among the hexahedra, which the per-element sweeps keep
+// far-form records of (rh_far.hpp), -1 for the other elements.
+std::vector<int32_t> hex_places(const PackedModel& P, int64_t* count);
+
 // Returns RH_OK or an error status with a message in *err.
 rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err);
 

@@ -666,4 +666,14 @@ int64_t rhc_vertex_probes(const double* xyz, int64_t n, double* probes)
     return int64_t(ids.size());
 }
 
+// Number of elements that a hexahedron record is kept for, -1 on error.
+int64_t rhc_hex_count(const rh_model_desc* d)
+{
+    rh::PackedModel P;
+    if (rh::pack_model(d, &P, &g_err) != RH_OK) return -1;
+    int64_t n = 0;
+    rh::hex_places(P, &n);
+    return n;
+}
+
 }  // extern "C"

@@ -52,48 +52,33 @@ __global__ __launch_bounds__(256) void k_far_records(DevModel m, double* __restr
     far_tet_record(m.data + m.off[m.kidx[k]], out + kFarTet * (k - m.koff[1]));
 }
 
-// Far-form records of the hexahedra among the general polyhedra, one wave each;
-// elements of the other kinds have none.
+// Far-form records of the hexahedra among the general polyhedra, one wave each,
+// at the places that `at` gives; an element that does not fit the topology has
+// none.
 __global__ __launch_bounds__(64) void k_hex_records(DevModel m, double* __restrict__ out, int32_t* __restrict__ at)
 {
     __shared__ double rec[kHexIn], o[kHex];
     __shared__ int id[8];
     __shared__ int ok;
-    const int64_t q = blockIdx.x, j = m.kidx[m.koff[2] + q];
+    const int64_t j = m.kidx[m.koff[2] + blockIdx.x];
+    const int64_t q = at[j];
+    if (q < 0) return;
     const double* src = m.data + m.off[j];
-    const bool hex = int(src[0]) == 8 && int(src[1]) == 12 && int(src[2]) == 6 && int(src[3]) == 24;
-    if (!hex) {
-        if (threadIdx.x == 0) at[j] = -1;
-        return;
-    }
     for (int i = threadIdx.x; i < kHexIn; i += 64) rec[i] = src[i];
     __syncthreads();
     if (threadIdx.x == 0) ok = hex_vertices(rec, id) ? 1 : 0;
     __syncthreads();
-    if (!ok) {
-        if (threadIdx.x == 0) at[j] = -1;
-        return;
-    }
-    bool fits = true;
-    if (threadIdx.x < 12) fits = hex_edge_record(rec, id, threadIdx.x, o);
-    else if (threadIdx.x < 17) fits = hex_face_record(rec, id, threadIdx.x - 12, o);
+    bool fits = ok;
+    if (fits && threadIdx.x < 12) fits = hex_edge_record(rec, id, threadIdx.x, o);
+    else if (fits && threadIdx.x < 17) fits = hex_face_record(rec, id, threadIdx.x - 12, o);
     if (__any(!fits)) {
         if (threadIdx.x == 0) at[j] = -1;
         return;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        hex_close_record(rec, id, o);
-        at[j] = int32_t(q);
-    }
+    if (threadIdx.x == 0) hex_close_record(rec, id, o);
     __syncthreads();
     for (int i = threadIdx.x; i < kHex; i += 64) out[kHex * q + i] = o[i];
-}
-
-__global__ __launch_bounds__(256) void k_no_hex(int64_t n, const int32_t* __restrict__ kidx, int32_t* __restrict__ at)
-{
-    const int64_t k = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (k < n) at[kidx[k]] = -1;
 }
 
 template <class T>
@@ -1901,16 +1886,18 @@ __global__ __launch_bounds__(256) void k_current(int64_t ns, const int32_t* __re
 
 // ---------------------------------------------------------------- launchers
 int64_t far_tet_doubles(int64_t ntet) { return kFarTet * ntet; }
-int64_t hex_doubles(int64_t ngen) { return kHex * ngen; }
+int64_t hex_doubles(int64_t nhex) { return kHex * nhex; }
 
-hipError_t launch_far_records(const DevModel& m, double* tet, double* hex, int32_t* hex_at, hipStream_t s)
+hipError_t launch_far_tets(const DevModel& m, double* tet, hipStream_t s)
 {
     const int64_t ntet = m.koff[2] - m.koff[1];
     if (ntet > 0) hipLaunchKernelGGL(k_far_records, dim3(unsigned((ntet + 255) / 256)), dim3(256), 0, s, m, tet);
+    return hipGetLastError();
+}
+
+hipError_t launch_hexes(const DevModel& m, double* hex, int32_t* hex_at, hipStream_t s)
+{
     const int64_t ngen = m.koff[3] - m.koff[2];
-    if (m.koff[2] > 0)
-        hipLaunchKernelGGL(k_no_hex, dim3(unsigned((m.koff[2] + 255) / 256)), dim3(256), 0, s, m.koff[2], m.kidx,
-                           hex_at);
     if (ngen > 0) hipLaunchKernelGGL(k_hex_records, dim3(unsigned(ngen)), dim3(64), 0, s, m, hex, hex_at);
     return hipGetLastError();
 }

@@ -57,12 +57,14 @@ struct DevModel {
     bool use_mesh = false;  // field sweeps use the mesh form (when active)
 };
 
-// Doubles of the far-form records of ntet tetrahedra and of ngen general
-// polyhedra (the hexahedra among them), and the kernels that build them from
-// the element records (once per model).
+// Doubles of the far-form records of ntet tetrahedra and of nhex hexahedra, and
+// the kernels that build them from the element records: hex_at holds an
+// element's place among the hexahedra, and -1 after launch_hexes where its
+// topology is another one.
 int64_t far_tet_doubles(int64_t ntet);
-int64_t hex_doubles(int64_t ngen);
-hipError_t launch_far_records(const DevModel& m, double* tet, double* hex, int32_t* hex_at, hipStream_t s);
+int64_t hex_doubles(int64_t nhex);
+hipError_t launch_far_tets(const DevModel& m, double* tet, hipStream_t s);
+hipError_t launch_hexes(const DevModel& m, double* hex, int32_t* hex_at, hipStream_t s);
 
 // Interaction-matrix rows of elements [r0, r1) into Q (row-major, leading
 // dimension ld elements of elem_bytes = 4 or 8; Q points at row 3*r0); the
