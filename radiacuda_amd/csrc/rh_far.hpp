@@ -11,12 +11,17 @@
 // keeps a relative error of a few ulp, where a logarithm of a ratio near 1
 // carries an absolute one, so far blocks are also the more accurate ones.
 //
-// Far means S >= 4 len for every edge and every lane.  Then every vertex is at
-// least 1.5 longest edges away, every face is seen under less than 0.23 sr
-// (half the angle has a tangent below 0.12), and X = 2 len / S <= 1/2, inside
-// the polynomials' ranges; the point is outside the element, so that the
-// fourth solid angle is minus the sum of the other three and the tensor is
-// traceless.  Against 64-bit sums the C-yoke's blocks carry 2.3e-15 of their
+// Far means S >= 4 len for every edge and every lane.  The cosine between the
+// directions of two vertices is then (R0^2 + R1^2 - len^2)/(2 R0 R1) >=
+// 15/16 - 1/16 = 7/8.  All vertices lie within one half-space of directions, so
+// that the point is outside the element, the fourth solid angle is minus the
+// sum of the other three and the tensor is traceless.  A face's half angle has
+// the tangent |u0 . (u1 x u2)| / (1 + u0.u1 + u1.u2 + u2.u0) of its vertices'
+// directions u, at most sqrt(1 - 3 c^2 + 2 c^3) / (1 + 3 c) = 0.058 at c = 7/8
+// (a face is seen under less than 0.115 sr), and X = 2 len / S <= 1/2: both
+// inside the polynomials' ranges.  The two ends of the longest edge are at
+// least 1.5 of it away, and any other vertex at least 1.2 (R2 >= 0.6 R0 by its
+// own edge).  Against 64-bit sums the C-yoke's blocks carry 2.3e-15 of their
 // norm (5.5e-15 by the general form), FP32 far blocks 5.4e-7 (8.0e-7).
 #pragma once
 

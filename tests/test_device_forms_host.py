@@ -143,3 +143,30 @@ def test_tetrahedron_block_next_to_a_vertex(L):  # noqa: F811
     H = _field(L, "rhc_field", P, M, pts)[1]
     assert np.abs(q[..., 2].sum(axis=1) - H).max() <= 1e-12
     rad.UtiDelAll()
+
+
+@pytest.mark.parametrize("shape", ["flat", "needle", "sliver", "limit"])
+def test_far_limit_of_thin_tetrahedra(L, shape):  # noqa: F811
+    """Around the limit of the far form (distance sums of four lengths on every
+    edge) for tetrahedra that are anything but regular."""
+    rng = np.random.default_rng(50)
+    if shape == "limit":
+        # all sums at least 4.01 lengths, one vertex 1.32 longest edges away
+        t = np.array([[0.624, 0.5, 0], [0.624, -0.5, 0], [0, 0, 0], [0.3, 0, 0.02]])
+        pts = np.array([[-1.32, 0, 0]]) + np.concatenate([np.zeros((1, 3)), 0.05 * rng.normal(size=(400, 3))])
+    else:
+        t = rng.normal(size=(4, 3)) * {"flat": [1, 1, 0.01], "needle": [1, 0.01, 0.01], "sliver": [1, 0.1, 0.001]}[shape]
+        u = rng.normal(size=(2000, 3))
+        size = np.linalg.norm(t[:, None] - t[None], axis=2).max()
+        pts = t.mean(0) + rng.uniform(1, 3, (2000, 1)) * size * u / np.linalg.norm(u, axis=1)[:, None]
+    rad.UtiDelAll()
+    P, _items = models.packed(rad.ObjPolyhdr(t.tolist(), [[1, 2, 3], [1, 2, 4], [1, 3, 4], [2, 3, 4]], [0, 0, 1]))
+    q, ins = _blocks(L, P, 1, pts)
+    assert not ins.any()
+    for a in range(3):
+        H = _field(L, "rhc_field", P, np.eye(3)[a][None], pts)[1]
+        # weights of order 1, 6 logarithms below 1 and 3 angles below 0.5, each
+        # to a few 1.1e-16 in either form: 9 x 6 x 1.1e-16 / (4 pi), doubled for
+        # the normals of the thin faces
+        assert np.abs(q[:, 0, :, a] - H).max() <= 1e-15
+    rad.UtiDelAll()
