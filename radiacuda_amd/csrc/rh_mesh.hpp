@@ -158,13 +158,12 @@ RH_FORM void mesh_sum(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b, R (&o)[N
 // product is formed, and the sums are those that the edges' integrals divide
 // by.  Next to a vertex the difference cancels.  FP64: a wave whose points all
 // have |im| < re / 32, the shortest arctangent's range, and a subtracted part t
-// of at most re (from about one edge away; the angle then carries less than a
-// unit of 1.1e-16, absolute) takes it; any other wave forms the dot products
-// (tri_re2), which keep their digits next to the vertices too.  On the C-yoke
-// 2.3 % of the waves' triangles do, and 1M points take 36.5 ms where the
-// difference alone took 35.8 (one vote |im| + t < re / 32, a comparison less,
-// sends 21 % there: 38.9).  FP32: the near test
-// (mesh32_near) keeps the points off the vertices.
+// below re (from about one edge away; the angle then carries less than a unit
+// of 1.1e-16, absolute) takes it, by one vote 32 |im| + t < re that costs what
+// the range alone would; any other wave forms the dot products (tri_re2), which
+// keep their digits next to the vertices too.  On the C-yoke 2.3 % of the
+// waves' triangles do.  FP32: the near test (mesh32_near) keeps the points off
+// the vertices.
 template <class R, int N>
 RH_FORM void mesh_tri_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& b,
                                                     const MeshVtxN<R, N>& c, const R (&sab)[N], const R (&sbc)[N],
@@ -179,7 +178,7 @@ RH_FORM void mesh_tri_half_omega(const MeshVtxN<R, N>& a, const MeshVtxN<R, N>& 
         im[i] = dot(a.r[i], v3(g.n0, g.n1, g.n2));
         const R t = c.d[i] * g.l01 + b.d[i] * g.l02 + a.d[i] * g.l12;
         re[i] = (sab[i] * sbc[i]) * sca[i] - t;
-        if constexpr (sizeof(R) == 8) far = far && fabs(im[i]) < 0.03125 * re[i] && t <= re[i];
+        if constexpr (sizeof(R) == 8) far = far && fma(32.0, fabs(im[i]), t) < re[i];
     }
     if constexpr (sizeof(R) == 8) {
         if (rh_all(far)) {
