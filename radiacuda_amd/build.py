@@ -34,7 +34,7 @@ def build(verbose=True):
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out + ".tmp"] + objs)
     os.replace(out + ".tmp", out)
     chk = os.path.join(HERE, "_rhcheck.so")
-    _run([HIPCC, "--offload-host-only", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-o",
+    _run([HIPCC, "--offload-host-only", "-no-hip-rt", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off", "-o",
           chk + ".tmp", "rh_hostcheck.cpp", "rh_geom.cpp"])
     os.replace(chk + ".tmp", chk)
     return out

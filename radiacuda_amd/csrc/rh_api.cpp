@@ -387,19 +387,17 @@ namespace {
 // memory left) the sweeps take the general form.
 hipError_t hex_records(rh_model* m)
 {
-    if (m->d_hex) return hipSuccess;
-    int64_t count = 0;
-    const std::vector<int32_t> at = rh::hex_places(m->host, &count);
-    if (count == 0) return hipSuccess;
-    if (dalloc(&m->d_hex, size_t(rh::hex_doubles(count))) != hipSuccess) {
+    const rh::PackedModel& P = m->host;
+    if (m->d_hex || P.nhex == 0) return hipSuccess;
+    if (dalloc(&m->d_hex, size_t(rh::hex_doubles(P.nhex))) != hipSuccess) {
         (void)hipGetLastError();
         m->d_hex = nullptr;
         return hipSuccess;
     }
     m->dev.hex = m->d_hex;
-    hipError_t e = hipMemcpyAsync(m->d_hex_at, at.data(), at.size() * sizeof(int32_t), hipMemcpyHostToDevice, m->stream);
+    hipError_t e = hipMemcpyAsync(m->d_hex_at, P.hex_at.data(), size_t(P.n) * sizeof(int32_t), hipMemcpyHostToDevice,
+                                  m->stream);
     if (e == hipSuccess) e = rh::launch_hexes(m->dev, m->d_hex, m->d_hex_at, m->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
     return e;
 }
 }  // namespace
@@ -436,6 +434,7 @@ rh_status rh_model_create(const rh_model_desc* desc, int device, void* stream, r
         e = dalloc(&m->d_charged, size_t(rh::kChargedTet * (P.kind_off[2] - P.kind_off[1])));
     if (e == hipSuccess) e = dalloc(&m->d_far, size_t(rh::far_tet_doubles(P.kind_off[2] - P.kind_off[1])));
     if (e == hipSuccess) e = dalloc(&m->d_hex_at, size_t(P.n));
+    // no records yet
     if (e == hipSuccess && P.n > 0) e = hipMemsetAsync(m->d_hex_at, 0xff, size_t(P.n) * sizeof(int32_t), s);
     rh::DevModel& d = m->dev;
     d.n = P.n;

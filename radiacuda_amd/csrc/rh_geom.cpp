@@ -385,6 +385,13 @@ rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err)
             if (P.rowt[9 * e + k] != ((k % 4 == 0) ? 1.0 : 0.0)) P.rowt_identity = false;
         }
     }
+    P.hex_at.assign(size_t(n), -1);
+    P.nhex = 0;
+    for (int64_t k = P.kind_off[2]; k < P.kind_off[3]; k++) {
+        const size_t j = size_t(P.kind_idx[size_t(k)]);
+        const double* r = P.data.data() + P.off[j];
+        if (r[0] == 8.0 && r[1] == 12.0 && r[2] == 6.0 && r[3] == 24.0) P.hex_at[j] = int32_t(P.nhex++);
+    }
     build_mesh_form(P);
     return RH_OK;
 }
@@ -460,19 +467,6 @@ ElemView view_elem(const PackedModel& P, int64_t j, std::vector<int32_t>& a)
     return {nv, ne, nf, verts, E + 6, kGenEdge, F, kGenFace, at};
 }
 }  // namespace
-
-std::vector<int32_t> hex_places(const PackedModel& P, int64_t* count)
-{
-    std::vector<int32_t> at(size_t(P.n), -1);
-    int32_t q = 0;
-    for (int64_t k = P.kind_off[2]; k < P.kind_off[3]; k++) {
-        const size_t j = size_t(P.kind_idx[size_t(k)]);
-        const double* r = P.data.data() + P.off[j];
-        if (r[0] == 8.0 && r[1] == 12.0 && r[2] == 6.0 && r[3] == 24.0) at[j] = q++;
-    }
-    *count = q;
-    return at;
-}
 
 void build_mesh_form(PackedModel& P)
 {

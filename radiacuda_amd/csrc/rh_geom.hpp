@@ -69,16 +69,16 @@ struct PackedModel {
     std::vector<int64_t> adj_off;   // [n+1]
     std::vector<double> adj;
     std::vector<int64_t> vert_off;  // [n+1] first vertex of each element in the caller's list
+    // every element's place among the nhex hexahedra, which the per-element
+    // sweeps keep far-form records of (rh_far.hpp), -1 for the others
+    std::vector<int32_t> hex_at;    // [n]
+    int64_t nhex = 0;
     MeshForm mesh;
 };
 
 // Builds P.mesh from the packed records (no-op when the model does not
 // qualify).
 void build_mesh_form(PackedModel& P);
-
-// Every element's place among the hexahedra, which the per-element sweeps keep
-// far-form records of (rh_far.hpp), -1 for the other elements.
-std::vector<int32_t> hex_places(const PackedModel& P, int64_t* count);
 
 // Returns RH_OK or an error status with a message in *err.
 rh_status pack_model(const rh_model_desc* d, PackedModel* out, std::string* err);

@@ -671,9 +671,7 @@ int64_t rhc_hex_count(const rh_model_desc* d)
 {
     rh::PackedModel P;
     if (rh::pack_model(d, &P, &g_err) != RH_OK) return -1;
-    int64_t n = 0;
-    rh::hex_places(P, &n);
-    return n;
+    return P.nhex;
 }
 
 }  // extern "C"
