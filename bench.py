@@ -37,8 +37,10 @@ sys.path.insert(0, ROOT)
 
 METRIC = "Q-blocks/s, rad.Solve s, Fld points/s: mixed vs FP64 GPU at stated error"
 # Algorithmic FLOPs per evaluation of the FP64 integrals, counted from the
-# kernel math instantiated with an op-counting scalar (tests/test_opcount.py
-# recounts them): + - * / sqrt count 1, a fused multiply-add 2, a log 20 and
+# general forms of the kernel math (a logarithm per edge, an arctangent per
+# face) instantiated with an op-counting scalar (tests/test_opcount.py recounts
+# them).  The mesh sweep and the far forms take series instead and execute
+# fewer, so rates by these counts are of work done, not of instructions: + - * / sqrt count 1, a fused multiply-add 2, a log 20 and
 # an atan2 30 (fixed weights).  Per (point, tetrahedron) field 480 and block
 # 669 (6 logs, 3 atan2, 4 sqrt); mesh form per (point, unique edge) 56 (1 log,
 # 2 sqrt), per (point, unique triangle) 93 (1 atan2, 3 sqrt).

@@ -1,4 +1,5 @@
-// rh_hostcheck.cpp -- host build of the packing and of the exact device math,
+// rh_hostcheck.cpp -- host build of the packing, of the general forms of the
+// integrals and of the forms that the kernels evaluate (second half),
 // for CPU unit tests of the formulation (no GPU).  This library is a test
 // aid: the product entry points in libradhip.so never call it.
 #include <string>
@@ -297,7 +298,7 @@ int rhc_opcount(const rh_model_desc* d, const double* M, const double* pts, int6
     return RH_OK;
 }
 
-// Field from the conforming-mesh form (host build of the device sweep):
+// Field from the conforming-mesh form by the general edge and face forms:
 // returns 2 when the model has no mesh form.  counts3 (may be null) gets the
 // numbers of unique edges, unique faces and inside records.
 int rhc_field_mesh(const rh_model_desc* d, const double* M, const double* pts, int64_t np,

@@ -489,7 +489,7 @@ __device__ __forceinline__ void field_store(double* __restrict__ B, double* __re
 constexpr int kRecTile = 64;
 constexpr int kRecStage = 6 + 3;
 // General polyhedra (FP64): hexahedron records and magnetizations likewise.
-// 2,048 points and 1,000 hexahedra 329 us by eval_gen, 128 now.
+// 2,048 points and 1,000 hexahedra 329 us by eval_gen, 134 now.
 constexpr int kHexTile = 16;
 constexpr int kHexStage = kHex + 3;
 
@@ -623,7 +623,7 @@ constexpr int kTetTile = 32;
 // mesh sweep with N points per lane: occupancy floor (waves per SIMD).  Two
 // points share a record's LDS reads, branches and votes and give each other
 // independent instructions; on the C-yoke (FP64, 1M points) two points at 3
-// waves (149 VGPRs, no spill) take 36.9 ms and at 4 waves 37.1 ms, one point
+// waves (155 VGPRs, no spill) take 35.7 ms and at 4 waves 0.2 ms more, one point
 // at 4 to 6 waves 40-47 ms; FP32 on the Halbach ring (250,007 points) two
 // points 37.5 ms at 4 waves and 39.7 at 3, one point 39.4 ms at 5.
 #ifndef RH_MESH_WAVES32
@@ -761,7 +761,7 @@ __global__ __launch_bounds__(256) void k_mesh_charge_in(MeshDev md, const double
 //
 // Bound by FP64 vector issue: 119 instructions per wave of points and
 // tetrahedron on the C-yoke (185 with logarithm-ratio edges, dot products and
-// one point per lane), 80 % of the issue slots.  1M points: 35.0 ms against
+// one point per lane), 80 % of the issue slots.  1M points: 35.7 ms against
 // 49.3; FP32 on the 20,000-element ring, 250,007 points: 35.4 ms against 45.8.
 // Reading the records through the scalar cache instead of LDS freed the vector
 // registers but left each wave waiting on scalar loads: 52 ms.
