@@ -383,8 +383,8 @@ namespace {
 // The far-form records of the model's hexahedra, 1.3 KB each, which the field
 // sweeps element by element and the gradient by the magnetization read: built
 // with the model where those sweeps carry its fields, at the first call that
-// reads them where the mesh form does.  Without them (no hexahedron, or no
-// memory left) the sweeps take the general form.
+// reads them where the mesh form does.  Without them (no hexahedron, no memory
+// left, a first call that must not allocate) the sweeps take the general form.
 hipError_t hex_records(rh_model* m)
 {
     const rh::PackedModel& P = m->host;
@@ -523,10 +523,6 @@ rh_status rh_model_set_field_form(rh_model* m, int32_t form)
     if (!m) return fail(RH_ERR_ARG, "null argument");
     if (form != 0 && form != 1) return fail(RH_ERR_ARG, "form must be 0 (automatic) or 1 (per element)");
     m->dev.use_mesh = (form == 0) && m->dev.mesh.active;
-    if (form == 1) {
-        RH_HIP(enter_device(m->device));
-        RH_HIP(hex_records(m));
-    }
     return RH_OK;
 }
 
@@ -1633,6 +1629,7 @@ rh_status rh_relax_tab(rh_matrix* q, const double* mats, const double* tab, int6
 static rh_status field_dev_impl(rh_model* m, const double* d_M, const double* d_pts, int64_t np,
                                 double* d_B, double* d_H, bool fp32, const char* family)
 {
+    if (!m->dev.use_mesh) RH_HIP(hex_records(m));
     const int64_t slices = rh::field_slices(m->dev, np);
     double* work = nullptr;
     if (slices > 1) {

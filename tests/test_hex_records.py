@@ -73,3 +73,34 @@ def test_sweeps_with_and_without_the_mesh_form(hexes, prisms, apart):
     assert np.array_equal(m.field(M, pts)[1], H)
     m.close()
     rad.UtiDelAll()
+
+
+@pytest.mark.gpu
+def test_form_chosen_during_a_capture():
+    """Choosing the per-element form touches no stream, so that it may happen
+    during a capture; the records come with the next field."""
+    import torch
+    print("case: hexahedron records, capture", flush=True)
+    rad.UtiDelAll()
+    ids = [models.hex_block([2.0 * a, 1.0 * b, 2.0 * c], np.array([2.0, 1.0, 2.0]), [0, 0, 1])
+           for a in range(5) for b in range(4) for c in range(2)]
+    P, items = models.packed(rad.ObjCnt(ids))
+    rng = np.random.default_rng(5)
+    M, pts = rng.uniform(-1, 1, (len(items), 3)), rng.uniform(-20, 20, (100, 3))
+    m = N.Model(P)
+    x = torch.zeros(8, device="cuda")
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x += 1.0
+        m.set_field_form(1)
+    Ho = _field(ctypes.CDLL(LIB), "rhc_field", P, M, pts)[1]
+    for k in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(x.cpu(), torch.full((8,), k + 1.0))
+        # 40 elements x 18 terms of order 1 to 10, each to a few 1.1e-16, over 4 pi
+        assert np.abs(m.field(M, pts)[1] - Ho).max() <= 1e-12
+        m.set_field_form(1)
+    m.close()
+    rad.UtiDelAll()
